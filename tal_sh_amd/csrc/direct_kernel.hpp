@@ -1,0 +1,580 @@
+// Direct contraction kernel (gfx950): D(m, n) (+)= alpha * sum_k A(m, k) * B(k, n)
+// for tensors in any dense layout, m, n and k being groups of tensor indices.
+// Replaces the GEMM call of gpu_tensor_block_contract_dlf
+// (tensor_algebra_gpu_nvidia.cu:6851-7060, cuBLAS/hipBLAS), its in-house
+// fallback gpu_matrix_multiply_tn__ (:2263-2312) and, where an operand or D
+// would only be transposed for its sake, the transposes around it.
+//
+// A workgroup of WM x WN waves computes a BM x BN tile of D (or one of the K
+// ranges of it) from 16x16x4 MFMAs:
+//   R8/C8: v_mfma_f64_16x16x4_f64   R4/C4: v_mfma_f32_16x16x4_f32
+// Complex products are four real MFMAs per step (re += ar*br - ai*bi, im +=
+// ar*bi + ai*br); conjugation is a sign put on while staging.  Operand lanes:
+// A lane l holds row l % 16, B lane l column l % 16; accumulator register r of
+// lane l holds C[4*(l/16)+r][l%16] for f32 and C[4*r+l/16][l%16] for f64.
+//
+// What bounds it: large products, the matrix cores (75 TFLOP/s at 9216^3 FP64
+// with the last round split along K, of 78.6 nominal); products of a few
+// tiles per CU, the latency of their K steps; narrow products, memory.  Hence:
+//  - K steps of KB are loaded PF steps ahead into registers and staged through
+//    two LDS buffers, one barrier per step.  The loads are pinned to the head
+//    of the step: left to itself the scheduler sinks them next to their use
+//    (1024^3 FP64, 64 x 64 tiles: 56 us with one step in flight, 38-42 with
+//    three pinned).  128 x 128 tiles have two workgroups per CU to hide
+//    latency and run best with one step in flight.
+//  - Each operand keeps the order it has in memory: rows of k for one that is
+//    contiguous along k, rows of m (n) otherwise, padded so that fragment
+//    reads are free of bank conflicts.  A lane reads KQ consecutive k of a
+//    k-contiguous tile at once (16 bytes) and uses them in KQ MFMA steps; the
+//    other operand follows the same order of k.  So neither layout is
+//    scattered while staging (4096^3 FP64: 72.4 TFLOP/s with both operands
+//    contiguous along k, 72.9 with both along their rows; the kernel before
+//    this one 65 and 48).
+//  - The K loop holds no branch and no bounds check: loads are buffer loads
+//    whose range check returns 0 for rows past the edge (offset kOutside), and
+//    the last, partial K step is peeled off and loaded element by element.
+//  - Tiles that do not fill a last round over the CUs are cut into K ranges in
+//    the same launch (direct_choose), their sums added in order by
+//    direct_reduce: 841 complex tiles on 256 CUs ran 890 us as four rounds
+//    and run 716 us.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "direct_index.hpp"
+
+namespace tal {
+
+namespace direct {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+template <typename S>
+struct Mfma;
+template <>
+struct Mfma<double> {
+  using acc_t = f64x4;
+  __device__ static int row(int lane, int r) { return 4 * r + (lane >> 4); }
+  __device__ static acc_t op(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Mfma<float> {
+  using acc_t = f32x4;
+  __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  __device__ static acc_t op(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+};
+
+__device__ inline __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)bytes, 0x00020000);
+}
+
+template <int BYTES>
+struct Raw;
+template <>
+struct Raw<4> {
+  using type = unsigned int;
+  __device__ static type load(__amdgpu_buffer_rsrc_t r, uint32_t o) { return __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, 0, 0); }
+};
+template <>
+struct Raw<8> {
+  using type = u32x2;
+  __device__ static type load(__amdgpu_buffer_rsrc_t r, uint32_t o) { return __builtin_amdgcn_raw_buffer_load_b64(r, (int)o, 0, 0); }
+};
+template <>
+struct Raw<16> {
+  using type = u32x4;
+  __device__ static type load(__amdgpu_buffer_rsrc_t r, uint32_t o) { return __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, 0, 0); }
+};
+
+template <typename S, int N>
+struct Vec {
+  S v[N];
+};
+template <typename S, int N>
+__device__ inline Vec<S, N> bload(__amdgpu_buffer_rsrc_t r, uint32_t o) {
+  const typename Raw<(int)sizeof(S) * N>::type u = Raw<(int)sizeof(S) * N>::load(r, o);
+  Vec<S, N> v;
+  __builtin_memcpy(&v, &u, sizeof(v));
+  return v;
+}
+// Tile t of C -> (bx, by): tiles are walked in groups of 8 tile-rows, column
+// by column inside a group (a bijection of [0, gx*gy)).
+__device__ inline void tile_xy(int t, int gx, int gy, int &bx, int &by) {
+  constexpr int G = 8;
+  const int group = t / (G * gy), first = group * G;
+  const int rows = min(G, gx - first), in = t - group * G * gy;
+  bx = first + in % rows;
+  by = in / rows;
+}
+
+// Unit u of n in dispatch order -> a number such that the units of one XCD
+// (workgroups are dealt round-robin over the 8 XCDs) are neighbours: XCD x
+// gets the x-th contiguous share (a bijection of [0, n)).
+__device__ inline int xcd_order(int u, int n) {
+  const int q = n >> 3, r = n & 7, x = u & 7;
+  return x * q + min(x, r) + (u >> 3);
+}
+
+// Values of one 16x16 accumulator block of this lane to D.  Along m (dn = 0):
+// the block is turned round through a wave-private LDS patch so that a store
+// covers 16 consecutive rows of 4 columns; along n the accumulator layout
+// already has 16 consecutive columns of 4 rows.  LDS accesses of one wave
+// complete in order, so the patch needs no barrier.
+// off[r]: byte offset of the lane's r-th element, negative when it is outside D.
+template <typename S, int NC, typename ACC>
+__device__ inline void emit_block(S *patch, int lane, const ACC (&acc)[NC], bool turn, char *__restrict__ D,
+                                  const int64_t (&off)[4], S ar, S ai, bool beta) {
+  constexpr int TP = 17;
+  const int tl = lane & 15, tg = lane >> 4;
+  Vec<S, NC> v[4];
+  if (turn) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) patch[tl * TP + Mfma<S>::row(lane, r)] = acc[c][r];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r].v[c] = patch[(4 * r + tg) * TP + tl];
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r].v[c] = acc[c][r];
+  }
+  Vec<S, NC> d[4];
+  if (beta) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (off[r] >= 0) d[r] = *reinterpret_cast<const Vec<S, NC> *>(D + off[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    Vec<S, NC> x;
+    if (NC == 1) {
+      x.v[0] = ar * v[r].v[0];
+    } else {
+      const S xr = v[r].v[0], xi = v[r].v[NC - 1];
+      x.v[0] = ar * xr - ai * xi;
+      x.v[NC - 1] = ar * xi + ai * xr;
+    }
+    if (beta) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) x.v[c] = d[r].v[c] + x.v[c];
+    }
+    if (off[r] >= 0) *reinterpret_cast<Vec<S, NC> *>(D + off[r]) = x;
+  }
+}
+
+// D offsets of a wave's TM x TN slab, one 16x16 block at a time.
+template <typename S, int SM, int SN>
+struct SlabOffsets {
+  int64_t o[SM * 4 + SN * 4];
+  // rows from m0, columns from n0; -1 past the edge (sums with it stay negative: |offsets| < 2^62)
+  __device__ SlabOffsets(const DirectArgs &p, int m0, int n0, int lane) {
+    constexpr int64_t kNone = -((int64_t)1 << 62);
+    const int fl = lane & 15, fg = lane >> 4;
+    if (!(p.flags & kDirectAlongN)) {
+#pragma unroll
+      for (int i = 0; i < SM; ++i) {
+        const int m = m0 + i * 16 + fl;
+        o[i] = m < p.M ? d_row(p, m) : kNone;
+      }
+#pragma unroll
+      for (int j = 0; j < SN * 4; ++j) {
+        const int n = n0 + (j >> 2) * 16 + 4 * (j & 3) + fg;
+        o[SM * 4 + j] = n < p.N ? d_col(p, n) : kNone;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < SM * 4; ++i) {
+        const int m = m0 + (i >> 2) * 16 + Mfma<S>::row(lane, i & 3);
+        o[i] = m < p.M ? d_row(p, m) : kNone;
+      }
+#pragma unroll
+      for (int j = 0; j < SN; ++j) {
+        const int n = n0 + j * 16 + fl;
+        o[SM * 4 + j] = n < p.N ? d_col(p, n) : kNone;
+      }
+    }
+  }
+  __device__ void block(bool dn, int i, int j, int64_t (&off)[4]) const {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t x = dn ? o[i * 4 + r] + o[SM * 4 + j] : o[i] + o[SM * 4 + j * 4 + r];
+      off[r] = x;
+    }
+  }
+};
+
+// KA / KBC: operand A / B is contiguous along k (else along its rows); WA /
+// WB: elements per load along that direction.  MODE says how a K step is
+// addressed:
+//   0  k is linear in both operands: 32-bit offsets advance by a constant
+//   1  k starts with a run of at least KB (or an operand is 2 GiB or more): a
+//      scalar base per step and, where the step crosses into the next run, one
+//      more scalar for the lanes past the crossing
+//   2  any k: every lane works its offset out
+template <typename S, int NC, int KA, int KBC, int WA, int WB, int BM, int BN, int KB, int WM, int WN, int PF, int OCC,
+          int MODE>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void direct_kernel(DirectArgs p) {
+  using MF = Mfma<S>;
+  using acc_t = typename MF::acc_t;
+  constexpr int NT = 64 * WM * WN;
+  constexpr int TM = BM / WM, TN = BN / WN, SM = TM / 16, SN = TN / 16;
+  constexpr int KQ = sizeof(S) == 8 ? 2 : 4;  // consecutive k per fragment read of a k-contiguous tile
+  constexpr int KPAD = KQ, RPAD = sizeof(S) == 8 ? 8 : 4;
+  // LDS tiles: [plane][row][k] for a k-contiguous operand, [plane][k][row] otherwise
+  constexpr int AL = KA ? BM : KB, AR = KA ? KB + KPAD : BM + RPAD;
+  constexpr int BL = KBC ? BN : KB, BR = KBC ? KB + KPAD : BN + RPAD;
+  __shared__ __attribute__((aligned(16))) S As[2][NC][AL][AR];
+  __shared__ __attribute__((aligned(16))) S Bs[2][NC][BL][BR];
+  constexpr int ALINE = (KA ? KB : BM) / WA, BLINE = (KBC ? KB : BN) / WB;
+  constexpr int NVA = BM * KB / WA / NT, NVB = BN * KB / WB / NT;
+  constexpr int ASTEP = NT / ALINE, BSTEP = NT / BLINE;
+  static_assert(NVA >= 1 && NVB >= 1 && NT % ALINE == 0 && NT % BLINE == 0, "tile split");
+  static_assert(KB % (4 * KQ) == 0, "fragment depth");
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  // units: the whole tiles, then the K ranges of the others
+  int u = blockIdx.x, tile, kpart = 0;
+  const bool part = u >= p.whole;
+  if (!part) {
+    tile = u = xcd_order(u, p.whole);
+  } else {
+    u = xcd_order(u - p.whole, p.rem * p.ksplit);
+    tile = u / p.ksplit;
+    kpart = u - tile * p.ksplit;
+    tile += p.whole;
+  }
+  int bx, by;
+  tile_xy(tile, p.gx, p.gy, bx, by);
+  const int m0 = bx * BM, n0 = by * BN;
+  const int kbeg = kpart * p.ksteps * KB;
+  const int kend = part ? min(p.K, kbeg + p.ksteps * KB) : p.K;
+  // A number with one dimension in an operand is linear there, and its offset
+  // from the tile's origin fits 32 bits (the host checks): the origin goes
+  // into the 64-bit base.
+  const bool ga = p.flags & kDirectGroupA, gb = p.flags & kDirectGroupB;
+  const int am0 = ga ? 0 : m0, bn0 = gb ? 0 : n0;
+  const char *abase = (const char *)p.A + (int64_t)blockIdx.y * p.sa + (int64_t)am0 * p.am1;
+  const char *bbase = (const char *)p.B + (int64_t)blockIdx.y * p.sb + (int64_t)bn0 * p.bn1;
+  if (MODE == 0) {
+    abase += (int64_t)kbeg * p.ka1;
+    bbase += (int64_t)kbeg * p.kb1;
+  }
+
+  // load j of a thread: vector at ac of line al + j * ASTEP (line = row of a
+  // k-contiguous operand, else k); a line of 64 or more threads is uniform per wave
+  const int ac = (tid % ALINE) * WA, bc = (tid % BLINE) * WB;
+  const int al = ALINE % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / ALINE) : tid / ALINE;
+  const int bl = BLINE % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / BLINE) : tid / BLINE;
+  uint32_t aro[KA ? NVA : 1], bro[KBC ? NVB : 1];
+#pragma unroll
+  for (int j = 0; j < (KA ? NVA : 1); ++j) {
+    const int r = m0 + (KA ? al + j * ASTEP : ac);
+    aro[j] = r >= p.M ? kOutside : ga ? group_offset32(p.am, (uint32_t)r) : (uint32_t)(r - am0) * (uint32_t)p.am1;
+  }
+#pragma unroll
+  for (int j = 0; j < (KBC ? NVB : 1); ++j) {
+    const int r = n0 + (KBC ? bl + j * BSTEP : bc);
+    bro[j] = r >= p.N ? kOutside : gb ? group_offset32(p.bn, (uint32_t)r) : (uint32_t)(r - bn0) * (uint32_t)p.bn1;
+  }
+
+  Vec<S, WA * NC> ra[PF][NVA];
+  Vec<S, WB * NC> rb[PF][NVB];
+  uint32_t av[NVA], bv[NVB];
+  if (MODE < 2) {
+#pragma unroll
+    for (int j = 0; j < NVA; ++j) av[j] = aro[KA ? j : 0] + (uint32_t)(KA ? ac : al + j * ASTEP) * (uint32_t)p.ka1;
+#pragma unroll
+    for (int j = 0; j < NVB; ++j) bv[j] = bro[KBC ? j : 0] + (uint32_t)(KBC ? bc : bl + j * BSTEP) * (uint32_t)p.kb1;
+  }
+  // mode 1: the leading run's extent, the offset from past its end to the next
+  // run (also where the second dimension wraps), k's place in its run and run's digit
+  RunWalk rw;
+  int kr = 0, kd1 = 0;
+  if (MODE == 1) {
+    rw = run_walk(p.k);
+    int64_t oa, ob;
+    run_start(p.k, kbeg, &oa, &ob, &kr, &kd1);
+    abase += oa;
+    bbase += ob;
+  }
+  // The next whole K step into a register set.  Past the last whole step the
+  // same step is loaded again and never multiplied.
+  int kload = kbeg;
+  auto load = [&](int set) {
+    const bool more = kload + 2 * KB <= kend;
+    if (MODE == 0) {
+      const auto rsa = rsrc(abase, kOutside), rsb = rsrc(bbase, kOutside);
+#pragma unroll
+      for (int j = 0; j < NVA; ++j) ra[set][j] = bload<S, WA * NC>(rsa, av[j]);
+#pragma unroll
+      for (int j = 0; j < NVB; ++j) rb[set][j] = bload<S, WB * NC>(rsb, bv[j]);
+      const uint32_t sa = more ? KB * (uint32_t)p.ka1 : 0, sb = more ? KB * (uint32_t)p.kb1 : 0;
+#pragma unroll
+      for (int j = 0; j < NVA; ++j) av[j] += sa;
+#pragma unroll
+      for (int j = 0; j < NVB; ++j) bv[j] += sb;
+    } else if (MODE == 1) {
+      const bool wrap = kd1 + 1 == (int)p.k.ext[1];
+      const int da = wrap ? rw.wrap[0] : rw.next[0], db = wrap ? rw.wrap[1] : rw.next[1];
+      const int cross = rw.e0 - kr;  // the step's elements from here on are in the next run: da / db further on
+      const auto rsa = rsrc(abase + min(da, 0), kOutside), rsb = rsrc(bbase + min(db, 0), kOutside);
+      const uint32_t a0 = (uint32_t)max(-da, 0), a1 = (uint32_t)max(da, 0);
+      const uint32_t b0 = (uint32_t)max(-db, 0), b1 = (uint32_t)max(db, 0);
+#pragma unroll
+      for (int j = 0; j < NVA; ++j)
+        ra[set][j] = bload<S, WA * NC>(rsa, av[j] + ((KA ? ac : al + j * ASTEP) >= cross ? a1 : a0));
+#pragma unroll
+      for (int j = 0; j < NVB; ++j)
+        rb[set][j] = bload<S, WB * NC>(rsb, bv[j] + ((KBC ? bc : bl + j * BSTEP) >= cross ? b1 : b0));
+      const bool over = kr + KB >= rw.e0;
+      if (more) {
+        abase += (int64_t)KB * p.ka1 + (over ? da : 0);
+        bbase += (int64_t)KB * p.kb1 + (over ? db : 0);
+        kr += over ? KB - rw.e0 : KB;
+        kd1 = !over ? kd1 : wrap ? 0 : kd1 + 1;
+      }
+    } else {
+      const auto rsa = rsrc(abase, kOutside), rsb = rsrc(bbase, kOutside);
+      uint32_t ka = 0, kb = 0, x;
+      if (KA) pair_offsets32(p.k, (uint32_t)(kload + ac), &ka, &kb);
+      if (KBC && !(KA && WA == WB)) pair_offsets32(p.k, (uint32_t)(kload + bc), &x, &kb);
+#pragma unroll
+      for (int j = 0; j < NVA; ++j) {
+        if (!KA) pair_offsets32(p.k, (uint32_t)(kload + al + j * ASTEP), &ka, &x);
+        ra[set][j] = bload<S, WA * NC>(rsa, aro[KA ? j : 0] + ka);
+      }
+#pragma unroll
+      for (int j = 0; j < NVB; ++j) {
+        if (!KBC) pair_offsets32(p.k, (uint32_t)(kload + bl + j * BSTEP), &x, &kb);
+        rb[set][j] = bload<S, WB * NC>(rsb, bro[KBC ? j : 0] + kb);
+      }
+    }
+    kload += more ? KB : 0;
+  };
+  // the last, partial K step, from k0: element by element, zeros past kend
+  auto load_tail = [&](int k0) {
+    const bool lin = MODE == 0 || (MODE == 1 && p.k.nd == 1);
+    const char *at = (const char *)p.A + (int64_t)blockIdx.y * p.sa + (int64_t)am0 * p.am1;
+    const char *bt = (const char *)p.B + (int64_t)blockIdx.y * p.sb + (int64_t)bn0 * p.bn1;
+    if (lin) {
+      at += (int64_t)k0 * p.ka1;
+      bt += (int64_t)k0 * p.kb1;
+    }
+    const auto rsa = rsrc(at, kOutside), rsb = rsrc(bt, kOutside);
+    auto off = [&](int k, int t) -> uint32_t {
+      if (k >= kend) return kOutside;
+      if (lin) return (uint32_t)(k - k0) * (uint32_t)(t ? p.kb1 : p.ka1);
+      uint32_t o[2];
+      pair_offsets32(p.k, (uint32_t)k, &o[0], &o[1]);
+      return o[t];
+    };
+#pragma unroll
+    for (int j = 0; j < NVA; ++j) {
+      if (KA) {
+#pragma unroll
+        for (int w = 0; w < WA; ++w) {
+          const Vec<S, NC> x = bload<S, NC>(rsa, aro[KA ? j : 0] + off(k0 + ac + w, 0));
+#pragma unroll
+          for (int c = 0; c < NC; ++c) ra[0][j].v[w * NC + c] = x.v[c];
+        }
+      } else {
+        ra[0][j] = bload<S, WA * NC>(rsa, aro[0] + off(k0 + al + j * ASTEP, 0));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NVB; ++j) {
+      if (KBC) {
+#pragma unroll
+        for (int w = 0; w < WB; ++w) {
+          const Vec<S, NC> x = bload<S, NC>(rsb, bro[KBC ? j : 0] + off(k0 + bc + w, 1));
+#pragma unroll
+          for (int c = 0; c < NC; ++c) rb[0][j].v[w * NC + c] = x.v[c];
+        }
+      } else {
+        rb[0][j] = bload<S, WB * NC>(rsb, bro[0] + off(k0 + bl + j * BSTEP, 1));
+      }
+    }
+  };
+  const S sgna = p.flags & kDirectConjA ? (S)-1 : (S)1, sgnb = p.flags & kDirectConjB ? (S)-1 : (S)1;
+  auto stage = [&](int buf, int set) {
+#pragma unroll
+    for (int j = 0; j < NVA; ++j) {
+      const int line = al + j * ASTEP;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        Vec<S, WA> x;
+#pragma unroll
+        for (int w = 0; w < WA; ++w) x.v[w] = c ? sgna * ra[set][j].v[w * NC + c] : ra[set][j].v[w * NC + c];
+        __builtin_memcpy(__builtin_assume_aligned(&As[buf][c][line][ac], sizeof(S) * WA), &x, sizeof(x));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NVB; ++j) {
+      const int line = bl + j * BSTEP;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        Vec<S, WB> x;
+#pragma unroll
+        for (int w = 0; w < WB; ++w) x.v[w] = c ? sgnb * rb[set][j].v[w * NC + c] : rb[set][j].v[w * NC + c];
+        __builtin_memcpy(__builtin_assume_aligned(&Bs[buf][c][line][bc], sizeof(S) * WB), &x, sizeof(x));
+      }
+    }
+  };
+
+  acc_t acc[SM][SN][NC];
+#pragma unroll
+  for (int i = 0; i < SM; ++i)
+#pragma unroll
+    for (int j = 0; j < SN; ++j)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[i][j][c] = acc_t{0, 0, 0, 0};
+
+  const int fl = lane & 15, fg = lane >> 4;
+  auto compute = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < KB / (4 * KQ); ++q) {
+      // lane group g holds k = 4 KQ q + KQ g + h in MFMA step h, in both operands
+      const int kk = q * 4 * KQ + fg * KQ;
+      Vec<S, KQ> fa[NC][SM], fb[NC][SN];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+#pragma unroll
+        for (int i = 0; i < SM; ++i) {
+          const int r = wm * TM + i * 16 + fl;
+          if (KA) __builtin_memcpy(&fa[c][i], __builtin_assume_aligned(&As[buf][c][r][kk], 16), 16);
+          else
+#pragma unroll
+            for (int h = 0; h < KQ; ++h) fa[c][i].v[h] = As[buf][c][kk + h][r];
+        }
+#pragma unroll
+        for (int j = 0; j < SN; ++j) {
+          const int r = wn * TN + j * 16 + fl;
+          if (KBC) __builtin_memcpy(&fb[c][j], __builtin_assume_aligned(&Bs[buf][c][r][kk], 16), 16);
+          else
+#pragma unroll
+            for (int h = 0; h < KQ; ++h) fb[c][j].v[h] = Bs[buf][c][kk + h][r];
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < KQ; ++h)
+#pragma unroll
+        for (int i = 0; i < SM; ++i)
+#pragma unroll
+          for (int j = 0; j < SN; ++j) {
+            if (NC == 1) {
+              acc[i][j][0] = MF::op(fa[0][i].v[h], fb[0][j].v[h], acc[i][j][0]);
+            } else {
+              const S ar = fa[0][i].v[h], ai = fa[NC - 1][i].v[h], br = fb[0][j].v[h], bi = fb[NC - 1][j].v[h];
+              acc[i][j][0] = MF::op(ar, br, acc[i][j][0]);
+              acc[i][j][0] = MF::op(-ai, bi, acc[i][j][0]);
+              acc[i][j][NC - 1] = MF::op(ar, bi, acc[i][j][NC - 1]);
+              acc[i][j][NC - 1] = MF::op(ai, br, acc[i][j][NC - 1]);
+            }
+          }
+    }
+  };
+
+  const int nfull = max(0, kend - kbeg) / KB;
+  if (nfull > 0) {
+#pragma unroll
+    for (int q = 0; q < PF; ++q) load(q);
+    stage(0, 0);
+    __syncthreads();
+  }
+  // K step kt: the loads of step kt + PF go out, step kt + 1 (loaded PF - 1
+  // steps ago) is staged into the other LDS buffer, step kt is multiplied
+  auto step = [&](int q, int buf) {
+    load(q);
+    __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+    if (PF > 1) stage(buf ^ 1, (q + 1) % PF);
+    compute(buf);
+    if (PF == 1) stage(buf ^ 1, 0);
+    __syncthreads();
+  };
+  constexpr int U = PF % 2 == 0 ? PF : 2 * PF;  // steps per loop round: register set and LDS buffer are constants
+  int kt = 0;
+  for (; kt + U <= nfull; kt += U) {
+#pragma unroll
+    for (int q = 0; q < U; ++q) step(q % PF, q & 1);
+  }
+#pragma unroll
+  for (int q = 0; q < U - 1; ++q)
+    if (kt + q < nfull) step(q % PF, q & 1);
+  if (kbeg + nfull * KB < kend) {
+    load_tail(kbeg + nfull * KB);
+    stage(0, 0);
+    __syncthreads();
+    compute(0);
+    __syncthreads();
+  }
+
+  if (part) {  // raw partial sums in accumulator order: element e of lane l at e * 64 + l
+    S *pb = (S *)p.part + ((int64_t)u * WM * WN + wave) * (SM * SN * NC * 4 * 64) + lane;
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+      for (int j = 0; j < SN; ++j)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pb[(((i * SN + j) * NC + c) * 4 + r) * 64] = acc[i][j][c][r];
+    return;
+  }
+  static_assert(sizeof(As) >= sizeof(S) * WM * WN * 16 * 17, "patches fit the A tiles' space");
+  S *patch = &As[0][0][0][0] + wave * 16 * 17;
+  const bool dn = p.flags & kDirectAlongN;
+  char *D = (char *)p.D + (int64_t)blockIdx.y * p.sd;
+  const SlabOffsets<S, SM, SN> so(p, m0 + wm * TM, n0 + wn * TN, lane);
+#pragma unroll
+  for (int i = 0; i < SM; ++i)
+#pragma unroll
+    for (int j = 0; j < SN; ++j) {
+      int64_t off[4];
+      so.block(dn, i, j, off);
+      emit_block<S, NC, acc_t>(patch, lane, acc[i][j], !dn, D, off, (S)p.ar, (S)p.ai, p.flags & kDirectBeta);
+    }
+}
+
+// Sums the ksplit partial blocks of each split tile in order; one wave per 16x16 block.
+template <typename S, int NC, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void direct_reduce(DirectArgs p) {
+  using acc_t = typename Mfma<S>::acc_t;
+  constexpr int TM = BM / WM, TN = BN / WN, SM = TM / 16, SN = TN / 16, PER = SM * SN * NC * 4 * 64;
+  __shared__ S patches[4][16 * 17];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = blockIdx.x * 4 + w;  // block index: (tile, wave, i, j)
+  constexpr int BPT = WM * WN * SM * SN;
+  const int tile = blk / BPT, in = blk % BPT;
+  if (tile >= p.rem) return;
+  const int wave = in / (SM * SN), ij = in % (SM * SN), i = ij / SN, j = ij % SN;
+  acc_t acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = acc_t{0, 0, 0, 0};
+  const S *pb = (const S *)p.part + ((int64_t)tile * p.ksplit * WM * WN + wave) * PER + (int64_t)ij * NC * 256 + lane;
+#pragma unroll 4
+  for (int q = 0; q < p.ksplit; ++q, pb += (int64_t)WM * WN * PER) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[c][r] += pb[(c * 4 + r) * 64];
+  }
+  int bx, by;
+  tile_xy(p.whole + tile, p.gx, p.gy, bx, by);
+  const SlabOffsets<S, 1, 1> so(p, bx * BM + (wave % WM) * TM + i * 16, by * BN + (wave / WM) * TN + j * 16, lane);
+  const bool dn = p.flags & kDirectAlongN;
+  int64_t off[4];
+  so.block(dn, 0, 0, off);
+  emit_block<S, NC, acc_t>(patches[w], lane, acc, !dn, (char *)p.D, off, (S)p.ar, (S)p.ai, p.flags & kDirectBeta);
+}
+
+}  // namespace direct
+}  // namespace tal

@@ -1,0 +1,49 @@
+// Instantiates the direct contraction kernels of one data kind: included by
+// direct_r4.hip, direct_r8.hip, direct_c4.hip and direct_c8.hip.
+#pragma once
+
+#include "direct.hpp"
+#include "direct_kernel.hpp"
+
+namespace tal {
+namespace direct {
+
+// A tile shape's kernel: BM x BN x KB by WM x WN waves, PF K steps of loads
+// in flight, OCC waves per SIMD.
+template <int BM_, int BN_, int KB_, int WM_, int WN_, int PF_, int OCC_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, KB = KB_, WM = WM_, WN = WN_, PF = PF_, OCC = OCC_;
+};
+
+template <typename S, int NC, class T, int KA, int KBC, int W, int MODE>
+void run(const DirectArgs &a, unsigned batch, hipStream_t s) {
+  direct_kernel<S, NC, KA, KBC, W, W, T::BM, T::BN, T::KB, T::WM, T::WN, T::PF, T::OCC, MODE>
+      <<<dim3((unsigned)(a.whole + a.rem * a.ksplit), batch), dim3(64 * T::WM * T::WN), 0, s>>>(a);
+  if (a.rem > 0) {
+    constexpr int kBlocks = (T::BM / 16) * (T::BN / 16);  // 16 x 16 blocks of a tile
+    direct_reduce<S, NC, T::BM, T::BN, T::WM, T::WN>
+        <<<dim3((unsigned)(((int64_t)a.rem * kBlocks + 3) / 4)), dim3(256), 0, s>>>(a);
+  }
+}
+
+template <typename S, int NC, class T, int W, int MODE>
+void run_layout(const DirectVariant &v, const DirectArgs &a, unsigned batch, hipStream_t s) {
+  if (v.ka && v.kb) run<S, NC, T, 1, 1, W, MODE>(a, batch, s);
+  else if (v.ka) run<S, NC, T, 1, 0, W, MODE>(a, batch, s);
+  else if (v.kb) run<S, NC, T, 0, 1, W, MODE>(a, batch, s);
+  else run<S, NC, T, 0, 0, W, MODE>(a, batch, s);
+}
+
+// Mode 2 (any k) is for small problems: element loads only.
+template <typename S, int NC, class T, int W>
+bool run_tile(const DirectVariant &v, const DirectArgs &a, unsigned batch, hipStream_t s) {
+  if (v.mode == 2) run_layout<S, NC, T, 1, 2>(v, a, batch, s);
+  else if (v.mode == 1 && v.width == W) run_layout<S, NC, T, W, 1>(v, a, batch, s);
+  else if (v.mode == 1) run_layout<S, NC, T, 1, 1>(v, a, batch, s);
+  else if (v.width == W) run_layout<S, NC, T, W, 0>(v, a, batch, s);
+  else run_layout<S, NC, T, 1, 0>(v, a, batch, s);
+  return true;
+}
+
+}  // namespace direct
+}  // namespace tal

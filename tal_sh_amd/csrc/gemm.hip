@@ -1,29 +1,16 @@
-// MFMA GEMM kernels for the TTGT contraction stage (gfx950).
+// Split R4 GEMMs (fast math) and the wide-address GEMM (gfx950).
 //
-// Replaces the GEMM call of gpu_tensor_block_contract_dlf
-// (tensor_algebra_gpu_nvidia.cu:6851-7060, cuBLAS/hipBLAS) and its in-house
-// fallback gpu_matrix_multiply_tn__ (:2263-2312).  Contract:
+// Contract of both (the GEMM call of gpu_tensor_block_contract_dlf,
+// tensor_algebra_gpu_nvidia.cu:6851-7060):
 //   C(MxN, column-major, ldc) = alpha * op(A) * op(B) + beta * C,  beta in {0,1}
-// with op(A) in {A, A^T} and op(B) in {B, B^T}, each optionally conjugated,
-// so that the contraction planner can feed tensor operands in whichever
-// matrix form their storage already has.
-//
-// Kernel shape: NW wave64s per workgroup (template parameter): single GEMMs
-// run 8 waves in a 2x4 grid (512 threads), batched GEMMs 4 waves in a 2x2
-// grid; each wave owns a (BM/2)x(BN/(NW/2)) slab of C built from 16x16
-// MFMA tiles:
-//   R8/C8: v_mfma_f64_16x16x4_f64   R4/C4: v_mfma_f32_16x16x4_f32
-// Operand tiles (BK=16) are double-buffered in LDS as K-contiguous rows padded
-// by one 16-byte vector (conflict-free fragment reads, aligned rows); the next
-// tile is loaded from HBM into registers with 16-byte accesses while the
-// current one is multiplied, so each K step needs a single barrier.  Blocks
-// are renumbered so that each XCD (dispatch round-robins workgroups over the
-// 8 XCDs) walks a compact band of C tiles and the operand panels it streams
-// stay in its own L2.  Complex products use four real MFMAs per step
-// (re += ar*br - ai*bi, im += ar*bi + ai*br), conjugation folded into the sign
-// of the imaginary operand.  MFMA fragment layout (16x16x4): A lane l holds
-// A[l%16][l/16], B lane l holds B[l/16][l%16]; accumulator register r of lane
-// l holds C[4*(l/16)+r][l%16] for f32 and C[4*r+l/16][l%16] for f64.
+// with op(A) in {A, A^T} and op(B) in {B, B^T}, complex operands optionally
+// conjugated.  Other products run on the direct contraction kernels
+// (direct_kernel.hpp).  Blocks are renumbered so that each XCD (dispatch
+// round-robins workgroups over the 8 XCDs) walks a compact band of C tiles and
+// the operand panels it streams stay in its own L2.  MFMA fragment layout
+// (16x16x4): A lane l holds A[l%16][l/16], B lane l holds B[l/16][l%16];
+// accumulator register r of lane l holds C[4*(l/16)+r][l%16] for f32 and
+// C[4*r+l/16][l%16] for f64.
 #include "kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -56,34 +43,6 @@ constexpr int kThreads = 256;
 constexpr int BK = 16;
 constexpr int kXcds = 8;
 
-// Waves per workgroup of gemm_kernel (template parameter NW), in 2 rows x
-// NW/2 columns: 8 (4 per SIMD) for single GEMMs — at 9216^3, against 4 waves
-// of 2 x 2: FP64 64.5 -> 65.6, FP32 124.8 -> 127.3, complex FP64 65.5 -> 66.8
-// TFLOP/s — and 4 (2 per SIMD) for batched ones, whose 16 x 1024^3 case ran
-// 48.1 TFLOP/s with 4 waves and 42.8 with 8.
-constexpr int kWavesSingle = 8, kWavesBatched = 4;
-// K step (template parameter KB): 16 for FP64 and complex tiles, 32 for FP32
-// 128 x 128 tiles (same LDS bytes as FP64 at 16; half the barriers per K for
-// MFMAs that take half as long: 9216^3 125.8 -> 129.3 TFLOP/s).
-
-// W scalars moved as one access (W*sizeof(S) is 16 bytes when vectorised).
-template <typename S, int W>
-struct Vec {
-  S v[W];
-};
-template <typename S, int W>
-__device__ inline Vec<S, W> ld(const S *p) {
-  Vec<S, W> r;
-  if constexpr (sizeof(S) * W == 16) {
-    const uint4 u = *reinterpret_cast<const uint4 *>(p);
-    __builtin_memcpy(&r, &u, 16);
-  } else {
-#pragma unroll
-    for (int i = 0; i < W; ++i) r.v[i] = p[i];
-  }
-  return r;
-}
-
 // Tile t of C -> (bx, by): tiles are walked in groups of 8 tile-rows, column
 // by column inside a group (a bijection of [0, gx*gy)).
 __device__ inline void tile_xy(int64_t t, int64_t gx, int64_t gy, int64_t &bx, int64_t &by) {
@@ -106,120 +65,68 @@ __device__ inline void tile_of(int64_t gx, int64_t gy, int64_t t0, int64_t count
   tile_xy(t0 + t, gx, gy, bx, by);
 }
 
-// layout codes: 0 = N, 1 = T; CJA/CJB conjugate the complex operand; W is the
-// vector width in scalars along each operand's contiguous axis.
-template <typename S, int NC, int OPA, int OPB, int CJA, int CJB, int BM, int BN, int W, int NW, int KB>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2))) void gemm_kernel(
-                                                        int64_t M, int64_t N, int64_t K, const S *__restrict__ A,
-                                                        int64_t lda, const S *__restrict__ B, int64_t ldb,
-                                                        S *__restrict__ C, int64_t ldc, S alpha_r, S alpha_i,
-                                                        int beta_one, int64_t gx, int64_t gy, int64_t bsa,
-                                                        int64_t bsb, int64_t bsc, int64_t t0, int64_t count,
-                                                        int ksplit, int64_t kchunk, S *__restrict__ part,
-                                                        const int64_t *__restrict__ cmap) {
-  // ksplit == 1: tiles [t0, t0 + count) of C, the whole K each.  ksplit > 1:
-  // workgroup q*ksplit + c computes K range [c*kchunk, (c+1)*kchunk) of tile
-  // t0 + q into its own BM x BN block of `part` (no alpha, no beta); a second
-  // kernel sums the ksplit blocks of each tile in order.  cmap (batch 1 only):
-  // element (m, n) of C is at C[cmap[m] + cmap[M + n]] instead of C[m + n*ldc].
+// Products whose operands the direct kernels cannot address (an operand of
+// 2 GiB or more with rows too far apart for 32-bit offsets within a tile):
+// every access works its 64-bit address out.  One tile shape per kind, 4 waves
+// in a 2 x 2 grid, element loads into a double-buffered LDS stage.
+// Layout codes: 0 = N, 1 = T; conja / conjb: sign of an operand's imaginary part.
+template <typename S, int NC, int OPA, int OPB, int BM, int BN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(
+    int64_t M, int64_t N, int64_t K, const S *__restrict__ A, int64_t lda, const S *__restrict__ B, int64_t ldb,
+    S *__restrict__ C, int64_t ldc, S alpha_r, S alpha_i, S sa, S sb, int beta_one, int64_t gx, int64_t gy,
+    int64_t bsa, int64_t bsb, int64_t bsc) {
   using MF = Mfma<S>;
-  // batch entry blockIdx.y: its operands start bsa, bsb, bsc scalars further on
+  using acc_t = typename MF::acc_t;
   A += (int64_t)blockIdx.y * bsa;
   B += (int64_t)blockIdx.y * bsb;
   C += (int64_t)blockIdx.y * bsc;
-  using acc_t = typename MF::acc_t;
-  // threads; columns of C per wave (waves form 2 rows x NW/2 columns)
-  constexpr int NT = 64 * NW, WBN = BN / (NW / 2);
-  constexpr int SM = BM / 32, SN = WBN / 16;  // 16x16 tiles per wave along M, N
-  constexpr int PAD = W;                     // keeps rows 16-byte aligned
-  constexpr int RS = KB + PAD;               // LDS row stride (scalars)
-  // A tile: BM x KB elements (BM*KB*NC scalars) moved in vectors of W scalars
-  // along the contiguous axis (m for 'N', k for 'T'; re/im interleaved).
-  constexpr int ACONT = (OPA == 0 ? BM : KB) * NC, BCONT = (OPB == 0 ? KB : BN) * NC;
-  constexpr int AVEC = BM * KB * NC / W / NT, BVEC = BN * KB * NC / W / NT;
-  static_assert(AVEC >= 1 && BVEC >= 1, "tile too small");
-  constexpr int ATPL = ACONT / W, BTPL = BCONT / W;  // threads per contiguous line
-  static_assert(NT % ATPL == 0 && NT % BTPL == 0, "line split");
+  constexpr int NT = 256, SM = BM / 32, SN = BN / 32, RS = BK + 2;
+  // tile elements are moved one by one along the contiguous axis (m for 'N', k for 'T')
+  constexpr int ATPL = OPA == 0 ? BM : BK, BTPL = OPB == 0 ? BK : BN;
+  constexpr int AVEC = BM * BK / NT, BVEC = BN * BK / NT, ALS = NT / ATPL, BLS = NT / BTPL;
   __shared__ S As[2][NC][BM][RS];
   __shared__ S Bs[2][NC][BN][RS];
-
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  int64_t bx, by, kbeg = 0, kend = K;
-  if (ksplit > 1) {
-    tile_xy(t0 + (int64_t)blockIdx.x / ksplit, gx, gy, bx, by);
-    kbeg = (int64_t)(blockIdx.x % ksplit) * kchunk;
-    kend = min(K, kbeg + kchunk);
-  } else {
-    tile_of(gx, gy, t0, count, bx, by);
-  }
+  int64_t bx, by;
+  tile_of(gx, gy, 0, gx * gy, bx, by);
   const int64_t m0 = bx * BM, n0 = by * BN;
-
-  // per-thread load coordinates: contiguous-axis scalar offset and line index
-  const int a_c = (tid % ATPL) * W, a_l = tid / ATPL;
-  const int b_c = (tid % BTPL) * W, b_l = tid / BTPL;
-  constexpr int ALS = NT / ATPL, BLS = NT / BTPL;  // line step per vector
-
-  Vec<S, W> ra[AVEC], rb[BVEC];
-
+  const int a_c = tid % ATPL, a_l = tid / ATPL, b_c = tid % BTPL, b_l = tid / BTPL;
+  S ra[AVEC][NC], rb[BVEC][NC];
   auto load_tiles = [&](int64_t k0) {
 #pragma unroll
     for (int e = 0; e < AVEC; ++e) {
       const int line = a_l + e * ALS;
-      int64_t m, k;
-      if (OPA == 0) { m = m0 + a_c / NC; k = k0 + line; }
-      else { m = m0 + line; k = k0 + a_c / NC; }
-      const bool ok = (m < M) && (k < kend);
-      const int64_t off = (OPA == 0) ? (m + k * lda) : (k + m * lda);
-      if (ok) {
-        ra[e] = ld<S, W>(A + off * NC + (a_c % NC));
-      } else {
+      const int64_t m = m0 + (OPA == 0 ? a_c : line), k = k0 + (OPA == 0 ? line : a_c);
+      const bool ok = m < M && k < K;
+      const int64_t off = OPA == 0 ? m + k * lda : k + m * lda;
 #pragma unroll
-        for (int i = 0; i < W; ++i) ra[e].v[i] = (S)0;
-      }
+      for (int c = 0; c < NC; ++c) ra[e][c] = ok ? A[off * NC + c] : (S)0;
     }
 #pragma unroll
     for (int e = 0; e < BVEC; ++e) {
       const int line = b_l + e * BLS;
-      int64_t n, k;
-      if (OPB == 0) { k = k0 + b_c / NC; n = n0 + line; }
-      else { k = k0 + line; n = n0 + b_c / NC; }
-      const bool ok = (n < N) && (k < kend);
-      const int64_t off = (OPB == 0) ? (k + n * ldb) : (n + k * ldb);
-      if (ok) {
-        rb[e] = ld<S, W>(B + off * NC + (b_c % NC));
-      } else {
+      const int64_t n = n0 + (OPB == 0 ? line : b_c), k = k0 + (OPB == 0 ? b_c : line);
+      const bool ok = n < N && k < K;
+      const int64_t off = OPB == 0 ? k + n * ldb : n + k * ldb;
 #pragma unroll
-        for (int i = 0; i < W; ++i) rb[e].v[i] = (S)0;
-      }
+      for (int c = 0; c < NC; ++c) rb[e][c] = ok ? B[off * NC + c] : (S)0;
     }
   };
-  // scatter register vectors into the K-contiguous LDS layout [c][row][k]
   auto store_tiles = [&](int buf) {
 #pragma unroll
     for (int e = 0; e < AVEC; ++e) {
       const int line = a_l + e * ALS;
 #pragma unroll
-      for (int i = 0; i < W; ++i) {
-        const int sc = a_c + i;  // scalar index along the contiguous axis
-        const int c = sc % NC, x = sc / NC;
-        if (OPA == 0) As[buf][c][x][line] = ra[e].v[i];
-        else As[buf][c][line][x] = ra[e].v[i];
-      }
+      for (int c = 0; c < NC; ++c) As[buf][c][OPA == 0 ? a_c : line][OPA == 0 ? line : a_c] = c ? sa * ra[e][c] : ra[e][c];
     }
 #pragma unroll
     for (int e = 0; e < BVEC; ++e) {
       const int line = b_l + e * BLS;
 #pragma unroll
-      for (int i = 0; i < W; ++i) {
-        const int sc = b_c + i;
-        const int c = sc % NC, x = sc / NC;
-        if (OPB == 0) Bs[buf][c][line][x] = rb[e].v[i];
-        else Bs[buf][c][x][line] = rb[e].v[i];
-      }
+      for (int c = 0; c < NC; ++c) Bs[buf][c][OPB == 0 ? line : b_c][OPB == 0 ? b_c : line] = c ? sb * rb[e][c] : rb[e][c];
     }
   };
-
   acc_t acc[NC][SM][SN];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -227,128 +134,38 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2)
     for (int i = 0; i < SM; ++i)
 #pragma unroll
       for (int j = 0; j < SN; ++j) acc[c][i][j] = acc_t{0, 0, 0, 0};
-
-  const S sa = CJA ? (S)-1 : (S)1;  // sign of A's imaginary part
-  const S sb = CJB ? (S)-1 : (S)1;
-  const int64_t nk = (kend - kbeg + KB - 1) / KB;
-
-  load_tiles(kbeg);
+  const int64_t nk = (K + BK - 1) / BK;
+  load_tiles(0);
   store_tiles(0);
   __syncthreads();
   for (int64_t kt = 0; kt < nk; ++kt) {
     const int buf = (int)(kt & 1);
-    if (kt + 1 < nk) load_tiles(kbeg + (kt + 1) * KB);
-    // interleave the LDS fragment reads with the MFMAs (+2 % on FP64, FP32 and complex)
-    __builtin_amdgcn_iglp_opt(1);
+    if (kt + 1 < nk) load_tiles((kt + 1) * BK);
 #pragma unroll
-    for (int ks = 0; ks < KB / 4; ++ks) {
+    for (int ks = 0; ks < BK / 4; ++ks) {
       const int kk = ks * 4 + (lane >> 4);
       S fa[NC][SM], fb[NC][SN];
 #pragma unroll
-      for (int i = 0; i < SM; ++i)
+      for (int c = 0; c < NC; ++c) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) fa[c][i] = As[buf][c][wm * (BM / 2) + i * 16 + (lane & 15)][kk];
+        for (int i = 0; i < SM; ++i) fa[c][i] = As[buf][c][wm * (BM / 2) + i * 16 + (lane & 15)][kk];
 #pragma unroll
-      for (int j = 0; j < SN; ++j)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) fb[c][j] = Bs[buf][c][wn * WBN + j * 16 + (lane & 15)][kk];
+        for (int j = 0; j < SN; ++j) fb[c][j] = Bs[buf][c][wn * (BN / 2) + j * 16 + (lane & 15)][kk];
+      }
 #pragma unroll
       for (int i = 0; i < SM; ++i)
 #pragma unroll
         for (int j = 0; j < SN; ++j) {
-          if (NC == 1) {
-            acc[0][i][j] = MF::op(fa[0][i], fb[0][j], acc[0][i][j]);
-          } else {
-            const S ai = sa * fa[NC - 1][i], bi = sb * fb[NC - 1][j];
-            acc[0][i][j] = MF::op(fa[0][i], fb[0][j], acc[0][i][j]);
-            acc[0][i][j] = MF::op(-ai, bi, acc[0][i][j]);
-            acc[NC - 1][i][j] = MF::op(fa[0][i], bi, acc[NC - 1][i][j]);
-            acc[NC - 1][i][j] = MF::op(ai, fb[0][j], acc[NC - 1][i][j]);
+          acc[0][i][j] = MF::op(fa[0][i], fb[0][j], acc[0][i][j]);
+          if (NC == 2) {
+            acc[0][i][j] = MF::op(-fa[NC - 1][i], fb[NC - 1][j], acc[0][i][j]);
+            acc[NC - 1][i][j] = MF::op(fa[0][i], fb[NC - 1][j], acc[NC - 1][i][j]);
+            acc[NC - 1][i][j] = MF::op(fa[NC - 1][i], fb[0][j], acc[NC - 1][i][j]);
           }
         }
     }
     if (kt + 1 < nk) store_tiles(buf ^ 1);
     __syncthreads();
-  }
-
-  // epilogue
-  if (ksplit > 1) {  // raw partial sums of this K range, BM x BN block column-major
-    S *pb = part + (int64_t)blockIdx.x * BM * BN * NC;
-#pragma unroll
-    for (int i = 0; i < SM; ++i)
-#pragma unroll
-      for (int j = 0; j < SN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int ml = wm * (BM / 2) + i * 16 + MF::row(lane, r), nl = wn * WBN + j * 16 + (lane & 15);
-#pragma unroll
-          for (int c = 0; c < NC; ++c) pb[(ml + nl * BM) * NC + c] = acc[c][i][j][r];
-        }
-    return;
-  }
-  // Short-K GEMMs (and GEMMs into plain column-major C) are store-bound:
-  // there each 16 x 16 block of the wave's accumulators is turned round
-  // through a wave-private LDS patch (the operand tiles' space, free after
-  // the last barrier of the K loop) so that every store covers 16
-  // consecutive rows (m, C's and D's contiguous axis) of 4 columns instead of
-  // 4 rows, or 4 rows 4 apart, of 16 columns: runs of 128 bytes (FP64) rather
-  // than 32.  Rank-6 contractions with K = 24 writing D in place ran 10-12 ->
-  // 14-18 TFLOP/s, and 18.5-23 with the offsets loaded ahead of the stores;
-  // a 5136^3 GEMM 47.3 -> 50.0; long-K GEMMs writing D in
-  // place lost 0.6-1 % with it and keep the direct stores.  LDS accesses of
-  // one wave complete in order, so the patch needs no barrier between its
-  // writes and reads.
-  if (!cmap || K <= 2048) {
-    constexpr int TP = 17;  // patch column stride (scalars)
-    static_assert(sizeof(As) >= sizeof(S) * NW * NC * 16 * TP, "patches fit the A tiles' space");
-    S *patch = &As[0][0][0][0] + wave * NC * 16 * TP;
-    const int tl = lane & 15, tg = lane >> 4;
-    // the lane's row and column offsets into C, all loaded before the first
-    // store (one table latency instead of one per store)
-    int64_t roff[SM], coff[SN][4];
-#pragma unroll
-    for (int i = 0; i < SM; ++i) {
-      const int64_t m = m0 + wm * (BM / 2) + i * 16 + tl;
-      roff[i] = m < M ? (cmap ? cmap[m] : m) : -1;
-    }
-#pragma unroll
-    for (int j = 0; j < SN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t n = n0 + wn * WBN + j * 16 + 4 * r + tg;
-        coff[j][r] = n < N ? (cmap ? cmap[M + n] : n * ldc) : -1;
-      }
-#pragma unroll
-    for (int i = 0; i < SM; ++i)
-#pragma unroll
-      for (int j = 0; j < SN; ++j) {
-        S v[NC][4];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) patch[(c * 16 + (lane & 15)) * TP + MF::row(lane, r)] = acc[c][i][j][r];
-          __builtin_amdgcn_wave_barrier();
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[c][r] = patch[(c * 16 + 4 * r + tg) * TP + tl];
-          __builtin_amdgcn_wave_barrier();
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (roff[i] >= 0 && coff[j][r] >= 0) {
-            S *c = C + (roff[i] + coff[j][r]) * NC;
-            if (NC == 1) {
-              const S x = alpha_r * v[0][r];
-              c[0] = beta_one ? c[0] + x : x;
-            } else {
-              const S xr = v[0][r], xi = v[NC - 1][r];
-              const S vr = alpha_r * xr - alpha_i * xi, vi = alpha_r * xi + alpha_i * xr;
-              c[0] = beta_one ? c[0] + vr : vr;
-              c[NC - 1] = beta_one ? c[NC - 1] + vi : vi;
-            }
-          }
-        }
-      }
-    return;
   }
 #pragma unroll
   for (int i = 0; i < SM; ++i)
@@ -357,16 +174,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t m = m0 + wm * (BM / 2) + i * 16 + MF::row(lane, r);
-        const int64_t n = n0 + wn * WBN + j * 16 + (lane & 15);
+        const int64_t n = n0 + wn * (BN / 2) + j * 16 + (lane & 15);
         if (m < M && n < N) {
-          S *c = C + (cmap ? cmap[m] + cmap[M + n] : m + n * ldc) * NC;
-          if (NC == 1) {
-            const S v = alpha_r * acc[0][i][j][r];
-            c[0] = beta_one ? c[0] + v : v;
-          } else {
-            const S xr = acc[0][i][j][r], xi = acc[NC - 1][i][j][r];
-            const S vr = alpha_r * xr - alpha_i * xi, vi = alpha_r * xi + alpha_i * xr;
-            c[0] = beta_one ? c[0] + vr : vr;
+          S *c = C + (m + n * ldc) * NC;
+          const S xr = acc[0][i][j][r], xi = acc[NC - 1][i][j][r];
+          const S vr = NC == 1 ? alpha_r * xr : alpha_r * xr - alpha_i * xi;
+          c[0] = beta_one ? c[0] + vr : vr;
+          if (NC == 2) {
+            const S vi = alpha_r * xi + alpha_i * xr;
             c[NC - 1] = beta_one ? c[NC - 1] + vi : vi;
           }
         }
@@ -417,177 +232,15 @@ __global__ __launch_bounds__(kThreads) void gemm_tail_reduce(int64_t M, int64_t 
 // Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
 // Higher-Precision Computations", ARITH 2019).  The dropped terms are below
 // 2^-24 relative; with FP32 accumulation the normwise error at K = 9216 is a
-// few 1e-7 (cf. ~1e-6 for the FP32 MFMA path).  Two kernels implement it:
-//  - gemm_bf16x6_kernel (launch_gemm with R4_SPLIT_BF16, no workspace):
-//    128 x 128 tiles; FP32 tiles come from HBM as for the FP32 kernel and the
-//    split happens once per element when the tile is written to LDS (three
-//    BF16 planes, rows padded to 80 bytes so the 16-byte fragment reads of 16
-//    lanes hit all 64 banks once);
-//  - gemm_bf16x6p_kernel (launch_gemm_split, used by talshTensorContract):
-//    both operands are split once into swizzled BF16 planes in a workspace by
-//    split_planes_kernel, then 256 x 128 tiles of 8 waves stream the planes
-//    with no VALU split work in the K loop; the last, mostly idle round of
-//    tiles is split along K into partials summed by gemm_tail_reduce.
-// MFMA 16x16x32 bf16
+// few 1e-7 (cf. ~1e-6 for the FP32 MFMA path).  Both operands are split once
+// into swizzled BF16 planes in a workspace by split_planes_kernel, then 256 x
+// 128 tiles of 8 waves stream the planes with no VALU split work in the K
+// loop; the last, mostly idle round of tiles is split along K into partials
+// summed by gemm_tail_reduce.  MFMA 16x16x32 bf16
 // layout: A lane l holds A[l%16][8*(l/16)..+7], B lane l holds
 // B[8*(l/16)..+7][l%16], accumulator register r of lane l holds
 // C[4*(l/16)+r][l%16].
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ inline void split3(float x, __bf16 &h, __bf16 &m, __bf16 &l) {
-  h = (__bf16)x;
-  const float r = x - (float)h;
-  m = (__bf16)r;
-  l = (__bf16)(r - (float)m);
-}
-
-// Block tile BM x BN with WM x WN waves (each wave (BM/WM) x (BN/WN)); BK = 32
-// (one MFMA depth).  Per K step each wave sums the five small products of a
-// 16x16 tile into a zero-started register and the dominant ah*bh product
-// into another, then adds both to the running FP32 accumulator, so the
-// accumulator is rounded once per K step instead of six times.
-template <int OPA, int OPB, int W, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void gemm_bf16x6_kernel(
-    int64_t M, int64_t N, int64_t K, const float *__restrict__ A, int64_t lda, const float *__restrict__ B,
-    int64_t ldb, float *__restrict__ C, int64_t ldc, float alpha, int beta_one, int64_t gx, int64_t gy) {
-  constexpr int NT = 64 * WM * WN, BKS = 32, RS = BKS + 8;
-  constexpr int TM = BM / WM, TN = BN / WN, SM = TM / 16, SN = TN / 16;
-  constexpr int ACONT = (OPA == 0 ? BM : BKS), BCONT = (OPB == 0 ? BKS : BN);
-  constexpr int AVEC = BM * BKS / W / NT, BVEC = BN * BKS / W / NT;
-  constexpr int ATPL = ACONT / W, BTPL = BCONT / W;
-  constexpr int ALS = NT / ATPL, BLS = NT / BTPL;
-  static_assert(AVEC >= 1 && BVEC >= 1 && NT % ATPL == 0 && NT % BTPL == 0, "tile split");
-  __shared__ __attribute__((aligned(16))) __bf16 As[3][BM][RS];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[3][BN][RS];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
-  int64_t bx, by;
-  tile_of(gx, gy, 0, gx * gy, bx, by);
-  const int64_t m0 = bx * BM, n0 = by * BN;
-  const int a_c = (tid % ATPL) * W, a_l = tid / ATPL;
-  const int b_c = (tid % BTPL) * W, b_l = tid / BTPL;
-  Vec<float, W> ra[AVEC], rb[BVEC];
-
-  auto load_tiles = [&](int64_t k0) {
-#pragma unroll
-    for (int e = 0; e < AVEC; ++e) {
-      const int line = a_l + e * ALS;
-      const int64_t m = OPA == 0 ? m0 + a_c : m0 + line, k = OPA == 0 ? k0 + line : k0 + a_c;
-      const int64_t off = OPA == 0 ? (m + k * lda) : (k + m * lda);
-      if (m < M && k < K) {
-        ra[e] = ld<float, W>(A + off);
-      } else {
-#pragma unroll
-        for (int i = 0; i < W; ++i) ra[e].v[i] = 0.0f;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < BVEC; ++e) {
-      const int line = b_l + e * BLS;
-      const int64_t n = OPB == 0 ? n0 + line : n0 + b_c, k = OPB == 0 ? k0 + b_c : k0 + line;
-      const int64_t off = OPB == 0 ? (k + n * ldb) : (n + k * ldb);
-      if (n < N && k < K) {
-        rb[e] = ld<float, W>(B + off);
-      } else {
-#pragma unroll
-        for (int i = 0; i < W; ++i) rb[e].v[i] = 0.0f;
-      }
-    }
-  };
-  // split each value into three BF16 planes; along K the W terms of a plane
-  // are contiguous and go out as one packed store
-  auto put = [&](__bf16 (*P)[BM > BN ? BM : BN][RS], const Vec<float, W> &v, int row, int col, bool kcont) {
-    __bf16 h[W], m[W], l[W];
-#pragma unroll
-    for (int i = 0; i < W; ++i) split3(v.v[i], h[i], m[i], l[i]);
-    if (kcont && W == 4) {
-      uint2 u;
-      __builtin_memcpy(&u, h, 8);
-      *reinterpret_cast<uint2 *>(&P[0][row][col]) = u;
-      __builtin_memcpy(&u, m, 8);
-      *reinterpret_cast<uint2 *>(&P[1][row][col]) = u;
-      __builtin_memcpy(&u, l, 8);
-      *reinterpret_cast<uint2 *>(&P[2][row][col]) = u;
-    } else {
-#pragma unroll
-      for (int i = 0; i < W; ++i) {
-        const int r = kcont ? row : row + i, c = kcont ? col + i : col;
-        P[0][r][c] = h[i];
-        P[1][r][c] = m[i];
-        P[2][r][c] = l[i];
-      }
-    }
-  };
-  auto store_tiles = [&]() {
-#pragma unroll
-    for (int e = 0; e < AVEC; ++e) {
-      const int line = a_l + e * ALS;
-      if (OPA == 1) put(reinterpret_cast<__bf16(*)[BM > BN ? BM : BN][RS]>(As), ra[e], line, a_c, true);
-      else put(reinterpret_cast<__bf16(*)[BM > BN ? BM : BN][RS]>(As), ra[e], a_c, line, false);
-    }
-#pragma unroll
-    for (int e = 0; e < BVEC; ++e) {
-      const int line = b_l + e * BLS;
-      if (OPB == 0) put(reinterpret_cast<__bf16(*)[BM > BN ? BM : BN][RS]>(Bs), rb[e], line, b_c, true);
-      else put(reinterpret_cast<__bf16(*)[BM > BN ? BM : BN][RS]>(Bs), rb[e], b_c, line, false);
-    }
-  };
-
-  f32x4 acc[SM][SN];
-#pragma unroll
-  for (int i = 0; i < SM; ++i)
-#pragma unroll
-    for (int j = 0; j < SN; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
-
-  const int64_t nk = (K + BKS - 1) / BKS;
-  const int kof = 8 * (lane >> 4);
-  const f32x4 zero = {0, 0, 0, 0};
-  load_tiles(0);
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    __syncthreads();
-    store_tiles();
-    __syncthreads();
-    if (kt + 1 < nk) load_tiles((kt + 1) * BKS);
-    bf16x8 fb[3][SN];
-#pragma unroll
-    for (int j = 0; j < SN; ++j)
-#pragma unroll
-      for (int t = 0; t < 3; ++t)
-        fb[t][j] = *reinterpret_cast<const bf16x8 *>(&Bs[t][wn * TN + j * 16 + (lane & 15)][kof]);
-#pragma unroll
-    for (int i = 0; i < SM; ++i) {
-      bf16x8 fa[3];
-#pragma unroll
-      for (int t = 0; t < 3; ++t)
-        fa[t] = *reinterpret_cast<const bf16x8 *>(&As[t][wm * TM + i * 16 + (lane & 15)][kof]);
-#pragma unroll
-      for (int j = 0; j < SN; ++j) {
-        f32x4 sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[2], fb[0][j], zero, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[1], fb[1][j], sm, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[2][j], sm, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[1], fb[0][j], sm, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[1][j], sm, 0, 0, 0);
-        const f32x4 hh = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[0][j], zero, 0, 0, 0);
-        acc[i][j] += hh + sm;
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < SM; ++i)
-#pragma unroll
-    for (int j = 0; j < SN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t m = m0 + wm * TM + i * 16 + 4 * (lane >> 4) + r;
-        const int64_t n = n0 + wn * TN + j * 16 + (lane & 15);
-        if (m < M && n < N) {
-          float *c = C + m + n * ldc;
-          const float v = alpha * acc[i][j][r];
-          *c = beta_one ? *c + v : v;
-        }
-      }
-}
 
 // ---------------------------------------------------------------------------
 // Pre-split GEMMs.  split_planes_kernel writes the planes of an operand once
@@ -1057,46 +710,6 @@ int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, 
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-template <int OPA, int OPB>
-int launch_bf16x6(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda, const void *B, int64_t ldb, void *C,
-                  int64_t ldc, double ar, int beta_one, hipStream_t s) {
-  const int64_t acont = OPA == 0 ? M : K, bcont = OPB == 0 ? K : N;
-  const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && acont % 4 == 0 && bcont % 4 == 0 &&
-                   lda % 4 == 0 && ldb % 4 == 0;
-  if (vec) {  // 128 x 128 tiles, 4 waves of 64 x 64
-    const int64_t gx = (M + 127) / 128, gy = (N + 127) / 128, nblk = gx * gy;
-    if (nblk > 0x7fffffffLL) return -4;
-    gemm_bf16x6_kernel<OPA, OPB, 4, 128, 128, 2, 2><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(
-        M, N, K, (const float *)A, lda, (const float *)B, ldb, (float *)C, ldc, (float)ar, beta_one, gx, gy);
-  } else {  // scalar accesses: 128 x 128 tiles, 4 waves of 64 x 64
-    const int64_t gx = (M + 127) / 128, gy = (N + 127) / 128, nblk = gx * gy;
-    if (nblk > 0x7fffffffLL) return -4;
-    gemm_bf16x6_kernel<OPA, OPB, 1, 128, 128, 2, 2><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(
-        M, N, K, (const float *)A, lda, (const float *)B, ldb, (float *)C, ldc, (float)ar, beta_one, gx, gy);
-  }
-  return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-// Workgroups of gemm_kernel<S, NC, ..., BM, BN> resident at once on the
-// current device (CUs x blocks per CU), cached per device.
-template <typename S, int NC, int BM, int BN, int NWS, int KB>
-int64_t gemm_slots() {
-  static int64_t cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (!cache[dev]) {
-    int cus = 0, per = 0;
-    constexpr int WV = (int)(16 / sizeof(S));
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, gemm_kernel<S, NC, 1, 0, 0, 0, BM, BN, WV, NWS, KB>,
-                                                     64 * NWS, 0) !=
-            hipSuccess)
-      return 0;
-    cache[dev] = (int64_t)cus * std::max(per, 1);
-  }
-  return cache[dev];
-}
-
 // The tiles of C are dealt to the resident workgroups in rounds.  When the
 // last round is at most a quarter full (or the whole GEMM is), its `rem`
 // tiles are computed as ksplit K ranges each (filling the GPU) plus a
@@ -1105,112 +718,27 @@ struct TailSplit {
   int64_t rem = 0;
   int ksplit = 1;
 };
-template <typename S, int NC, int BM, int BN, int NWS, int KB>
-TailSplit tail_split(int64_t M, int64_t N, int64_t K, int64_t batch) {
-  TailSplit t;
-  if (batch != 1 || M <= 0 || N <= 0) return t;
-  const int64_t T = ((M + BM - 1) / BM) * ((N + BN - 1) / BN), slots = gemm_slots<S, NC, BM, BN, NWS, KB>();
-  if (slots <= 0) return t;
-  const int64_t rem = T % slots;
-  if (rem == 0 || rem * 4 > slots) return t;
-  // up to 64 K ranges per tile (a 312 x 312 x 97,344 product: 16 ranges ran
-  // 30.7 TFLOP/s, 20 ran 36.5); the partials never exceed one round of tiles
-  const int64_t ks = std::min<int64_t>(std::min<int64_t>(64, slots / rem), ((K + KB - 1) / KB) / 8);
-  if (ks < 2) return t;
-  t.rem = rem;
-  t.ksplit = (int)ks;
-  return t;
-}
 template <typename S, int NC, int BM, int BN>
-size_t tail_bytes(const TailSplit &t) {
-  return t.ksplit > 1 ? (size_t)t.rem * t.ksplit * BM * BN * NC * sizeof(S) : 0;
-}
-
-template <typename S, int NC, int OPA, int OPB, int CJA, int CJB, int BM, int BN, int NWS, int KB>
-int launch_typed(int64_t M, int64_t N, int64_t K, const void *A, int64_t lda, const void *B, int64_t ldb,
-                 void *C, int64_t ldc, double ar, double ai, int beta_one, int64_t batch, int64_t sa, int64_t sb,
-                 int64_t sc, void *ws, size_t ws_bytes, const int64_t *cmap, hipStream_t s) {
+int launch_wide(int opa, int opb, int cja, int cjb, int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
+                const void *B, int64_t ldb, void *C, int64_t ldc, double ar, double ai, int beta_one, int64_t batch,
+                int64_t sa, int64_t sb, int64_t sc, hipStream_t s) {
   const int64_t gx = (M + BM - 1) / BM, gy = (N + BN - 1) / BN;
-  const int64_t nblk = gx * gy;
-  if (nblk > 0x7fffffffLL) return -4;
-  // 16-byte accesses need every contiguous run (and every base, every batch entry) to split into whole vectors
-  constexpr int WV = (int)(16 / sizeof(S));
-  const int64_t acont = (OPA == 0 ? M : K) * NC, bcont = (OPB == 0 ? K : N) * NC;
-  const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && acont % WV == 0 &&
-                   bcont % WV == 0 && (lda * NC) % WV == 0 && (ldb * NC) % WV == 0 &&
-                   (batch == 1 || ((sa * NC) % WV == 0 && (sb * NC) % WV == 0));
-  TailSplit ts = tail_split<S, NC, BM, BN, NWS, KB>(M, N, K, batch);
-  if (!ws || tail_bytes<S, NC, BM, BN>(ts) > ws_bytes) ts = TailSplit{};
-  const int64_t full = nblk - ts.rem;  // tiles computed whole, in the first launch
-  const int64_t kchunk = ts.ksplit > 1 ? (((K + KB - 1) / KB + ts.ksplit - 1) / ts.ksplit) * KB : 0;
-  // batch entries go to grid.y, at most 65535 per launch
-  for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
-    const unsigned nb = (unsigned)std::min<int64_t>(65535, batch - b0);
+  if (gx * gy > 0x7fffffffLL) return -4;
+  for (int64_t b0 = 0; b0 < batch; b0 += 65535) {  // batch entries go to grid.y, at most 65535 per launch
+    const dim3 grid((unsigned)(gx * gy), (unsigned)std::min<int64_t>(65535, batch - b0));
     const S *a = (const S *)A + b0 * sa * NC, *b = (const S *)B + b0 * sb * NC;
     S *c = (S *)C + b0 * sc * NC;
-    if (full > 0) {
-      const dim3 grid((unsigned)full, nb);
-      const int64_t bsa = sa * NC, bsb = sb * NC, bsc = sc * NC;
-      if (batch > 1 && vec)
-        gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, WV, kWavesBatched, KB><<<grid, dim3(64 * kWavesBatched), 0, s>>>(
-            M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, beta_one, gx, gy, bsa, bsb, bsc, 0, full, 1, 0, nullptr,
-            cmap);
-      else if (batch > 1)
-        gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, 1, kWavesBatched, KB><<<grid, dim3(64 * kWavesBatched), 0, s>>>(
-            M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, beta_one, gx, gy, bsa, bsb, bsc, 0, full, 1, 0, nullptr,
-            cmap);
-      else if (vec)
-        gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, WV, NWS, KB><<<grid, dim3(64 * NWS), 0, s>>>(
-            M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, beta_one, gx, gy, bsa, bsb, bsc, 0, full, 1, 0, nullptr,
-            cmap);
-      else
-        gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, 1, NWS, KB><<<grid, dim3(64 * NWS), 0, s>>>(
-            M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, beta_one, gx, gy, bsa, bsb, bsc, 0, full, 1, 0, nullptr,
-            cmap);
-    }
-  }
-  if (ts.ksplit > 1) {
-    const unsigned nw = (unsigned)(ts.rem * ts.ksplit);
-    if (vec)
-      gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, WV, NWS, KB><<<dim3(nw), dim3(64 * NWS), 0, s>>>(
-          M, N, K, (const S *)A, lda, (const S *)B, ldb, (S *)C, ldc, (S)ar, (S)ai, beta_one, gx, gy, 0, 0, 0, full,
-          ts.rem, ts.ksplit, kchunk, (S *)ws, cmap);
-    else
-      gemm_kernel<S, NC, OPA, OPB, CJA, CJB, BM, BN, 1, NWS, KB><<<dim3(nw), dim3(64 * NWS), 0, s>>>(
-          M, N, K, (const S *)A, lda, (const S *)B, ldb, (S *)C, ldc, (S)ar, (S)ai, beta_one, gx, gy, 0, 0, 0, full,
-          ts.rem, ts.ksplit, kchunk, (S *)ws, cmap);
-    const int64_t nel = ts.rem * BM * BN;
-    gemm_tail_reduce<S, NC, BM, BN><<<dim3((unsigned)((nel + kThreads - 1) / kThreads)), dim3(kThreads), 0, s>>>(
-        M, N, (const S *)ws, ts.ksplit, (S *)C, ldc, (S)ar, (S)ai, beta_one, gx, gy, full, ts.rem, cmap);
+#define TAL_WIDE(a_, b_)                                                                                          \
+  gemm_wide_kernel<S, NC, a_, b_, BM, BN><<<grid, dim3(256), 0, s>>>(                                             \
+      M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, (S)(cja ? -1 : 1), (S)(cjb ? -1 : 1), beta_one, gx, gy,      \
+      sa * NC, sb * NC, sc * NC)
+    if (opa == 0 && opb == 0) TAL_WIDE(0, 0);
+    else if (opa == 0) TAL_WIDE(0, 1);
+    else if (opb == 0) TAL_WIDE(1, 0);
+    else TAL_WIDE(1, 1);
+#undef TAL_WIDE
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-template <typename S, int NC, int BM, int BN, int NWS, int KB>
-int dispatch_ops(int opa, int opb, int cja, int cjb, int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
-                 const void *B, int64_t ldb, void *C, int64_t ldc, double ar, double ai, int beta_one,
-                 int64_t batch, int64_t sa, int64_t sb, int64_t sc, void *ws, size_t ws_bytes,
-                 const int64_t *cmap, hipStream_t s) {
-#define TAL_GEMM_CASE(a, b, ca, cb)                                                                      \
-  if (opa == a && opb == b && cja == ca && cjb == cb)                                                    \
-    return launch_typed<S, NC, a, b, ca, cb, BM, BN, NWS, KB>(M, N, K, A, lda, B, ldb, C, ldc, ar, ai, beta_one, \
-                                                              batch, sa, sb, sc, ws, ws_bytes, cmap, s);
-#define TAL_GEMM_LAYOUTS(ca, cb) \
-  TAL_GEMM_CASE(0, 0, ca, cb)    \
-  TAL_GEMM_CASE(0, 1, ca, cb)    \
-  TAL_GEMM_CASE(1, 0, ca, cb)    \
-  TAL_GEMM_CASE(1, 1, ca, cb)
-  if constexpr (NC == 1) {
-    TAL_GEMM_LAYOUTS(0, 0)
-  } else {
-    TAL_GEMM_LAYOUTS(0, 0)
-    TAL_GEMM_LAYOUTS(0, 1)
-    TAL_GEMM_LAYOUTS(1, 0)
-    TAL_GEMM_LAYOUTS(1, 1)
-  }
-#undef TAL_GEMM_LAYOUTS
-#undef TAL_GEMM_CASE
-  return -1;
 }
 
 int op_code(char t) {
@@ -1353,56 +881,9 @@ int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_
              : launch_presplit<3>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, cmap, s);
 }
 
-// Real single GEMMs whose 128 x 128 tiles would not fill one round of the
-// resident workgroups run 64 x 64 tiles: four times the tiles, so a 1024^3
-// product spreads over the whole GPU.  FP64 uses 8 waves (32 x 16 of C each)
-// and a K step of 32, one 256-tile round with no K split (1024^3: 54 us,
-// against 62 us for 4 waves with a K step of 16 split in two plus the
-// summing pass); FP32 keeps 4 waves (32 x 32 each) and a K step of 16.
-template <typename S>
-bool small_real(int64_t M, int64_t N, int64_t batch) {
-  if (batch != 1) return false;
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
-  return t128 < gemm_slots<S, 1, 128, 128, kWavesSingle, sizeof(S) == 4 ? 2 * BK : BK>();
-}
-
-// Real GEMMs with at most 32 columns and many 128-row tiles (the N = 24
-// contractions of the reference's benchmark list) are latency-bound
-// on their A tile loads: 128 x 32 tiles of 4 waves (64 x 16 of C each) keep
-// more workgroups, and so more of A, in flight per CU than 128 x 128 tiles
-// of which three quarters of the columns are empty.  Those GEMMs ran 6-10 ->
-// 16-28 TFLOP/s in FP64 and 9-20 -> 20-49 in FP32 (K = 48-312, M = 97,344
-// to 5,308,416); up to 96 columns, three narrow tiles still beat one wide
-// one from 4,096 rows (5184 x 72 x 5184: 12.8 -> 19.2 TFLOP/s per step).
-bool skinny_real(int64_t M, int64_t N, int64_t batch) {
-  return batch == 1 && ((N <= 32 && M >= 128 * 512) || (N <= 96 && M >= 4096));
-}
-
-size_t gemm_tail_workspace(int dk, int64_t M, int64_t N, int64_t K, int64_t batch) {
-  switch (dk) {
-    case 8:
-      if (skinny_real(M, N, batch))
-        return tail_bytes<double, 1, 128, 32>(tail_split<double, 1, 128, 32, 4, BK>(M, N, K, batch));
-      return small_real<double>(M, N, batch)
-                 ? tail_bytes<double, 1, 64, 64>(tail_split<double, 1, 64, 64, kWavesSingle, 2 * BK>(M, N, K, batch))
-                 : tail_bytes<double, 1, 128, 128>(tail_split<double, 1, 128, 128, kWavesSingle, BK>(M, N, K, batch));
-    case 4:
-      if (skinny_real(M, N, batch))
-        return tail_bytes<float, 1, 128, 32>(tail_split<float, 1, 128, 32, 4, 2 * BK>(M, N, K, batch));
-      return small_real<float>(M, N, batch)
-                 ? tail_bytes<float, 1, 64, 64>(tail_split<float, 1, 64, 64, 4, BK>(M, N, K, batch))
-                 : tail_bytes<float, 1, 128, 128>(
-                       tail_split<float, 1, 128, 128, kWavesSingle, 2 * BK>(M, N, K, batch));
-    case 18: return tail_bytes<double, 2, 64, 64>(tail_split<double, 2, 64, 64, kWavesSingle, BK>(M, N, K, batch));
-    case 14: return tail_bytes<float, 2, 64, 64>(tail_split<float, 2, 64, 64, kWavesSingle, BK>(M, N, K, batch));
-    default: return 0;
-  }
-}
-
-int launch_gemm(int dk, int r4mode, char ta, char tb, int conja, int conjb, int64_t M, int64_t N, int64_t K,
-                double ar, double ai, const void *A, int64_t lda, const void *B, int64_t ldb, int beta_one, void *C,
-                int64_t ldc, hipStream_t s, int64_t batch, int64_t sa, int64_t sb, int64_t sc, void *ws,
-                size_t ws_bytes, const int64_t *cmap) {
+int launch_gemm(int dk, char ta, char tb, int conja, int conjb, int64_t M, int64_t N, int64_t K, double ar, double ai,
+                const void *A, int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc,
+                hipStream_t s, int64_t batch, int64_t sa, int64_t sb, int64_t sc) {
   const bool cplx = (dk == 14 || dk == 18);
   const int opa = op_code(ta), opb = op_code(tb);
   const int cja = (cplx && conja) ? 1 : 0, cjb = (cplx && conjb) ? 1 : 0;
@@ -1412,34 +893,14 @@ int launch_gemm(int dk, int r4mode, char ta, char tb, int conja, int conjb, int6
   if (lda < std::max<int64_t>(1, opa == 0 ? M : K)) return -1;
   if (ldb < std::max<int64_t>(1, opb == 0 ? K : N)) return -1;
   if (batch > 1 && (sa < 0 || sb < 0 || sc < ldc * N)) return -1;  // batch entries of C may not overlap
-  if (cmap && (batch > 1 || (dk == 4 && r4mode == R4_SPLIT_BF16))) return -1;
-  if (dk == 4 && r4mode == R4_SPLIT_BF16) {
-    for (int64_t q = 0; q < batch; ++q) {
-      const float *a = (const float *)A + q * sa, *b = (const float *)B + q * sb;
-      float *c = (float *)C + q * sc;
-      int e;
-      if (opa == 0 && opb == 0) e = launch_bf16x6<0, 0>(M, N, K, a, lda, b, ldb, c, ldc, ar, beta_one, s);
-      else if (opa == 0 && opb == 1) e = launch_bf16x6<0, 1>(M, N, K, a, lda, b, ldb, c, ldc, ar, beta_one, s);
-      else if (opa == 1 && opb == 0) e = launch_bf16x6<1, 0>(M, N, K, a, lda, b, ldb, c, ldc, ar, beta_one, s);
-      else e = launch_bf16x6<1, 1>(M, N, K, a, lda, b, ldb, c, ldc, ar, beta_one, s);
-      if (e) return e;
-    }
-    return 0;
-  }
-#define TAL_GEMM_KIND(S, NC, BM, BN, NWS, KB)                                                                    \
-  dispatch_ops<S, NC, BM, BN, NWS, KB>(opa, opb, cja, cjb, M, N, K, A, lda, B, ldb, C, ldc, ar, ai, beta_one, batch, \
-                                       sa, sb, sc, ws, ws_bytes, cmap, s)
+#define TAL_GEMM_KIND(S, NC, BM, BN)                                                                              \
+  launch_wide<S, NC, BM, BN>(opa, opb, cja, cjb, M, N, K, A, lda, B, ldb, C, ldc, ar, ai, beta_one, batch, sa, sb, \
+                             sc, s)
   switch (dk) {
-    case 8:
-      if (skinny_real(M, N, batch)) return TAL_GEMM_KIND(double, 1, 128, 32, 4, BK);
-      return small_real<double>(M, N, batch) ? TAL_GEMM_KIND(double, 1, 64, 64, kWavesSingle, 2 * BK)
-                                             : TAL_GEMM_KIND(double, 1, 128, 128, kWavesSingle, BK);
-    case 4:
-      if (skinny_real(M, N, batch)) return TAL_GEMM_KIND(float, 1, 128, 32, 4, 2 * BK);
-      return small_real<float>(M, N, batch) ? TAL_GEMM_KIND(float, 1, 64, 64, 4, BK)
-                                            : TAL_GEMM_KIND(float, 1, 128, 128, kWavesSingle, 2 * BK);
-    case 18: return TAL_GEMM_KIND(double, 2, 64, 64, kWavesSingle, BK);
-    case 14: return TAL_GEMM_KIND(float, 2, 64, 64, kWavesSingle, BK);
+    case 8: return TAL_GEMM_KIND(double, 1, 128, 128);
+    case 4: return TAL_GEMM_KIND(float, 1, 128, 128);
+    case 18: return TAL_GEMM_KIND(double, 2, 64, 64);
+    case 14: return TAL_GEMM_KIND(float, 2, 64, 64);
     default: return -1;
   }
 #undef TAL_GEMM_KIND

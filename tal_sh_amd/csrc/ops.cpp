@@ -12,6 +12,7 @@
 // gpu_tensor_block_{init,scale,copy,add,contract_dlf,place}
 // (tensor_algebra_gpu_nvidia.cu:4089-7188); coherence letters as in
 // DOC/TALSH_manual.txt:719-750 (D discard, M move, T temporary, K keep).
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -21,6 +22,7 @@
 #include <vector>
 
 #include "contract.hpp"
+#include "direct.hpp"
 #include "plan.hpp"
 #include "runtime.hpp"
 #include "talsh_amd.h"
@@ -106,6 +108,16 @@ class Op {
     return TALSH_SUCCESS;
   }
   void *temp(int i) const { return temps_[i]; }
+  // One more temporary if the pool has room for it now: its index, else -1.
+  int acquire_optional(size_t bytes) {
+    void *p = nullptr;
+    int h = -1;
+    if (dev_alloc(g_, bytes, &p, &h)) return -1;
+    temps_.push_back(p);
+    temp_handles_.push_back(h);
+    temp_bytes_.push_back(bytes);
+    return (int)temps_.size() - 1;
+  }
 
   // Starts the task: stream, ordering against earlier work, input transfers.
   // clock: the kernels launched until end() carry dispatch timestamps, which
@@ -494,18 +506,68 @@ void ttgt_cache_clear() {
   c.chunks.clear();
 }
 
+namespace {
+
+// How a plan runs for a data kind: a plain product by the direct kernels
+// straight from the tensors, or on copies of the operands the planner
+// transposes (with D written in place or through D'); split: the fast-math
+// GEMMs.  Depends on the plan, the kind and the fast-math mode only.
+enum Route { kRouteDirect, kRouteCopies, kRouteWide, kRouteSplit };
+
+// Straight from the tensors where the transposes would cost more than the
+// reads in place do.  Measured (R8): a K step that walks runs of k costs 4 %
+// of a product in 128 x 128 tiles (9216^3: 21.99 -> 22.66 ms) and about a
+// quarter in smaller ones (1024^3: 41 -> 50 us); one whose every lane works
+// its offsets out, 40 %; D written 8 bytes apart, about four times its bytes.
+// A transpose moves 4.6 TB/s and takes about 4 us beside that.
+Route plan_route(const ContractPlan &plan, int dk) {
+  if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) return kRouteSplit;
+  const bool mat_ok = direct_addressable(plan.mat, dk);
+  if (plan.direct_ok && direct_addressable(plan.direct, dk)) {
+    const DirectForm &f = plan.direct;
+    const int esz = dk_size(dk);
+    const bool d_copy = plan.d_transpose && !plan.mat_d_in_place;
+    if (mat_ok && !plan.a.transpose && !plan.b.transpose && !d_copy) return kRouteCopies;  // nothing to copy
+    const double avol = (double)f.avol * esz, bvol = (double)f.bvol * esz;
+    const double dvol = (double)f.M * (double)f.N * (double)f.batch * esz;
+    const bool ta = plan.swap ? plan.b.transpose : plan.a.transpose, tb = plan.swap ? plan.a.transpose : plan.b.transpose;
+    const double copies =
+        (2 * ((ta ? avol : 0) + (tb ? bvol : 0) + (d_copy ? dvol : 0))) / 4.6e6 + ((ta || tb) ? 4 : 0) + (d_copy ? 4 : 0);
+    const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
+    const double gemm = c.us;
+    double extra = 0;
+    if (plan.direct_krun) extra += (plan.direct_krun < 32 ? 0.4 : c.tile == 0 ? 0.05 : 0.25) * gemm;
+    if (plan.direct_run && plan.direct_run < 8) extra += 0.3 * gemm;
+    if (plan.direct_conflict) extra += std::min(avol, bvol) > 4e6 ? 1e9 : 0.5 * gemm;
+    if (plan.direct_scatter) extra += 4 * dvol / 4.6e6;
+    if (!mat_ok || copies > extra) return kRouteDirect;
+  }
+  return mat_ok ? kRouteCopies : kRouteWide;
+}
+
+}  // namespace
+
 TtgtTemps ttgt_temp_bytes(const ContractPlan &plan, int dk, size_t lbytes, size_t rbytes, size_t dbytes) {
   TtgtTemps t;
+  const Route route = plan_route(plan, dk);
+  if (route == kRouteDirect) {
+    const DirectForm &f = plan.direct;
+    t.s = direct_choose(dk, f.M, f.N, f.K, f.batch).part_bytes;
+    return t;
+  }
   if (plan.a.transpose) t.a = plan.swap ? rbytes : lbytes;
   if (plan.b.transpose) t.b = plan.swap ? lbytes : rbytes;
-  int nm = 0, nn = 0;
-  if (d_in_place(plan, &nm, &nn)) t.d = (size_t)(plan.M + plan.N) * sizeof(int64_t);  // the C map
-  else if (plan.d_transpose) t.d = dbytes;
-  if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) {
+  if (route == kRouteCopies) {
+    if (plan.d_transpose && !plan.mat_d_in_place) t.d = dbytes;
+    t.s = direct_choose(dk, plan.M, plan.N, plan.K, plan.batch).part_bytes;
+  } else if (route == kRouteWide) {
+    if (plan.d_transpose) t.d = dbytes;
+  } else {
+    int nm = 0, nn = 0;
+    if (d_in_place(plan, &nm, &nn)) t.d = (size_t)(plan.M + plan.N) * sizeof(int64_t);  // the C map
+    else if (plan.d_transpose) t.d = dbytes;
     t.split = rt().split_method;
     t.w = gemm_split_workspace(t.split, plan.M, plan.N, plan.K);
-  } else {
-    t.s = gemm_tail_workspace(dk, plan.M, plan.N, plan.K, plan.batch);
   }
   return t;
 }
@@ -514,6 +576,17 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
                  void *D, const void *L, const void *R, const int *ddims, const int *ldims, const int *rdims,
                  const TtgtBuffers &tmp, hipStream_t s, hipEvent_t gemm_start, hipEvent_t gemm_end) {
   const bool cplx = (dk == C4 || dk == C8);
+  int lconj = (p.conj >> 1) & 1, rconj = (p.conj >> 2) & 1;
+  if (p.conj & 1) { lconj ^= 1; rconj ^= 1; }
+  if (!cplx) lconj = rconj = 0;
+  const Route route = tmp.split >= 0 ? kRouteSplit : plan_route(plan, dk);
+  if (route == kRouteDirect) {
+    if (gemm_start) (void)hipEventRecord(gemm_start, s);
+    if (launch_direct(dk, plan.direct, L, R, D, ar, cplx ? ai : 0.0, lconj, rconj, acc, tmp.s, tmp.s_bytes, s))
+      return TALSH_FAILURE;
+    if (gemm_end) (void)hipEventRecord(gemm_end, s);
+    return TALSH_SUCCESS;
+  }
   const void *X = plan.swap ? R : L, *Y = plan.swap ? L : R;
   const int *xd = plan.swap ? rdims : ldims, *yd = plan.swap ? ldims : rdims;
   const int xr = plan.swap ? p.rrank : p.lrank, yr = plan.swap ? p.lrank : p.rrank;
@@ -535,9 +608,9 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
     B = tmp.b;
   }
   int nm = 0, nn = 0;
-  const bool in_place = d_in_place(plan, &nm, &nn);
+  const bool in_place = route == kRouteCopies ? plan.mat_d_in_place : route == kRouteSplit && d_in_place(plan, &nm, &nn);
   const int64_t *cmap = nullptr;
-  if (in_place) {
+  if (route == kRouteSplit && in_place) {
     // D' dim t is D dim i with d_o2n[i] == t; its D stride is the product of the extents before i
     if (!tmp.d || (int)plan.d_o2n.size() != p.drank) return TALSH_FAILURE;
     OffsetMap map;
@@ -559,20 +632,20 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
       if (launch_offset_map(map, (int64_t *)tmp.d, s)) return TALSH_FAILURE;
       cmap = (const int64_t *)tmp.d;
     }
-  } else if (plan.d_transpose) {
+  } else if (plan.d_transpose && !in_place) {
     if (!tmp.d) return TALSH_FAILURE;
     C = tmp.d;
     if (acc && launch_permute(dk, D, C, p.drank, ddims, plan.d_o2n.data(), PERM_COPY, 1, 0, 0, s))
       return TALSH_FAILURE;
   }
-  int lconj = (p.conj >> 1) & 1, rconj = (p.conj >> 2) & 1;
-  if (p.conj & 1) { lconj ^= 1; rconj ^= 1; }
-  if (!cplx) lconj = rconj = 0;
+  const int aconj = plan.swap ? rconj : lconj, bconj = plan.swap ? lconj : rconj;
   if (gemm_start) (void)hipEventRecord(gemm_start, s);
-  const bool split = tmp.split >= 0;
   // hyper indices: plan.batch products of M x N x K, each operand strided by one matrix
   const int64_t sa = plan.M * plan.K, sb = plan.K * plan.N, sc = plan.M * plan.N;
-  if (split) {
+  if (route == kRouteCopies) {
+    if (launch_direct(dk, plan.mat, A, B, C, ar, cplx ? ai : 0.0, aconj, bconj, acc, tmp.s, tmp.s_bytes, s))
+      return TALSH_FAILURE;
+  } else if (route == kRouteSplit) {
     if (!tmp.w) return TALSH_FAILURE;
     for (int64_t q = 0; q < plan.batch; ++q)  // the planes workspace is reused in stream order
       if (launch_gemm_split(tmp.split, plan.a.op, plan.b.op, plan.M, plan.N, plan.K, ar,
@@ -580,9 +653,9 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
                             (const float *)B + q * sb, plan.b.ld, acc ? 1 : 0, (float *)C + q * sc,
                             std::max<int64_t>(1, plan.M), tmp.w, s, cmap))
         return TALSH_FAILURE;
-  } else if (launch_gemm(dk, R4_FP32, plan.a.op, plan.b.op, plan.swap ? rconj : lconj, plan.swap ? lconj : rconj,
-                         plan.M, plan.N, plan.K, ar, cplx ? ai : 0.0, A, plan.a.ld, B, plan.b.ld, acc ? 1 : 0, C,
-                         std::max<int64_t>(1, plan.M), s, plan.batch, sa, sb, sc, tmp.s, tmp.s_bytes, cmap)) {
+  } else if (launch_gemm(dk, plan.a.op, plan.b.op, aconj, bconj, plan.M, plan.N, plan.K, ar, cplx ? ai : 0.0, A,
+                         plan.a.ld, B, plan.b.ld, acc ? 1 : 0, C, std::max<int64_t>(1, plan.M), s, plan.batch, sa, sb,
+                         sc)) {
     return TALSH_FAILURE;
   }
   if (gemm_end) (void)hipEventRecord(gemm_end, s);
@@ -849,13 +922,14 @@ int talshTensorContract(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *lt
   // temporaries: [A'], [B'], [D'], [split-BF16 planes]
   const TtgtTemps tb = ttgt_temp_bytes(plan, dk, op.operand(1).bytes, op.operand(2).bytes, op.operand(0).bytes);
   std::vector<size_t> temps;
-  int ia = -1, ib = -1, id = -1, iw = -1, is = -1;
+  int ia = -1, ib = -1, id = -1, iw = -1;
   if (tb.a) { ia = (int)temps.size(); temps.push_back(tb.a); }
   if (tb.b) { ib = (int)temps.size(); temps.push_back(tb.b); }
   if (tb.d) { id = (int)temps.size(); temps.push_back(tb.d); }
   if (tb.w) { iw = (int)temps.size(); temps.push_back(tb.w); }
-  if (tb.s) { is = (int)temps.size(); temps.push_back(tb.s); }
   if (int e = op.acquire(temps)) return deferred(g, e);
+  // room for partial sums only helps: without it the product runs in whole tiles
+  const int is = tb.s ? op.acquire_optional(tb.s) : -1;
   if (int e = op.begin(dk, copy_ctrl)) return e;
   TtgtBuffers bufs;
   bufs.a = ia >= 0 ? op.temp(ia) : nullptr;
@@ -863,7 +937,7 @@ int talshTensorContract(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *lt
   bufs.d = id >= 0 ? op.temp(id) : nullptr;
   bufs.w = iw >= 0 ? op.temp(iw) : nullptr;
   bufs.s = is >= 0 ? op.temp(is) : nullptr;
-  bufs.s_bytes = tb.s;
+  bufs.s_bytes = is >= 0 ? tb.s : 0;
   bufs.split = tb.split;
   op.gemm_events();
   if (int e = enqueue_ttgt(p, plan, dk, acc, scale_real, scale_imag, op.operand(0).dptr, op.operand(1).dptr,

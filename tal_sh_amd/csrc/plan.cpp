@@ -209,6 +209,93 @@ int plan_contraction(const DigitalPattern &p, const int *ddims, const int *ldims
 
 namespace {
 
+// Strides by symbol of a tensor whose dimensions are `seq`, first fastest (0: symbol absent).
+std::vector<int64_t> seq_strides(const std::vector<int> &seq, const std::vector<int64_t> &ext, int nsym) {
+  std::vector<int64_t> s(nsym, 0);
+  int64_t a = 1;
+  for (int x : seq) {
+    s[x] = a;
+    a *= ext[x];
+  }
+  return s;
+}
+
+// The product straight from the tensors (A = L, B = R).  Rows of an input
+// that is contiguous along them are taken in its own order, so that its loads
+// run along memory; otherwise in D's.  Contracted indices follow the input
+// that is contiguous along one of them.
+template <class IsHyper>
+void make_direct(const ContractPlan &c, const std::vector<int> &sl, const std::vector<int> &sr,
+                 const std::vector<int> &sd, const std::vector<int> &hyper, const IsHyper &is_hyper,
+                 const std::vector<int64_t> &ext, const std::vector<int64_t> (&str)[3], ContractPlan *out) {
+  out->direct_ok = false;
+  auto first = [&](const std::vector<int> &seq) {
+    for (int x : seq)
+      if (ext[x] > 1) return x;
+    return -1;
+  };
+  auto contracted = [](int x) { return x >= kContr; };
+  auto by_stride = [&](std::vector<int> v, int t) {
+    std::sort(v.begin(), v.end(), [&](int x, int y) { return str[t][x] < str[t][y]; });
+    return v;
+  };
+  std::vector<int> m, n, k;
+  for (int x : sl)
+    if (ext[x] > 1 && !is_hyper(x)) (contracted(x) ? k : m).push_back(x);
+  for (int x : sr)
+    if (ext[x] > 1 && !is_hyper(x) && !contracted(x)) n.push_back(x);
+  const int fl = first(sl), fr = first(sr), fd = first(sd);
+  const bool kl = fl >= 0 && contracted(fl), kr = fr >= 0 && !is_hyper(fr) && std::find(k.begin(), k.end(), fr) != k.end();
+  DirectForm f;
+  f.M = c.swap ? c.N : c.M;
+  f.N = c.swap ? c.M : c.N;
+  f.K = c.K;
+  f.batch = c.batch;
+  for (int x : sl) f.avol = f.avol ? f.avol * ext[x] : ext[x];
+  for (int x : sr) f.bvol = f.bvol ? f.bvol * ext[x] : ext[x];
+  if (sl.empty()) f.avol = 1;
+  if (sr.empty()) f.bvol = 1;
+  out->direct_conflict = kl && kr && fl != fr;
+  if (kl && (!out->direct_conflict || f.avol >= f.bvol)) k = by_stride(k, 0);
+  else if (kr) k = by_stride(k, 1);
+  else {
+    // either order will do: the one with the longer leading run
+    const std::vector<int> l = by_stride(k, 0), r = by_stride(k, 1);
+    std::vector<DirectDim> dl, dr;
+    for (int x : l) direct_dim(&dl, ext[x], str[0][x], str[1][x]);
+    for (int x : r) direct_dim(&dr, ext[x], str[0][x], str[1][x]);
+    k = !dr.empty() && dr[0].ext > dl[0].ext ? r : l;
+  }
+  m = by_stride(m, kl ? 2 : 0);
+  n = by_stride(n, kr ? 2 : 1);
+  for (int x : m) direct_dim(&f.m, ext[x], str[0][x], str[2][x]);
+  for (int x : n) direct_dim(&f.n, ext[x], str[1][x], str[2][x]);
+  for (int x : k) direct_dim(&f.k, ext[x], str[0][x], str[1][x]);
+  // hyper indices: one batch stride per tensor
+  int64_t e = 1;
+  for (int x : hyper) {
+    if (ext[x] == 1) continue;
+    if (e == 1) {
+      f.sa = str[0][x];
+      f.sb = str[1][x];
+      f.sd = str[2][x];
+    } else if (str[0][x] != f.sa * e || str[1][x] != f.sb * e || str[2][x] != f.sd * e) {
+      return;
+    }
+    e *= ext[x];
+  }
+  // an input whose contiguous index is a hyper index has no run along rows or k
+  if ((fl >= 0 && is_hyper(fl)) || (fr >= 0 && is_hyper(fr))) return;
+  out->direct_krun = f.k.size() > 1 ? (int)std::min<int64_t>(f.k[0].ext, 1 << 30) : 0;
+  out->direct_scatter = fd >= 0 && !is_hyper(fd) && !(!f.m.empty() && f.m[0].s[1] == 1) && !(!f.n.empty() && f.n[0].s[1] == 1);
+  int64_t run = 0;
+  if (!kl && !f.m.empty()) run = f.m[0].ext;
+  if (!kr && !f.n.empty() && (run == 0 || f.n[0].ext < run)) run = f.n[0].ext;
+  out->direct_run = (int)std::min<int64_t>(run, 1 << 30);
+  out->direct = f;
+  out->direct_ok = true;
+}
+
 int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, const int *rdims, int accumulative,
                   ContractPlan *plan) {
   const int nd = p.drank, nl = p.lrank, nr = p.rrank;
@@ -269,6 +356,7 @@ int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, c
 
   bool have = false;
   ContractPlan best;
+  std::vector<int> best_m, best_n, best_k;
   int best_ntrans = 99;
   bool best_d0_first = false;
   for (int swap = 0; swap < 2; ++swap) {
@@ -356,6 +444,9 @@ int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, c
               (c.moved_elems == best.moved_elems &&
                (ntrans < best_ntrans || (ntrans == best_ntrans && d0_first && !best_d0_first)))) {
             best = c;
+            best_m = M;
+            best_n = N;
+            best_k = K;
             best_ntrans = ntrans;
             best_d0_first = d0_first;
             have = true;
@@ -366,6 +457,51 @@ int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, c
           (void)ydims;
         }
   }
+  // strides of every symbol in the tensors, and in the matrices the transposes leave
+  const int nsym = kContr + nl + 1;
+  std::vector<int64_t> str[3];
+  const std::vector<int> *seqs[3] = {&sl, &sr, &sd};
+  for (int t = 0; t < 3; ++t) str[t] = seq_strides(*seqs[t], ext_of, nsym);
+  make_direct(best, sl, sr, sd, hyper, is_hyper, ext_of, str, &best);
+  const std::vector<int> xt = cat(cat(best_k, best_m), hyper), xn = cat(cat(best_m, best_k), hyper);
+  const std::vector<int> yn = cat(cat(best_k, best_n), hyper), yt = cat(cat(best_n, best_k), hyper);
+  const std::vector<int64_t> ax = seq_strides(best.a.op == 'T' ? xt : xn, ext_of, nsym);
+  const std::vector<int64_t> by = seq_strides(best.b.op == 'N' ? yn : yt, ext_of, nsym);
+  std::vector<int64_t> dp = seq_strides(cat(cat(best_m, best_n), hyper), ext_of, nsym);
+  // D is written where it lies if it does not need D' at all, or if its
+  // contiguous index leads m or n with runs of at least 16 elements, or D is
+  // small enough to be put together in the L2 caches; hyper indices must chain
+  best.mat_d_in_place = false;
+  if (best.d_transpose) {
+    std::vector<DirectDim> m, n;
+    for (int x : best_m) direct_dim(&m, ext_of[x], ax[x], str[2][x]);
+    for (int x : best_n) direct_dim(&n, ext_of[x], by[x], str[2][x]);
+    int64_t run = 0;
+    for (const auto *g : {&m, &n})
+      if (!g->empty() && (*g)[0].s[1] == 1) run = (*g)[0].ext;
+    std::vector<DirectDim> h;
+    for (int x : hyper) direct_dim(&h, ext_of[x], ax[x], str[2][x]);
+    best.mat_d_in_place = (run >= 16 || vd <= 1048576) && h.size() <= 1;
+  }
+  const std::vector<int64_t> &ds = best.d_transpose && !best.mat_d_in_place ? dp : str[2];
+  DirectForm f;
+  f.M = best.M;
+  f.N = best.N;
+  f.K = best.K;
+  f.batch = best.batch;
+  for (int x : best_m) direct_dim(&f.m, ext_of[x], ax[x], ds[x]);
+  for (int x : best_n) direct_dim(&f.n, ext_of[x], by[x], ds[x]);
+  for (int x : best_k) direct_dim(&f.k, ext_of[x], ax[x], by[x]);
+  for (int x : hyper)
+    if (ext_of[x] > 1) {
+      f.sa = ax[x];
+      f.sb = by[x];
+      f.sd = ds[x];
+      break;
+    }
+  f.avol = (int64_t)(best.swap ? vr : vl);
+  f.bvol = (int64_t)(best.swap ? vl : vr);
+  best.mat = f;
   *plan = best;
   return 0;
 }

@@ -4,6 +4,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "direct_form.hpp"
+
 namespace tal {
 
 // Digital form of a symbolic pattern (TAL-SH convention, 1-based):
@@ -43,6 +45,19 @@ struct ContractPlan {
   std::vector<int> d_back_o2n;   // D' -> D
   std::vector<int> dprime_dims;  // extents of D' in its own order
   double moved_elems = 0;        // elements copied by the transposes
+  // The product as the direct kernels take it (direct.hpp), A = L and B = R:
+  // straight from the tensors, and of the operands as the transposes above
+  // leave them (A = L's copy where L is copied; D written in place where
+  // `mat_d_in_place`, else into D').
+  bool direct_ok = false;        // `direct` can be formed (hyper indices chain in all three tensors)
+  DirectForm direct, mat;
+  bool mat_d_in_place = false;
+  // what reading the tensors in place costs beside a plain product
+  bool direct_conflict = false;  // both inputs are contiguous along contracted indices, but not the same one:
+                                 // the smaller input is read in pieces of one element
+  int direct_krun = 0;           // extent of the contracted run the kernel walks (0: one run)
+  bool direct_scatter = false;   // D's contiguous index leads neither m nor n
+  int direct_run = 0;            // shortest contiguous run of an input along its rows (0: none is read along rows)
 };
 
 // Validates the pattern against the extents and picks the matricization that

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "contract.hpp"
+#include "direct.hpp"
 #include "plan.hpp"
 #include "runtime.hpp"
 #include "talsh_amd.h"
@@ -243,7 +244,7 @@ int talshTensorContractXL(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *
     for (int j = 0; j < p.rrank; ++j)
       if (rid[j] < nd) N *= t[rid[j]];
     if (dk == R4 && r.r4mode == R4_SPLIT_BF16) b += gemm_split_workspace(r.split_method, M, N, K);
-    else b += gemm_tail_workspace(dk, M, N, K, 1);
+    else b += direct_choose(dk, M, N, K, 1).part_bytes;
     return b;
   };
   size_t budget = dev.arena.largest_free() / 10 * 9;
