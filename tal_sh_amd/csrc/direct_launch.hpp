@@ -4,6 +4,7 @@
 
 #include "direct.hpp"
 #include "direct_kernel.hpp"
+#include "kernels.hpp"
 
 namespace tal {
 namespace direct {
@@ -17,13 +18,17 @@ struct Tile {
 
 template <typename S, int NC, class T, int KA, int KBC, int W, int MODE>
 void run(const DirectArgs &a, unsigned batch, hipStream_t s) {
-  direct_kernel<S, NC, KA, KBC, W, W, T::BM, T::BN, T::KB, T::WM, T::WN, T::PF, T::OCC, MODE>
-      <<<dim3((unsigned)(a.whole + a.rem * a.ksplit), batch), dim3(64 * T::WM * T::WN), 0, s>>>(a);
-  if (a.rem > 0) {
-    constexpr int kBlocks = (T::BM / 16) * (T::BN / 16);  // 16 x 16 blocks of a tile
-    direct_reduce<S, NC, T::BM, T::BN, T::WM, T::WN>
-        <<<dim3((unsigned)(((int64_t)a.rem * kBlocks + 3) / 4)), dim3(256), 0, s>>>(a);
+  const dim3 grid((unsigned)(a.whole + a.rem * a.ksplit), batch), block(64 * T::WM * T::WN);
+  constexpr auto kernel =
+      direct_kernel<S, NC, KA, KBC, W, W, T::BM, T::BN, T::KB, T::WM, T::WN, T::PF, T::OCC, MODE>;
+  if (a.rem == 0) {
+    launch_last(kernel, grid, block, s, a);
+    return;
   }
+  kernel<<<grid, block, 0, s>>>(a);
+  constexpr int kBlocks = (T::BM / 16) * (T::BN / 16);  // 16 x 16 blocks of a tile
+  launch_last(direct_reduce<S, NC, T::BM, T::BN, T::WM, T::WN>, dim3((unsigned)(((int64_t)a.rem * kBlocks + 3) / 4)),
+              dim3(256), s, a);
 }
 
 template <typename S, int NC, class T, int W, int MODE>

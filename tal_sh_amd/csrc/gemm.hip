@@ -833,21 +833,28 @@ static int launch_presplit(int opa, int opb, int64_t M, int64_t N, int64_t K, do
   const int64_t ksteps = ts.ksplit > 1 ? (nsteps + ts.ksplit - 1) / ts.ksplit : 0;
   const int64_t apl = l.Mp * l.Kp / 8, bpl = l.Np * l.Kp / 8;
   auto gemm = [&](int64_t blocks, int64_t t0, int64_t count, int ksplit, int64_t kst, float *pt) {
-    if (NP == 3)
-      gemm_bf16x6p_kernel<<<dim3((unsigned)blocks), dim3(512), 0, s>>>(
-          M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C, ldc, (float)ar, beta_one, gx, gy,
-          t0, count, ksplit, kst, pt, cmap);
+    const dim3 grid((unsigned)blocks), block(512);
+    const bool last = ts.ksplit <= 1;  // no other launch follows
+    if (NP == 3 && last)
+      launch_last(gemm_bf16x6p_kernel, grid, block, s, M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl,
+                  (float *)C, ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, cmap);
+    else if (NP == 3)
+      gemm_bf16x6p_kernel<<<grid, block, 0, s>>>(M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C,
+                                                 ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, cmap);
+    else if (last)
+      launch_last(gemm_f16x3p_kernel, grid, block, s, M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl,
+                  (float *)C, ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, ua, ub, cmap);
     else
-      gemm_f16x3p_kernel<<<dim3((unsigned)blocks), dim3(512), 0, s>>>(
-          M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C, ldc, (float)ar, beta_one, gx, gy,
-          t0, count, ksplit, kst, pt, ua, ub, cmap);
+      gemm_f16x3p_kernel<<<grid, block, 0, s>>>(M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C,
+                                                ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, ua, ub,
+                                                cmap);
   };
   if (full > 0) gemm(full, 0, full, 1, 0, nullptr);
   if (ts.ksplit > 1) {
     gemm(ts.rem * ts.ksplit, full, ts.rem, ts.ksplit, ksteps, part);
     const int64_t nel = ts.rem * PBM * PBN;
-    gemm_tail_reduce<float, 1, PBM, PBN><<<dim3((unsigned)((nel + kThreads - 1) / kThreads)), dim3(kThreads), 0, s>>>(
-        M, N, part, ts.ksplit, (float *)C, ldc, (float)ar, 0.0f, beta_one, gx, gy, full, ts.rem, cmap);
+    launch_last(gemm_tail_reduce<float, 1, PBM, PBN>, dim3((unsigned)((nel + kThreads - 1) / kThreads)), dim3(kThreads), s,
+                M, N, part, ts.ksplit, (float *)C, ldc, (float)ar, 0.0f, beta_one, gx, gy, full, ts.rem, cmap);
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -121,7 +121,10 @@ class Op {
 
   // Starts the task: stream, ordering against earlier work, input transfers.
   // clock: the kernels launched until end() carry dispatch timestamps, which
-  // talshTaskTime reports as the compute time.
+  // talshTaskTime reports as the compute time.  A blocking call has no handle
+  // to ask for times: it records none, its completion event goes onto its last
+  // kernel, and as it holds the runtime's lock until that event, no later
+  // operation has to be ordered against it.
   int begin(int data_kind, int coh_ctrl, bool clock = false) {
     Device &d = rt().gpus[g_];
     (void)hipSetDevice(d.hip_id);
@@ -135,7 +138,8 @@ class Op {
     for (size_t i = 0; i < temps_.size(); ++i) weight += 2.0 * (double)temp_bytes_[i] / 64.0;
     task_ = task_new(g_, weight);
     s_ = task_->stream;
-    (void)hipEventRecord(task_->ev_start->ev, s_);
+    task_->timed = user_ != nullptr;
+    if (task_->timed) (void)hipEventRecord(task_->ev_start->ev, s_);
     bool moved = false;
     for (auto &o : ops_) {
       if (o.resident) {
@@ -154,9 +158,12 @@ class Op {
     for (size_t i = 0; i < temps_.size(); ++i) hazard_wait_write(temps_[i], temp_bytes_[i], s_);
     // with no input transfer the input stage is empty: its end is the start
     // (one event record less on the launch path of a short task)
-    if (moved) (void)hipEventRecord(task_->ev_in->ev, s_);
+    if (moved && task_->timed) (void)hipEventRecord(task_->ev_in->ev, s_);
     else task_->ev_in = task_->ev_start;
-    if (clock) {
+    kernel_clock() = KernelClock();
+    if (!task_->timed) {
+      kernel_clock().done = task_->ev_done->ev;
+    } else if (clock) {
       task_->ev_k0 = new_event(g_);
       task_->ev_k1 = new_event(g_);
       KernelClock &c = kernel_clock();
@@ -173,22 +180,32 @@ class Op {
   hipStream_t stream() const { return s_; }
   Task *task() { return task_; }
 
-  // Events that bracket the GEMM (talshTaskTime's mmul); the enqueuer records them.
-  void gemm_events() {
-    task_->ev_mm0 = new_event(g_);
-    task_->ev_mm1 = new_event(g_);
+  // Events that bracket the GEMM (talshTaskTime's mmul); the enqueuer records
+  // the ones it is given.  Nothing before (after) the GEMM: the input stage's
+  // end (the task's) is its start (end).
+  void gemm_events(bool before, bool after) {
+    if (!task_->timed) return;
+    task_->ev_mm0 = before ? new_event(g_) : task_->ev_in;
+    bool back = after;
+    for (auto &o : ops_) back = back || copied_back(o);
+    task_->ev_mm1 = back ? new_event(g_) : task_->ev_done;
+    mm0_ = before ? task_->ev_mm0->ev : nullptr;
+    mm1_ = back ? task_->ev_mm1->ev : nullptr;
   }
+  hipEvent_t gemm_start() const { return mm0_; }
+  hipEvent_t gemm_end() const { return mm1_; }
 
   // Ends the task: output transfers, completion event, coherence bookkeeping.
   int end(double flops) {
     Device &d = rt().gpus[g_];
     KernelClock &clk = kernel_clock();
     task_->kclock = clk.on && clk.started;
+    const bool done_set = clk.done_set;
     clk = KernelClock();
     bool back = false;
     for (auto &o : ops_) back = back || copied_back(o);
     // likewise an empty output stage starts where the task ends
-    if (back) (void)hipEventRecord(task_->ev_comp->ev, s_);
+    if (back && task_->timed) (void)hipEventRecord(task_->ev_comp->ev, s_);
     else task_->ev_comp = task_->ev_done;
     for (auto &o : ops_) {
       if (copied_back(o)) {
@@ -198,18 +215,22 @@ class Op {
         d.traffic_out += (double)o.bytes;
       }
     }
-    (void)hipEventRecord(task_->ev_done->ev, s_);
+    if (back || !done_set) (void)hipEventRecord(task_->ev_done->ev, s_);
     if (hipGetLastError() != hipSuccess) return TALSH_FAILURE;
     // ordering state of every buffer touched; a non-resident output's source
     // image is written only when the result is copied back to it
-    for (auto &o : ops_) {
-      if (o.output) hazard_set_writer(o.dptr, o.bytes, task_->ev_done);
-      else hazard_add_reader(o.dptr, o.bytes, task_->ev_done);
-      if (o.resident) continue;
-      if (copied_back(o)) hazard_set_writer(o.src_p, o.bytes, task_->ev_done);
-      else hazard_add_reader(o.src_p, o.bytes, task_->ev_done);
+    if (task_->timed) {
+      for (auto &o : ops_) {
+        if (o.output) hazard_set_writer(o.dptr, o.bytes, task_->ev_done);
+        else hazard_add_reader(o.dptr, o.bytes, task_->ev_done);
+        if (o.resident) continue;
+        if (copied_back(o)) hazard_set_writer(o.src_p, o.bytes, task_->ev_done);
+        else hazard_add_reader(o.src_p, o.bytes, task_->ev_done);
+      }
+      for (size_t i = 0; i < temps_.size(); ++i) hazard_set_writer(temps_[i], temp_bytes_[i], task_->ev_done);
+    } else {
+      rt().hazard_epoch++;  // images may have moved
     }
-    for (size_t i = 0; i < temps_.size(); ++i) hazard_set_writer(temps_[i], temp_bytes_[i], task_->ev_done);
     // output images other than the source become stale
     for (auto &o : ops_)
       if (o.output) {
@@ -337,6 +358,7 @@ class Op {
   Task *task_ = nullptr;
   hipStream_t s_ = nullptr;
   bool committed_ = false;
+  hipEvent_t mm0_ = nullptr, mm1_ = nullptr;
   int data_kind_ = NO_TYPE, coh_ctrl_ = 0;
 };
 
@@ -587,6 +609,10 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
     if (gemm_end) (void)hipEventRecord(gemm_end, s);
     return TALSH_SUCCESS;
   }
+  // the completion event of a blocking call belongs to the last kernel only
+  KernelClock &clock = kernel_clock();
+  const hipEvent_t done = clock.done;
+  clock.done = nullptr;
   const void *X = plan.swap ? R : L, *Y = plan.swap ? L : R;
   const int *xd = plan.swap ? rdims : ldims, *yd = plan.swap ? ldims : rdims;
   const int xr = plan.swap ? p.rrank : p.lrank, yr = plan.swap ? p.lrank : p.rrank;
@@ -640,6 +666,8 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
   }
   const int aconj = plan.swap ? rconj : lconj, bconj = plan.swap ? lconj : rconj;
   if (gemm_start) (void)hipEventRecord(gemm_start, s);
+  const bool d_back = plan.d_transpose && !in_place;
+  if (!d_back) clock.done = done;
   // hyper indices: plan.batch products of M x N x K, each operand strided by one matrix
   const int64_t sa = plan.M * plan.K, sb = plan.K * plan.N, sc = plan.M * plan.N;
   if (route == kRouteCopies) {
@@ -659,7 +687,8 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
     return TALSH_FAILURE;
   }
   if (gemm_end) (void)hipEventRecord(gemm_end, s);
-  if (plan.d_transpose && !in_place &&
+  clock.done = done;
+  if (d_back &&
       launch_permute(dk, C, D, (int)plan.dprime_dims.size(), plan.dprime_dims.data(), plan.d_back_o2n.data(),
                      PERM_COPY, 1, 0, 0, s))
     return TALSH_FAILURE;
@@ -939,10 +968,10 @@ int talshTensorContract(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *lt
   bufs.s = is >= 0 ? op.temp(is) : nullptr;
   bufs.s_bytes = is >= 0 ? tb.s : 0;
   bufs.split = tb.split;
-  op.gemm_events();
+  op.gemm_events(tb.a || tb.b || tb.d, tb.d);
   if (int e = enqueue_ttgt(p, plan, dk, acc, scale_real, scale_imag, op.operand(0).dptr, op.operand(1).dptr,
                            op.operand(2).dptr, dtens->shape_p->dims, ltens->shape_p->dims, rtens->shape_p->dims,
-                           bufs, op.stream(), op.task()->ev_mm0->ev, op.task()->ev_mm1->ev))
+                           bufs, op.stream(), op.gemm_start(), op.gemm_end()))
     return e;
   const double flops = (cplx ? 8.0 : 2.0) * (double)plan.M * (double)plan.N * (double)plan.K * (double)plan.batch;
   if (int e = op.end(flops)) return e;

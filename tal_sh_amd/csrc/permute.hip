@@ -772,6 +772,7 @@ int launch_perm_typed(const T *src, T *dst, int rank, const int *dims, const int
   kc.started = false;
   kc.t0 = ev[0];
   kc.t1 = ev[1];
+  kc.done = nullptr;
   const int e = launch_plan(src, dst, pl, op, ar, ai, conj, s);
   kc = op_clock;
   if (op_clock.on) {
@@ -1137,9 +1138,9 @@ static int launch_norm2_typed(const T *x, size_t vol, double *partials, void *ou
   const int64_t packs = aligned ? n / VW : n;
   const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kNormBlocks, (packs + 4 * kThreads - 1) / (4 * kThreads)));
   if (aligned)
-    launch_clocked(norm2_stage1<T, VW>, dim3(nb), dim3(kThreads), s, x, n, partials);
+    launch_clocked<false>(norm2_stage1<T, VW>, dim3(nb), dim3(kThreads), s, x, n, partials);
   else
-    launch_clocked(norm2_stage1<T, 1>, dim3(nb), dim3(kThreads), s, x, n, partials);
+    launch_clocked<false>(norm2_stage1<T, 1>, dim3(nb), dim3(kThreads), s, x, n, partials);
   launch_clocked(norm2_stage2<T>, dim3(1), dim3(kThreads), s, partials, nb, (T *)out);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

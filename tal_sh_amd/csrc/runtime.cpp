@@ -387,7 +387,7 @@ int task_finalize(Task *t, bool block) {
     d.tasks_completed++;
     d.flops += t->flops;
     float ms = 0;
-    if (hipEventElapsedTime(&ms, t->ev_start->ev, t->ev_done->ev) == hipSuccess) t->exec_time = ms * 1e-3;
+    if (t->timed && hipEventElapsedTime(&ms, t->ev_start->ev, t->ev_done->ev) == hipSuccess) t->exec_time = ms * 1e-3;
   } else {
     t->status = TALSH_TASK_ERROR;
     t->error = (int)q;

@@ -94,6 +94,7 @@ struct Task {
   EvRef ev_start, ev_in, ev_comp, ev_done, ev_mm0, ev_mm1;
   EvRef ev_k0, ev_k1;   // dispatch timestamps of the first / last kernel (KernelClock)
   bool kclock = false;  // ev_k0 / ev_k1 were recorded
+  bool timed = true;    // ev_start ... were recorded (not for a blocking call, only ev_done is)
   int status = TALSH_TASK_EMPTY;
   int error = 0;  // HIP status of a failed task
   double flops = 0, bytes = 0, exec_time = 0;
