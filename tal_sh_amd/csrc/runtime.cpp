@@ -93,7 +93,13 @@ EvRef new_event(int g) {
   return h;
 }
 
-static bool ev_done(const EvRef &e) { return !e || !e->ev || hipEventQuery(e->ev) == hipSuccess; }
+// Events in the hazard table are recorded ones, so one that was found complete
+// stays so until its owner records it again (and clears the mark).
+static bool ev_done(const EvRef &e) {
+  if (!e || !e->ev || e->seen_done) return true;
+  e->seen_done = hipEventQuery(e->ev) == hipSuccess;
+  return e->seen_done;
+}
 
 namespace {
 
@@ -245,6 +251,7 @@ void host_free(void *p, int handle, size_t bytes) {
 // ------------------------------------------------------------------ images
 int image_add(talsh_tens_t *t, int dev_id, void *p, int buf_entry, int attached, int dk) {
   if (t->ndev >= t->dev_rsc_len) return -1;
+  rt().image_epoch++;
   const int i = t->ndev++;
   t->dev_rsc[i].dev_id = canonical_dev(dev_id);
   t->dev_rsc[i].gmem_p = p;
@@ -256,6 +263,7 @@ int image_add(talsh_tens_t *t, int dev_id, void *p, int buf_entry, int attached,
 }
 
 void image_release(talsh_dev_rsc_t *r, size_t bytes) {
+  rt().image_epoch++;
   if (r->gmem_p && !r->mem_attached) {
     const int g = gpu_index(r->dev_id);
     if (r->dev_id == DEV_HOST)
@@ -315,6 +323,17 @@ int tensor_healthy(const talsh_tens_t *t) {
 // launches and the short kernels of a small contraction).
 constexpr double kTaskOverheadBytes = 4.0e6;
 
+static bool backlog_empty(std::deque<std::pair<EvRef, double>> &q) {
+  while (!q.empty() && hipEventQuery(q.front().first->ev) != hipErrorNotReady) q.pop_front();
+  return q.empty();
+}
+
+bool device_idle(int g) {
+  bool idle = true;
+  for (auto &q : rt().gpus[g].backlog) idle = backlog_empty(q) && idle;
+  return idle;
+}
+
 Task *task_new(int g, double weight) {
   Task *t = new Task();
   t->dev = g;
@@ -325,7 +344,7 @@ Task *task_new(int g, double weight) {
   double best_w = 0.0;
   for (size_t i = 0; i < d.streams.size(); ++i) {
     auto &q = d.backlog[i];
-    while (!q.empty() && hipEventQuery(q.front().first->ev) != hipErrorNotReady) q.pop_front();
+    (void)backlog_empty(q);
     double w = 0.0;
     for (auto &e : q) w += e.second;
     if (i == 0 || w < best_w) {

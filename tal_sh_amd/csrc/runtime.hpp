@@ -24,6 +24,7 @@ namespace tal {
 struct EvHandle {
   int dev = -1;
   hipEvent_t ev = nullptr;
+  bool seen_done = false;  // found complete since it was last recorded (hazard table entries)
   ~EvHandle();
 };
 using EvRef = std::shared_ptr<EvHandle>;
@@ -82,6 +83,8 @@ struct Runtime {
   // bumped by every change of the hazard table: a caller that saw the same
   // value before knows every entry is still what it left there
   uint64_t hazard_epoch = 0;
+  // bumped whenever a tensor gains, loses or moves an image
+  uint64_t image_epoch = 0;
   std::recursive_mutex mu;
 };
 
@@ -120,6 +123,9 @@ void hazard_add_reader(const void *p, size_t n, const EvRef &e);
 void hazard_set_writer(const void *p, size_t n, const EvRef &e);
 void hazard_drain(const void *p, size_t n);  // blocks until all work on overlapping memory is done, forgets it
 size_t image_bytes(const talsh_tens_t *t, int i);  // bytes of image i's body
+
+// Whether nothing that was submitted to GPU g is still running (completed tasks are dropped from the backlog).
+bool device_idle(int g);
 
 // Device memory (buffer pool) and host memory (pinned pool, malloc fallback).
 int dev_alloc(int g, size_t bytes, void **p, int *handle);
