@@ -61,6 +61,7 @@ struct Device {
   long long tasks_submitted = 0, tasks_completed = 0, tasks_deferred = 0, tasks_failed = 0;
   double flops = 0, traffic_in = 0, traffic_out = 0, time_start = 0;
   int active = 0;
+  int unreaped = 0;  // blocking calls since their stream was last synchronized
 };
 
 struct Runtime {
