@@ -17,6 +17,7 @@
 // and the write side are full contiguous runs.  The elementwise add uses a
 // separately rounded multiply and add, matching the reference CPU path bit
 // for bit; copies are pure data movement.
+#include "batch_item.hpp"
 #include "kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -108,43 +109,54 @@ struct Real<double2> {
 // block moves kElems elements with all of its loads issued before any store.
 // NO: capacity for outer dims (a launch of two permutations packs both
 // argument sets into the kernel arguments, so it uses a short form).
+//
+// The block index is taken apart with 32-bit multiply-high divisions by
+// divisors prepared on the host (64-bit divisions take some 150 scalar
+// instructions each, up to two per dimension and block), and within a block
+// every access of a thread is its first one plus a multiple of the strides
+// that is the same for the whole block.  Both are worth 1-3 % (16^6 R8
+// reversal 58.5 -> 57 us, 83x83x41x41 R4 adds 47.4 -> 46.0): the transposes
+// are bound by how they touch memory, not by their arithmetic.
+struct PermOuter {
+  uint32_t e, mg, sh, pad;  // extent and its divider
+  int64_t is, os;           // input and output strides
+};
 template <int NO>
 struct PermArgsT {
   int nouter;
+  int tc;                      // tile size along c (<= TCMAX of the kernel)
+  int tb_log;                  // row mode: log2 of the tile size along b
+  uint32_t nta, mga, sha;      // tiles along a, b and c, with dividers
+  uint32_t ntb, mgb, shb;
+  uint32_t ntc, mgc, shc;
   int64_t ea, eb, ec;          // tile-dim extents
   int64_t isb, isc;            // input strides of b and c (a has stride 1)
   int64_t osa, osb, osc;       // output strides of a, b, c
-  int64_t ntile_a, ntile_b, ntile_c;
-  int tc;                      // tile size along c (<= TCMAX of the kernel)
-  int tb_log;                  // row mode: log2 of the tile size along b
-  int64_t oe[NO];              // outer extents
-  int64_t ois[NO];             // outer input strides
-  int64_t oos[NO];             // outer output strides
+  PermOuter o[NO];             // outer dims
 };
 using PermArgs = PermArgsT<kMaxRank>;
 constexpr int kPairOuter = 6;
 
 template <class PA>
-__device__ inline void tile_origin(const PA &p, int64_t blk, int TA, int TB, int64_t &a0, int64_t &b0,
+__device__ inline void tile_origin(const PA &p, uint32_t blk, int TA, int TB, int64_t &a0, int64_t &b0,
                                    int64_t &c0, int64_t &ib, int64_t &ob) {
-  int64_t t = blk % p.ntile_a;
-  blk /= p.ntile_a;
-  a0 = t * TA;
-  t = blk % p.ntile_b;
-  blk /= p.ntile_b;
-  b0 = t * TB;
-  t = blk % p.ntile_c;
-  blk /= p.ntile_c;
-  c0 = t * p.tc;
+  uint32_t q = divide(blk, p.mga, p.sha);
+  a0 = (int64_t)(blk - q * p.nta) * TA;
+  blk = q;
+  q = divide(blk, p.mgb, p.shb);
+  b0 = (int64_t)(blk - q * p.ntb) * TB;
+  blk = q;
+  q = divide(blk, p.mgc, p.shc);
+  c0 = (int64_t)(blk - q * p.ntc) * p.tc;
+  blk = q;
   ib = a0 + b0 * p.isb + c0 * p.isc;
   ob = a0 * p.osa + b0 * p.osb + c0 * p.osc;
   for (int k = 0; k < p.nouter; ++k) {
-    const int64_t e = p.oe[k];
-    const int64_t q = blk / e;
-    const int64_t r = blk - q * e;
+    q = divide(blk, p.o[k].mg, p.o[k].sh);
+    const uint32_t r = blk - q * p.o[k].e;
     blk = q;
-    ib += r * p.ois[k];
-    ob += r * p.oos[k];
+    ib += (int64_t)r * p.o[k].is;
+    ob += (int64_t)r * p.o[k].os;
   }
 }
 
@@ -215,26 +227,28 @@ __device__ inline void emit(T *o, Pack<T, V> x, typename Real<T>::type ar, typen
 // chosen at launch (p.tb_log) to fit the extent of b, so a small b does not
 // leave most of the block idle; c takes the rest of the block.
 template <typename T, int TA, int V, int OP, class PA>
-__device__ inline void perm_rows_body(const T *__restrict__ src, T *__restrict__ dst, const PA &p, int64_t blk,
+__device__ inline void perm_rows_body(const T *__restrict__ src, T *__restrict__ dst, const PA &p, uint32_t blk,
                                       typename Real<T>::type ar, typename Real<T>::type ai, int conj) {
-  constexpr int EPB = elems_per_block<T>(), N = EPB / kThreads / V, AV = TA / V;
+  constexpr int EPB = elems_per_block<T>(), N = EPB / kThreads / V, AV = TA / V, LINES = kThreads / AV;
   const int tbl = p.tb_log, tb = 1 << tbl;
   int64_t a0, b0, c0, ib, ob;
   tile_origin(p, blk, TA, tb, a0, b0, c0, ib, ob);
   const int na = (int)min<int64_t>(TA, p.ea - a0), nb = (int)min<int64_t>(tb, p.eb - b0);
   const int nc = (int)min<int64_t>(p.tc, p.ec - c0);
+  // the block's lines (b, c) in order: line l is b = l % tb, c = l / tb
+  const int ia = (threadIdx.x % AV) * V, l0 = threadIdx.x / AV;
+  src += ib + ia;
+  dst += ob + ia;
   Pack<T, V> v[N];
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    const int u = threadIdx.x + q * kThreads;
-    const int ia = (u % AV) * V, jb = (u / AV) & (tb - 1), kc = (u / AV) >> tbl;
-    if (ia < na && jb < nb && kc < nc) v[q] = ldv<T, V>(src + ib + ia + jb * p.isb + kc * p.isc);
+    const int l = l0 + q * LINES, jb = l & (tb - 1), kc = l >> tbl;
+    if (ia < na && jb < nb && kc < nc) v[q] = ldv<T, V>(src + jb * p.isb + kc * p.isc);
   }
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    const int u = threadIdx.x + q * kThreads;
-    const int ia = (u % AV) * V, jb = (u / AV) & (tb - 1), kc = (u / AV) >> tbl;
-    if (ia < na && jb < nb && kc < nc) emit<T, V, OP>(dst + ob + ia + jb * p.osb + kc * p.osc, v[q], ar, ai, conj);
+    const int l = l0 + q * LINES, jb = l & (tb - 1), kc = l >> tbl;
+    if (ia < na && jb < nb && kc < nc) emit<T, V, OP>(dst + jb * p.osb + kc * p.osc, v[q], ar, ai, conj);
   }
 }
 template <typename T, int TA, int V, int OP>
@@ -244,49 +258,84 @@ __global__ __launch_bounds__(kThreads) void perm_rows_kernel(const T *__restrict
   perm_rows_body<T, TA, V, OP>(src, dst, p, blockIdx.x, ar, ai, conj);
 }
 
+// Offset of line l0 + q * LINES of a tile's lines (i fast with extent E, k
+// slow) as the offset of line l0 plus a block-uniform multiple of the strides:
+// either LINES is a multiple of E (the lines step along k only) or E of LINES.
+template <int E, int LINES>
+__device__ inline int64_t line_step(int q, int64_t si, int64_t sk) {
+  if constexpr (LINES >= E) return q * (LINES / E) * sk;
+  else return (q % (E / LINES)) * LINES * si + (q / (E / LINES)) * sk;
+}
+
+// Threads and elements of one block of a tile problem.  The wide tiles serve
+// element accesses, whose runs start anywhere: see plan_perm.
+template <int TB>
+constexpr int tile_threads() {
+  return TB == 128 ? 512 : kThreads;
+}
+template <typename T, int TB>
+constexpr int tile_elems() {
+  return TB == 128 ? 4096 : TB == 64 ? 2048 : elems_per_block<T>();
+}
+
 // Tile mode: stage a (a x b x c) tile through LDS (+1 pad on the a axis) so
 // the reads run along a and the writes along b, V elements per access on
 // both sides (the host guarantees V | extents of a and b when V > 1).
 template <typename T, int TA, int TB, int V, int OP, class PA>
-__device__ inline void perm_tile_body(const T *__restrict__ src, T *__restrict__ dst, const PA &p, int64_t blk,
+__device__ inline void perm_tile_body(const T *__restrict__ src, T *__restrict__ dst, const PA &p, uint32_t blk,
                                       typename Real<T>::type ar, typename Real<T>::type ai, int conj) {
-  constexpr int EPB = elems_per_block<T>(), N = EPB / kThreads / V, TCMAX = EPB / (TA * TB);
+  constexpr int EPB = tile_elems<T, TB>(), NT = tile_threads<TB>();
+  constexpr int N = EPB / NT / V, TCMAX = EPB / (TA * TB);
   constexpr int AV = TA / V, BV = TB / V;
+  constexpr int AL = NT / AV, BL = NT / BV;  // lines per round of the block, reading and writing
   __shared__ T tile[TCMAX][TB][TA + 1];
   int64_t a0, b0, c0, ib, ob;
   tile_origin(p, blk, TA, TB, a0, b0, c0, ib, ob);
   const int na = (int)min<int64_t>(TA, p.ea - a0), nb = (int)min<int64_t>(TB, p.eb - b0);
   const int nc = (int)min<int64_t>(p.tc, p.ec - c0);
   Pack<T, V> v[N];
+  {
+    const int ia = (threadIdx.x % AV) * V, l0 = threadIdx.x / AV;  // lines: b fast, c slow
+    const T *s = src + ib + ia + (l0 % TB) * p.isb + (l0 / TB) * p.isc;
 #pragma unroll
-  for (int q = 0; q < N; ++q) {
-    const int u = threadIdx.x + q * kThreads;
-    const int ia = (u % AV) * V, jb = (u / AV) % TB, kc = u / (AV * TB);
-    if (ia < na && jb < nb && kc < nc) v[q] = ldv<T, V>(src + ib + ia + jb * p.isb + kc * p.isc);
+    for (int q = 0; q < N; ++q) {
+      const int l = l0 + q * AL, jb = l % TB, kc = l / TB;
+      if (ia < na && jb < nb && kc < nc) v[q] = ldv<T, V>(s + line_step<TB, AL>(q, p.isb, p.isc));
+    }
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const int l = l0 + q * AL, jb = l % TB, kc = l / TB;
+      if (ia < na && jb < nb && kc < nc)
+#pragma unroll
+        for (int t = 0; t < V; ++t) tile[kc][jb][ia + t] = v[q].v[t];
+    }
   }
+  const int jb = (threadIdx.x % BV) * V, l0 = threadIdx.x / BV;  // lines: a fast, c slow
+  T *d = dst + ob + jb + (l0 % TA) * p.osa + (l0 / TA) * p.osc;
+  if constexpr (OP == PERM_ADD) {  // the old values are read in one go too, before any store
 #pragma unroll
-  for (int q = 0; q < N; ++q) {
-    const int u = threadIdx.x + q * kThreads;
-    const int ia = (u % AV) * V, jb = (u / AV) % TB, kc = u / (AV * TB);
-    if (ia < na && jb < nb && kc < nc)
-#pragma unroll
-      for (int t = 0; t < V; ++t) tile[kc][jb][ia + t] = v[q].v[t];
+    for (int q = 0; q < N; ++q) {
+      const int l = l0 + q * BL, ia = l % TA, kc = l / TA;
+      if (ia < na && jb < nb && kc < nc) v[q] = ldv<T, V>(d + line_step<TA, BL>(q, p.osa, p.osc));
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    const int u = threadIdx.x + q * kThreads;
-    const int jb = (u % BV) * V, ia = (u / BV) % TA, kc = u / (BV * TA);
+    const int l = l0 + q * BL, ia = l % TA, kc = l / TA;
     if (ia < na && jb < nb && kc < nc) {
       Pack<T, V> x;
 #pragma unroll
-      for (int t = 0; t < V; ++t) x.v[t] = tile[kc][jb + t][ia];
-      emit<T, V, OP>(dst + ob + jb + ia * p.osa + kc * p.osc, x, ar, ai, conj);
+      for (int t = 0; t < V; ++t) x.v[t] = Elem<T>::conj(tile[kc][jb + t][ia], conj);
+      if constexpr (OP == PERM_ADD)
+#pragma unroll
+        for (int t = 0; t < V; ++t) x.v[t] = Elem<T>::axpy(v[q].v[t], x.v[t], ar, ai);
+      stv<T, V>(d + line_step<TA, BL>(q, p.osa, p.osc), x);
     }
   }
 }
 template <typename T, int TA, int TB, int V, int OP>
-__global__ __launch_bounds__(kThreads) void perm_tile_kernel(const T *__restrict__ src, T *__restrict__ dst,
+__global__ __launch_bounds__(tile_threads<TB>()) void perm_tile_kernel(const T *__restrict__ src, T *__restrict__ dst,
                                                              PermArgs p, typename Real<T>::type ar,
                                                              typename Real<T>::type ai, int conj) {
   perm_tile_body<T, TA, TB, V, OP>(src, dst, p, blockIdx.x, ar, ai, conj);
@@ -301,12 +350,12 @@ struct PermPair {
   const T *src[2];
   T *dst[2];
   PermArgsT<kPairOuter> p[2];
-  int64_t nblk0;
+  uint32_t nblk0;
 };
 template <typename T, int TA, int TB, int V, bool ROWS>
-__global__ __launch_bounds__(kThreads) void perm_pair_kernel(PermPair<T> q) {
+__global__ __launch_bounds__(tile_threads<TB>()) void perm_pair_kernel(PermPair<T> q) {
   using R = typename Real<T>::type;
-  const int64_t b = blockIdx.x;
+  const uint32_t b = blockIdx.x;
   if constexpr (ROWS) {
     if (b < q.nblk0) perm_rows_body<T, TA, V, PERM_COPY>(q.src[0], q.dst[0], q.p[0], b, (R)1, (R)0, 0);
     else perm_rows_body<T, TA, V, PERM_COPY>(q.src[1], q.dst[1], q.p[1], b - q.nblk0, (R)1, (R)0, 0);
@@ -338,19 +387,30 @@ __global__ __launch_bounds__(kThreads) void perm_flat_kernel(const T *__restrict
     emit<T, 1, OP>(dst + e, ldv<T, 1>(src + e), ar, ai, conj);
 }
 
-template <typename T>
+// One V-wide access per thread (16 bytes on aligned bodies), the remainder by
+// element: element accesses ran 3.4 TB/s (init) and 4.6 TB/s (scale) on a
+// 46 MB R4 tensor, 5.0 and 6.1 TB/s now.
+template <typename T, int V>
 __global__ __launch_bounds__(kThreads) void init_kernel(T *__restrict__ d, int64_t n, T v) {
-  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (; i < n; i += stride) d[i] = v;
+  const int64_t nvec = n / V, stride = (int64_t)gridDim.x * kThreads, t0 = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  Pack<T, V> x;
+#pragma unroll
+  for (int t = 0; t < V; ++t) x.v[t] = v;
+  for (int64_t i = t0; i < nvec; i += stride) stv<T, V>(d + i * V, x);
+  for (int64_t e = nvec * V + t0; e < n; e += stride) d[e] = v;
 }
 
-template <typename T>
+template <typename T, int V>
 __global__ __launch_bounds__(kThreads) void scale_kernel(T *__restrict__ d, int64_t n, typename Real<T>::type ar,
                                                          typename Real<T>::type ai) {
-  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (; i < n; i += stride) d[i] = Elem<T>::scale(d[i], ar, ai);
+  const int64_t nvec = n / V, stride = (int64_t)gridDim.x * kThreads, t0 = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  for (int64_t i = t0; i < nvec; i += stride) {
+    Pack<T, V> x = ldv<T, V>(d + i * V);
+#pragma unroll
+    for (int t = 0; t < V; ++t) x.v[t] = Elem<T>::scale(x.v[t], ar, ai);
+    stv<T, V>(d + i * V, x);
+  }
+  for (int64_t e = nvec * V + t0; e < n; e += stride) d[e] = Elem<T>::scale(d[e], ar, ai);
 }
 
 // ------------------------------------------------------------------ norm2
@@ -444,10 +504,10 @@ template <typename T, int TA, int TB, int V>
 void launch_tile(const T *src, T *dst, const PermArgs &p, int op, typename Real<T>::type ar,
                  typename Real<T>::type ai, int conj, int64_t nblk, hipStream_t s) {
   if (op == PERM_COPY)
-    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_COPY>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p, ar, ai,
+    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_COPY>, dim3((unsigned)nblk), dim3(tile_threads<TB>()), s, src, dst, p, ar, ai,
                                                                                               conj);
   else
-    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_ADD>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p, ar, ai,
+    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_ADD>, dim3((unsigned)nblk), dim3(tile_threads<TB>()), s, src, dst, p, ar, ai,
                                                                                              conj);
 }
 
@@ -565,35 +625,56 @@ int plan_perm(const T *src, T *dst, int rank, const int *dims, const int *o2n, P
     if (k != b && k != c) outer.push_back(k);
   if (variant == 2) std::stable_sort(outer.begin(), outer.end(), [&](int x, int y) { return fos[x] < fos[y]; });
   for (int k : outer) {
-    p.oe[p.nouter] = fe[k];
-    p.ois[p.nouter] = fis[k];
-    p.oos[p.nouter] = fos[k];
-    p.nouter++;
+    if (fe[k] > 0x7fffffffLL) return -4;
+    const Divider dv = make_divider((uint32_t)fe[k]);
+    p.o[p.nouter++] = PermOuter{(uint32_t)fe[k], dv.magic, dv.shift, 0, fis[k], fos[k]};
     nouter_vol *= fe[k];
   }
-  constexpr int EPB = elems_per_block<T>();
+  // vector accesses need V | extent on each contiguous side (so every other
+  // stride is a multiple of V) and 16-byte aligned bodies
+  const bool vec = aligned && (p.ea % VW == 0) && (rows || p.eb % VW == 0) && VW > 1;
+  int epb = elems_per_block<T>();
   int ta, tb;
   if (rows) {
     ta = p.ea >= 64 ? 64 : p.ea >= 32 ? 32 : p.ea >= 16 ? 16 : 8;
     // b: the smallest power of two covering its extent, within the block
     p.tb_log = 0;
-    while ((1 << p.tb_log) < p.eb && (ta << (p.tb_log + 1)) <= EPB) ++p.tb_log;
+    while ((1 << p.tb_log) < p.eb && (ta << (p.tb_log + 1)) <= epb) ++p.tb_log;
     tb = 1 << p.tb_log;
   } else {
     const int64_t m = std::min(p.ea, p.eb);
     if (m >= 24) { ta = 32; tb = 32; }
     else if (m >= 12) { ta = 16; tb = 16; }
     else { ta = 8; tb = 8; }
+    // Without vector accesses the written runs start at any element, and each
+    // partial cache line at the two ends of a run is written twice, so longer
+    // runs are worth lanes that fall off the end: 128 elements where b has
+    // more than 64, unless two 64-wide tiles cover it with a fifth fewer.
+    // Measured with 32x32, 32x64 and 32x128 tiles, us: 1681 x 6889 R4 adds
+    // 45/37/33 (copies 30/26/24), 83x83x41x41 with 83 swapped 46/41/33
+    // (29/27/22), b of 41 in a 83x41x83x41 reversal 54/44/53 (36/31/37), of 59
+    // 39/30/31 (22/18/24); 8-byte copies 55/48/45, 54/53/38, 61/53/54 and
+    // 52/41/41, their adds 1-17 % faster.  With 16-byte elements a run is long
+    // already and the three are within 3 %.
+    if (ta == 32 && !vec && sizeof(T) <= 8 && p.eb > 32) {
+      const int64_t w64 = (p.eb + 63) / 64 * 64, w128 = (p.eb + 127) / 128 * 128;
+      tb = p.eb > 64 && w128 * 4 <= w64 * 5 ? 128 : 64;
+      epb = tb == 128 ? tile_elems<T, 128>() : tile_elems<T, 64>();
+    }
   }
-  p.tc = (int)std::min<int64_t>(p.ec, EPB / (ta * tb));
-  p.ntile_a = (p.ea + ta - 1) / ta;
-  p.ntile_b = (p.eb + tb - 1) / tb;
-  p.ntile_c = (p.ec + p.tc - 1) / p.tc;
-  const int64_t nblk = p.ntile_a * p.ntile_b * p.ntile_c * nouter_vol;
+  p.tc = (int)std::min<int64_t>(p.ec, epb / (ta * tb));
+  const int64_t nta = (p.ea + ta - 1) / ta, ntb = (p.eb + tb - 1) / tb, ntc = (p.ec + p.tc - 1) / p.tc;
+  const int64_t nblk = nta * ntb * ntc * nouter_vol;
   if (nblk <= 0 || nblk > 0x7fffffffLL) return -4;
-  // vector accesses need V | extent on each contiguous side (so every other
-  // stride is a multiple of V) and 16-byte aligned bodies
-  const bool vec = aligned && (p.ea % VW == 0) && (rows || p.eb % VW == 0) && VW > 1;
+  auto tiles = [](int64_t n, uint32_t *nt, uint32_t *mg, uint32_t *sh) {
+    const Divider dv = make_divider((uint32_t)n);
+    *nt = (uint32_t)n;
+    *mg = dv.magic;
+    *sh = dv.shift;
+  };
+  tiles(nta, &p.nta, &p.mga, &p.sha);
+  tiles(ntb, &p.ntb, &p.mgb, &p.shb);
+  tiles(ntc, &p.ntc, &p.mgc, &p.shc);
   pl->mode = rows ? 2 : 3;
   pl->ta = ta;
   pl->tb = tb;
@@ -641,7 +722,12 @@ int launch_plan(const T *src, T *dst, const PermPlan &pl, int op, double ar_, do
 #define TAL_TILE(A, B)                                                         \
   (vec ? launch_tile<T, A, B, VW>(src, dst, p, op, ar, ai, conj, nblk, s)      \
        : launch_tile<T, A, B, 1>(src, dst, p, op, ar, ai, conj, nblk, s))
-    if (ta == 32) TAL_TILE(32, 32);
+    if constexpr (sizeof(T) <= 8) {
+      if (pl.tb == 128) launch_tile<T, 32, 128, 1>(src, dst, p, op, ar, ai, conj, nblk, s);
+      else if (pl.tb == 64) launch_tile<T, 32, 64, 1>(src, dst, p, op, ar, ai, conj, nblk, s);
+    }
+    if (pl.tb > 32) {}
+    else if (ta == 32) TAL_TILE(32, 32);
     else if (ta == 16) TAL_TILE(16, 16);
     else TAL_TILE(8, 8);
 #undef TAL_TILE
@@ -784,7 +870,7 @@ int launch_perm_typed(const T *src, T *dst, int rank, const int *dims, const int
 
 template <typename T, int TA, int TB, int V, bool ROWS>
 void launch_pair(const PermPair<T> &q, int64_t nblk, hipStream_t s) {
-  launch_clocked(perm_pair_kernel<T, TA, TB, V, ROWS>, dim3((unsigned)nblk), dim3(kThreads), s, q);
+  launch_clocked(perm_pair_kernel<T, TA, TB, V, ROWS>, dim3((unsigned)nblk), dim3(tile_threads<TB>()), s, q);
 }
 
 // Two permutation copies: one launch when both take the same kernel (row or
@@ -808,23 +894,21 @@ int launch_perm_pair_typed(const T *src0, T *dst0, int rank0, const int *dims0, 
   q.dst[0] = dst0;
   q.src[1] = src1;
   q.dst[1] = dst1;
-  q.nblk0 = a.nblk;
+  q.nblk0 = (uint32_t)a.nblk;
   const PermPlan *pl[2] = {&a, &b};
   for (int j = 0; j < 2; ++j) {
     const PermArgs &x = pl[j]->p;
     auto &y = q.p[j];
     y.nouter = x.nouter;
+    y.tc = x.tc;
+    y.tb_log = x.tb_log;
+    y.nta = x.nta, y.mga = x.mga, y.sha = x.sha;
+    y.ntb = x.ntb, y.mgb = x.mgb, y.shb = x.shb;
+    y.ntc = x.ntc, y.mgc = x.mgc, y.shc = x.shc;
     y.ea = x.ea, y.eb = x.eb, y.ec = x.ec;
     y.isb = x.isb, y.isc = x.isc;
     y.osa = x.osa, y.osb = x.osb, y.osc = x.osc;
-    y.ntile_a = x.ntile_a, y.ntile_b = x.ntile_b, y.ntile_c = x.ntile_c;
-    y.tc = x.tc;
-    y.tb_log = x.tb_log;
-    for (int k = 0; k < x.nouter; ++k) {
-      y.oe[k] = x.oe[k];
-      y.ois[k] = x.ois[k];
-      y.oos[k] = x.oos[k];
-    }
+    for (int k = 0; k < x.nouter; ++k) y.o[k] = x.o[k];
   }
   constexpr int VW = vec_width<T>();
   const int64_t n = a.nblk + b.nblk;
@@ -839,7 +923,12 @@ int launch_perm_pair_typed(const T *src0, T *dst0, int rank0, const int *dims0, 
   } else {
 #define TAL_PAIR_TILE(A) \
   (a.vec ? launch_pair<T, A, A, VW, false>(q, n, s) : launch_pair<T, A, A, 1, false>(q, n, s))
-    if (a.ta == 32) TAL_PAIR_TILE(32);
+    if constexpr (sizeof(T) <= 8) {
+      if (a.tb == 128) launch_pair<T, 32, 128, 1, false>(q, n, s);
+      else if (a.tb == 64) launch_pair<T, 32, 64, 1, false>(q, n, s);
+    }
+    if (a.tb > 32) {}
+    else if (a.ta == 32) TAL_PAIR_TILE(32);
     else if (a.ta == 16) TAL_PAIR_TILE(16);
     else TAL_PAIR_TILE(8);
 #undef TAL_PAIR_TILE
@@ -1070,29 +1159,48 @@ int launch_slice(int dk, int mode, const void *src, void *dst, int rank, const i
   }
 }
 
+template <typename T>
+static void launch_init_typed(T *d, int64_t n, T v, hipStream_t s) {
+  constexpr int VW = vec_width<T>();
+  if (VW > 1 && (uintptr_t)d % 16 == 0)
+    launch_clocked(init_kernel<T, VW>, dim3(grid_for(n / VW)), dim3(kThreads), s, d, n, v);
+  else
+    launch_clocked(init_kernel<T, 1>, dim3(grid_for(n)), dim3(kThreads), s, d, n, v);
+}
+
 int launch_init(int dk, void *d, size_t vol, double vr, double vi, hipStream_t s) {
   if (!d) return -1;
   if (vol == 0) return 0;
-  const int g = grid_for((int64_t)vol);
+  const int64_t n = (int64_t)vol;
   switch (dk) {
-    case 4: launch_clocked(init_kernel<float>, dim3(g), dim3(kThreads), s, (float *)d, vol, make_val<float>(vr, vi)); break;
-    case 8: launch_clocked(init_kernel<double>, dim3(g), dim3(kThreads), s, (double *)d, vol, make_val<double>(vr, vi)); break;
-    case 14: launch_clocked(init_kernel<float2>, dim3(g), dim3(kThreads), s, (float2 *)d, vol, make_val<float2>(vr, vi)); break;
-    case 18: launch_clocked(init_kernel<double2>, dim3(g), dim3(kThreads), s, (double2 *)d, vol, make_val<double2>(vr, vi)); break;
+    case 4: launch_init_typed((float *)d, n, make_val<float>(vr, vi), s); break;
+    case 8: launch_init_typed((double *)d, n, make_val<double>(vr, vi), s); break;
+    case 14: launch_init_typed((float2 *)d, n, make_val<float2>(vr, vi), s); break;
+    case 18: launch_init_typed((double2 *)d, n, make_val<double2>(vr, vi), s); break;
     default: return -1;
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+template <typename T>
+static void launch_scale_typed(T *d, int64_t n, double ar, double ai, hipStream_t s) {
+  using R = typename Real<T>::type;
+  constexpr int VW = vec_width<T>();
+  if (VW > 1 && (uintptr_t)d % 16 == 0)
+    launch_clocked(scale_kernel<T, VW>, dim3(grid_for(n / VW)), dim3(kThreads), s, d, n, (R)ar, (R)ai);
+  else
+    launch_clocked(scale_kernel<T, 1>, dim3(grid_for(n)), dim3(kThreads), s, d, n, (R)ar, (R)ai);
+}
+
 int launch_scale(int dk, void *d, size_t vol, double ar, double ai, hipStream_t s) {
   if (!d) return -1;
   if (vol == 0) return 0;
-  const int g = grid_for((int64_t)vol);
+  const int64_t n = (int64_t)vol;
   switch (dk) {
-    case 4: launch_clocked(scale_kernel<float>, dim3(g), dim3(kThreads), s, (float *)d, vol, (float)ar, (float)ai); break;
-    case 8: launch_clocked(scale_kernel<double>, dim3(g), dim3(kThreads), s, (double *)d, vol, ar, ai); break;
-    case 14: launch_clocked(scale_kernel<float2>, dim3(g), dim3(kThreads), s, (float2 *)d, vol, (float)ar, (float)ai); break;
-    case 18: launch_clocked(scale_kernel<double2>, dim3(g), dim3(kThreads), s, (double2 *)d, vol, ar, ai); break;
+    case 4: launch_scale_typed((float *)d, n, ar, ai, s); break;
+    case 8: launch_scale_typed((double *)d, n, ar, ai, s); break;
+    case 14: launch_scale_typed((float2 *)d, n, ar, ai, s); break;
+    case 18: launch_scale_typed((double2 *)d, n, ar, ai, s); break;
     default: return -1;
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
