@@ -17,6 +17,13 @@
 // tasks one TTGT schedule (up to 4 transposes + a GEMM launch) at a time
 // (tensor_algebra_gpu_nvidia.cu:5847-7188).
 //
+// What bounds it: 4,096 FP64 contractions of ranks 2-4 (0.70 GB of operands,
+// 0.33 GB of D) take 0.40 ms, 3.1 TB/s of 4.8 for a copy: the address unit is
+// busy 63 % of the time (17 lines an access, as runs are 2-24 elements long),
+// MFMA and VALU 23 % each; 4, 5 or 6 resident workgroups per CU make no
+// difference beyond the 3 of the default register budget (407, 397, 411 us at
+// 3, 4, 5), so latency is covered.
+//
 // Each D element is produced by exactly one item, in a fixed order of the
 // contracted indices, so results are deterministic and independent of the
 // batch composition and of the schedule.
@@ -224,43 +231,68 @@ __device__ __forceinline__ void item_body(const BatchItem &it, int tid, const Ba
   asm volatile("" ::"s"(pf0), "s"(pf1), "s"(pf2), "s"(pf3));
 }
 
-// Queue q holds items [qstart[q], qstart[q + 1]); counters[kCounterStride * q]
-// counts the positions taken from it.  Workgroup b starts on queue b % nq
-// and, once a fetch comes back past the end of a queue, moves on to the next
-// one; after a fetch past the end of all nq queues it exits, so every
-// workgroup exits and the grid drains.  Thread 0 fetches; the position is
-// published through a two-slot LDS word behind a barrier.
+// Queue q holds items [qstart[q], qstart[q + 1]).  Workgroup b starts on
+// queue b % nq with that queue's item b / nq; counters[kCounterStride * q]
+// counts the positions fetched from it after those.  Once a fetch comes back
+// past a queue's end, the counters of all queues are read at once and the
+// workgroup goes to the one with the most items left, or exits: each turn of
+// that loop ends in an item, in a queue seen empty (never chosen again, the
+// counters only grow) or in the exit, so every workgroup exits and the grid
+// drains.  (Visiting the other queues one by one took seven round trips of
+// about 1 us: 1,024 small contractions 58 -> 48 us.)  The last workgroup to
+// leave clears the counters for the next launch: every queue's workgroups count
+// down in a line of their own, the last of each in one common line.
+// Thread 0 fetches; the position is published through a two-slot LDS word
+// behind a barrier.
 constexpr int kCounterStride = 64;  // one 256-byte line per counter
 
-__global__ void batch_reset_kernel(unsigned *counters, int nq) {
-  if ((int)threadIdx.x < nq) counters[kCounterStride * threadIdx.x] = 0u;
+__global__ void batch_reset_kernel(unsigned *counters, int n) {
+  if ((int)threadIdx.x < n) counters[kCounterStride * threadIdx.x] = 0u;
 }
 
+// Workgroups that start on queue q.
+__device__ inline int starters(int q, int nq) { return ((int)gridDim.x - q + nq - 1) / nq; }
+
 template <typename S>
-__global__ __launch_bounds__(kThreads) void batch_contract_kernel(const BatchItem *__restrict__ items,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void batch_contract_kernel(const BatchItem *__restrict__ items,
                                                                  const int *__restrict__ qstart,
                                                                  unsigned *counters, int nq) {
   __shared__ TileLds<S> lds;
-  __shared__ int s_pos[2];
-  const int tid = threadIdx.x;
-  int q = (int)blockIdx.x % nq, visited = 1, slot = 0;
-  if (tid == 0) s_pos[0] = (int)atomicAdd(&counters[kCounterStride * q], 1u);
-  __syncthreads();
-  int cur = s_pos[0];
+  __shared__ int s_pos[2], s_queue;
+  const int tid = threadIdx.x, q0 = (int)blockIdx.x % nq;
+  int q = q0, slot = 0, cur = (int)blockIdx.x / nq;
   while (true) {
     const int base = qstart[q], end = qstart[q + 1];
     slot ^= 1;  // the other slot was last read before the barrier that published `cur`
     if (base + cur >= end) {
-      if (visited == nq) break;
-      q = q + 1 == nq ? 0 : q + 1;
-      ++visited;
-      if (tid == 0) s_pos[slot] = (int)atomicAdd(&counters[kCounterStride * q], 1u);
+      if (tid < 64) {  // wave 0: the items left in queue `tid`, then the largest of all
+        int left = 0;
+        if (tid < nq) {
+          const unsigned taken = (unsigned)starters(tid, nq) +
+                                 __hip_atomic_load(&counters[kCounterStride * tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          left = max(0, qstart[tid + 1] - qstart[tid] - (int)taken);
+        }
+        // a queue number in the low bits; rotated, so that workgroups of
+        // different queues spread over equally full ones
+        int64_t key = left ? (int64_t)left << 8 | (tid + nq - q0) % nq : -1;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) key = max(key, (int64_t)__shfl_xor(key, o));
+        if (tid == 0) {
+          const int to = key < 0 ? -1 : ((int)(key & 255) + q0) % nq;
+          if (to >= 0) s_pos[slot] = starters(to, nq) + (int)atomicAdd(&counters[kCounterStride * to], 1u);
+          s_queue = to;
+        }
+      }
       __syncthreads();
+      const int to = s_queue;
       cur = s_pos[slot];
+      __syncthreads();
+      if (to < 0) break;
+      q = to;
       continue;
     }
     unsigned next = 0;
-    if (tid == 0) next = atomicAdd(&counters[kCounterStride * q], 1u);
+    if (tid == 0) next = (unsigned)starters(q, nq) + atomicAdd(&counters[kCounterStride * q], 1u);
     const BatchItem &it = items[base + cur];
     // (BI - 1) | (BJ - 1) << 2 | along-k bits of L and R, uniform over the workgroup
 #define TAL_ITEM(BI, BJ, AK, BK)                                         \
@@ -284,6 +316,13 @@ __global__ __launch_bounds__(kThreads) void batch_contract_kernel(const BatchIte
     __syncthreads();
     cur = s_pos[slot];
   }
+  if (tid == 0) {
+    unsigned *leave = counters + kCounterStride * nq;
+    if (atomicAdd(&leave[kCounterStride * q0], 1u) + 1 == (unsigned)starters(q0, nq) &&
+        atomicAdd(&leave[kCounterStride * nq], 1u) + 1 == (unsigned)min(nq, (int)gridDim.x))
+      for (int i = 0; i < 2 * nq + 1; ++i)
+        __hip_atomic_store(&counters[kCounterStride * i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 }  // namespace
@@ -302,8 +341,7 @@ int batch_blocks_per_cu(int dk, int *blocks) {
 
 int batch_launch(int dk, const BatchItem *items, const int *qstart, unsigned *counters, int nq, int nblocks,
                  hipStream_t s) {
-  if (!items || !qstart || !counters || nq <= 0 || nq > kThreads || nblocks <= 0) return -1;
-  batch_reset_kernel<<<1, kThreads, 0, s>>>(counters, nq);
+  if (!items || !qstart || !counters || nq <= 0 || nq > kBatchMaxQueues || nblocks <= 0) return -1;
   switch (dk) {
     case 8: batch_contract_kernel<double><<<nblocks, kThreads, 0, s>>>(items, qstart, counters, nq); break;
     case 4: batch_contract_kernel<float><<<nblocks, kThreads, 0, s>>>(items, qstart, counters, nq); break;
@@ -312,6 +350,12 @@ int batch_launch(int dk, const BatchItem *items, const int *qstart, unsigned *co
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-size_t batch_counter_bytes(int nq) { return (size_t)nq * kCounterStride * sizeof(unsigned); }
+size_t batch_counter_bytes(int nq) { return (size_t)(2 * nq + 1) * kCounterStride * sizeof(unsigned); }
+
+int batch_counter_reset(unsigned *counters, int nq, hipStream_t s) {
+  if (!counters || nq <= 0 || nq > kBatchMaxQueues) return -1;
+  batch_reset_kernel<<<1, kThreads, 0, s>>>(counters, 2 * nq + 1);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
 
 }  // namespace tal

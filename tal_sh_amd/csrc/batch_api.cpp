@@ -169,7 +169,7 @@ int upload(int g, int dk, const std::vector<HostTask> &hts, hipStream_t s, Devic
   if (hipMemcpyAsync((void *)db->qstart, qstart.data(), 4 * qstart.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
       (!ordered.empty() && hipMemcpyAsync((void *)db->items, ordered.data(), sizeof(BatchItem) * ordered.size(),
                                           hipMemcpyHostToDevice, s) != hipSuccess) ||
-      hipStreamSynchronize(s) != hipSuccess) {
+      batch_counter_reset(db->counters, kXcds, s) != 0 || hipStreamSynchronize(s) != hipSuccess) {
     dev_free(g, db->base, db->handle);
     return TALSH_FAILURE;
   }
@@ -367,7 +367,7 @@ int build(talshAmdBatch *b, int g) {
   b->nblocks = nblocks;
   b->g = g;
   b->dk = dk;
-  // capture [clear the queue counters, persistent launch] once; executions replay it
+  // capture the persistent launch once; executions replay it
   hipStream_t cs;
   if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) return TALSH_FAILURE;
   int err = TALSH_SUCCESS;

@@ -83,7 +83,7 @@ struct BatchItem {
   double alpha;
   BatchGroup gm;  // rows: tensors (L, D)
   BatchGroup gn;  // columns: tensors (R, D)
-  BatchGroup gk;  // contracted: tensors (L, R)
+  BatchGroup gk;  // contracted: tensors (L, R); L and R may be the contraction's right and left operand
   int32_t pad1[10];
 };
 static_assert(sizeof(BatchGroup) == 48, "BatchGroup layout");

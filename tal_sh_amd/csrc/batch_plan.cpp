@@ -90,29 +90,41 @@ int batch_task_geometry(const DigitalPattern &p, const int *ddims, const int *ld
   }
   const int lf = fastest(p.lrank, ldims), rf = fastest(p.rrank, rdims);
   const bool l_kfast = lf >= 0 && p.dig[(size_t)lf] < 0, r_kfast = rf >= 0 && p.dig[(size_t)(p.lrank + rf)] < 0;
-  const int kby = (r_kfast && !l_kfast) ? 1 : 0;
   g->l_along_k = l_kfast;
   g->r_along_k = r_kfast;
-  if (!make_group(m, 0, esz, &g->gm, &g->M, &g->ndims_m) || !make_group(n, 0, esz, &g->gn, &g->N, &g->ndims_n) ||
+  // D's fastest index goes to the columns
+  const int df = fastest(p.drank, ddims);
+  g->swapped = false;
+  for (const Dim &d : m) g->swapped = g->swapped || (df >= 0 && d.ext > 1 && d.s1 == ds[(size_t)df]);
+  if (g->swapped) {
+    std::swap(m, n);
+    for (Dim &d : k) std::swap(d.s0, d.s1);
+  }
+  const bool ak = g->swapped ? r_kfast : l_kfast;
+  const int kby = (r_kfast && !l_kfast) != g->swapped ? 1 : 0;
+  int ndm = 0, ndn = 0;
+  if (!make_group(m, ak ? 1 : 0, esz, &g->gm, &g->M, &ndm) || !make_group(n, 1, esz, &g->gn, &g->N, &ndn) ||
       !make_group(k, kby, esz, &g->gk, &g->K, &g->ndims_k))
     return 2;
+  g->ndims_m = g->swapped ? ndn : ndm;
+  g->ndims_n = g->swapped ? ndm : ndn;
   return 0;
 }
 
 void batch_task_items(const BatchTaskGeom &g, uint64_t L, uint64_t R, uint64_t D, uint64_t lbytes, uint64_t rbytes,
                       uint64_t dbytes, double alpha, bool accumulate, WaveTile tile, std::vector<BatchItem> *out) {
   BatchItem it{};
-  it.L = L;
-  it.R = R;
+  it.L = g.swapped ? R : L;
+  it.R = g.swapped ? L : R;
   it.D = D;
-  it.lbytes = (uint32_t)lbytes;
-  it.rbytes = (uint32_t)rbytes;
+  it.lbytes = (uint32_t)(g.swapped ? rbytes : lbytes);
+  it.rbytes = (uint32_t)(g.swapped ? lbytes : rbytes);
   it.dbytes = (uint32_t)dbytes;
   it.M = g.M;
   it.N = g.N;
   it.K = g.K;
-  it.shape = (tile.tm / 32 - 1) | ((tile.tn / 32 - 1) << 2) | (accumulate ? 16 : 0) | (g.l_along_k ? 32 : 0) |
-             (g.r_along_k ? 64 : 0);
+  it.shape = (tile.tm / 32 - 1) | ((tile.tn / 32 - 1) << 2) | (accumulate ? 16 : 0) |
+             ((g.swapped ? g.r_along_k : g.l_along_k) ? 32 : 0) | ((g.swapped ? g.l_along_k : g.r_along_k) ? 64 : 0);
   it.alpha = alpha;
   it.gm = g.gm;
   it.gn = g.gn;
