@@ -65,6 +65,13 @@ __device__ inline void tile_of(int64_t gx, int64_t gy, int64_t t0, int64_t count
   tile_xy(t0 + t, gx, gy, bx, by);
 }
 
+// Unit u of n in dispatch order -> a number such that the units of one XCD are
+// neighbours, for any n (a bijection of [0, n)).
+__device__ inline int64_t xcd_order(int64_t u, int64_t n) {
+  const int64_t q = n / kXcds, r = n % kXcds, x = u % kXcds;
+  return x * q + min(x, r) + u / kXcds;
+}
+
 // Products whose operands the direct kernels cannot address (an operand of
 // 2 GiB or more with rows too far apart for 32-bit offsets within a tile):
 // every access works its 64-bit address out.  One tile shape per kind, 4 waves
@@ -188,41 +195,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       }
 }
 
-// Second pass of a K-split tile range: sums the ksplit partial blocks of
-// tiles [t0, t0 + ntiles) in order and applies C = alpha * sum (+ C).
-template <typename S, int NC, int BM, int BN>
-__global__ __launch_bounds__(kThreads) void gemm_tail_reduce(int64_t M, int64_t N, const S *__restrict__ part,
-                                                             int ksplit, S *__restrict__ C, int64_t ldc, S alpha_r,
-                                                             S alpha_i, int beta_one, int64_t gx, int64_t gy,
-                                                             int64_t t0, int64_t ntiles,
-                                                             const int64_t *__restrict__ cmap) {
-  const int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (e >= ntiles * BM * BN) return;
-  const int64_t q = e / (BM * BN);
-  const int rem = (int)(e % (BM * BN)), ml = rem % BM, nl = rem / BM;
-  int64_t bx, by;
-  tile_xy(t0 + q, gx, gy, bx, by);
-  const int64_t m = bx * BM + ml, n = by * BN + nl;
-  if (m >= M || n >= N) return;
-  S x[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) x[c] = (S)0;
-  for (int ch = 0; ch < ksplit; ++ch) {
-    const S *pb = part + ((q * ksplit + ch) * BM * BN + ml + (int64_t)nl * BM) * NC;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) x[c] += pb[c];
-  }
-  S *cp = C + (cmap ? cmap[m] + cmap[M + n] : m + n * ldc) * NC;
-  if (NC == 1) {
-    const S v = alpha_r * x[0];
-    cp[0] = beta_one ? cp[0] + v : v;
-  } else {
-    const S vr = alpha_r * x[0] - alpha_i * x[NC - 1], vi = alpha_r * x[NC - 1] + alpha_i * x[0];
-    cp[0] = beta_one ? cp[0] + vr : vr;
-    cp[NC - 1] = beta_one ? cp[NC - 1] + vi : vi;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // R4 GEMM as 3-term split-BF16 products (bf16x6): every FP32 operand value x
 // is split exactly into x = h + m + l with h = bf16(x), m = bf16(x - h),
@@ -235,8 +207,8 @@ __global__ __launch_bounds__(kThreads) void gemm_tail_reduce(int64_t M, int64_t 
 // few 1e-7 (cf. ~1e-6 for the FP32 MFMA path).  Both operands are split once
 // into swizzled BF16 planes in a workspace by split_planes_kernel, then 256 x
 // 128 tiles of 8 waves stream the planes with no VALU split work in the K
-// loop; the last, mostly idle round of tiles is split along K into partials
-// summed by gemm_tail_reduce.  MFMA 16x16x32 bf16
+// loop; a partial last round of tiles is split along K into partials summed by
+// presplit_reduce_kernel.  MFMA 16x16x32 bf16
 // layout: A lane l holds A[l%16][8*(l/16)..+7], B lane l holds
 // B[8*(l/16)..+7][l%16], accumulator register r of lane l holds
 // C[4*(l/16)+r][l%16].
@@ -244,11 +216,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // ---------------------------------------------------------------------------
 // Pre-split GEMMs.  split_planes_kernel writes the planes of an operand once
-// into a workspace (row r, column k of a plane at r*Kp + k; rows padded to the
-// GEMM tile, K padded to 32, zeros in the padding), so the GEMM's inner loop
-// only moves bytes and issues MFMAs: no split arithmetic (which the on-the-fly
-// kernel above repeats for every C tile that reads an element) and no bounds
-// checks.  The dominant product of the leading terms goes to one accumulator
+// into a workspace (layout: plane_chunk; rows padded to the GEMM tile, K padded
+// to 32, zeros in the padding), so the GEMM's inner loop only moves bytes and
+// issues MFMAs: no split arithmetic and no bounds checks.  The dominant product of the leading terms goes to one accumulator
 // and the small products to a second, so the main accumulator is rounded once
 // per K step of 32 without any VALU adds; the two are summed in the epilogue.
 //
@@ -270,14 +240,18 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 //    FP32's exponent range, has no such limit.  The epilogue multiplies by
 //    2^(ea + eb), which is exact.
 //
-// Block tile 256 x 128, 8 waves of 64 x 64 (two per SIMD), BK = 32.  LDS
-// holds two stages of both operands (2 x (16 + 8) KB per plane); a plane row
-// is 64 bytes (four 16-byte chunks) and chunk c of row r is stored at slot
-// c ^ (((r >> 1) ^ (r >> 3)) & 3), so the 16-byte fragment reads are free of
-// bank conflicts whether the LDS serves them 8 lanes over 32 banks or 16 lanes
-// over 64 banks per cycle.
-// The next K step is loaded into registers while the current one is multiplied;
-// one barrier per K step.
+// Block tile 256 x 128, 8 waves of 64 x 64 (two per SIMD), K steps of 32.  The
+// planes lie in memory as the blocks an LDS stage holds (plane_chunk), so a
+// stage is filled by loads straight to LDS, 1 KB a wave and instruction, with
+// no registers, no address arithmetic and no LDS store instructions; fragment
+// reads are free of bank conflicts.  What bounds it: fp16x3, where a step is 48
+// MFMAs a wave, the latency of the next step's loads and the LDS (1,400 of
+// 1,536 cycles a step); hence three stages, two steps in flight.  bf16x6 has
+// twice the MFMAs and room for two stages.  One barrier per K step.  Rates of
+// the 16-bit products: fp16x3 at 5184^3 772 -> 1,100 TFLOP/s (1080 -> 757 us
+// with the last round split), bf16x6 at 9216^3 1,146 -> 1,376 (8.19 -> 6.82 ms),
+// against loads through registers one step ahead of rows with a stride of K; a
+// bf16 library product reaches 1,230-1,320 on this card.
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 __device__ inline void split3_finite(float x, __bf16 &h, __bf16 &m, __bf16 &l) {
@@ -312,163 +286,166 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t *__restrict__ p,
   if (i < n) p[i] = 0u;
 }
 
-// U[r] = max over k < K of the bit pattern of |X(r, k)| (for non-negative
-// floats the pattern orders as the value; NaN patterns sort above Inf), U
-// zeroed beforehand.  Block = 4 waves; grid.x = row groups, grid.y = K
-// segments of kseg.  KC = 1 (X(r, k) at X[r*ld + k]): one wave per row, lanes
-// along k.  KC = 0 (X(r, k) at X[r + k*ld]): lanes along r, the four waves
-// share the segment.
-// vec (KC = 1): X 16-byte aligned and ld a multiple of 4, so whole rounds of
-// 256 floats of a segment (kseg a multiple of 256) are read as float4.
 __device__ inline uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 
-template <int KC>
-__global__ __launch_bounds__(256) void row_absmax_kernel(const float *__restrict__ X, int64_t ld, int64_t R,
-                                                         int64_t K, int64_t kseg, int vec, uint32_t *__restrict__ U) {
+// U[r] = max over k < K of the bit pattern of |X(r, k)| with X(r, k) at
+// X[r + k*ld] (for non-negative floats the pattern orders as the value; NaN
+// patterns sort above Inf), U zeroed beforehand.  Block = 4 waves, lanes along
+// r; grid.x = row groups, grid.y = K segments of kseg, which the four waves share.
+__global__ __launch_bounds__(256) void row_absmax_kernel(const float *__restrict__ X, int64_t ld, int64_t R, int64_t K,
+                                                         int64_t kseg, uint32_t *__restrict__ U) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t k0 = (int64_t)blockIdx.y * kseg, k1 = min(K, k0 + kseg);
   uint32_t m = 0;
-  if (KC) {
-    const int64_t r = (int64_t)blockIdx.x * 4 + wave;
-    if (r < R) {
-      const float *x = X + r * ld;
-      int64_t k = k0;
-      if (vec) {
-        const int64_t kv = k0 + ((k1 - k0) & ~(int64_t)255);
-#pragma unroll 4
-        for (int64_t q = k0 + 4 * lane; q < kv; q += 256) {
-          const float4 v = *reinterpret_cast<const float4 *>(x + q);
-          m = max(m, max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w))));
-        }
-        k = kv;
-      }
-#pragma unroll 4
-      for (k += lane; k < k1; k += 64) m = max(m, abs_bits(x[k]));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
-    if (lane == 0 && r < R && m) atomicMax(U + r, m);
-  } else {
-    const int64_t r = (int64_t)blockIdx.x * 64 + lane;
-    if (r < R) {
+  const int64_t r = (int64_t)blockIdx.x * 64 + lane;
+  if (r >= R) return;
 #pragma unroll 8
-      for (int64_t k = k0 + wave; k < k1; k += 4) m = max(m, abs_bits(X[r + k * ld]));
-      if (m) atomicMax(U + r, m);
-    }
-  }
+  for (int64_t k = k0 + wave; k < k1; k += 4) m = max(m, abs_bits(X[r + k * ld]));
+  if (m) atomicMax(U + r, m);
 }
 
-// fp16x3 planes of op(X) when its rows are K-contiguous (X(r, k) at
-// X[r*ld + k]): one block per padded row finds the row's largest magnitude
-// (U[r], 0 for padding rows), then splits the row, whose second read comes
-// from L2, so HBM sees each element once.  vec as for row_absmax_kernel.
-__global__ __launch_bounds__(256) void split_rows_f16_kernel(const float *__restrict__ X, int64_t ld, int64_t R,
-                                                             int64_t K, int64_t Kp, uint16_t *__restrict__ P,
-                                                             int64_t plane, int vec, uint32_t *__restrict__ U) {
-  __shared__ uint32_t red[4];
-  const int64_t r = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const float *x = X + r * ld;
-  uint32_t m = 0;
-  if (r < R) {
-    int64_t k = 0;
-    if (vec) {
-      const int64_t kv = K & ~(int64_t)3;
-#pragma unroll 8
-      for (int64_t q = 4 * tid; q < kv; q += 1024) {
-        const float4 v = *reinterpret_cast<const float4 *>(x + q);
-        m = max(m, max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w))));
-      }
-      k = kv;
-    }
-    for (k += tid; k < K; k += 256) m = max(m, abs_bits(x[k]));
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
-  if (lane == 0) red[wave] = m;
-  __syncthreads();
-  m = max(max(red[0], red[1]), max(red[2], red[3]));
-  if (tid == 0) U[r] = m;
-  const int e = row_exp(m);
-#pragma unroll 4
-  for (int64_t kc = tid; kc < Kp / 8; kc += 256) {
-    const int64_t k0 = kc * 8;
-    float v[8];
-    if (vec && r < R && k0 + 8 <= K) {
-      const float4 a = *reinterpret_cast<const float4 *>(x + k0);
-      const float4 b = *reinterpret_cast<const float4 *>(x + k0 + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (r < R && k0 + i < K) ? x[k0 + i] : 0.0f;
-    }
-    _Float16 h[8], l[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) split2_scaled(v[i], e, h[i], l[i]);
-    uint4 u;
-    __builtin_memcpy(&u, h, 16);
-    *reinterpret_cast<uint4 *>(P + r * Kp + k0) = u;
-    __builtin_memcpy(&u, l, 16);
-    *reinterpret_cast<uint4 *>(P + plane + r * Kp + k0) = u;
-  }
+// Plane layout: blocks of kPRows rows x PBK contracted indices, 8 KB each and
+// contiguous, along K first; in a block row r holds its four 16-byte chunks at
+// slots c ^ pswz(r).  A K step of the GEMM reads whole blocks, as they lie, and
+// they are the image its LDS stage needs.
+constexpr int kPRows = 128, PBK = 32;
+__device__ inline int pswz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
+// Address of chunk kc (8 contracted indices) of row r, in chunks; nks: K steps of the plane.
+__device__ inline int64_t plane_chunk(int64_t r, int64_t kc, int64_t nks) {
+  const int rr = (int)(r % kPRows), c = (int)(kc & 3);
+  return ((r / kPRows * nks + (kc >> 2)) * kPRows + rr) * 4 + (c ^ pswz(rr));
 }
 
-// KC = 1: source element (r, k) at X[r*ld + k]; KC = 0: at X[r + k*ld].
-// One thread per 8 consecutive k of one row (KC = 1: lanes along k, KC = 0:
-// lanes along r, so source reads are coalesced either way).  NP = 3: BF16
-// planes; NP = 2: FP16 planes of the row scaled by the exponent from U.
-template <int KC, int NP>
-__global__ __launch_bounds__(256) void split_planes_kernel(const float *__restrict__ X, int64_t ld, int64_t R,
-                                                           int64_t K, int64_t Rp, int64_t Kp,
-                                                           uint16_t *__restrict__ P, int64_t plane, int vec,
-                                                           const uint32_t *__restrict__ U) {
-  const int64_t kcn = Kp / 8;
-  const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (item >= Rp * kcn) return;
-  const int64_t r = KC ? item / kcn : item % Rp, kc = KC ? item % kcn : item / Rp;
-  const int64_t k0 = kc * 8;
-  float v[8];
-  if (KC && vec && r < R && k0 + 8 <= K) {
-    const float4 a = *reinterpret_cast<const float4 *>(X + r * ld + k0);
-    const float4 b = *reinterpret_cast<const float4 *>(X + r * ld + k0 + 4);
+// 8 consecutive k of row x (contiguous along k), zeros past n.
+__device__ inline void load8(const float *x, int64_t k0, int64_t n, bool vec, float (&v)[8]) {
+  if (vec && k0 + 8 <= n) {
+    const float4 a = *reinterpret_cast<const float4 *>(x + k0);
+    const float4 b = *reinterpret_cast<const float4 *>(x + k0 + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t k = k0 + i;
-      v[i] = (r < R && k < K) ? (KC ? X[r * ld + k] : X[r + k * ld]) : 0.0f;
-    }
+    for (int i = 0; i < 8; ++i) v[i] = k0 + i < n ? x[k0 + i] : 0.0f;
   }
+}
+
+// The NP planes of 8 values to their chunk; e: exponent of the row (NP = 2).
+template <int NP>
+__device__ inline void split_store(const float (&v)[8], int e, uint4 *__restrict__ P, int64_t plane, int64_t at) {
   uint4 u;
-  const int64_t off = r * Kp + k0;
   if constexpr (NP == 3) {
     __bf16 h[8], m[8], l[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) split3_finite(v[i], h[i], m[i], l[i]);
     __builtin_memcpy(&u, h, 16);
-    *reinterpret_cast<uint4 *>(P + off) = u;
+    P[at] = u;
     __builtin_memcpy(&u, m, 16);
-    *reinterpret_cast<uint4 *>(P + plane + off) = u;
+    P[plane + at] = u;
     __builtin_memcpy(&u, l, 16);
-    *reinterpret_cast<uint4 *>(P + 2 * plane + off) = u;
+    P[2 * plane + at] = u;
   } else {
-    const int e = r < R ? row_exp(U[r]) : 0;
     _Float16 h[8], m[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) split2_scaled(v[i], e, h[i], m[i]);
     __builtin_memcpy(&u, h, 16);
-    *reinterpret_cast<uint4 *>(P + off) = u;
+    P[at] = u;
     __builtin_memcpy(&u, m, 16);
-    *reinterpret_cast<uint4 *>(P + plane + off) = u;
+    P[plane + at] = u;
   }
 }
 
-constexpr int PBM = 256, PBN = 128, PBK = 32;
+// fp16x3 planes of op(X) when its rows are K-contiguous (X(r, k) at
+// X[r*ld + k]).  A block takes two padded rows, 256 threads each: it finds their
+// largest magnitudes (U[r], 0 for padding rows) and splits them, four threads on
+// the 32 k of a row's part of a plane block (128 bytes read; 128 written, the
+// two rows side by side).  The first kHeld chunks of a thread stay in registers
+// between the two, so rows of up to 8,192 are read once; longer ones' other
+// chunks are read again.  vec: X 16-byte aligned and ld a multiple of 4.
+// Memory-bound: 5184 x 5184 in 46 us, 4.7 TB/s
+// (two passes over a row per block: 60).
+constexpr int kSplitThreads = 512;
+__global__ __launch_bounds__(kSplitThreads) void split_rows_f16_kernel(const float *__restrict__ X, int64_t ld,
+                                                                       int64_t R, int64_t K, int64_t nks,
+                                                                       uint4 *__restrict__ P, int64_t plane, int vec,
+                                                                       uint32_t *__restrict__ U) {
+  constexpr int kHeld = 4, kRound = kSplitThreads / 8;  // K steps per round of the block
+  __shared__ uint32_t red[2][8];
+  const int tid = threadIdx.x, c = tid & 3, row = (tid >> 2) & 1, lane = tid & 63, wave = tid >> 6;
+  const int64_t r = (int64_t)blockIdx.x * 2 + row, n = r < R ? K : 0;
+  const float *x = X + r * ld;
+  float v[kHeld][8];
+  uint32_t m = 0;
+#pragma unroll
+  for (int q = 0; q < kHeld; ++q) {
+    const int64_t ks = (tid >> 3) + q * kRound;
+    load8(x, ks * PBK + c * 8, n, vec, v[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < kHeld; ++q)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = max(m, abs_bits(v[q][i]));
+  for (int64_t ks = (tid >> 3) + kHeld * kRound; ks < nks; ks += kRound) {
+    float w[8];
+    load8(x, ks * PBK + c * 8, n, vec, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = max(m, abs_bits(w[i]));
+  }
+  // lane bit 2 is the row
+#pragma unroll
+  for (int o = 32; o > 4; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+#pragma unroll
+  for (int o = 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+  if ((lane & ~4) == 0) red[row][wave] = m;
+  __syncthreads();
+  m = 0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) m = max(m, red[row][w]);
+  if ((tid & ~4) == 0) U[r] = m;
+  const int e = row_exp(m);
+#pragma unroll
+  for (int q = 0; q < kHeld; ++q) {
+    const int64_t ks = (tid >> 3) + q * kRound;
+    if (ks < nks) split_store<2>(v[q], e, P, plane, plane_chunk(r, ks * 4 + c, nks));
+  }
+  for (int64_t ks = (tid >> 3) + kHeld * kRound; ks < nks; ks += kRound) {
+    float w[8];
+    load8(x, ks * PBK + c * 8, n, vec, w);
+    split_store<2>(w, e, P, plane, plane_chunk(r, ks * 4 + c, nks));
+  }
+}
 
-__device__ inline int pswz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
-__device__ inline int pslot(int r, int c) { return r * 4 + (c ^ pswz(r)); }
+// KC = 1: source element (r, k) at X[r*ld + k]; KC = 0: at X[r + k*ld].  A
+// thread splits 8 consecutive k of one row.  KC = 1: a block covers kSplitRows
+// rows of 64 / kSplitRows K steps, four threads on a row's 32 k (9216 x 9216 in
+// 141 us, 6.0 TB/s; 2, 4, 16 and 64 rows 149, 147, 147 and 165); KC = 0: 64
+// rows of one K step, lanes along the rows; so source reads are coalesced
+// either way.  NP = 3: BF16 planes; NP = 2: FP16 planes of the row scaled by
+// the exponent from U.
+constexpr int kSplitRows = 8;
+template <int KC, int NP>
+__global__ __launch_bounds__(256) void split_planes_kernel(const float *__restrict__ X, int64_t ld, int64_t R,
+                                                           int64_t K, int64_t nks, uint4 *__restrict__ P,
+                                                           int64_t plane, int vec, const uint32_t *__restrict__ U) {
+  const int tid = threadIdx.x;
+  constexpr int ROWS = KC ? kSplitRows : 64, STEPS = 64 / ROWS;  // of a block
+  const int64_t nkb = (nks + STEPS - 1) / STEPS, rg = blockIdx.x / nkb;
+  const int64_t r = rg * ROWS + (KC ? (tid >> 2) % ROWS : tid & 63);
+  const int64_t ks = (blockIdx.x - rg * nkb) * STEPS + (KC ? tid / (4 * ROWS) : 0);
+  const int c = KC ? tid & 3 : tid >> 6;
+  if (ks >= nks) return;
+  const int64_t k0 = ks * PBK + c * 8;
+  float v[8];
+  if (KC) {
+    load8(X + r * ld, k0, r < R ? K : 0, vec, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (r < R && k0 + i < K) ? X[r + (k0 + i) * ld] : 0.0f;
+  }
+  const int e = NP == 2 && r < R ? row_exp(U[r]) : 0;
+  split_store<NP>(v, e, P, plane, plane_chunk(r, ks * 4 + c, nks));
+}
+
+constexpr int PBM = 256, PBN = 128;
 
 template <int NP>
 __device__ inline f32x4 pmfma(uint4 a, uint4 b, f32x4 c) {
@@ -480,67 +457,76 @@ __device__ inline f32x4 pmfma(uint4 a, uint4 b, f32x4 c) {
                                                   0, 0);
 }
 
-// aplane / bplane / row strides in 16-byte chunks.  ksplit > 1: workgroup
-// q*ksplit + c computes K steps [c*ksteps, (c+1)*ksteps) of tile t0 + q into
-// its own PBM x PBN block of `part` (big + small, scaled by 2^(ea + eb) for
-// NP = 2, no alpha, no beta).  UA / UB (NP = 2): row maxima of op(A) and
-// column maxima of op(B), Mp and Np entries.
+struct SplitArgs {
+  const uint4 *a, *b;      // planes of op(A) and op(B)
+  int64_t apl, bpl, nks;   // chunks per plane, K steps
+  float *C;
+  const int64_t *cmap;     // element offsets of C's rows, then its columns; null: m + n * ldc
+  float *part;             // partial sums of the tiles cut into K ranges, PBM x PBN each
+  const uint32_t *ua, *ub; // NP = 2: row maxima of op(A), column maxima of op(B)
+  int64_t M, N, ldc;
+  int64_t gx, gy, whole;   // tiles; the first `whole` are computed by one workgroup each
+  int64_t rem, ksteps;     // the others by ksplit workgroups, `ksteps` K steps each
+  int ksplit;
+  int beta_one;
+  float alpha;
+};
+
+// 16 bytes a lane from base + off to the LDS bytes from `lds` on, lane after
+// lane: no registers, no LDS store instructions.  The compiler neither knows
+// the load nor waits for it; presplit_gemm_kernel's loop does.
+__device__ inline void dma16(uint32_t lds, const char *base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+
+template <int N>
+__device__ inline void wait_dma() {  // at most N of the wave's loads in flight, its LDS reads done
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int NP>
-__device__ __forceinline__ void presplit_gemm(int64_t M, int64_t N, int64_t Kp, const uint4 *__restrict__ Ap,
-                                              int64_t aplane, const uint4 *__restrict__ Bp, int64_t bplane,
-                                              float *__restrict__ C, int64_t ldc, float alpha, int beta_one,
-                                              int64_t gx, int64_t gy, int64_t t0, int64_t count, int ksplit,
-                                              int64_t ksteps, float *__restrict__ part,
-                                              const uint32_t *__restrict__ UA, const uint32_t *__restrict__ UB,
-                                              const int64_t *__restrict__ cmap) {
-  __shared__ uint4 As[2][NP][PBM * 4];
-  __shared__ uint4 Bs[2][NP][PBN * 4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void presplit_gemm_kernel(SplitArgs p) {
+  constexpr int NS = NP == 2 ? 3 : 2;             // LDS stages
+  constexpr int PIECE = kPRows * 4, PIECES = 3;   // chunks of a plane block; blocks of a plane: two of A, one of B
+  constexpr int LOADS = NP * PIECES;              // a wave's loads per K step
+  __shared__ uint4 S[NS][NP][PIECES][PIECE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 3, wn = wave >> 2;
-  int64_t bx, by, kt0 = 0, kt1 = Kp / PBK;
-  if (ksplit > 1) {
-    tile_xy(t0 + (int64_t)blockIdx.x / ksplit, gx, gy, bx, by);
-    kt0 = (int64_t)(blockIdx.x % ksplit) * ksteps;
-    kt1 = min(kt1, kt0 + ksteps);
+  // units: the whole tiles, then the K ranges of the others
+  const int64_t whole = p.whole;
+  int64_t tile, kt0 = 0, kt1 = p.nks, unit = (int64_t)blockIdx.x - whole;
+  const bool range = unit >= 0;
+  if (!range) {
+    tile = xcd_order(blockIdx.x, whole);
   } else {
-    tile_of(gx, gy, t0, count, bx, by);
+    unit = xcd_order(unit, p.rem * p.ksplit);
+    tile = unit / p.ksplit;
+    kt0 = (unit - tile * p.ksplit) * p.ksteps;
+    kt1 = min(kt1, kt0 + p.ksteps);
+    tile += whole;
   }
-  const int64_t kpc = Kp / 8;  // chunks per plane row
-  // thread tid loads chunk (tid & 3) of row (tid >> 2) [+128] of each plane
-  const int lr = tid >> 2, lc = tid & 3;
-  // block-uniform bases (scalar registers) plus one 32-bit per-thread byte offset
-  const char *ag = reinterpret_cast<const char *>(Ap + bx * PBM * kpc);
-  const char *bg = reinterpret_cast<const char *>(Bp + by * PBN * kpc);
-  const uint32_t voff = (uint32_t)((lr * kpc + lc) * 16);
-  const int ls = pslot(lr, lc);
-  const int64_t a1 = 128 * kpc;
-  // prefetch registers: A planes t rows lr and lr+128; B planes t row lr
-  uint4 a0, a1r, a2, a3, a4, a5, b0, b1, b2;
-#define TAL_PG(base, chunk) (*reinterpret_cast<const uint4 *>((base) + (chunk) * 16 + voff))
-#define TAL_PLOAD(kc)                                                                  \
-  a0 = TAL_PG(ag, (kc));                                                               \
-  a1r = TAL_PG(ag, a1 + (kc));                                                         \
-  a2 = TAL_PG(ag, aplane + (kc));                                                      \
-  a3 = TAL_PG(ag, aplane + a1 + (kc));                                                 \
-  if constexpr (NP == 3) {                                                             \
-    a4 = TAL_PG(ag, 2 * aplane + (kc));                                                \
-    a5 = TAL_PG(ag, 2 * aplane + a1 + (kc));                                           \
-  }                                                                                    \
-  b0 = TAL_PG(bg, (kc));                                                               \
-  b1 = TAL_PG(bg, bplane + (kc));                                                      \
-  if constexpr (NP == 3) b2 = TAL_PG(bg, 2 * bplane + (kc));
-#define TAL_PSTORE(st)                                                                 \
-  As[st][0][ls] = a0;                                                                  \
-  As[st][0][ls + 512] = a1r;                                                           \
-  As[st][1][ls] = a2;                                                                  \
-  As[st][1][ls + 512] = a3;                                                            \
-  if constexpr (NP == 3) {                                                             \
-    As[st][NP - 1][ls] = a4;                                                           \
-    As[st][NP - 1][ls + 512] = a5;                                                     \
-  }                                                                                    \
-  Bs[st][0][ls] = b0;                                                                  \
-  Bs[st][1][ls] = b1;                                                                  \
-  if constexpr (NP == 3) Bs[st][NP - 1][ls] = b2;
+  int64_t bx, by;
+  tile_xy(tile, p.gx, p.gy, bx, by);
+  const int64_t nk = kt1 - kt0;  // may be <= 0 for a trailing K range: its partial sums are zeros
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4 *)&S[0][0][0][0] + wave * 1024;
+  const uint32_t voff = (uint32_t)lane * 16;
+  const char *ab = reinterpret_cast<const char *>(p.a + (2 * bx * p.nks + kt0) * PIECE) + wave * 1024;
+  const char *bb = reinterpret_cast<const char *>(p.b + (by * p.nks + kt0) * PIECE) + wave * 1024;
+  const int64_t ablk = p.nks * PIECE * 16, apl = p.apl * 16, bpl = p.bpl * 16;
+  auto load = [&](int st) {
+    const uint32_t l = lds0 + (uint32_t)st * (NP * PIECES * PIECE * 16);
+#pragma unroll
+    for (int t = 0; t < NP; ++t) {
+      dma16(l + (t * PIECES + 0) * PIECE * 16, ab + t * apl, voff);
+      dma16(l + (t * PIECES + 1) * PIECE * 16, ab + t * apl + ablk, voff);
+      dma16(l + (t * PIECES + 2) * PIECE * 16, bb + t * bpl, voff);
+    }
+  };
 
   f32x4 big[4][4], small[4][4];
 #pragma unroll
@@ -550,115 +536,146 @@ __device__ __forceinline__ void presplit_gemm(int64_t M, int64_t N, int64_t Kp, 
 
   // fragment slot of row 16*x + (lane & 15), chunk lane >> 4: the swizzle of
   // that row is pswz(lane & 15), with bit 1 flipped when x is odd
-  const int fs[2] = {pslot(lane & 15, lane >> 4), (lane & 15) * 4 + ((lane >> 4) ^ pswz(lane & 15) ^ 2)};
-  const int64_t nk = kt1 - kt0;  // may be <= 0 for a trailing K range: its partial sums are zeros
-  if (nk > 0) {
-    TAL_PLOAD(kt0 * (PBK / 8))
-    TAL_PSTORE(0)
-  }
-  __syncthreads();
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    const int cur = (int)(kt & 1);
-    if (kt + 1 < nk) {
-      TAL_PLOAD((kt0 + kt + 1) * (PBK / 8))
-    }
+  const int fc = lane >> 4, fr = lane & 15;
+  const int fs[2] = {fr * 4 + (fc ^ pswz(fr)), fr * 4 + (fc ^ pswz(fr) ^ 2)};
+  const int am = (wm >> 1) * PIECE + (wm & 1) * 256, bn = 2 * PIECE + wn * 256;  // the wave's rows and columns
+  auto compute = [&](int st) {
+    const uint4 *s = &S[st][0][0][0];
     uint4 fb[NP][4];
 #pragma unroll
     for (int t = 0; t < NP; ++t)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) fb[t][j] = Bs[cur][t][(wn * 64 + j * 16) * 4 + fs[j & 1]];
+      for (int j = 0; j < 4; ++j) fb[t][j] = s[t * PIECES * PIECE + bn + j * 64 + fs[j & 1]];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint4 fa[NP];
 #pragma unroll
-      for (int t = 0; t < NP; ++t) fa[t] = As[cur][t][(wm * 64 + i * 16) * 4 + fs[i & 1]];
+      for (int t = 0; t < NP; ++t) fa[t] = s[t * PIECES * PIECE + am + i * 64 + fs[i & 1]];
+      // B is the first operand, so that a lane's column of the accumulators is a row of C
       if constexpr (NP == 3) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fa[2], fb[0][j], small[i][j]);
+        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fb[0][j], fa[2], small[i][j]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fa[1], fb[1][j], small[i][j]);
+        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fb[1][j], fa[1], small[i][j]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fa[0], fb[2][j], small[i][j]);
+        for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fb[2][j], fa[0], small[i][j]);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fa[1], fb[0][j], small[i][j]);
+      for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fb[0][j], fa[1], small[i][j]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fa[0], fb[1][j], small[i][j]);
+      for (int j = 0; j < 4; ++j) small[i][j] = pmfma<NP>(fb[1][j], fa[0], small[i][j]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) big[i][j] = pmfma<NP>(fa[0], fb[0][j], big[i][j]);
+      for (int j = 0; j < 4; ++j) big[i][j] = pmfma<NP>(fb[0][j], fa[0], big[i][j]);
     }
-    if (kt + 1 < nk) {
-      TAL_PSTORE(cur ^ 1)
+  };
+
+  // K step kt is multiplied while the loads of step kt + NS - 1 are in flight.
+  // A stage is loaded again only behind the barrier that every wave reaches
+  // after its reads of it.  Past the last step that step is loaded again, into
+  // stages nobody reads, so that the number of loads in flight is a constant.
+  if (nk > 0) {
+    int64_t left = nk - 1;  // steps whose loads have not gone out
+    auto next = [&] {
+      const int64_t d = left > 0 ? PIECE * 16 : 0;
+      ab += d;
+      bb += d;
+      left -= left > 0;
+    };
+#pragma unroll
+    for (int q = 0; q < NS - 1; ++q) {
+      load(q);
+      next();
     }
-    __syncthreads();
+    int64_t kt = 0;
+    for (; kt + NS <= nk; kt += NS) {
+#pragma unroll
+      for (int q = 0; q < NS; ++q) {
+        wait_dma<(NS - 2) * LOADS>();
+        load((q + NS - 1) % NS);
+        next();
+        __builtin_amdgcn_sched_barrier(0);
+        compute(q);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NS - 1; ++q) {
+      if (kt + q < nk) {
+        wait_dma<(NS - 2) * LOADS>();
+        load((q + NS - 1) % NS);
+        next();
+        compute(q);
+      }
+    }
+    wait_dma<0>();  // LDS is given back only when nothing writes to it any more
   }
-#undef TAL_PG
-#undef TAL_PLOAD
-#undef TAL_PSTORE
-  // NP = 2: exponents of this lane's 16 rows (i, r) and 4 columns (j); every
-  // index is below Mp / Np, the sizes of UA / UB
-  int ea[4][4] = {}, eb[4] = {};
+
+  // NP = 2: exponents of this lane's 4 rows (i) and 16 columns (j, r); every
+  // index is below the padded sizes of ua / ub
+  const int64_t m0 = bx * PBM + wm * 64 + fr, n0 = by * PBN + wn * 64 + 4 * fc;
+  int ea[4] = {}, eb[4][4] = {};
   if constexpr (NP == 2) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ea[i][r] = row_exp(UA[bx * PBM + wm * 64 + i * 16 + 4 * (lane >> 4) + r]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) eb[j] = row_exp(UB[by * PBN + wn * 64 + j * 16 + (lane & 15)]);
-  }
-  if (ksplit > 1) {
-    float *pb = part + (int64_t)blockIdx.x * PBM * PBN;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int ml = wm * 64 + i * 16 + 4 * (lane >> 4) + r, nl = wn * 64 + j * 16 + (lane & 15);
-          const float s = big[i][j][r] + small[i][j][r];
-          pb[ml + nl * PBM] = NP == 2 ? ldexpf(s, ea[i][r] + eb[j]) : s;
-        }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) ea[i] = row_exp(p.ua[m0 + i * 16]);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t m = bx * PBM + wm * 64 + i * 16 + 4 * (lane >> 4) + r;
-        const int64_t n = by * PBN + wn * 64 + j * 16 + (lane & 15);
-        if (m < M && n < N) {
-          float *c = C + (cmap ? cmap[m] + cmap[M + n] : m + n * ldc);
-          const float s = big[i][j][r] + small[i][j][r];
-          const float v = alpha * (NP == 2 ? ldexpf(s, ea[i][r] + eb[j]) : s);
-          *c = beta_one ? *c + v : v;
+      for (int r = 0; r < 4; ++r) eb[j][r] = row_exp(p.ub[n0 + j * 16 + r]);
+  }
+  if (range) {
+    float *pb = p.part + unit * PBM * PBN;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int ml = wm * 64 + i * 16 + fr, nl = wn * 64 + j * 16 + 4 * fc + r;
+          const float x = big[i][j][r] + small[i][j][r];
+          pb[ml + nl * PBM] = NP == 2 ? ldexpf(x, ea[i] + eb[j][r]) : x;
         }
+    return;
+  }
+  int64_t om[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) om[i] = m0 + i * 16 >= p.M ? -1 : p.cmap ? p.cmap[m0 + i * 16] : m0 + i * 16;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t n = n0 + j * 16 + r;
+      if (n >= p.N) continue;
+      float *c = p.C + (p.cmap ? p.cmap[p.M + n] : n * p.ldc);
+      float old[4];
+      if (p.beta_one) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) old[i] = om[i] >= 0 ? c[om[i]] : 0.0f;
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = big[i][j][r] + small[i][j][r];
+        const float v = p.alpha * (NP == 2 ? ldexpf(x, ea[i] + eb[j][r]) : x);
+        if (om[i] >= 0) c[om[i]] = p.beta_one ? old[i] + v : v;
+      }
+    }
 }
 
-__global__ __launch_bounds__(512) void gemm_bf16x6p_kernel(int64_t M, int64_t N, int64_t Kp,
-                                                           const uint4 *__restrict__ Ap, int64_t aplane,
-                                                           const uint4 *__restrict__ Bp, int64_t bplane,
-                                                           float *__restrict__ C, int64_t ldc, float alpha,
-                                                           int beta_one, int64_t gx, int64_t gy, int64_t t0,
-                                                           int64_t count, int ksplit, int64_t ksteps,
-                                                           float *__restrict__ part, const int64_t *__restrict__ cmap) {
-  presplit_gemm<3>(M, N, Kp, Ap, aplane, Bp, bplane, C, ldc, alpha, beta_one, gx, gy, t0, count, ksplit, ksteps,
-                   part, nullptr, nullptr, cmap);
-}
-
-__global__ __launch_bounds__(512) void gemm_f16x3p_kernel(int64_t M, int64_t N, int64_t Kp,
-                                                          const uint4 *__restrict__ Ap, int64_t aplane,
-                                                          const uint4 *__restrict__ Bp, int64_t bplane,
-                                                          float *__restrict__ C, int64_t ldc, float alpha,
-                                                          int beta_one, int64_t gx, int64_t gy, int64_t t0,
-                                                          int64_t count, int ksplit, int64_t ksteps,
-                                                          float *__restrict__ part, const uint32_t *__restrict__ UA,
-                                                          const uint32_t *__restrict__ UB,
-                                                          const int64_t *__restrict__ cmap) {
-  presplit_gemm<2>(M, N, Kp, Ap, aplane, Bp, bplane, C, ldc, alpha, beta_one, gx, gy, t0, count, ksplit, ksteps,
-                   part, UA, UB, cmap);
+// Sums the ksplit partial blocks of the tiles cut into K ranges in order and applies C = alpha * sum (+ C).
+__global__ __launch_bounds__(kThreads) void presplit_reduce_kernel(SplitArgs p) {
+  const int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (e >= p.rem * PBM * PBN) return;
+  const int64_t q = e / (PBM * PBN);
+  const int in = (int)(e % (PBM * PBN)), ml = in % PBM, nl = in / PBM;
+  int64_t bx, by;
+  tile_xy(p.whole + q, p.gx, p.gy, bx, by);
+  const int64_t m = bx * PBM + ml, n = by * PBN + nl;
+  if (m >= p.M || n >= p.N) return;
+  const float *pb = p.part + q * p.ksplit * (PBM * PBN) + in;
+  float x = 0.0f;
+#pragma unroll 4
+  for (int ch = 0; ch < p.ksplit; ++ch) x += pb[(int64_t)ch * (PBM * PBN)];
+  float *c = p.C + (p.cmap ? p.cmap[m] + p.cmap[p.M + n] : m + n * p.ldc);
+  const float v = p.alpha * x;
+  *c = p.beta_one ? *c + v : v;
 }
 
 int64_t round_up(int64_t x, int64_t q) { return (x + q - 1) / q * q; }
@@ -679,41 +696,36 @@ __global__ __launch_bounds__(256) void offset_map_kernel(OffsetMap map, int64_t 
 // Splits op(X) (rows R, depth K) into NP planes at P (NP = 2: also the row
 // maxima into U, Rp entries, used for the scaling); returns 0 or a launch error.
 template <int NP>
-int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, int64_t Rp, int64_t Kp,
-                  uint16_t *P, uint32_t *U, hipStream_t s) {
-  const int64_t items = Rp * (Kp / 8), nblk = (items + 255) / 256;
+int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, int64_t Rp, int64_t Kp, uint4 *P,
+                  uint32_t *U, hipStream_t s) {
+  const int64_t nks = Kp / PBK, plane = Rp * Kp / 8;
+  const int64_t steps = kcont ? 64 / kSplitRows : 1, nblk = Rp / (64 / steps) * ((nks + steps - 1) / steps);
   if (nblk > 0x7fffffffLL) return -4;
   const int vec = ((uintptr_t)X % 16 == 0) && ld % 4 == 0;
   if (NP == 2 && kcont) {  // maxima and planes in one pass over HBM
-    if (Rp > 0x7fffffffLL) return -4;
-    split_rows_f16_kernel<<<dim3((unsigned)Rp), dim3(256), 0, s>>>(X, ld, R, K, Kp, P, Rp * Kp, vec, U);
+    if (Rp / 2 > 0x7fffffffLL) return -4;
+    split_rows_f16_kernel<<<dim3((unsigned)(Rp / 2)), dim3(kSplitThreads), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
     return hipGetLastError() == hipSuccess ? 0 : -2;
   }
   if constexpr (NP == 2) {
     fill_u32_kernel<<<dim3((unsigned)((Rp + 255) / 256)), dim3(256), 0, s>>>(U, Rp);
     if (R > 0 && K > 0) {
-      const int64_t rows = kcont ? 4 : 64;
-      int64_t kseg = kcont ? 2048 : 512;
-      kseg = std::max(kseg, round_up((K + 65534) / 65535, 256));
-      if ((R + rows - 1) / rows > 0x7fffffffLL) return -4;
-      const dim3 grid((unsigned)((R + rows - 1) / rows), (unsigned)((K + kseg - 1) / kseg));
-      if (kcont)
-        row_absmax_kernel<1><<<grid, dim3(256), 0, s>>>(X, ld, R, K, kseg, vec, U);
-      else
-        row_absmax_kernel<0><<<grid, dim3(256), 0, s>>>(X, ld, R, K, kseg, vec, U);
+      const int64_t kseg = std::max<int64_t>(512, round_up((K + 65534) / 65535, 256));
+      if ((R + 63) / 64 > 0x7fffffffLL) return -4;
+      const dim3 grid((unsigned)((R + 63) / 64), (unsigned)((K + kseg - 1) / kseg));
+      row_absmax_kernel<<<grid, dim3(256), 0, s>>>(X, ld, R, K, kseg, U);
     }
   }
   if (kcont)
-    split_planes_kernel<1, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, Rp, Kp, P, Rp * Kp, vec, U);
+    split_planes_kernel<1, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
   else
-    split_planes_kernel<0, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, Rp, Kp, P, Rp * Kp, vec, U);
+    split_planes_kernel<0, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// The tiles of C are dealt to the resident workgroups in rounds.  When the
-// last round is at most a quarter full (or the whole GEMM is), its `rem`
-// tiles are computed as ksplit K ranges each (filling the GPU) plus a
-// summing pass; ksplit = 1 means no split.
+// The tiles of C are dealt to the resident workgroups in rounds.  The `rem`
+// tiles of a partial last round may be computed as ksplit K ranges each; ksplit
+// = 1 means no split.
 struct TailSplit {
   int64_t rem = 0;
   int ksplit = 1;
@@ -764,28 +776,36 @@ static int64_t presplit_slots() {
     int cus = 0, per = 0;
     hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess)
-      e = NP == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, gemm_bf16x6p_kernel, 512, 0)
-                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, gemm_f16x3p_kernel, 512, 0);
+      e = NP == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, presplit_gemm_kernel<3>, 512, 0)
+                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, presplit_gemm_kernel<2>, 512, 0);
     if (e != hipSuccess) return 0;
     cache[dev] = (int64_t)cus * std::max(per, 1);
   }
   return cache[dev];
 }
 
-// K split of a mostly idle last round of tiles (as for the FP32/FP64 GEMM).
+// K split of a partial last round of tiles: as many ranges as make it shortest,
+// counted in K steps.  A range costs about 8 steps beside its own (its first
+// loads, its partial sums written and read again): 5184^3 in fp16x3 has 861
+// tiles on 256 slots, and its 93 last ones run as 5 ranges each, 0.5 of a round
+// instead of a whole one (and 20 us of summing against 110 saved).
 template <int NP>
 static TailSplit presplit_tail(int64_t M, int64_t N, int64_t K) {
   TailSplit t;
   if (M <= 0 || N <= 0) return t;
   const int64_t T = (round_up(M, PBM) / PBM) * (round_up(N, PBN) / PBN), slots = presplit_slots<NP>();
   if (slots <= 0) return t;
-  const int64_t rem = T % slots;
-  if (rem == 0 || rem * 4 > slots) return t;
-  const int64_t ksteps = round_up(std::max<int64_t>(K, 1), PBK) / PBK;
-  const int64_t ks = std::min<int64_t>(std::min<int64_t>(16, slots / rem), ksteps / 8);
-  if (ks < 2) return t;
-  t.rem = rem;
-  t.ksplit = (int)ks;
+  const int64_t rem = T % slots, nks = round_up(std::max<int64_t>(K, 1), PBK) / PBK;
+  if (rem == 0) return t;
+  int64_t best = nks;
+  for (int64_t ks = 2; ks <= 16 && ks * 8 <= nks; ++ks) {
+    const int64_t cost = (rem * ks + slots - 1) / slots * ((nks + ks - 1) / ks + 8);
+    if (cost < best) {
+      best = cost;
+      t.rem = rem;
+      t.ksplit = (int)ks;
+    }
+  }
   return t;
 }
 
@@ -820,41 +840,40 @@ static int launch_presplit(int opa, int opb, int64_t M, int64_t N, int64_t K, do
                            const int64_t *cmap, hipStream_t s) {
   const SplitLayout l = split_layout<NP>(M, N, K);
   char *w = (char *)ws;
-  uint16_t *pa = (uint16_t *)(w + l.a), *pb = (uint16_t *)(w + l.b);
+  uint4 *pa = (uint4 *)(w + l.a), *pb = (uint4 *)(w + l.b);
   uint32_t *ua = NP == 2 ? (uint32_t *)(w + l.ua) : nullptr, *ub = NP == 2 ? (uint32_t *)(w + l.ub) : nullptr;
-  float *part = (float *)(w + l.part);
   // A 'T' (KxM) and B 'N' (KxN) already have K contiguous per row of the plane
   if (int e = split_operand<NP>(opa == 1, (const float *)A, lda, M, K, l.Mp, l.Kp, pa, ua, s)) return e;
   if (int e = split_operand<NP>(opb == 0, (const float *)B, ldb, N, K, l.Np, l.Kp, pb, ub, s)) return e;
-  const int64_t gx = l.Mp / PBM, gy = l.Np / PBN;
-  if (gx * gy > 0x7fffffffLL) return -4;
-  const TailSplit ts = l.tail;
-  const int64_t full = gx * gy - ts.rem, nsteps = l.Kp / PBK;
-  const int64_t ksteps = ts.ksplit > 1 ? (nsteps + ts.ksplit - 1) / ts.ksplit : 0;
-  const int64_t apl = l.Mp * l.Kp / 8, bpl = l.Np * l.Kp / 8;
-  auto gemm = [&](int64_t blocks, int64_t t0, int64_t count, int ksplit, int64_t kst, float *pt) {
-    const dim3 grid((unsigned)blocks), block(512);
-    const bool last = ts.ksplit <= 1;  // no other launch follows
-    if (NP == 3 && last)
-      launch_last(gemm_bf16x6p_kernel, grid, block, s, M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl,
-                  (float *)C, ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, cmap);
-    else if (NP == 3)
-      gemm_bf16x6p_kernel<<<grid, block, 0, s>>>(M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C,
-                                                 ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, cmap);
-    else if (last)
-      launch_last(gemm_f16x3p_kernel, grid, block, s, M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl,
-                  (float *)C, ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, ua, ub, cmap);
-    else
-      gemm_f16x3p_kernel<<<grid, block, 0, s>>>(M, N, l.Kp, (const uint4 *)pa, apl, (const uint4 *)pb, bpl, (float *)C,
-                                                ldc, (float)ar, beta_one, gx, gy, t0, count, ksplit, kst, pt, ua, ub,
-                                                cmap);
-  };
-  if (full > 0) gemm(full, 0, full, 1, 0, nullptr);
-  if (ts.ksplit > 1) {
-    gemm(ts.rem * ts.ksplit, full, ts.rem, ts.ksplit, ksteps, part);
-    const int64_t nel = ts.rem * PBM * PBN;
-    launch_last(gemm_tail_reduce<float, 1, PBM, PBN>, dim3((unsigned)((nel + kThreads - 1) / kThreads)), dim3(kThreads), s,
-                M, N, part, ts.ksplit, (float *)C, ldc, (float)ar, 0.0f, beta_one, gx, gy, full, ts.rem, cmap);
+  SplitArgs p;
+  p.a = pa;
+  p.b = pb;
+  p.apl = l.Mp * l.Kp / 8;
+  p.bpl = l.Np * l.Kp / 8;
+  p.nks = l.Kp / PBK;
+  p.C = (float *)C;
+  p.cmap = cmap;
+  p.part = (float *)(w + l.part);
+  p.ua = ua;
+  p.ub = ub;
+  p.M = M;
+  p.N = N;
+  p.ldc = ldc;
+  p.gx = l.Mp / PBM;
+  p.gy = l.Np / PBN;
+  p.rem = l.tail.rem;
+  p.whole = p.gx * p.gy - p.rem;
+  p.ksplit = l.tail.ksplit;
+  p.ksteps = (p.nks + p.ksplit - 1) / p.ksplit;
+  p.beta_one = beta_one;
+  p.alpha = (float)ar;
+  if (p.gx * p.gy > 0x7fffffffLL - 16 * p.rem) return -4;
+  const dim3 grid((unsigned)(p.whole + p.rem * p.ksplit)), block(512);
+  if (p.rem == 0) {
+    launch_last(presplit_gemm_kernel<NP>, grid, block, s, p);
+  } else {
+    presplit_gemm_kernel<NP><<<grid, block, 0, s>>>(p);
+    launch_last(presplit_reduce_kernel, dim3((unsigned)(p.rem * PBM * PBN / kThreads)), dim3(kThreads), s, p);
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
