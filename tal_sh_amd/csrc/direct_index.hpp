@@ -13,6 +13,9 @@
 
 #include "batch_item.hpp"
 
+// Inlined before anything else is done, so that the kernel's arguments stay scalar loads.
+#define TAL_INLINE __attribute__((always_inline))
+
 namespace tal {
 
 constexpr int kDirectDims = 6;
@@ -31,7 +34,7 @@ struct DirectPair {
 };
 
 // Byte offset of x: 64-bit (D), and 32-bit for operands shorter than kOutside bytes.
-TAL_HD inline int64_t group_offset64(const DirectGroup &g, uint32_t x) {
+TAL_HD TAL_INLINE inline int64_t group_offset64(const DirectGroup &g, uint32_t x) {
   int64_t o = 0;
 #if defined(__HIPCC__)
 #pragma unroll
@@ -44,7 +47,7 @@ TAL_HD inline int64_t group_offset64(const DirectGroup &g, uint32_t x) {
   }
   return o + (int64_t)x * g.s[kDirectDims - 1];
 }
-TAL_HD inline uint32_t group_offset32(const DirectGroup &g, uint32_t x) {
+TAL_HD TAL_INLINE inline uint32_t group_offset32(const DirectGroup &g, uint32_t x) {
   uint32_t o = 0;
 #if defined(__HIPCC__)
 #pragma unroll
@@ -57,7 +60,7 @@ TAL_HD inline uint32_t group_offset32(const DirectGroup &g, uint32_t x) {
   }
   return o + x * (uint32_t)g.s[kDirectDims - 1];
 }
-TAL_HD inline void pair_offsets32(const DirectPair &g, uint32_t x, uint32_t *oa, uint32_t *ob) {
+TAL_HD TAL_INLINE inline void pair_offsets32(const DirectPair &g, uint32_t x, uint32_t *oa, uint32_t *ob) {
   uint32_t a = 0, b = 0;
 #if defined(__HIPCC__)
 #pragma unroll
@@ -85,7 +88,7 @@ struct RunWalk {
   int32_t e0;
   int32_t next[2], wrap[2];
 };
-TAL_HD inline RunWalk run_walk(const DirectPair &g) {
+TAL_HD TAL_INLINE inline RunWalk run_walk(const DirectPair &g) {
   RunWalk w;
   w.e0 = g.nd > 1 ? (int32_t)g.ext[0] : 0x7fffffff;
   for (int t = 0; t < 2; ++t) {
@@ -96,7 +99,7 @@ TAL_HD inline RunWalk run_walk(const DirectPair &g) {
   return w;
 }
 // Offsets of k, its place r in its run and the run's digit in the second dimension.
-TAL_HD inline void run_start(const DirectPair &g, int k, int64_t *oa, int64_t *ob, int *r, int *d1) {
+TAL_HD TAL_INLINE inline void run_start(const DirectPair &g, int k, int64_t *oa, int64_t *ob, int *r, int *d1) {
   if (g.nd == 1) {
     *oa = (int64_t)k * g.s[0][0];
     *ob = (int64_t)k * g.s[1][0];
@@ -139,10 +142,10 @@ struct DirectArgs {
   DirectGroup dm, dn;           // m and n in D
 };
 
-TAL_HD inline int64_t d_row(const DirectArgs &p, int m) {
+TAL_HD TAL_INLINE inline int64_t d_row(const DirectArgs &p, int m) {
   return p.flags & kDirectGroupDm ? group_offset64(p.dm, (uint32_t)m) : (int64_t)m * p.dm1;
 }
-TAL_HD inline int64_t d_col(const DirectArgs &p, int n) {
+TAL_HD TAL_INLINE inline int64_t d_col(const DirectArgs &p, int n) {
   return p.flags & kDirectGroupDn ? group_offset64(p.dn, (uint32_t)n) : (int64_t)n * p.dn1;
 }
 

@@ -41,6 +41,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "direct_index.hpp"
 
 namespace tal {
@@ -51,6 +53,14 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// The kernels read their arguments where they lie.  As a by-value parameter
+// the compiler keeps a private copy of all of them wherever a branch picks one
+// of two groups: 784 bytes of scratch memory a lane, and launches that took
+// 17-33 us longer.
+__device__ TAL_INLINE inline const DirectArgs &kernel_args() {
+  return *(const DirectArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+}
 
 template <typename S>
 struct Mfma;
@@ -118,15 +128,23 @@ __device__ inline int xcd_order(int u, int n) {
   return x * q + min(x, r) + (u >> 3);
 }
 
+template <typename S, int NC>
+__device__ TAL_INLINE inline void old_values(const char *__restrict__ D, const int64_t (&off)[4], Vec<S, NC> (&d)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (off[r] >= 0) d[r] = *reinterpret_cast<const Vec<S, NC> *>(D + off[r]);
+}
+
 // Values of one 16x16 accumulator block of this lane to D.  Along m (dn = 0):
 // the block is turned round through a wave-private LDS patch so that a store
 // covers 16 consecutive rows of 4 columns; along n the accumulator layout
 // already has 16 consecutive columns of 4 rows.  LDS accesses of one wave
 // complete in order, so the patch needs no barrier.
 // off[r]: byte offset of the lane's r-th element, negative when it is outside D.
+// old: D's values there (beta), read before.
 template <typename S, int NC, typename ACC>
-__device__ inline void emit_block(S *patch, int lane, const ACC (&acc)[NC], bool turn, char *__restrict__ D,
-                                  const int64_t (&off)[4], S ar, S ai, bool beta) {
+__device__ TAL_INLINE inline void emit_block(S *patch, int lane, const ACC (&acc)[NC], bool turn, char *__restrict__ D,
+                                             const int64_t (&off)[4], S ar, S ai, bool beta, const Vec<S, NC> (&old)[4]) {
   constexpr int TP = 17;
   const int tl = lane & 15, tg = lane >> 4;
   Vec<S, NC> v[4];
@@ -146,12 +164,6 @@ __device__ inline void emit_block(S *patch, int lane, const ACC (&acc)[NC], bool
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r].v[c] = acc[c][r];
   }
-  Vec<S, NC> d[4];
-  if (beta) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (off[r] >= 0) d[r] = *reinterpret_cast<const Vec<S, NC> *>(D + off[r]);
-  }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     Vec<S, NC> x;
@@ -164,50 +176,36 @@ __device__ inline void emit_block(S *patch, int lane, const ACC (&acc)[NC], bool
     }
     if (beta) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) x.v[c] = d[r].v[c] + x.v[c];
+      for (int c = 0; c < NC; ++c) x.v[c] = old[r].v[c] + x.v[c];
     }
     if (off[r] >= 0) *reinterpret_cast<Vec<S, NC> *>(D + off[r]) = x;
   }
 }
 
+// D offsets of rows and columns; past the edge, a value whose sum with any offset is negative (|offsets| < 2^62).
+constexpr int64_t kNone = -((int64_t)1 << 62);
+__device__ TAL_INLINE inline int64_t row_or_none(const DirectArgs &p, int m) { return m < p.M ? d_row(p, m) : kNone; }
+__device__ TAL_INLINE inline int64_t col_or_none(const DirectArgs &p, int n) { return n < p.N ? d_col(p, n) : kNone; }
+
 // D offsets of a wave's TM x TN slab, one 16x16 block at a time.
-template <typename S, int SM, int SN>
+// DN: stored along n.  A template parameter: with indexes that depend on a
+// variable the arrays would live in scratch memory.
+template <typename S, int SM, int SN, bool DN>
 struct SlabOffsets {
-  int64_t o[SM * 4 + SN * 4];
-  // rows from m0, columns from n0; -1 past the edge (sums with it stay negative: |offsets| < 2^62)
-  __device__ SlabOffsets(const DirectArgs &p, int m0, int n0, int lane) {
-    constexpr int64_t kNone = -((int64_t)1 << 62);
+  static constexpr int RR = DN ? 4 : 1, CC = DN ? 1 : 4;
+  int64_t rows[SM * RR], cols[SN * CC];
+  // row(m), col(n): offsets of the slab's m-th row and n-th column
+  template <class R, class C>
+  __device__ TAL_INLINE SlabOffsets(int lane, R row, C col) {
     const int fl = lane & 15, fg = lane >> 4;
-    if (!(p.flags & kDirectAlongN)) {
 #pragma unroll
-      for (int i = 0; i < SM; ++i) {
-        const int m = m0 + i * 16 + fl;
-        o[i] = m < p.M ? d_row(p, m) : kNone;
-      }
+    for (int i = 0; i < SM * RR; ++i) rows[i] = row(DN ? (i / RR) * 16 + Mfma<S>::row(lane, i % RR) : i * 16 + fl);
 #pragma unroll
-      for (int j = 0; j < SN * 4; ++j) {
-        const int n = n0 + (j >> 2) * 16 + 4 * (j & 3) + fg;
-        o[SM * 4 + j] = n < p.N ? d_col(p, n) : kNone;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < SM * 4; ++i) {
-        const int m = m0 + (i >> 2) * 16 + Mfma<S>::row(lane, i & 3);
-        o[i] = m < p.M ? d_row(p, m) : kNone;
-      }
-#pragma unroll
-      for (int j = 0; j < SN; ++j) {
-        const int n = n0 + j * 16 + fl;
-        o[SM * 4 + j] = n < p.N ? d_col(p, n) : kNone;
-      }
-    }
+    for (int j = 0; j < SN * CC; ++j) cols[j] = col(DN ? j * 16 + fl : (j / CC) * 16 + 4 * (j % CC) + fg);
   }
-  __device__ void block(bool dn, int i, int j, int64_t (&off)[4]) const {
+  __device__ TAL_INLINE void block(int i, int j, int64_t (&off)[4]) const {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t x = dn ? o[i * 4 + r] + o[SM * 4 + j] : o[i] + o[SM * 4 + j * 4 + r];
-      off[r] = x;
-    }
+    for (int r = 0; r < 4; ++r) off[r] = DN ? rows[i * RR + r % RR] + cols[j] : rows[i] + cols[j * CC + r % CC];
   }
 };
 
@@ -218,10 +216,18 @@ struct SlabOffsets {
 //   1  k starts with a run of at least KB (or an operand is 2 GiB or more): a
 //      scalar base per step and, where the step crosses into the next run, one
 //      more scalar for the lanes past the crossing
-//   2  any k: every lane works its offset out
+//   2  any k: offsets by table.  The offsets of each row, column and contracted
+//      index are worked out once, by one thread, and read from LDS, those of k a
+//      step ahead of the loads that use them and with offsets outside the
+//      operands past k's end, so that the last, partial step is like the others.
+//      Worked out for every load they took 6 KB of code a step, and a small
+//      product ran as long as its code took to arrive: 77 x 72 by 60 R8 9.7 ->
+//      8.1 us of kernel, 399 x 440 by 195 18.0 -> 13.6 (R4, whose compilation
+//      needed scratch memory, 50 -> 14).
 template <typename S, int NC, int KA, int KBC, int WA, int WB, int BM, int BN, int KB, int WM, int WN, int PF, int OCC,
           int MODE>
-__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void direct_kernel(DirectArgs p) {
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void direct_kernel(DirectArgs) {
+  const DirectArgs &p = kernel_args();
   using MF = Mfma<S>;
   using acc_t = typename MF::acc_t;
   constexpr int NT = 64 * WM * WN;
@@ -274,16 +280,51 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   const int ac = (tid % ALINE) * WA, bc = (tid % BLINE) * WB;
   const int al = ALINE % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / ALINE) : tid / ALINE;
   const int bl = BLINE % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / BLINE) : tid / BLINE;
+  // Mode 2: offsets by table.  Rows, columns and D's of both once; k in two
+  // halves of kHalf, one filled while loads read the other.
+  constexpr bool TAB = MODE == 2;
+  constexpr int kHalf = 256;
+  static_assert(!TAB || (WA == 1 && WB == 1 && kHalf % KB == 0 && kHalf <= NT && kHalf >= PF * KB), "tables");
+  __shared__ uint32_t arow_t[TAB ? BM : 1], brow_t[TAB ? BN : 1];
+  __shared__ int64_t drow_t[TAB ? BM : 1], dcol_t[TAB ? BN : 1];
+  __shared__ uint2 k_t[TAB ? 2 * kHalf : 1];
+  auto arow = [&](int r) TAL_INLINE -> uint32_t {
+    return r >= p.M ? kOutside : ga ? group_offset32(p.am, (uint32_t)r) : (uint32_t)(r - am0) * (uint32_t)p.am1;
+  };
+  auto brow = [&](int r) TAL_INLINE -> uint32_t {
+    return r >= p.N ? kOutside : gb ? group_offset32(p.bn, (uint32_t)r) : (uint32_t)(r - bn0) * (uint32_t)p.bn1;
+  };
+  auto fill_k = [&](int h) TAL_INLINE {  // half h of this K range; past its end, offsets outside both operands
+    if (kHalf == NT || tid < kHalf) {
+      const int k = kbeg + h * kHalf + tid;
+      uint2 o = make_uint2(kOutside, kOutside);
+      if (k < kend) pair_offsets32(p.k, (uint32_t)k, &o.x, &o.y);
+      k_t[(h & 1) * kHalf + tid] = o;
+    }
+  };
+  if (TAB) {
+    fill_k(0);
+    if (kbeg + kHalf < kend) fill_k(1);
+    static_assert(!TAB || BM + BN <= NT, "a thread per row and column");
+    if (tid < BM) {
+      arow_t[tid] = arow(m0 + tid);
+      drow_t[tid] = row_or_none(p, m0 + tid);
+    } else if (tid < BM + BN) {
+      brow_t[tid - BM] = brow(n0 + tid - BM);
+      dcol_t[tid - BM] = col_or_none(p, n0 + tid - BM);
+    }
+    __syncthreads();
+  }
   uint32_t aro[KA ? NVA : 1], bro[KBC ? NVB : 1];
 #pragma unroll
   for (int j = 0; j < (KA ? NVA : 1); ++j) {
-    const int r = m0 + (KA ? al + j * ASTEP : ac);
-    aro[j] = r >= p.M ? kOutside : ga ? group_offset32(p.am, (uint32_t)r) : (uint32_t)(r - am0) * (uint32_t)p.am1;
+    const int r = KA ? al + j * ASTEP : ac;
+    aro[j] = TAB ? arow_t[r] : arow(m0 + r);
   }
 #pragma unroll
   for (int j = 0; j < (KBC ? NVB : 1); ++j) {
-    const int r = n0 + (KBC ? bl + j * BSTEP : bc);
-    bro[j] = r >= p.N ? kOutside : gb ? group_offset32(p.bn, (uint32_t)r) : (uint32_t)(r - bn0) * (uint32_t)p.bn1;
+    const int r = KBC ? bl + j * BSTEP : bc;
+    bro[j] = TAB ? brow_t[r] : brow(n0 + r);
   }
 
   Vec<S, WA * NC> ra[PF][NVA];
@@ -306,10 +347,27 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
     abase += oa;
     bbase += ob;
   }
+  // What the K loop needs of the arguments, held in scalar registers: read again
+  // in the loop, they come with branches around the loads (4096^3 R4 987 -> 1013 us).
+  uint32_t astep = KB * (uint32_t)p.ka1, bstep = KB * (uint32_t)p.kb1;
+  int64_t abase_step = KB * p.ka1, bbase_step = KB * p.kb1;
+  uint32_t kext1 = MODE == 1 ? p.k.ext[1] : 0;
+  asm volatile("" : "+s"(astep), "+s"(bstep), "+s"(abase_step), "+s"(bbase_step), "+s"(kext1));
   // The next whole K step into a register set.  Past the last whole step the
   // same step is loaded again and never multiplied.
   int kload = kbeg;
-  auto load = [&](int set) {
+  // mode 2: the table's offsets for the step at kload, read a step ahead of
+  // their use (but by 128 x 128 tiles, which have no registers for that)
+  constexpr bool AHEAD = BM * BN < 128 * 128;
+  auto next_k = [&]() TAL_INLINE {
+    const uint2 *t = k_t + ((kload - kbeg) & (2 * kHalf - 1));
+#pragma unroll
+    for (int j = 0; j < NVA; ++j) av[j] = t[KA ? ac : al + j * ASTEP].x;
+#pragma unroll
+    for (int j = 0; j < NVB; ++j) bv[j] = t[KBC ? bc : bl + j * BSTEP].y;
+  };
+  if (TAB && AHEAD) next_k();
+  auto load = [&](int set) TAL_INLINE {
     const bool more = kload + 2 * KB <= kend;
     if (MODE == 0) {
       const auto rsa = rsrc(abase, kOutside), rsb = rsrc(bbase, kOutside);
@@ -317,13 +375,13 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
       for (int j = 0; j < NVA; ++j) ra[set][j] = bload<S, WA * NC>(rsa, av[j]);
 #pragma unroll
       for (int j = 0; j < NVB; ++j) rb[set][j] = bload<S, WB * NC>(rsb, bv[j]);
-      const uint32_t sa = more ? KB * (uint32_t)p.ka1 : 0, sb = more ? KB * (uint32_t)p.kb1 : 0;
+      const uint32_t sa = more ? astep : 0, sb = more ? bstep : 0;
 #pragma unroll
       for (int j = 0; j < NVA; ++j) av[j] += sa;
 #pragma unroll
       for (int j = 0; j < NVB; ++j) bv[j] += sb;
     } else if (MODE == 1) {
-      const bool wrap = kd1 + 1 == (int)p.k.ext[1];
+      const bool wrap = kd1 + 1 == (int)kext1;
       const int da = wrap ? rw.wrap[0] : rw.next[0], db = wrap ? rw.wrap[1] : rw.next[1];
       const int cross = rw.e0 - kr;  // the step's elements from here on are in the next run: da / db further on
       const auto rsa = rsrc(abase + min(da, 0), kOutside), rsb = rsrc(bbase + min(db, 0), kOutside);
@@ -337,31 +395,31 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
         rb[set][j] = bload<S, WB * NC>(rsb, bv[j] + ((KBC ? bc : bl + j * BSTEP) >= cross ? b1 : b0));
       const bool over = kr + KB >= rw.e0;
       if (more) {
-        abase += (int64_t)KB * p.ka1 + (over ? da : 0);
-        bbase += (int64_t)KB * p.kb1 + (over ? db : 0);
+        abase += abase_step + (over ? da : 0);
+        bbase += bbase_step + (over ? db : 0);
         kr += over ? KB - rw.e0 : KB;
         kd1 = !over ? kd1 : wrap ? 0 : kd1 + 1;
       }
     } else {
       const auto rsa = rsrc(abase, kOutside), rsb = rsrc(bbase, kOutside);
-      uint32_t ka = 0, kb = 0, x;
-      if (KA) pair_offsets32(p.k, (uint32_t)(kload + ac), &ka, &kb);
-      if (KBC && !(KA && WA == WB)) pair_offsets32(p.k, (uint32_t)(kload + bc), &x, &kb);
+      if (!AHEAD) next_k();
 #pragma unroll
-      for (int j = 0; j < NVA; ++j) {
-        if (!KA) pair_offsets32(p.k, (uint32_t)(kload + al + j * ASTEP), &ka, &x);
-        ra[set][j] = bload<S, WA * NC>(rsa, aro[KA ? j : 0] + ka);
-      }
+      for (int j = 0; j < NVA; ++j) ra[set][j] = bload<S, WA * NC>(rsa, aro[KA ? j : 0] + av[j]);
 #pragma unroll
-      for (int j = 0; j < NVB; ++j) {
-        if (!KBC) pair_offsets32(p.k, (uint32_t)(kload + bl + j * BSTEP), &x, &kb);
-        rb[set][j] = bload<S, WB * NC>(rsb, bro[KBC ? j : 0] + kb);
+      for (int j = 0; j < NVB; ++j) rb[set][j] = bload<S, WB * NC>(rsb, bro[KBC ? j : 0] + bv[j]);
+      const int next = kload + KB;
+      if (next < kend) {
+        kload = next;
+        const int h = (kload - kbeg) / kHalf;
+        if ((kload - kbeg) % kHalf == 0 && kload + kHalf < kend) fill_k(h + 1);  // half h - 1 is no longer read
+        if (AHEAD) next_k();
       }
+      return;
     }
     kload += more ? KB : 0;
   };
   // the last, partial K step, from k0: element by element, zeros past kend
-  auto load_tail = [&](int k0) {
+  auto load_tail = [&](int k0) TAL_INLINE {
     const bool lin = MODE == 0 || (MODE == 1 && p.k.nd == 1);
     const char *at = (const char *)p.A + (int64_t)blockIdx.y * p.sa + (int64_t)am0 * p.am1;
     const char *bt = (const char *)p.B + (int64_t)blockIdx.y * p.sb + (int64_t)bn0 * p.bn1;
@@ -370,7 +428,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
       bt += (int64_t)k0 * p.kb1;
     }
     const auto rsa = rsrc(at, kOutside), rsb = rsrc(bt, kOutside);
-    auto off = [&](int k, int t) -> uint32_t {
+    auto off = [&](int k, int t) TAL_INLINE -> uint32_t {
       if (k >= kend) return kOutside;
       if (lin) return (uint32_t)(k - k0) * (uint32_t)(t ? p.kb1 : p.ka1);
       uint32_t o[2];
@@ -405,7 +463,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
     }
   };
   const S sgna = p.flags & kDirectConjA ? (S)-1 : (S)1, sgnb = p.flags & kDirectConjB ? (S)-1 : (S)1;
-  auto stage = [&](int buf, int set) {
+  auto stage = [&](int buf, int set) TAL_INLINE {
 #pragma unroll
     for (int j = 0; j < NVA; ++j) {
       const int line = al + j * ASTEP;
@@ -438,8 +496,24 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
       for (int c = 0; c < NC; ++c) acc[i][j][c] = acc_t{0, 0, 0, 0};
 
+  // Where a wave has one block and offsets come from tables, it reads D ahead of its products.
+  constexpr bool EARLY = TAB && SM * SN == 1;
+  const bool dn = p.flags & kDirectAlongN, beta = p.flags & kDirectBeta;
+  char *D = (char *)p.D + (int64_t)blockIdx.y * p.sd;
+  auto drow = [&](int m) TAL_INLINE { return TAB ? drow_t[wm * TM + m] : row_or_none(p, m0 + wm * TM + m); };
+  auto dcol = [&](int n) TAL_INLINE { return TAB ? dcol_t[wn * TN + n] : col_or_none(p, n0 + wn * TN + n); };
+  int64_t off0[4];
+  Vec<S, NC> old[4];
+  auto read_old = [&]() TAL_INLINE {
+    if (EARLY && !part) {
+      if (dn) SlabOffsets<S, SM, SN, true>(lane, drow, dcol).block(0, 0, off0);
+      else SlabOffsets<S, SM, SN, false>(lane, drow, dcol).block(0, 0, off0);
+      if (beta) old_values(D, off0, old);
+    }
+  };
+
   const int fl = lane & 15, fg = lane >> 4;
-  auto compute = [&](int buf) {
+  auto compute = [&](int buf) TAL_INLINE {
 #pragma unroll
     for (int q = 0; q < KB / (4 * KQ); ++q) {
       // lane group g holds k = 4 KQ q + KQ g + h in MFMA step h, in both operands
@@ -483,16 +557,20 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
     }
   };
 
-  const int nfull = max(0, kend - kbeg) / KB;
+  // whole K steps; in mode 2 the last step may be a partial one like any other
+  const int nfull = TAB ? (max(0, kend - kbeg) + KB - 1) / KB : max(0, kend - kbeg) / KB;
   if (nfull > 0) {
 #pragma unroll
     for (int q = 0; q < PF; ++q) load(q);
+    read_old();
     stage(0, 0);
     __syncthreads();
+  } else {
+    read_old();
   }
   // K step kt: the loads of step kt + PF go out, step kt + 1 (loaded PF - 1
   // steps ago) is staged into the other LDS buffer, step kt is multiplied
-  auto step = [&](int q, int buf) {
+  auto step = [&](int q, int buf) TAL_INLINE {
     load(q);
     __builtin_amdgcn_sched_barrier(0);  // the loads go out first
     if (PF > 1) stage(buf ^ 1, (q + 1) % PF);
@@ -509,7 +587,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
   for (int q = 0; q < U - 1; ++q)
     if (kt + q < nfull) step(q % PF, q & 1);
-  if (kbeg + nfull * KB < kend) {
+  if (!TAB && kbeg + nfull * KB < kend) {
     load_tail(kbeg + nfull * KB);
     stage(0, 0);
     __syncthreads();
@@ -531,22 +609,42 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   }
   static_assert(sizeof(As) >= sizeof(S) * WM * WN * 16 * 17, "patches fit the A tiles' space");
   S *patch = &As[0][0][0][0] + wave * 16 * 17;
-  const bool dn = p.flags & kDirectAlongN;
-  char *D = (char *)p.D + (int64_t)blockIdx.y * p.sd;
-  const SlabOffsets<S, SM, SN> so(p, m0 + wm * TM, n0 + wn * TN, lane);
+  if constexpr (EARLY) {
+    emit_block<S, NC, acc_t>(patch, lane, acc[0][0], !dn, D, off0, (S)p.ar, (S)p.ai, beta, old);
+  } else {
+    auto emit = [&](auto along_n) TAL_INLINE {
+      constexpr bool DN = decltype(along_n)::value;
+      const SlabOffsets<S, SM, SN, DN> so(lane, drow, dcol);
+      // D's old values are read DIST blocks before theirs are stored: a wave that
+      // reads and stores block by block waits for memory at every block (C4
+      // rank-6 product of K = 24, 755 MB of D: 541 -> 516 us).  The largest real
+      // tiles have no registers for it (R8: 313 us, 463 with DIST = 4), but more
+      // waves that wait in turn.
+      constexpr int NBLK = SM * SN, DIST = NC == 1 && NBLK > 2 ? 0 : NBLK < 4 ? NBLK : 4;
+      int64_t off[DIST + 1][4];
+      Vec<S, NC> d[DIST + 1][4];
+      auto fetch = [&](int b) TAL_INLINE {
+        so.block(b / SN, b % SN, off[b % (DIST + 1)]);
+        if (beta) old_values(D, off[b % (DIST + 1)], d[b % (DIST + 1)]);
+      };
 #pragma unroll
-  for (int i = 0; i < SM; ++i)
+      for (int b = 0; b < DIST; ++b) fetch(b);
 #pragma unroll
-    for (int j = 0; j < SN; ++j) {
-      int64_t off[4];
-      so.block(dn, i, j, off);
-      emit_block<S, NC, acc_t>(patch, lane, acc[i][j], !dn, D, off, (S)p.ar, (S)p.ai, p.flags & kDirectBeta);
-    }
+      for (int b = 0; b < NBLK; ++b) {
+        if (b + DIST < NBLK) fetch(b + DIST);
+        emit_block<S, NC, acc_t>(patch, lane, acc[b / SN][b % SN], !DN, D, off[b % (DIST + 1)], (S)p.ar, (S)p.ai, beta,
+                                 d[b % (DIST + 1)]);
+      }
+    };
+    if (dn) emit(std::true_type());
+    else emit(std::false_type());
+  }
 }
 
 // Sums the ksplit partial blocks of each split tile in order; one wave per 16x16 block.
 template <typename S, int NC, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256) void direct_reduce(DirectArgs p) {
+__global__ __launch_bounds__(256) void direct_reduce(DirectArgs) {
+  const DirectArgs &p = kernel_args();
   using acc_t = typename Mfma<S>::acc_t;
   constexpr int TM = BM / WM, TN = BN / WN, SM = TM / 16, SN = TN / 16, PER = SM * SN * NC * 4 * 64;
   __shared__ S patches[4][16 * 17];
@@ -556,6 +654,17 @@ __global__ __launch_bounds__(256) void direct_reduce(DirectArgs p) {
   const int tile = blk / BPT, in = blk % BPT;
   if (tile >= p.rem) return;
   const int wave = in / (SM * SN), ij = in % (SM * SN), i = ij / SN, j = ij % SN;
+  int bx, by;
+  tile_xy(p.whole + tile, p.gx, p.gy, bx, by);
+  const int mb = bx * BM + (wave % WM) * TM + i * 16, nb = by * BN + (wave / WM) * TN + j * 16;
+  auto drow = [&](int m) TAL_INLINE { return row_or_none(p, mb + m); };
+  auto dcol = [&](int n) TAL_INLINE { return col_or_none(p, nb + n); };
+  const bool dn = p.flags & kDirectAlongN, beta = p.flags & kDirectBeta;
+  int64_t off[4];
+  if (dn) SlabOffsets<S, 1, 1, true>(lane, drow, dcol).block(0, 0, off);
+  else SlabOffsets<S, 1, 1, false>(lane, drow, dcol).block(0, 0, off);
+  Vec<S, NC> old[4];
+  if (beta) old_values((const char *)p.D, off, old);
   acc_t acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = acc_t{0, 0, 0, 0};
@@ -567,13 +676,7 @@ __global__ __launch_bounds__(256) void direct_reduce(DirectArgs p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[c][r] += pb[(c * 4 + r) * 64];
   }
-  int bx, by;
-  tile_xy(p.whole + tile, p.gx, p.gy, bx, by);
-  const SlabOffsets<S, 1, 1> so(p, bx * BM + (wave % WM) * TM + i * 16, by * BN + (wave / WM) * TN + j * 16, lane);
-  const bool dn = p.flags & kDirectAlongN;
-  int64_t off[4];
-  so.block(dn, 0, 0, off);
-  emit_block<S, NC, acc_t>(patches[w], lane, acc, !dn, (char *)p.D, off, (S)p.ar, (S)p.ai, p.flags & kDirectBeta);
+  emit_block<S, NC, acc_t>(patches[w], lane, acc, !dn, (char *)p.D, off, (S)p.ar, (S)p.ai, beta, old);
 }
 
 }  // namespace direct

@@ -39,10 +39,15 @@ void run_layout(const DirectVariant &v, const DirectArgs &a, unsigned batch, hip
   else run<S, NC, T, 0, 0, W, MODE>(a, batch, s);
 }
 
-// Mode 2 (any k) is for small problems: element loads only.
+// Mode 2 (any k, offsets by table) is for small problems: element loads only.
+// 32 x 32 tiles take it for every k of several dimensions, also where its
+// leading run would do for mode 1, whose steps carry more code (418 x 420 by
+// 475 R8 22.7 -> 19.2 us, by 105 C8 17.4 -> 15.8, by 665 R4 20.5 -> 18.4; with
+// one dimension mode 0 is the faster one, 9.0 against 9.8).
 template <typename S, int NC, class T, int W>
 bool run_tile(const DirectVariant &v, const DirectArgs &a, unsigned batch, hipStream_t s) {
-  if (v.mode == 2) run_layout<S, NC, T, 1, 2>(v, a, batch, s);
+  const bool tables = v.mode == 2 || (v.mode == 1 && a.k.nd > 1 && T::BM * T::BN == 32 * 32);
+  if (tables) run_layout<S, NC, T, 1, 2>(v, a, batch, s);
   else if (v.mode == 1 && v.width == W) run_layout<S, NC, T, W, 1>(v, a, batch, s);
   else if (v.mode == 1) run_layout<S, NC, T, 1, 1>(v, a, batch, s);
   else if (v.width == W) run_layout<S, NC, T, W, 0>(v, a, batch, s);
