@@ -539,8 +539,12 @@ enum Route { kRouteDirect, kRouteCopies, kRouteWide, kRouteSplit };
 // Straight from the tensors where the transposes would cost more than the
 // reads in place do.  Measured (R8): a K step that walks runs of k costs 4 %
 // of a product in 128 x 128 tiles (9216^3: 21.99 -> 22.66 ms) and about a
-// quarter in smaller ones (1024^3: 41 -> 50 us); one whose every lane works
-// its offsets out, 40 %; D written 8 bytes apart, about four times its bytes.
+// quarter in smaller ones (1024^3: 41 -> 50 us), there with runs of any length,
+// as offsets then come from tables (runs of 20-24 by copies and in place: R8
+// 930 x 957 by 616 60 -> 56 us, 1480 x 1189 by 280 55 -> 51, C4 311 x 336 by
+// 600 40 -> 34, C8 550 x 552 by 420 64 -> 65; runs of 32, R8 1024^3, 72 -> 79);
+// in 128 x 128 tiles short runs cost 40 %; D written 8 bytes apart, about four
+// times its bytes.
 // A transpose moves 4.6 TB/s and takes about 4 us beside that.
 Route plan_route(const ContractPlan &plan, int dk) {
   if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) return kRouteSplit;
@@ -558,7 +562,7 @@ Route plan_route(const ContractPlan &plan, int dk) {
     const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
     const double gemm = c.us;
     double extra = 0;
-    if (plan.direct_krun) extra += (plan.direct_krun < 32 ? 0.4 : c.tile == 0 ? 0.05 : 0.25) * gemm;
+    if (plan.direct_krun) extra += (c.tile ? 0.25 : plan.direct_krun < 32 ? 0.4 : 0.05) * gemm;
     if (plan.direct_run && plan.direct_run < 8) extra += 0.3 * gemm;
     if (plan.direct_conflict) extra += std::min(avol, bvol) > 4e6 ? 1e9 : 0.5 * gemm;
     if (plan.direct_scatter) extra += 4 * dvol / 4.6e6;
