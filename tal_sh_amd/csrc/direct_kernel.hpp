@@ -258,9 +258,15 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   if (!part) {
     tile = u = xcd_order(u, p.whole);
   } else {
+    // by K range, then by tile: the tiles of one range read the same panels,
+    // side by side on an XCD, so its L2 serves them.  A call by tile first and
+    // by range first, us: 189 x 278 by 147864 R8 (27 tiles in 56 ranges) 600 and
+    // 443, 240 x 264 by 70400 322 and 236, 300 x 400 by 60000 R4 281 and 160; 76
+    // x 5254 by 20952, whose tiles share one panel only, 478 and 504.
     u = xcd_order(u - p.whole, p.rem * p.ksplit);
-    tile = u / p.ksplit;
-    kpart = u - tile * p.ksplit;
+    kpart = u / p.rem;
+    tile = u - kpart * p.rem;
+    u = tile * p.ksplit + kpart;  // place of the partial sums
     tile += p.whole;
   }
   int bx, by;

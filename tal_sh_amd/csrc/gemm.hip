@@ -503,9 +503,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (!range) {
     tile = xcd_order(blockIdx.x, whole);
   } else {
+    // by K range, then by tile: the tiles of one range share panels in an XCD's L2
     unit = xcd_order(unit, p.rem * p.ksplit);
-    tile = unit / p.ksplit;
-    kt0 = (unit - tile * p.ksplit) * p.ksteps;
+    const int64_t kpart = unit / p.rem;
+    tile = unit - kpart * p.rem;
+    unit = tile * p.ksplit + kpart;  // place of the partial sums
+    kt0 = kpart * p.ksteps;
     kt1 = min(kt1, kt0 + p.ksteps);
     tile += whole;
   }
