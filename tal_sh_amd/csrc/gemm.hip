@@ -355,59 +355,60 @@ __device__ inline void split_store(const float (&v)[8], int e, uint4 *__restrict
 }
 
 // fp16x3 planes of op(X) when its rows are K-contiguous (X(r, k) at
-// X[r*ld + k]).  A block takes two padded rows, 256 threads each: it finds their
-// largest magnitudes (U[r], 0 for padding rows) and splits them, four threads on
-// the 32 k of a row's part of a plane block (128 bytes read; 128 written, the
-// two rows side by side).  The first kHeld chunks of a thread stay in registers
+// X[r*ld + k]).  A block takes 2^rows_log padded rows: it finds their largest
+// magnitudes (U[r], 0 for padding rows) and splits them, four threads on the 32
+// k of a row's part of a plane block (128 bytes read, 64 written, the block's
+// rows side by side).  The first kHeld chunks of a thread stay in registers
 // between the two, so rows of up to 8,192 are read once; longer ones' other
 // chunks are read again.  vec: X 16-byte aligned and ld a multiple of 4.
-// Memory-bound: 5184 x 5184 in 46 us, 4.7 TB/s
-// (two passes over a row per block: 60).
-constexpr int kSplitThreads = 512;
+// Memory-bound: 5184 x 5184, two rows a block, in 46 us, 4.7 TB/s (two passes
+// over a row per block: 60).  Short rows go many to a block, as long as their
+// chunks stay in registers and there are blocks for all CUs (split_rows_log).
+constexpr int kSplitThreads = 512, kHeld = 4;
+int split_rows_log(int64_t nks, int64_t Rp) {
+  int l = 1;
+  while (l < 7 && (kSplitThreads / 8 >> l) * kHeld >= nks && Rp >> l > 1024) ++l;
+  return l;
+}
 __global__ __launch_bounds__(kSplitThreads) void split_rows_f16_kernel(const float *__restrict__ X, int64_t ld,
                                                                        int64_t R, int64_t K, int64_t nks,
                                                                        uint4 *__restrict__ P, int64_t plane, int vec,
-                                                                       uint32_t *__restrict__ U) {
-  constexpr int kHeld = 4, kRound = kSplitThreads / 8;  // K steps per round of the block
-  __shared__ uint32_t red[2][8];
-  const int tid = threadIdx.x, c = tid & 3, row = (tid >> 2) & 1, lane = tid & 63, wave = tid >> 6;
-  const int64_t r = (int64_t)blockIdx.x * 2 + row, n = r < R ? K : 0;
+                                                                       uint32_t *__restrict__ U, int rows_log) {
+  __shared__ uint32_t red[kSplitThreads / 4];
+  const int tid = threadIdx.x, c = tid & 3, row = tid >> 2 & ((1 << rows_log) - 1);
+  const int ks0 = tid >> (2 + rows_log), round = kSplitThreads / 4 >> rows_log;  // K steps per round of the block
+  const int64_t r = ((int64_t)blockIdx.x << rows_log) + row, n = r < R ? K : 0;
   const float *x = X + r * ld;
+  if (tid < kSplitThreads / 4) red[tid] = 0;
   float v[kHeld][8];
   uint32_t m = 0;
 #pragma unroll
-  for (int q = 0; q < kHeld; ++q) {
-    const int64_t ks = (tid >> 3) + q * kRound;
-    load8(x, ks * PBK + c * 8, n, vec, v[q]);
-  }
+  for (int q = 0; q < kHeld; ++q) load8(x, (int64_t)(ks0 + q * round) * PBK + c * 8, n, vec, v[q]);
 #pragma unroll
   for (int q = 0; q < kHeld; ++q)
 #pragma unroll
     for (int i = 0; i < 8; ++i) m = max(m, abs_bits(v[q][i]));
-  for (int64_t ks = (tid >> 3) + kHeld * kRound; ks < nks; ks += kRound) {
+  for (int64_t ks = ks0 + kHeld * round; ks < nks; ks += round) {
     float w[8];
     load8(x, ks * PBK + c * 8, n, vec, w);
 #pragma unroll
     for (int i = 0; i < 8; ++i) m = max(m, abs_bits(w[i]));
   }
-  // lane bit 2 is the row
-#pragma unroll
-  for (int o = 32; o > 4; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
-#pragma unroll
-  for (int o = 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
-  if ((lane & ~4) == 0) red[row][wave] = m;
+  // the four threads of a chunk row, then the wave's and the block's others in LDS
+  m = max(m, (uint32_t)__shfl_xor((int)m, 1));
+  m = max(m, (uint32_t)__shfl_xor((int)m, 2));
   __syncthreads();
-  m = 0;
-#pragma unroll
-  for (int w = 0; w < 8; ++w) m = max(m, red[row][w]);
-  if ((tid & ~4) == 0) U[r] = m;
+  if (c == 0) atomicMax(&red[row], m);
+  __syncthreads();
+  m = red[row];
+  if (ks0 == 0 && c == 0) U[r] = m;
   const int e = row_exp(m);
 #pragma unroll
   for (int q = 0; q < kHeld; ++q) {
-    const int64_t ks = (tid >> 3) + q * kRound;
+    const int64_t ks = ks0 + q * round;
     if (ks < nks) split_store<2>(v[q], e, P, plane, plane_chunk(r, ks * 4 + c, nks));
   }
-  for (int64_t ks = (tid >> 3) + kHeld * kRound; ks < nks; ks += kRound) {
+  for (int64_t ks = ks0 + kHeld * round; ks < nks; ks += round) {
     float w[8];
     load8(x, ks * PBK + c * 8, n, vec, w);
     split_store<2>(w, e, P, plane, plane_chunk(r, ks * 4 + c, nks));
@@ -641,25 +642,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   int64_t om[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) om[i] = m0 + i * 16 >= p.M ? -1 : p.cmap ? p.cmap[m0 + i * 16] : m0 + i * 16;
+  // The columns' offsets are read together and the old values of four columns
+  // while the four before are stored: one after the other, a lone tile's 16
+  // columns wait for memory 32 times (products of 300 x 280 by 500 53 us each).
+  int64_t on[4][4];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int64_t n = n0 + j * 16 + r;
-      if (n >= p.N) continue;
-      float *c = p.C + (p.cmap ? p.cmap[p.M + n] : n * p.ldc);
-      float old[4];
-      if (p.beta_one) {
+      on[j][r] = n >= p.N ? -1 : p.cmap ? p.cmap[p.M + n] : n * p.ldc;
+    }
+  float old[2][4][4];
+  auto fetch = [&](int j) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) old[i] = om[i] >= 0 ? c[om[i]] : 0.0f;
-      }
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) old[j & 1][r][i] = on[j][r] >= 0 && om[i] >= 0 ? p.C[on[j][r] + om[i]] : 0.0f;
+  };
+  if (p.beta_one) fetch(0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (p.beta_one && j < 3) fetch(j + 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float x = big[i][j][r] + small[i][j][r];
         const float v = p.alpha * (NP == 2 ? ldexpf(x, ea[i] + eb[j][r]) : x);
-        if (om[i] >= 0) c[om[i]] = p.beta_one ? old[i] + v : v;
+        if (on[j][r] >= 0 && om[i] >= 0) p.C[on[j][r] + om[i]] = p.beta_one ? old[j & 1][r][i] + v : v;
       }
-    }
+  }
 }
 
 // Sums the ksplit partial blocks of the tiles cut into K ranges in order and applies C = alpha * sum (+ C).
@@ -707,7 +720,9 @@ int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, 
   const int vec = ((uintptr_t)X % 16 == 0) && ld % 4 == 0;
   if (NP == 2 && kcont) {  // maxima and planes in one pass over HBM
     if (Rp / 2 > 0x7fffffffLL) return -4;
-    split_rows_f16_kernel<<<dim3((unsigned)(Rp / 2)), dim3(kSplitThreads), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
+    const int rows_log = split_rows_log(nks, Rp);  // at most the 128 rows that Rp is a multiple of
+    split_rows_f16_kernel<<<dim3((unsigned)(Rp >> rows_log)), dim3(kSplitThreads), 0, s>>>(X, ld, R, K, nks, P, plane,
+                                                                                         vec, U, rows_log);
     return hipGetLastError() == hipSuccess ? 0 : -2;
   }
   if constexpr (NP == 2) {
@@ -788,7 +803,7 @@ static int64_t presplit_slots() {
 }
 
 // K split of a partial last round of tiles: as many ranges as make it shortest,
-// counted in K steps.  A range costs about 8 steps beside its own (its first
+// counted in K steps.  A range costs about 4 steps beside its own (its first
 // loads, its partial sums written and read again): 5184^3 in fp16x3 has 861
 // tiles on 256 slots, and its 93 last ones run as 5 ranges each, 0.5 of a round
 // instead of a whole one (and 20 us of summing against 110 saved).
@@ -802,7 +817,7 @@ static TailSplit presplit_tail(int64_t M, int64_t N, int64_t K) {
   if (rem == 0) return t;
   int64_t best = nks;
   for (int64_t ks = 2; ks <= 16 && ks * 8 <= nks; ++ks) {
-    const int64_t cost = (rem * ks + slots - 1) / slots * ((nks + ks - 1) / ks + 8);
+    const int64_t cost = (rem * ks + slots - 1) / slots * ((nks + ks - 1) / ks + 4);
     if (cost < best) {
       best = cost;
       t.rem = rem;

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 # a, b, c of D(a,b)+=L(..)*R(..)
 SIZES = [(1, 1, 1), (5, 3, 33), (257, 129, 31), (130, 70, 65), (255, 128, 97), (300, 260, 128), (96, 80, 8229),
-         (70, 40, 16411), (2100, 2053, 515), (1537, 1281, 1030)]
+         (70, 40, 16411), (2100, 2053, 515), (1537, 1281, 1030),
+         (3000, 33, 48), (700, 600, 250), (300, 200, 2049)]
 PATTERNS = ["D(a,b)+=L(c,a)*R(c,b)", "D(a,b)+=L(a,c)*R(b,c)", "D(b,a)+=L(a,c)*R(c,b)"]
 
 
