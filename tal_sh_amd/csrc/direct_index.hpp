@@ -114,6 +114,21 @@ TAL_HD TAL_INLINE inline void run_start(const DirectPair &g, int k, int64_t *oa,
   *ob = (int64_t)*r * g.s[1][0] + (int64_t)*d1 * g.s[1][1] + (int64_t)y * g.s[1][2];
 }
 
+// Offset tables of contracted indices: two halves of `half` entries, in which
+// half h of a K range takes the place of half h - 2.  The walk has advanced to
+// step offset `at` of a range of `len` (steps of kb): the half to fill now, or
+// -1.  Between two calls lies a barrier, but none within one, so the half that
+// is written over must be one that no wave reads any more in this call.  A
+// kernel that reads a step's entries a call ahead has read the last ones of
+// half h - 1 in the call before it comes to half h; one that reads them in the
+// call that uses them reads those in the very call that comes to half h, and
+// fills one call later.
+TAL_HD TAL_INLINE inline int table_refill(int at, int len, int kb, int half, bool ahead) {
+  const int h = at / half;
+  if (h < 1 || at % half != (ahead ? 0 : kb) || (h + 1) * half >= len) return -1;
+  return h + 1;
+}
+
 // Arguments of one launch.  Byte strides and sizes throughout.  What every
 // launch reads comes first; a group is read only where its flag says that the
 // number has more than one dimension in that tensor (kernel arguments come

@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   // halves of kHalf, one filled while loads read the other.
   constexpr bool TAB = MODE == 2;
   constexpr int kHalf = 256;
-  static_assert(!TAB || (WA == 1 && WB == 1 && kHalf % KB == 0 && kHalf <= NT && kHalf >= PF * KB), "tables");
+  static_assert(!TAB || (WA == 1 && WB == 1 && kHalf % KB == 0 && kHalf <= NT && kHalf > (PF + 1) * KB), "tables");
   __shared__ uint32_t arow_t[TAB ? BM : 1], brow_t[TAB ? BN : 1];
   __shared__ int64_t drow_t[TAB ? BM : 1], dcol_t[TAB ? BN : 1];
   __shared__ uint2 k_t[TAB ? 2 * kHalf : 1];
@@ -421,8 +421,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
       const int next = kload + KB;
       if (next < kend) {
         kload = next;
-        const int h = (kload - kbeg) / kHalf;
-        if ((kload - kbeg) % kHalf == 0 && kload + kHalf < kend) fill_k(h + 1);  // half h - 1 is no longer read
+        const int h = table_refill(kload - kbeg, kend - kbeg, KB, kHalf, AHEAD);
+        if (h >= 0) fill_k(h);
         if (AHEAD) next_k();
       }
       return;

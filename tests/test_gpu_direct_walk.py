@@ -1,0 +1,42 @@
+"""Direct contractions in 128 x 128 tiles with offsets by table, over K ranges of several table halves. The bodies hold
+small whole numbers, so every sum is exact in both precisions and in any order."""
+import math
+
+import pytest
+import torch
+
+from tal_common import R4, R8
+from test_direct_walk import SHORT_RUNS, labels_of
+
+pytestmark = pytest.mark.gpu
+
+
+def matrix(body, labels, ext, rows, cols):
+    """A body (its shape is the labels reversed) as a matrix in 64 bits."""
+    order = [len(labels) - 1 - labels.index(x) for x in rows + cols]
+    return body.view([ext[x] for x in labels][::-1]).permute(order).reshape(
+        math.prod([ext[x] for x in rows]), -1).to(torch.float64).contiguous()
+
+
+@pytest.mark.parametrize("dk", (R4, R8))
+@pytest.mark.parametrize("case", SHORT_RUNS)
+def test_short_runs_in_large_tiles(talsh_gpu, dk, case):
+    ts = talsh_gpu
+    pattern, ext = case
+    print("[case] short runs", dk, pattern, ext, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    labels = labels_of(pattern)
+    dtype = torch.float32 if dk == R4 else torch.float64
+    # |sum| <= 64 K + 8 < 2^24
+    body = [torch.randint(-8, 9, (math.prod(ext[x] for x in lab),), generator=gen, device="cuda").to(dtype)
+            for lab in labels]
+    d, l, r = labels
+    k = [x for x in l if x in r and x not in d]
+    m, n = [x for x in d if x in l], [x for x in d if x in r]
+    want = matrix(body[0], d, ext, m, n) + matrix(body[1], l, ext, m, k) @ matrix(body[2], r, ext, k, n)
+    torch.cuda.synchronize()
+    ten = [ts.Tensor(dk, [ext[x] for x in lab], ts.gpu_flat(0), ext=b.data_ptr()) for lab, b in zip(labels, body)]
+    ts.check(ts.contract(pattern, ten[0], ten[1], ten[2], alpha=1.0, accumulative=ts.YEP), "contract")
+    assert torch.equal(matrix(body[0], d, ext, m, n), want)
+    for t in ten:
+        t.destruct()
