@@ -122,15 +122,36 @@ bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, Direct
   if (!reach(a->am, f.M, a->ka1, abytes) || !reach(a->bn, f.N, a->kb1, bbytes)) return false;
   // loads of rows past the edge: what is added to kOutside stays below 2^31
   if (32 * a->ka1 >= (int64_t)kOutside || 32 * a->kb1 >= (int64_t)kOutside) return false;
+  // Mode 1 puts the way to a step's next run into the base where it is
+  // negative, and gives it back in the offsets of the lanes before the crossing:
+  // up to |way| beyond the operand's own span.  Where that could leave the range
+  // (or, past the edge, wrap round into it), offsets go by table: they are those
+  // in the operand.
+  auto walks = [&](const DirectGroup &g, bool grouped, const std::vector<DirectDim> &rows, int64_t nrows, int t) {
+    int64_t span = (int64_t)(kstep - 1) * a->k.s[t][0] + 16, way = 0;
+    if (!grouped) span += (std::min<int64_t>(nrows, 128) - 1) * g.s[0];
+    else
+      for (const DirectDim &d : rows) span += (d.ext - 1) * d.s[0] * esz;
+    const int64_t past = f.k[0].ext * a->k.s[t][0], next = a->k.s[t][1] - past;
+    way = next < 0 ? -next : next;
+    if (a->k.nd > 2) {
+      const int64_t wrap = a->k.s[t][2] - (f.k[1].ext - 1) * a->k.s[t][1] - past;
+      way = std::max(way, wrap < 0 ? -wrap : wrap);
+    }
+    return span + way < (int64_t)kOutside;
+  };
   if (a->k.nd == 1) v->mode = small ? 0 : 1;
-  else v->mode = a->k.nd <= 3 && f.k[0].ext >= kstep ? 1 : 2;
+  else
+    v->mode = a->k.nd <= 3 && f.k[0].ext >= kstep && walks(a->am, a->am.nd > 1, f.m, f.M, 0) &&
+                      walks(a->bn, a->bn.nd > 1, f.n, f.N, 1)
+                  ? 1
+                  : 2;
   return true;
 }
 
-bool direct_addressable(const DirectForm &f, int dk) {
+bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v) {
   DirectArgs a;
-  DirectVariant v;
-  return direct_args(f, direct_elem(dk), direct_width(dk), 16, &a, &v);
+  return direct_args(f, direct_elem(dk), direct_width(dk), 16, &a, v);
 }
 
 const DirectTile *direct_tiles(int dk) {

@@ -25,8 +25,8 @@ struct DirectVariant {
 // false when the kernel cannot address the form (more than kDirectDims
 // dimensions in a group, extents or strides past 32 bits).
 bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, DirectArgs *a, DirectVariant *v);
-// Whether direct_args accepts the form for data kind dk at every tile, either way round.
-bool direct_addressable(const DirectForm &f, int dk);
+// Whether direct_args accepts the form for data kind dk at every tile, either way round; the variant at K steps of 16.
+bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v);
 
 // Tile shapes of a kind, largest first.  unit / stream: microseconds that one
 // tile of K = 1024 takes alone on a CU, and per tile when several share the CU.

@@ -83,7 +83,8 @@ TAL_HD TAL_INLINE inline void pair_offsets32(const DirectPair &g, uint32_t x, ui
 // Walking k in steps no longer than its leading run, k of up to three
 // dimensions (or one).  next / wrap: how much further on than the position
 // just past a run's end the next run starts in A and B, where the second
-// dimension goes on / wraps; below 2^31 for operands below 2 GiB.
+// dimension goes on / wraps; direct_args lets only those walk whose ways, with
+// what the lanes add, stay within 32-bit offsets.
 struct RunWalk {
   int32_t e0;
   int32_t next[2], wrap[2];

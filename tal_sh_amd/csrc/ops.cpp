@@ -543,13 +543,14 @@ enum Route { kRouteDirect, kRouteCopies, kRouteWide, kRouteSplit };
 // as offsets then come from tables (runs of 20-24 by copies and in place: R8
 // 930 x 957 by 616 60 -> 56 us, 1480 x 1189 by 280 55 -> 51, C4 311 x 336 by
 // 600 40 -> 34, C8 550 x 552 by 420 64 -> 65; runs of 32, R8 1024^3, 72 -> 79);
-// in 128 x 128 tiles short runs cost 40 %; D written 8 bytes apart, about four
+// in 128 x 128 tiles short runs, and any runs by table, cost 40 %; D written 8 bytes apart, about four
 // times its bytes.
 // A transpose moves 4.6 TB/s and takes about 4 us beside that.
 Route plan_route(const ContractPlan &plan, int dk) {
   if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) return kRouteSplit;
-  const bool mat_ok = direct_addressable(plan.mat, dk);
-  if (plan.direct_ok && direct_addressable(plan.direct, dk)) {
+  DirectVariant v;
+  const bool mat_ok = direct_addressable(plan.mat, dk, &v);
+  if (plan.direct_ok && direct_addressable(plan.direct, dk, &v)) {
     const DirectForm &f = plan.direct;
     const int esz = dk_size(dk);
     const bool d_copy = plan.d_transpose && !plan.mat_d_in_place;
@@ -562,7 +563,7 @@ Route plan_route(const ContractPlan &plan, int dk) {
     const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
     const double gemm = c.us;
     double extra = 0;
-    if (plan.direct_krun) extra += (c.tile ? 0.25 : plan.direct_krun < 32 ? 0.4 : 0.05) * gemm;
+    if (plan.direct_krun) extra += (c.tile ? 0.25 : plan.direct_krun < 32 || v.mode == 2 ? 0.4 : 0.05) * gemm;
     if (plan.direct_run && plan.direct_run < 8) extra += 0.3 * gemm;
     if (plan.direct_conflict) extra += std::min(avol, bvol) > 4e6 ? 1e9 : 0.5 * gemm;
     if (plan.direct_scatter) extra += 4 * dvol / 4.6e6;

@@ -1,6 +1,7 @@
 """CPU tests of how the direct contraction kernels walk through their K steps (tal_sh_amd/csrc/direct_index.hpp)."""
 import ctypes
 import os
+import random
 import subprocess
 
 import pytest
@@ -55,3 +56,58 @@ def variant(walk, pattern, ext, dk):
 def test_short_runs_take_tables_in_large_tiles(walk, dk, case):
     mode, tile, krange = variant(walk, *case, dk)
     assert (mode, tile) == (2, 0) and krange > 512
+
+
+def lane_offsets(walk, pattern, ext, dk):
+    dims = [(ctypes.c_int * len(lab))(*[ext[x] for x in lab]) for lab in labels_of(pattern)]
+    modes = ctypes.c_int()
+    return walk.lane_offsets(pattern.encode(), *dims, dk, ctypes.byref(modes)), modes.value
+
+
+# R below 2 GiB, its next run of k far lower in memory than the end of the one before
+BACKWARDS = [("D(a,b,c)+=L(i,a,j)*R(b,j,i,c)", dict(a=128, b=1500, c=2, i=20, j=3300)),
+             ("D(a,b,c)+=L(i,a,j)*R(b,j,i,c)", dict(a=64, b=1600, c=4, i=18, j=2000)),
+             ("D(a,b)+=L(i,a,j,k)*R(k,j,b,i)", dict(a=64, b=37, i=18, j=500, k=700)),
+             ("D(a,b,c)+=L(i,a,j)*R(b,i,c,j)", dict(a=40, b=300, c=1200, i=33, j=21))]
+
+
+@pytest.mark.parametrize("case", BACKWARDS)
+def test_large_operands_stay_in_range_backwards(walk, case):
+    """Every lane's 32-bit offset stays in its resource's range where the element is inside the operand."""
+    assert lane_offsets(walk, *case, 8)[0] in (0, -1)
+
+
+@pytest.mark.parametrize("dk", (4, 8, 14, 18))
+def test_operands_up_to_2gib_stay_in_range(walk, dk):
+    rng = random.Random(dk)
+    seen = 0
+    size = {4: 4, 8: 8, 14: 8, 18: 16}[dk]
+    for _ in range(60):
+        nl, nr, nk = rng.randint(1, 2), rng.randint(1, 2), rng.randint(1, 3)
+        x = [chr(ord("a") + i) for i in range(nl + nr + nk)]
+        lu, ru, cc = x[:nl], x[nl:nl + nr], x[nl + nr:]
+        ext = {q: rng.choice((3, 9, 18, 33, 40)) for q in cc}
+        ext.update({q: rng.choice((5, 16, 129)) for q in lu})
+        ext.update({q: 2 for q in ru})
+        # one index of R grows until R is just below 2 GiB, or a third of that
+        grow, goal = rng.choice(ru + cc), rng.choice((1.0, 1.0, 0.34)) * (0x7FFFFF00 / size)
+        rest = 1
+        for q in ru + cc:
+            rest *= ext[q] if q != grow else 1
+        ext[grow] = max(1, int(goal / rest))
+        k = 1
+        for q in cc:
+            k *= ext[q]
+        left = 1
+        for q in lu + cc:
+            left *= ext[q]
+        if k > 60000 or left * size > 0x7FFFFF00:
+            continue
+        l, r, d = lu + cc, ru + cc, lu + ru
+        for q in (l, r, d):
+            rng.shuffle(q)
+        pattern = "D(%s)+=L(%s)*R(%s)" % (",".join(d), ",".join(l), ",".join(r))
+        rc, modes = lane_offsets(walk, pattern, ext, dk)
+        assert rc in (0, -1), (rc, pattern, ext)
+        seen |= modes
+    assert seen & 7 == 7

@@ -1,12 +1,13 @@
-"""Direct contractions in 128 x 128 tiles with offsets by table, over K ranges of several table halves. The bodies hold
-small whole numbers, so every sum is exact in both precisions and in any order."""
+"""Direct contractions in 128 x 128 tiles with offsets by table, over K ranges of several table halves, and of operands
+whose runs of k lie far back from each other. The bodies hold small whole numbers, so every sum is exact in both
+precisions and in any order."""
 import math
 
 import pytest
 import torch
 
 from tal_common import R4, R8
-from test_direct_walk import SHORT_RUNS, labels_of
+from test_direct_walk import BACKWARDS, SHORT_RUNS, labels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -18,16 +19,12 @@ def matrix(body, labels, ext, rows, cols):
         math.prod([ext[x] for x in rows]), -1).to(torch.float64).contiguous()
 
 
-@pytest.mark.parametrize("dk", (R4, R8))
-@pytest.mark.parametrize("case", SHORT_RUNS)
-def test_short_runs_in_large_tiles(talsh_gpu, dk, case):
-    ts = talsh_gpu
-    pattern, ext = case
-    print("[case] short runs", dk, pattern, ext, flush=True)
+def check(ts, dk, pattern, ext):
+    print("[case] walk", dk, pattern, ext, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(7)
     labels = labels_of(pattern)
     dtype = torch.float32 if dk == R4 else torch.float64
-    # |sum| <= 64 K + 8 < 2^24
+    # |sum| <= 64 K + 8: below 2^24 for every R4 case
     body = [torch.randint(-8, 9, (math.prod(ext[x] for x in lab),), generator=gen, device="cuda").to(dtype)
             for lab in labels]
     d, l, r = labels
@@ -40,3 +37,14 @@ def test_short_runs_in_large_tiles(talsh_gpu, dk, case):
     assert torch.equal(matrix(body[0], d, ext, m, n), want)
     for t in ten:
         t.destruct()
+
+
+@pytest.mark.parametrize("dk", (R4, R8))
+@pytest.mark.parametrize("case", SHORT_RUNS)
+def test_short_runs_in_large_tiles(talsh_gpu, dk, case):
+    check(talsh_gpu, dk, *case)
+
+
+@pytest.mark.parametrize("case", BACKWARDS)
+def test_runs_far_back(talsh_gpu, case):
+    check(talsh_gpu, R8, *case)
