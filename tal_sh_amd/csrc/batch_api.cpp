@@ -429,17 +429,22 @@ int talshAmdBatchExecute(talshAmdBatch *b, int dev_id, int dev_kind, talsh_task_
   (void)hipSetDevice(dev.hip_id);
   // Replay fast path: same GPU, graph built, hazard table unchanged since the
   // last execution, so every operand's ordering state is exactly `hz` and one
-  // wait on it covers all of them (no per-tensor lookups).
-  const bool fast = b->built && b->g == g && b->hz && rt().hazard_epoch == b->epoch;
+  // wait on it covers all of them (no per-tensor lookups); and no tensor gained
+  // or lost an image (a caller's body leaves no trace in the hazard table when
+  // its tensor is destructed).
+  const bool planned = b->built && b->g == g && rt().image_epoch == b->images;
+  const bool fast = planned && b->hz && rt().hazard_epoch == b->epoch;
   // Where something else ran meanwhile, the operands' bodies are still the
   // ones planned for if no image moved anywhere and no task that may hold one
   // is unfinalized (a batch of 4,096 looks 12,288 operands up otherwise: 0.3 ms).
-  const bool same = b->built && b->g == g && rt().image_epoch == b->images && rt().tens_tasks.empty();
-  if (!fast && !same && (!b->built || b->g != g || signature(b, g) != b->sig)) {
-    const int e = build(b, g);
-    if (e) return e;
+  const bool same = planned && rt().tens_tasks.empty();
+  if (!fast && !same) {
+    if (!b->built || b->g != g || signature(b, g) != b->sig) {
+      const int e = build(b, g);
+      if (e) return e;
+    }
+    b->images = rt().image_epoch;
   }
-  b->images = rt().image_epoch;
   // nothing running anywhere: no operand has anything to wait for (3-4 ms of
   // per-range lookups for 12,288 operands otherwise)
   bool idle = !fast;
