@@ -299,6 +299,8 @@ int choose_policy(int g, int dk, std::vector<HostTask> hts, hipStream_t s, int *
 }
 
 void release_build(talshAmdBatch *b) {
+  // an asynchronous execution still reads its items and queue counters, which no hazard entry covers
+  if (b->hz) (void)hipEventSynchronize(b->hz->ev);
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;

@@ -60,3 +60,35 @@ def test_rebuilt_operand(talsh_gpu, dk, which):
     b.destroy()
     for t in ten:
         t.destruct()
+
+
+@pytest.mark.parametrize("dk", (R8, R4))
+def test_added_while_it_runs(talsh_gpu, dk):
+    """A contraction added behind an asynchronous execution: the plan is made anew, and both executions are whole."""
+    ts = talsh_gpu
+    print("[case] added while it runs", dk, flush=True)
+    dtype = torch.float64 if dk == R8 else torch.float32
+    n = 512
+    bodies = [body(dtype, n * n, i) for i in range(4)]
+    out = [torch.zeros(n * n, dtype=dtype, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    mk = lambda x: ts.Tensor(dk, [n, n], ts.gpu_flat(0), ext=x.data_ptr())  # noqa: E731
+    ten, d = [mk(x) for x in bodies], [mk(x) for x in out]
+    want = [(bodies[2 * i + 1].double().view(n, n) @ bodies[2 * i].double().view(n, n)).reshape(-1) for i in range(2)]
+    for rep in range(3):
+        b = ts.Batch()
+        assert b.add("D(a,b)+=L(a,k)*R(k,b)", d[0], ten[0], ten[1], alpha=1.0, accumulative=ts.NOPE) == 0
+        first, second = ts.Task(), ts.Task()
+        assert b.execute(first) == 0
+        assert b.add("D(a,b)+=L(a,k)*R(k,b)", d[1], ten[2], ten[3], alpha=1.0, accumulative=ts.NOPE) == 0
+        assert b.execute(second) == 0
+        for t in (first, second):
+            t.wait()
+            t.destruct()
+        for o, w in zip(out, want):
+            assert torch.equal(o.double(), w), rep
+            o.zero_()
+        torch.cuda.synchronize()
+        b.destroy()
+    for t in ten + d:
+        t.destruct()
