@@ -1,6 +1,7 @@
 // Contractions as the direct kernels see them.  No HIP: planned and tested on the CPU.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 #include <vector>
 
@@ -31,6 +32,14 @@ inline void direct_dim(std::vector<DirectDim> *v, int64_t ext, int64_t s0, int64
     }
   }
   v->push_back(DirectDim{ext, {s0, s1}});
+}
+
+// Most dimensions a number may have in one tensor, neighbours that chain there counted as one.
+constexpr int kDirectDims = 6;
+inline int direct_chains(const std::vector<DirectDim> &v, int t) {
+  int n = 0;
+  for (size_t i = 0; i < v.size(); ++i) n += i == 0 || v[i - 1].s[t] * v[i - 1].ext != v[i].s[t];
+  return n;
 }
 
 }  // namespace tal

@@ -12,13 +12,12 @@
 #include <cstdint>
 
 #include "batch_item.hpp"
+#include "direct_form.hpp"
 
 // Inlined before anything else is done, so that the kernel's arguments stay scalar loads.
 #define TAL_INLINE __attribute__((always_inline))
 
 namespace tal {
-
-constexpr int kDirectDims = 6;
 
 // Digits x -> (d0, ..., d[nd-1]) over ext[0..nd-2], the last digit unbounded.
 struct DirectGroup {

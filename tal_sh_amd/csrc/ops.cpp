@@ -24,6 +24,7 @@
 #include "contract.hpp"
 #include "direct.hpp"
 #include "plan.hpp"
+#include "route.hpp"
 #include "runtime.hpp"
 #include "talsh_amd.h"
 
@@ -528,51 +529,12 @@ void ttgt_cache_clear() {
   c.chunks.clear();
 }
 
-namespace {
-
-// How a plan runs for a data kind: a plain product by the direct kernels
-// straight from the tensors, or on copies of the operands the planner
-// transposes (with D written in place or through D'); split: the fast-math
-// GEMMs.  Depends on the plan, the kind and the fast-math mode only.
-enum Route { kRouteDirect, kRouteCopies, kRouteWide, kRouteSplit };
-
-// Straight from the tensors where the transposes would cost more than the
-// reads in place do.  Measured (R8): a K step that walks runs of k costs 4 %
-// of a product in 128 x 128 tiles (9216^3: 21.99 -> 22.66 ms) and about a
-// quarter in smaller ones (1024^3: 41 -> 50 us), there with runs of any length,
-// as offsets then come from tables (runs of 20-24 by copies and in place: R8
-// 930 x 957 by 616 60 -> 56 us, 1480 x 1189 by 280 55 -> 51, C4 311 x 336 by
-// 600 40 -> 34, C8 550 x 552 by 420 64 -> 65; runs of 32, R8 1024^3, 72 -> 79);
-// in 128 x 128 tiles short runs, and any runs by table, cost 40 %; D written 8 bytes apart, about four
-// times its bytes.
-// A transpose moves 4.6 TB/s and takes about 4 us beside that.
-Route plan_route(const ContractPlan &plan, int dk) {
+// Depends on the plan, the kind, the fast-math mode and the device only.
+static Route plan_route(const ContractPlan &plan, int dk) {
   if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) return kRouteSplit;
-  DirectVariant v;
-  const bool mat_ok = direct_addressable(plan.mat, dk, &v);
-  if (plan.direct_ok && direct_addressable(plan.direct, dk, &v)) {
-    const DirectForm &f = plan.direct;
-    const int esz = dk_size(dk);
-    const bool d_copy = plan.d_transpose && !plan.mat_d_in_place;
-    if (mat_ok && !plan.a.transpose && !plan.b.transpose && !d_copy) return kRouteCopies;  // nothing to copy
-    const double avol = (double)f.avol * esz, bvol = (double)f.bvol * esz;
-    const double dvol = (double)f.M * (double)f.N * (double)f.batch * esz;
-    const bool ta = plan.swap ? plan.b.transpose : plan.a.transpose, tb = plan.swap ? plan.a.transpose : plan.b.transpose;
-    const double copies =
-        (2 * ((ta ? avol : 0) + (tb ? bvol : 0) + (d_copy ? dvol : 0))) / 4.6e6 + ((ta || tb) ? 4 : 0) + (d_copy ? 4 : 0);
-    const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
-    const double gemm = c.us;
-    double extra = 0;
-    if (plan.direct_krun) extra += (c.tile ? 0.25 : plan.direct_krun < 32 || v.mode == 2 ? 0.4 : 0.05) * gemm;
-    if (plan.direct_run && plan.direct_run < 8) extra += 0.3 * gemm;
-    if (plan.direct_conflict) extra += std::min(avol, bvol) > 4e6 ? 1e9 : 0.5 * gemm;
-    if (plan.direct_scatter) extra += 4 * dvol / 4.6e6;
-    if (!mat_ok || copies > extra) return kRouteDirect;
-  }
-  return mat_ok ? kRouteCopies : kRouteWide;
+  const DirectForm &f = plan.direct;
+  return contract_route(plan, dk, direct_choose(dk, f.M, f.N, f.K, f.batch));
 }
-
-}  // namespace
 
 TtgtTemps ttgt_temp_bytes(const ContractPlan &plan, int dk, size_t lbytes, size_t rbytes, size_t dbytes) {
   TtgtTemps t;

@@ -470,7 +470,8 @@ int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, c
   std::vector<int64_t> dp = seq_strides(cat(cat(best_m, best_n), hyper), ext_of, nsym);
   // D is written where it lies if it does not need D' at all, or if its
   // contiguous index leads m or n with runs of at least 16 elements, or D is
-  // small enough to be put together in the L2 caches; hyper indices must chain
+  // small enough to be put together in the L2 caches; hyper indices must chain,
+  // and D's rows and columns be numbers that the kernels can take apart
   best.mat_d_in_place = false;
   if (best.d_transpose) {
     std::vector<DirectDim> m, n;
@@ -481,7 +482,8 @@ int plan_uncached(const DigitalPattern &p, const int *ddims, const int *ldims, c
       if (!g->empty() && (*g)[0].s[1] == 1) run = (*g)[0].ext;
     std::vector<DirectDim> h;
     for (int x : hyper) direct_dim(&h, ext_of[x], ax[x], str[2][x]);
-    best.mat_d_in_place = (run >= 16 || vd <= 1048576) && h.size() <= 1;
+    best.mat_d_in_place = (run >= 16 || vd <= 1048576) && h.size() <= 1 && direct_chains(m, 1) <= kDirectDims &&
+                          direct_chains(n, 1) <= kDirectDims;
   }
   const std::vector<int64_t> &ds = best.d_transpose && !best.mat_d_in_place ? dp : str[2];
   DirectForm f;

@@ -190,6 +190,17 @@ int lane_offsets(const char *pattern, const int *ddims, const int *ldims, const 
   return *modes ? 0 : -1;
 }
 
+// Whether the product on the planner's operands (copied where it copies them)
+// is one that the direct kernels take; *in_place: D is written where it lies.
+int mat_addressable(const char *pattern, const int *ddims, const int *ldims, const int *rdims, int dk, int *in_place) {
+  DigitalPattern p;
+  ContractPlan plan;
+  if (parse_pattern(pattern, &p) || plan_contraction(p, ddims, ldims, rdims, 1, &plan)) return -1;
+  *in_place = plan.mat_d_in_place;
+  DirectVariant v;
+  return direct_addressable(plan.mat, dk, &v) ? 1 : 0;
+}
+
 // Mode, tile and K range (in K) that a contraction gets straight from the
 // tensors on a GPU of `cus` compute units, with tile's K step.
 int direct_variant(const char *pattern, const int *ddims, const int *ldims, const int *rdims, int dk, int cus, int *out) {

@@ -111,3 +111,29 @@ def test_operands_up_to_2gib_stay_in_range(walk, dk):
         assert rc in (0, -1), (rc, pattern, ext)
         seen |= modes
     assert seen & 7 == 7
+
+
+def high_rank(rng):
+    """A contraction of many indices of extent 2: the labels of D, L and R."""
+    nl, nr, nk = rng.choice(((9, 9, 6), (10, 9, 6), (10, 10, 6), (8, 9, 3)))
+    x = ["x%d" % i for i in range(nl + nr + nk)]
+    l, r, d = x[:nl] + x[nl + nr:], x[nl:], x[:nl + nr]
+    for q in (l, r, d):
+        rng.shuffle(q)
+    return d, l, r
+
+
+def test_high_ranks_are_addressable(walk):
+    """Contractions of many short indices: where D's rows or columns are too many numbers to be written in place, D'
+    takes their place and the product is a plain one."""
+    rng = random.Random(5)
+    seen = set()
+    for _ in range(60):
+        d, l, r = high_rank(rng)
+        pattern = "D(%s)+=L(%s)*R(%s)" % (",".join(d), ",".join(l), ",".join(r))
+        dims = [(ctypes.c_int * len(lab))(*[2] * len(lab)) for lab in (d, l, r)]
+        in_place = ctypes.c_int()
+        for dk in (4, 8, 14, 18):
+            assert walk.mat_addressable(pattern.encode(), *dims, dk, ctypes.byref(in_place)) == 1, pattern
+        seen.add(in_place.value)
+    assert seen == {0, 1}
