@@ -111,7 +111,9 @@ bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, Direct
                  : 1;
   // 32-bit addressing of the operands: whole ones from their first element,
   // or, where a tile's origin can go into the 64-bit base (one dimension in
-  // both numbers), a tile's rows over one K step
+  // both numbers), a tile's rows over one K step; else, with one dimension in
+  // both, a 64-bit address per load: k 64 MiB apart or more (8.4 million rows
+  // of R8), or 128 rows that span 2 GiB (2.1 million contracted indices)
   const int64_t abytes = f.avol * esz, bbytes = f.bvol * esz;
   const bool small = abytes < (int64_t)kOutside && bbytes < (int64_t)kOutside;
   auto reach = [&](const DirectGroup &g, int64_t rows, int64_t kstride, int64_t bytes) {
@@ -119,9 +121,12 @@ bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, Direct
     if (a->k.nd > 1 || g.nd > 1) return false;
     return (std::min<int64_t>(rows, 128) - 1) * g.s[0] + 32 * kstride + 64 * esz < (int64_t)kOutside;
   };
-  if (!reach(a->am, f.M, a->ka1, abytes) || !reach(a->bn, f.N, a->kb1, bbytes)) return false;
   // loads of rows past the edge: what is added to kOutside stays below 2^31
-  if (32 * a->ka1 >= (int64_t)kOutside || 32 * a->kb1 >= (int64_t)kOutside) return false;
+  if (!reach(a->am, f.M, a->ka1, abytes) || !reach(a->bn, f.N, a->kb1, bbytes) ||
+      32 * a->ka1 >= (int64_t)kOutside || 32 * a->kb1 >= (int64_t)kOutside) {
+    v->mode = 3;
+    return a->k.nd == 1 && a->am.nd == 1 && a->bn.nd == 1;
+  }
   // Mode 1 puts the way to a step's next run into the base where it is
   // negative, and gives it back in the offsets of the lanes before the crossing:
   // up to |way| beyond the operand's own span.  Where that could leave the range

@@ -23,7 +23,8 @@ struct DirectVariant {
 // Fills the layout part of the kernel arguments and the variant for elements
 // of esz bytes, loads of up to full_width elements and K steps of kstep;
 // false when the kernel cannot address the form (more than kDirectDims
-// dimensions in a group, extents or strides past 32 bits).
+// dimensions in a group, extents past 31 bits, strides past 32 bits where rows
+// or k have several dimensions).
 bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, DirectArgs *a, DirectVariant *v);
 // Whether direct_args accepts the form for data kind dk at every tile, either way round; the variant at K steps of 16.
 bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v);

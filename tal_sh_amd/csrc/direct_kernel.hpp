@@ -110,6 +110,15 @@ __device__ inline Vec<S, N> bload(__amdgpu_buffer_rsrc_t r, uint32_t o) {
   __builtin_memcpy(&v, &u, sizeof(v));
   return v;
 }
+// The same from a 64-bit address in device memory.
+template <typename S, int N>
+__device__ inline Vec<S, N> gload(const char *a) {
+  typedef typename Raw<(int)sizeof(S) * N>::type __attribute__((address_space(1), aligned(sizeof(S)))) G;
+  const auto u = *(const G *)(uintptr_t)a;
+  Vec<S, N> v;
+  __builtin_memcpy(&v, &u, sizeof(v));
+  return v;
+}
 // Tile t of C -> (bx, by): tiles are walked in groups of 8 tile-rows, column
 // by column inside a group (a bijection of [0, gx*gy)).
 __device__ inline void tile_xy(int t, int gx, int gy, int &bx, int &by) {
@@ -224,6 +233,15 @@ struct SlabOffsets {
 //      product ran as long as its code took to arrive: 77 x 72 by 60 R8 9.7 ->
 //      8.1 us of kernel, 399 x 440 by 195 18.0 -> 13.6 (R4, whose compilation
 //      needed scratch memory, 50 -> 14).
+//   3  rows and k linear, operands whose rows or contracted indices lie too far
+//      apart for 32-bit offsets within a tile: a 64-bit address per load and
+//      lane, advanced by a constant. Rows past the edge read the last row again
+//      (their products are never stored).
+//      R8, in us, by the wide-address kernel that ran them before and now: 208^3
+//      rows by 208 and 208 24,400 -> 18,000, 9,000,000 by 24 and 24 3,090 ->
+//      1,460; C8 8,000,000 by 32 and 32 4,990 -> 2,430; R8 130 x 130 by
+//      2,200,000 along k, one tile there and cut into K ranges here, 364,000 ->
+//      3,300.
 template <typename S, int NC, int KA, int KBC, int WA, int WB, int BM, int BN, int KB, int WM, int WN, int PF, int OCC,
           int MODE>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OCC))) void direct_kernel(DirectArgs) {
@@ -293,7 +311,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   const int bl = BLINE % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / BLINE) : tid / BLINE;
   // Mode 2: offsets by table.  Rows, columns and D's of both once; k in two
   // halves of kHalf, one filled while loads read the other.
-  constexpr bool TAB = MODE == 2;
+  constexpr bool TAB = MODE == 2, FAR = MODE == 3;
   constexpr int kHalf = 256;
   static_assert(!TAB || (WA == 1 && WB == 1 && kHalf % KB == 0 && kHalf <= NT && kHalf > (PF + 1) * KB), "tables");
   __shared__ uint32_t arow_t[TAB ? BM : 1], brow_t[TAB ? BN : 1];
@@ -327,15 +345,32 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
     __syncthreads();
   }
   uint32_t aro[KA ? NVA : 1], bro[KBC ? NVB : 1];
+  // Mode 3: the address of load j of row r0 (clamped to the operand) and contracted index k.
+  auto afar = [&](int j, int k) TAL_INLINE {
+    const int r = min(m0 + (KA ? al + j * ASTEP : ac), p.M - (KA ? 1 : WA));
+    return (const char *)p.A + (int64_t)blockIdx.y * p.sa + (int64_t)r * p.am1 + (int64_t)k * p.ka1;
+  };
+  auto bfar = [&](int j, int k) TAL_INLINE {
+    const int r = min(n0 + (KBC ? bl + j * BSTEP : bc), p.N - (KBC ? 1 : WB));
+    return (const char *)p.B + (int64_t)blockIdx.y * p.sb + (int64_t)r * p.bn1 + (int64_t)k * p.kb1;
+  };
+  const char *af[FAR ? NVA : 1], *bf[FAR ? NVB : 1];
+  if (FAR) {
 #pragma unroll
-  for (int j = 0; j < (KA ? NVA : 1); ++j) {
-    const int r = KA ? al + j * ASTEP : ac;
-    aro[j] = TAB ? arow_t[r] : arow(m0 + r);
-  }
+    for (int j = 0; j < NVA; ++j) af[FAR ? j : 0] = afar(j, kbeg + (KA ? ac : al + j * ASTEP));
 #pragma unroll
-  for (int j = 0; j < (KBC ? NVB : 1); ++j) {
-    const int r = KBC ? bl + j * BSTEP : bc;
-    bro[j] = TAB ? brow_t[r] : brow(n0 + r);
+    for (int j = 0; j < NVB; ++j) bf[FAR ? j : 0] = bfar(j, kbeg + (KBC ? bc : bl + j * BSTEP));
+  } else {
+#pragma unroll
+    for (int j = 0; j < (KA ? NVA : 1); ++j) {
+      const int r = KA ? al + j * ASTEP : ac;
+      aro[j] = TAB ? arow_t[r] : arow(m0 + r);
+    }
+#pragma unroll
+    for (int j = 0; j < (KBC ? NVB : 1); ++j) {
+      const int r = KBC ? bl + j * BSTEP : bc;
+      bro[j] = TAB ? brow_t[r] : brow(n0 + r);
+    }
   }
 
   Vec<S, WA * NC> ra[PF][NVA];
@@ -411,6 +446,16 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
         kr += over ? KB - rw.e0 : KB;
         kd1 = !over ? kd1 : wrap ? 0 : kd1 + 1;
       }
+    } else if (FAR) {
+#pragma unroll
+      for (int j = 0; j < NVA; ++j) ra[set][j] = gload<S, WA * NC>(af[FAR ? j : 0]);
+#pragma unroll
+      for (int j = 0; j < NVB; ++j) rb[set][j] = gload<S, WB * NC>(bf[FAR ? j : 0]);
+      const int64_t sa = more ? abase_step : 0, sb = more ? bbase_step : 0;
+#pragma unroll
+      for (int j = 0; j < NVA; ++j) af[FAR ? j : 0] += sa;
+#pragma unroll
+      for (int j = 0; j < NVB; ++j) bf[FAR ? j : 0] += sb;
     } else {
       const auto rsa = rsrc(abase, kOutside), rsb = rsrc(bbase, kOutside);
       if (!AHEAD) next_k();
@@ -431,6 +476,29 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   };
   // the last, partial K step, from k0: element by element, zeros past kend
   auto load_tail = [&](int k0) TAL_INLINE {
+    if (FAR) {  // indices past kend read the last one, and count as zeros in both operands
+#pragma unroll
+      for (int j = 0; j < NVA; ++j)
+#pragma unroll
+        for (int w = 0; w < (KA ? WA : 1); ++w) {
+          const int k = k0 + (KA ? ac + w : al + j * ASTEP);
+          constexpr int L = KA ? NC : WA * NC;
+          const Vec<S, L> x = gload<S, L>(afar(j, min(k, kend - 1)));
+#pragma unroll
+          for (int c = 0; c < L; ++c) ra[0][j].v[w * L + c] = k < kend ? x.v[c] : (S)0;
+        }
+#pragma unroll
+      for (int j = 0; j < NVB; ++j)
+#pragma unroll
+        for (int w = 0; w < (KBC ? WB : 1); ++w) {
+          const int k = k0 + (KBC ? bc + w : bl + j * BSTEP);
+          constexpr int L = KBC ? NC : WB * NC;
+          const Vec<S, L> x = gload<S, L>(bfar(j, min(k, kend - 1)));
+#pragma unroll
+          for (int c = 0; c < L; ++c) rb[0][j].v[w * L + c] = k < kend ? x.v[c] : (S)0;
+        }
+      return;
+    }
     const bool lin = MODE == 0 || (MODE == 1 && p.k.nd == 1);
     const char *at = (const char *)p.A + (int64_t)blockIdx.y * p.sa + (int64_t)am0 * p.am1;
     const char *bt = (const char *)p.B + (int64_t)blockIdx.y * p.sb + (int64_t)bn0 * p.bn1;

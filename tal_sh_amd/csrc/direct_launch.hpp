@@ -48,6 +48,8 @@ template <typename S, int NC, class T, int W>
 bool run_tile(const DirectVariant &v, const DirectArgs &a, unsigned batch, hipStream_t s) {
   const bool tables = v.mode == 2 || (v.mode == 1 && a.k.nd > 1 && T::BM * T::BN == 32 * 32);
   if (tables) run_layout<S, NC, T, 1, 2>(v, a, batch, s);
+  else if (v.mode == 3 && v.width == W) run_layout<S, NC, T, W, 3>(v, a, batch, s);
+  else if (v.mode == 3) run_layout<S, NC, T, 1, 3>(v, a, batch, s);
   else if (v.mode == 1 && v.width == W) run_layout<S, NC, T, W, 1>(v, a, batch, s);
   else if (v.mode == 1) run_layout<S, NC, T, 1, 1>(v, a, batch, s);
   else if (v.width == W) run_layout<S, NC, T, W, 0>(v, a, batch, s);

@@ -18,7 +18,7 @@ namespace tal {
 Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c) {
   DirectVariant v;
   const bool mat_ok = direct_addressable(plan.mat, dk, &v);
-  if (plan.direct_ok && direct_addressable(plan.direct, dk, &v)) {
+  if (plan.direct_ok && direct_addressable(plan.direct, dk, &v) && v.mode < 3) {
     const DirectForm &f = plan.direct;
     const int esz = direct_elem(dk);
     const bool d_copy = plan.d_transpose && !plan.mat_d_in_place;

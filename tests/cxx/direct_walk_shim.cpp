@@ -1,5 +1,5 @@
 // C entry points for the CPU test tests/test_direct_walk.py, which builds this
-// file with g++ beside tal_sh_amd/csrc/plan.cpp and direct_args.cpp: the walk
+// file with g++ beside tal_sh_amd/csrc/plan.cpp, direct_args.cpp and route.cpp: the walk
 // of a direct contraction kernel through its K steps.
 #include <cstdint>
 #include <cstring>
@@ -8,6 +8,7 @@
 
 #include "direct_args.hpp"
 #include "plan.hpp"
+#include "route.hpp"
 
 using namespace tal;
 
@@ -103,6 +104,7 @@ int64_t true_k(const DirectForm &f, int esz, int t, int64_t k) {
 // 2: a row past the edge comes back into the range.
 int check_operand(const DirectForm &f, const DirectArgs &a, const DirectVariant &v, const Operand &o, int esz, int kb,
                   int width) {
+  if (v.mode == 3) return 0;  // 64-bit addresses
   const int64_t tiles = (o.nrows + o.tile - 1) / o.tile;
   std::set<int64_t> which = {0, tiles / 2, tiles - 1};
   for (int64_t tile : which) {
@@ -199,6 +201,26 @@ int mat_addressable(const char *pattern, const int *ddims, const int *ldims, con
   *in_place = plan.mat_d_in_place;
   DirectVariant v;
   return direct_addressable(plan.mat, dk, &v) ? 1 : 0;
+}
+
+// The route of a contraction without fast math on a GPU of `cus` compute units;
+// out: mode and width of the product that it runs, and its tile.
+int route_of(const char *pattern, const int *ddims, const int *ldims, const int *rdims, int dk, int cus, int *out) {
+  DigitalPattern p;
+  ContractPlan plan;
+  if (parse_pattern(pattern, &p) || plan_contraction(p, ddims, ldims, rdims, 1, &plan)) return -1;
+  const DirectForm &d = plan.direct;
+  const Route r = contract_route(plan, dk, direct_choose(dk, d.M, d.N, d.K, d.batch, cus));
+  const DirectForm &f = r == kRouteDirect ? plan.direct : plan.mat;
+  const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch, cus);
+  DirectArgs a;
+  DirectVariant v;
+  if (!direct_args(c.swap ? direct_swapped(f) : f, direct_elem(dk), direct_width(dk), direct_tiles(dk)[c.tile].kb, &a, &v))
+    return r;
+  out[0] = v.mode;
+  out[1] = v.width;
+  out[2] = c.tile;
+  return r;
 }
 
 // Mode, tile and K range (in K) that a contraction gets straight from the

@@ -13,7 +13,7 @@ def build(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("walk") / "libdirect_walk.so")
     csrc = os.path.join(REPO, "tal_sh_amd", "csrc")
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I" + csrc, "-I" + os.path.join(REPO, "include"),
-                    os.path.join(csrc, "direct_args.cpp"), os.path.join(csrc, "plan.cpp"),
+                    os.path.join(csrc, "direct_args.cpp"), os.path.join(csrc, "plan.cpp"), os.path.join(csrc, "route.cpp"),
                     os.path.join(REPO, "tests", "cxx", "direct_walk_shim.cpp"), "-o", out], check=True)
     return ctypes.CDLL(out)
 
@@ -137,3 +137,33 @@ def test_high_ranks_are_addressable(walk):
             assert walk.mat_addressable(pattern.encode(), *dims, dk, ctypes.byref(in_place)) == 1, pattern
         seen.add(in_place.value)
     assert seen == {0, 1}
+
+
+# Operands whose rows or contracted indices lie 64 MiB or more apart: tall ones along their rows, long ones along k.
+MODE_FAR, ROUTE_COPIES = 3, 1
+FAR = {8: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=8400000, p=37, q=24)),      # 16-byte loads, a partial K step
+           ("D(a,q)+=L(a,p)*R(q,p)", dict(a=8400001, p=16, q=47)),      # element loads, a partial tile
+           ("D(q,a)+=L(p,q)*R(a,p)", dict(a=8400003, p=5, q=70)),       # K below a step
+           ("D(a,q)+=L(a,p)*R(p,q)", dict(a=8388610, p=33, q=130)),
+           ("D(a,b,c,q)+=L(a,b,c,p)*R(p,q)", dict(a=210, b=200, c=201, p=40, q=9)),
+           ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=30, k=2200001)),     # both along k, element loads
+           ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=140, k=2200002)),
+           ("D(a,b)+=L(k,a)*R(b,k)", dict(a=129, b=31, k=2200000)),
+           ("D(b,a)+=L(a,k)*R(k,b)", dict(a=30, b=135, k=2150002))],
+       4: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=16800000, p=35, q=24)),
+           ("D(a,q)+=L(a,p)*R(q,p)", dict(a=16800001, p=64, q=33)),
+           ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=33, k=4400001)),
+           ("D(a,b)+=L(k,a)*R(b,k)", dict(a=130, b=33, k=4400000))],
+       18: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=4200001, p=35, q=24)),
+            ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=33, k=1100001))],
+       14: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=8400001, p=35, q=24)),
+            ("D(a,b)+=L(k,a)*R(b,k)", dict(a=130, b=33, k=2200001))]}
+
+
+@pytest.mark.parametrize("dk", (4, 8, 14, 18))
+def test_far_operands_take_the_direct_kernels(walk, dk):
+    for pattern, ext in FAR[dk]:
+        dims = [(ctypes.c_int * len(lab))(*[ext[x] for x in lab]) for lab in labels_of(pattern)]
+        out = (ctypes.c_int * 3)()
+        assert walk.route_of(pattern.encode(), *dims, dk, 256, out) == ROUTE_COPIES, (pattern, ext)
+        assert out[0] == MODE_FAR, (pattern, ext)

@@ -1,6 +1,6 @@
-"""Direct contractions in 128 x 128 tiles with offsets by table, over K ranges of several table halves, and of operands
-whose runs of k lie far back from each other. The bodies hold small whole numbers, so every sum is exact in both
-precisions and in any order."""
+"""Direct contractions where their walk through the operands is long: in 128 x 128 tiles with offsets by table, over K
+ranges of several table halves; with runs of k that lie far back from each other; with rows too far apart for 32-bit
+offsets; with many indices. The bodies hold small whole numbers, so every sum is exact and in any order."""
 import math
 import random
 
@@ -8,30 +8,41 @@ import numpy as np
 import pytest
 import torch
 
-from tal_common import R4, R8
-from test_direct_walk import BACKWARDS, SHORT_RUNS, high_rank, labels_of
+from tal_common import C4, C8, R4, R8
+from test_direct_walk import BACKWARDS, FAR, SHORT_RUNS, high_rank, labels_of
 
 pytestmark = pytest.mark.gpu
+
+
+DTYPE = {R4: torch.float32, R8: torch.float64, C4: torch.complex64, C8: torch.complex128}
 
 
 def matrix(body, labels, ext, rows, cols):
     """A body (its shape is the labels reversed) as a matrix in 64 bits."""
     order = [len(labels) - 1 - labels.index(x) for x in rows + cols]
     return body.view([ext[x] for x in labels][::-1]).permute(order).reshape(
-        math.prod([ext[x] for x in rows]), -1).to(torch.float64).contiguous()
+        math.prod([ext[x] for x in rows]), -1).to(torch.complex128 if body.is_complex() else torch.float64).contiguous()
 
 
-def check(ts, dk, pattern, ext):
+def check(ts, dk, pattern, ext, largest=8):
+    """largest: magnitude of the bodies' whole numbers; no sum may leave the kind's exact range."""
     print("[case] walk", dk, pattern, ext, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(7)
     labels = labels_of(pattern)
-    dtype = torch.float32 if dk == R4 else torch.float64
-    # |sum| <= 64 K + 8: below 2^24 for every R4 case
-    body = [torch.randint(-8, 9, (math.prod(ext[x] for x in lab),), generator=gen, device="cuda").to(dtype)
-            for lab in labels]
+
+    def draw(n):
+        x = torch.empty(n, dtype=torch.float32, device="cuda")
+        return x.random_(-largest, largest + 1, generator=gen)
+
+    body = []
+    for lab in labels:
+        n = math.prod(ext[x] for x in lab)
+        body.append((torch.complex(draw(n), draw(n)) if dk in (C4, C8) else draw(n)).to(DTYPE[dk]))
     d, l, r = labels
     k = [x for x in l if x in r and x not in d]
     m, n = [x for x in d if x in l], [x for x in d if x in r]
+    total = math.prod(ext[x] for x in k) * largest ** 2 * (2 if dk in (C4, C8) else 1) + largest
+    assert total < (2 ** 24 if dk in (R4, C4) else 2 ** 53)
     want = matrix(body[0], d, ext, m, n) + matrix(body[1], l, ext, m, k) @ matrix(body[2], r, ext, k, n)
     torch.cuda.synchronize()
     ten = [ts.Tensor(dk, [ext[x] for x in lab], ts.gpu_flat(0), ext=b.data_ptr()) for lab, b in zip(labels, body)]
@@ -77,3 +88,11 @@ def test_high_ranks(talsh_gpu, seed):
     assert np.array_equal(mat(0, d, m, n), want)
     for t in ten:
         t.destruct()
+
+
+@pytest.mark.parametrize("dk,case", [(dk, i) for dk in FAR for i in range(len(FAR[dk]))])
+def test_far_operands(talsh_gpu, dk, case):
+    """Rows or contracted indices 64 MiB and more apart."""
+    pattern, ext = FAR[dk][case]
+    check(talsh_gpu, dk, pattern, ext, largest=1 if dk in (R4, C4) else 8)
+    torch.cuda.empty_cache()
