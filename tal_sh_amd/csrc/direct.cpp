@@ -47,7 +47,7 @@ int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, voi
     c.ksplit = 1;
     c.ksteps = 0;
   }
-  if (c.gx * c.gy > 0x7fffffff / 64) return -4;
+  if (c.us < 0) return -4;  // more tiles than 31 bits number
   DirectForm swapped;
   const DirectForm *p = &f;
   if (c.swap) {

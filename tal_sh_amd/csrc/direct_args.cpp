@@ -81,7 +81,7 @@ bool wide(const std::vector<DirectDim> &rows, const std::vector<DirectDim> &k, i
 
 bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, DirectArgs *a, DirectVariant *v) {
   std::memset(a, 0, sizeof(*a));
-  constexpr int64_t kMax = 0x7fffffff - 1024;
+  constexpr int64_t kMax = 0x7fffffff - 127;  // a tile past the edge is still numbered in 31 bits
   if (f.M < 1 || f.N < 1 || f.K < 0 || f.batch < 1 || f.M > kMax || f.N > kMax || f.K > kMax) return false;
   if (!single_group(f.m, 0, esz, &a->am) || !single_group(f.n, 0, esz, &a->bn) || !single_group(f.m, 1, esz, &a->dm) ||
       !single_group(f.n, 1, esz, &a->dn) || !pair_group(f.k, esz, &a->k))
@@ -184,7 +184,7 @@ DirectChoice direct_choose(int dk, int64_t M, int64_t N, int64_t K, int64_t batc
   const DirectTile *tiles = direct_tiles(dk);
   const int esz = direct_elem(dk);
   DirectChoice best;
-  best.us = -1;
+  best.us = -1;  // stays where every tile shape makes too many
   for (int swap = 0; swap < 2; ++swap) {
     const int64_t m = swap ? N : M, n = swap ? M : N;
     for (int t = 0; t < kDirectTiles; ++t) {
@@ -193,6 +193,7 @@ DirectChoice direct_choose(int dk, int64_t M, int64_t N, int64_t K, int64_t batc
       const int64_t gx = (m + ti.bm - 1) / ti.bm, gy = (n + ti.bn - 1) / ti.bn, T = gx * gy;
       const int64_t nk = std::max<int64_t>(1, (K + ti.kb - 1) / ti.kb);
       const double k = (double)nk * ti.kb / 1024;
+      if (T > 0x7fffffff - 64 * (int64_t)cus) continue;  // units are numbered in 31 bits, K ranges of `rem` < cus tiles included
       auto consider = [&](int64_t whole, int64_t rem, int ks, int64_t steps, double us, size_t bytes) {
         if (best.us >= 0 && us >= best.us) return;
         best.swap = swap != 0;

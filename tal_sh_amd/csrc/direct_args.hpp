@@ -29,6 +29,13 @@ bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, Direct
 // Whether direct_args accepts the form for data kind dk at every tile, either way round; the variant at K steps of 16.
 bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v);
 
+// Units of one launch of workgroups of `threads`, from unit `at` of `units` on: a
+// grid may not hold 2^32 threads or more (products of more than 2^30 rows).
+inline int64_t direct_launch_units(int64_t units, int64_t at, unsigned threads) {
+  const int64_t most = (int64_t)(0xffffffffu / threads) / 8 * 8;  // whole rounds over the XCDs
+  return units - at < most ? units - at : most;
+}
+
 // Tile shapes of a kind, largest first.  unit / stream: microseconds that one
 // tile of K = 1024 takes alone on a CU, and per tile when several share the CU.
 constexpr int kDirectTiles = 4;

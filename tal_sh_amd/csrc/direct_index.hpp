@@ -147,7 +147,8 @@ struct DirectArgs {
   int32_t gx, gy;               // tiles along m and n
   int32_t whole;                // tiles [0, whole) take all of K, one workgroup each
   int32_t rem, ksplit, ksteps;  // the rem tiles after them are cut into ksplit ranges of ksteps K steps
-  int32_t pad0, pad1;
+  int32_t first;                // unit of the launch's first workgroup (a grid holds fewer than 2^32 threads)
+  int32_t pad0;
   int64_t am1, bn1, dm1, dn1;   // strides of m and n where they have one dimension
   int64_t ka1, kb1;             // strides of k's first dimension
   double ar, ai;

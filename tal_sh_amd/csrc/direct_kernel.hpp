@@ -271,7 +271,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   // smaller tiles, and four levels of priority cost R4 23 %).
   if (BM * BN == 128 * 128 && (blockIdx.x >> 8 & 1)) __builtin_amdgcn_s_setprio(1);
   // units: the whole tiles, then the K ranges of the others
-  int u = blockIdx.x, tile, kpart = 0;
+  int u = p.first + (int)blockIdx.x, tile, kpart = 0;
   const bool part = u >= p.whole;
   if (!part) {
     tile = u = xcd_order(u, p.whole);

@@ -17,15 +17,19 @@ struct Tile {
 };
 
 template <typename S, int NC, class T, int KA, int KBC, int W, int MODE>
-void run(const DirectArgs &a, unsigned batch, hipStream_t s) {
-  const dim3 grid((unsigned)(a.whole + a.rem * a.ksplit), batch), block(64 * T::WM * T::WN);
+void run(DirectArgs a, unsigned batch, hipStream_t s) {
+  constexpr unsigned NT = 64 * T::WM * T::WN;
   constexpr auto kernel =
       direct_kernel<S, NC, KA, KBC, W, W, T::BM, T::BN, T::KB, T::WM, T::WN, T::PF, T::OCC, MODE>;
-  if (a.rem == 0) {
-    launch_last(kernel, grid, block, s, a);
-    return;
+  const int64_t units = a.whole + (int64_t)a.rem * a.ksplit;
+  int64_t at = 0;
+  for (int64_t n; (n = direct_launch_units(units, at, NT)) > 0; at += n) {
+    const dim3 grid((unsigned)n, batch), block(NT);
+    a.first = (int32_t)at;
+    if (a.rem == 0 && at + n == units) launch_last(kernel, grid, block, s, a);
+    else kernel<<<grid, block, 0, s>>>(a);
   }
-  kernel<<<grid, block, 0, s>>>(a);
+  if (a.rem == 0) return;
   constexpr int kBlocks = (T::BM / 16) * (T::BN / 16);  // 16 x 16 blocks of a tile
   launch_last(direct_reduce<S, NC, T::BM, T::BN, T::WM, T::WN>, dim3((unsigned)(((int64_t)a.rem * kBlocks + 3) / 4)),
               dim3(256), s, a);

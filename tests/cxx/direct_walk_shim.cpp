@@ -223,6 +223,16 @@ int route_of(const char *pattern, const int *ddims, const int *ldims, const int 
   return r;
 }
 
+// Units of the launch that begins at unit `at`.
+long long launch_units(long long units, long long at, unsigned threads) { return direct_launch_units(units, at, threads); }
+
+// Whether a product has a tile shape, and its number of workgroups and threads of each.
+int choose_units(int dk, long long M, long long N, long long K, int cus, long long *units) {
+  const DirectChoice c = direct_choose(dk, M, N, K, 1, cus);
+  *units = c.whole + c.rem * c.ksplit;
+  return c.us >= 0;
+}
+
 // Mode, tile and K range (in K) that a contraction gets straight from the
 // tensors on a GPU of `cus` compute units, with tile's K step.
 int direct_variant(const char *pattern, const int *ddims, const int *ldims, const int *rdims, int dk, int cus, int *out) {

@@ -167,3 +167,24 @@ def test_far_operands_take_the_direct_kernels(walk, dk):
         out = (ctypes.c_int * 3)()
         assert walk.route_of(pattern.encode(), *dims, dk, 256, out) == ROUTE_COPIES, (pattern, ext)
         assert out[0] == MODE_FAR, (pattern, ext)
+
+
+@pytest.mark.parametrize("dk", (4, 8, 14, 18))
+def test_launches_hold_fewer_threads_than_a_grid_can(walk, dk):
+    """Products of up to 2^31 rows: every unit is launched once, in grids of fewer than 2^32 threads."""
+    LL = ctypes.c_longlong
+    walk.launch_units.restype, walk.launch_units.argtypes = LL, [LL, LL, ctypes.c_uint]
+    walk.choose_units.argtypes = [ctypes.c_int, LL, LL, LL, ctypes.c_int, ctypes.POINTER(LL)]
+    for M in (1, 1000, 536870913, 1073741825, 1100000000, 2147483520):
+        for N in (1, 24, 100):
+            for swap in (0, 1):
+                units = LL()
+                assert walk.choose_units(dk, N if swap else M, M if swap else N, 2, 256, ctypes.byref(units)) == 1
+                assert 0 < units.value < 2 ** 31
+                for threads in (256, 512):
+                    at = 0
+                    while at < units.value:
+                        n = walk.launch_units(units.value, at, threads)
+                        assert n > 0 and n * threads < 2 ** 32
+                        at += n
+                    assert at == units.value and walk.launch_units(units.value, at, threads) == 0

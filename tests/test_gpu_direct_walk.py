@@ -96,3 +96,22 @@ def test_far_operands(talsh_gpu, dk, case):
     pattern, ext = FAR[dk][case]
     check(talsh_gpu, dk, pattern, ext, largest=1 if dk in (R4, C4) else 8)
     torch.cuda.empty_cache()
+
+
+def test_more_rows_than_one_grid_holds(talsh_gpu):
+    ts = talsh_gpu
+    M = 1100000000
+    print("[case] rows", M, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    L = torch.empty(2 * M, device="cuda").random_(-8, 9, generator=gen)
+    R = torch.tensor([3.0, -2.0], device="cuda")
+    D = torch.full((M,), 5.0, device="cuda")
+    torch.cuda.synchronize()
+    ten = [ts.Tensor(R4, d, ts.gpu_flat(0), ext=b.data_ptr()) for d, b in (([M], D), ([M, 2], L), ([2], R))]
+    ts.check(ts.contract("D(a)+=L(a,k)*R(k)", *ten, alpha=1.0, accumulative=ts.YEP), "contract")
+    for at in range(0, M, 1 << 28):  # a piece at a time
+        b = slice(at, min(M, at + (1 << 28)))
+        assert torch.equal(D[b], 5.0 + 3.0 * L[:M][b] - 2.0 * L[M:][b]), at
+    for t in ten:
+        t.destruct()
+    torch.cuda.empty_cache()
