@@ -40,6 +40,17 @@ int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, voi
                   bool conjb, bool accumulate, void *ws, size_t ws_bytes, hipStream_t s) {
   const int esz = direct_elem(dk);
   if (!esz || !A || !B || !D) return -1;
+  if (f.K > kDirectMaxK) {
+    if (f.k.size() != 1) return -4;
+    DirectForm g = f;
+    for (int64_t k0 = 0; k0 < f.K; k0 += g.K) {
+      g.K = g.k[0].ext = std::min(kDirectMaxK, f.K - k0);
+      if (int e = launch_direct(dk, g, (const char *)A + k0 * f.k[0].s[0] * esz, (const char *)B + k0 * f.k[0].s[1] * esz,
+                                D, ar, ai, conja, conjb, accumulate || k0 > 0, ws, ws_bytes, s))
+        return e;
+    }
+    return 0;
+  }
   DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
   if (c.part_bytes > ws_bytes || (c.part_bytes && !ws)) {  // no room for partial sums: whole tiles
     c.whole = c.gx * c.gy;

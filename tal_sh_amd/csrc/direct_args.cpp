@@ -82,7 +82,7 @@ bool wide(const std::vector<DirectDim> &rows, const std::vector<DirectDim> &k, i
 bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, DirectArgs *a, DirectVariant *v) {
   std::memset(a, 0, sizeof(*a));
   constexpr int64_t kMax = 0x7fffffff - 127;  // a tile past the edge is still numbered in 31 bits
-  if (f.M < 1 || f.N < 1 || f.K < 0 || f.batch < 1 || f.M > kMax || f.N > kMax || f.K > kMax) return false;
+  if (f.M < 1 || f.N < 1 || f.K < 0 || f.batch < 1 || f.M > kMax || f.N > kMax || f.K > kDirectMaxK) return false;
   if (!single_group(f.m, 0, esz, &a->am) || !single_group(f.n, 0, esz, &a->bn) || !single_group(f.m, 1, esz, &a->dm) ||
       !single_group(f.n, 1, esz, &a->dn) || !pair_group(f.k, esz, &a->k))
     return false;
@@ -156,6 +156,12 @@ bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, Direct
 
 bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v) {
   DirectArgs a;
+  if (f.K > kDirectMaxK) {
+    if (f.k.size() != 1) return false;
+    DirectForm g = f;
+    g.K = g.k[0].ext = kDirectMaxK;
+    return direct_addressable(g, dk, v);
+  }
   return direct_args(f, direct_elem(dk), direct_width(dk), 16, &a, v);
 }
 
@@ -183,6 +189,7 @@ constexpr size_t kMaxPart = (size_t)64 << 20;
 DirectChoice direct_choose(int dk, int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
   const DirectTile *tiles = direct_tiles(dk);
   const int esz = direct_elem(dk);
+  K = std::min(K, kDirectMaxK);  // of the first of several launches
   DirectChoice best;
   best.us = -1;  // stays where every tile shape makes too many
   for (int swap = 0; swap < 2; ++swap) {

@@ -26,7 +26,10 @@ struct DirectVariant {
 // dimensions in a group, extents past 31 bits, strides past 32 bits where rows
 // or k have several dimensions).
 bool direct_args(const DirectForm &f, int esz, int full_width, int kstep, DirectArgs *a, DirectVariant *v);
-// Whether direct_args accepts the form for data kind dk at every tile, either way round; the variant at K steps of 16.
+// Longest K of one launch: a longer product (k of one dimension) is summed into D range after range.
+constexpr int64_t kDirectMaxK = (int64_t)1 << 30;
+
+// Whether the direct kernels take the form for data kind dk at every tile, either way round; the variant at K steps of 16.
 bool direct_addressable(const DirectForm &f, int dk, DirectVariant *v);
 
 // Units of one launch of workgroups of `threads`, from unit `at` of `units` on: a

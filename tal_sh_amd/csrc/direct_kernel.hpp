@@ -237,7 +237,7 @@ struct SlabOffsets {
 //      apart for 32-bit offsets within a tile: a 64-bit address per load and
 //      lane, advanced by a constant. Rows past the edge read the last row again
 //      (their products are never stored).
-//      R8, in us, by the wide-address kernel that ran them before and now: 208^3
+//      R8, in us, by the kernel with 64-bit index arithmetic before and now: 208^3
 //      rows by 208 and 208 24,400 -> 18,000, 9,000,000 by 24 and 24 3,090 ->
 //      1,460; C8 8,000,000 by 32 and 32 4,990 -> 2,430; R8 130 x 130 by
 //      2,200,000 along k, one tile there and cut into K ranges here, 364,000 ->

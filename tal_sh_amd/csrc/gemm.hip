@@ -1,16 +1,12 @@
-// Split R4 GEMMs (fast math) and the wide-address GEMM (gfx950).
+// Split R4 GEMMs (fast math, gfx950).
 //
-// Contract of both (the GEMM call of gpu_tensor_block_contract_dlf,
+// Contract (the GEMM call of gpu_tensor_block_contract_dlf,
 // tensor_algebra_gpu_nvidia.cu:6851-7060):
 //   C(MxN, column-major, ldc) = alpha * op(A) * op(B) + beta * C,  beta in {0,1}
-// with op(A) in {A, A^T} and op(B) in {B, B^T}, complex operands optionally
-// conjugated.  Other products run on the direct contraction kernels
-// (direct_kernel.hpp).  Blocks are renumbered so that each XCD (dispatch
-// round-robins workgroups over the 8 XCDs) walks a compact band of C tiles and
-// the operand panels it streams stay in its own L2.  MFMA fragment layout
-// (16x16x4): A lane l holds A[l%16][l/16], B lane l holds B[l/16][l%16];
-// accumulator register r of lane l holds C[4*(l/16)+r][l%16] for f32 and
-// C[4*r+l/16][l%16] for f64.
+// with op(A) in {A, A^T} and op(B) in {B, B^T}.  All other products run on the
+// direct contraction kernels (direct_kernel.hpp).  Blocks are renumbered so that
+// each XCD (dispatch round-robins workgroups over the 8 XCDs) walks a compact
+// band of C tiles and the operand panels it streams stay in its own L2.
 #include "kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -21,26 +17,9 @@ namespace tal {
 
 namespace {
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <typename S>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  using acc_t = f64x4;
-  __device__ static int row(int lane, int r) { return 4 * r + (lane >> 4); }
-  __device__ static acc_t op(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-};
-template <>
-struct Mfma<float> {
-  using acc_t = f32x4;
-  __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-  __device__ static acc_t op(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-};
-
 constexpr int kThreads = 256;
-constexpr int BK = 16;
 constexpr int kXcds = 8;
 
 // Tile t of C -> (bx, by): tiles are walked in groups of 8 tile-rows, column
@@ -55,144 +34,11 @@ __device__ inline void tile_xy(int64_t t, int64_t gx, int64_t gy, int64_t &bx, i
   by = in / rows;
 }
 
-// Tile of this workgroup among the `count` tiles starting at t0, renumbered
-// so that consecutive tiles of one XCD are neighbours: XCD x (= launch index
-// % 8) gets the x-th contiguous slice of them.
-__device__ inline void tile_of(int64_t gx, int64_t gy, int64_t t0, int64_t count, int64_t &bx, int64_t &by) {
-  const int64_t id = (int64_t)blockIdx.x;
-  int64_t t = id;
-  if (count >= kXcds * 4 && count % kXcds == 0) t = (id % kXcds) * (count / kXcds) + id / kXcds;
-  tile_xy(t0 + t, gx, gy, bx, by);
-}
-
 // Unit u of n in dispatch order -> a number such that the units of one XCD are
 // neighbours, for any n (a bijection of [0, n)).
 __device__ inline int64_t xcd_order(int64_t u, int64_t n) {
   const int64_t q = n / kXcds, r = n % kXcds, x = u % kXcds;
   return x * q + min(x, r) + u / kXcds;
-}
-
-// Products whose operands the direct kernels cannot address (an operand of
-// 2 GiB or more with rows too far apart for 32-bit offsets within a tile):
-// every access works its 64-bit address out.  One tile shape per kind, 4 waves
-// in a 2 x 2 grid, element loads into a double-buffered LDS stage.
-// Layout codes: 0 = N, 1 = T; conja / conjb: sign of an operand's imaginary part.
-template <typename S, int NC, int OPA, int OPB, int BM, int BN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(
-    int64_t M, int64_t N, int64_t K, const S *__restrict__ A, int64_t lda, const S *__restrict__ B, int64_t ldb,
-    S *__restrict__ C, int64_t ldc, S alpha_r, S alpha_i, S sa, S sb, int beta_one, int64_t gx, int64_t gy,
-    int64_t bsa, int64_t bsb, int64_t bsc) {
-  using MF = Mfma<S>;
-  using acc_t = typename MF::acc_t;
-  A += (int64_t)blockIdx.y * bsa;
-  B += (int64_t)blockIdx.y * bsb;
-  C += (int64_t)blockIdx.y * bsc;
-  constexpr int NT = 256, SM = BM / 32, SN = BN / 32, RS = BK + 2;
-  // tile elements are moved one by one along the contiguous axis (m for 'N', k for 'T')
-  constexpr int ATPL = OPA == 0 ? BM : BK, BTPL = OPB == 0 ? BK : BN;
-  constexpr int AVEC = BM * BK / NT, BVEC = BN * BK / NT, ALS = NT / ATPL, BLS = NT / BTPL;
-  __shared__ S As[2][NC][BM][RS];
-  __shared__ S Bs[2][NC][BN][RS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  int64_t bx, by;
-  tile_of(gx, gy, 0, gx * gy, bx, by);
-  const int64_t m0 = bx * BM, n0 = by * BN;
-  const int a_c = tid % ATPL, a_l = tid / ATPL, b_c = tid % BTPL, b_l = tid / BTPL;
-  S ra[AVEC][NC], rb[BVEC][NC];
-  auto load_tiles = [&](int64_t k0) {
-#pragma unroll
-    for (int e = 0; e < AVEC; ++e) {
-      const int line = a_l + e * ALS;
-      const int64_t m = m0 + (OPA == 0 ? a_c : line), k = k0 + (OPA == 0 ? line : a_c);
-      const bool ok = m < M && k < K;
-      const int64_t off = OPA == 0 ? m + k * lda : k + m * lda;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) ra[e][c] = ok ? A[off * NC + c] : (S)0;
-    }
-#pragma unroll
-    for (int e = 0; e < BVEC; ++e) {
-      const int line = b_l + e * BLS;
-      const int64_t n = n0 + (OPB == 0 ? line : b_c), k = k0 + (OPB == 0 ? b_c : line);
-      const bool ok = n < N && k < K;
-      const int64_t off = OPB == 0 ? k + n * ldb : n + k * ldb;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) rb[e][c] = ok ? B[off * NC + c] : (S)0;
-    }
-  };
-  auto store_tiles = [&](int buf) {
-#pragma unroll
-    for (int e = 0; e < AVEC; ++e) {
-      const int line = a_l + e * ALS;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) As[buf][c][OPA == 0 ? a_c : line][OPA == 0 ? line : a_c] = c ? sa * ra[e][c] : ra[e][c];
-    }
-#pragma unroll
-    for (int e = 0; e < BVEC; ++e) {
-      const int line = b_l + e * BLS;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) Bs[buf][c][OPB == 0 ? line : b_c][OPB == 0 ? b_c : line] = c ? sb * rb[e][c] : rb[e][c];
-    }
-  };
-  acc_t acc[NC][SM][SN];
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int i = 0; i < SM; ++i)
-#pragma unroll
-      for (int j = 0; j < SN; ++j) acc[c][i][j] = acc_t{0, 0, 0, 0};
-  const int64_t nk = (K + BK - 1) / BK;
-  load_tiles(0);
-  store_tiles(0);
-  __syncthreads();
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    const int buf = (int)(kt & 1);
-    if (kt + 1 < nk) load_tiles((kt + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kk = ks * 4 + (lane >> 4);
-      S fa[NC][SM], fb[NC][SN];
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-#pragma unroll
-        for (int i = 0; i < SM; ++i) fa[c][i] = As[buf][c][wm * (BM / 2) + i * 16 + (lane & 15)][kk];
-#pragma unroll
-        for (int j = 0; j < SN; ++j) fb[c][j] = Bs[buf][c][wn * (BN / 2) + j * 16 + (lane & 15)][kk];
-      }
-#pragma unroll
-      for (int i = 0; i < SM; ++i)
-#pragma unroll
-        for (int j = 0; j < SN; ++j) {
-          acc[0][i][j] = MF::op(fa[0][i], fb[0][j], acc[0][i][j]);
-          if (NC == 2) {
-            acc[0][i][j] = MF::op(-fa[NC - 1][i], fb[NC - 1][j], acc[0][i][j]);
-            acc[NC - 1][i][j] = MF::op(fa[0][i], fb[NC - 1][j], acc[NC - 1][i][j]);
-            acc[NC - 1][i][j] = MF::op(fa[NC - 1][i], fb[0][j], acc[NC - 1][i][j]);
-          }
-        }
-    }
-    if (kt + 1 < nk) store_tiles(buf ^ 1);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < SM; ++i)
-#pragma unroll
-    for (int j = 0; j < SN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t m = m0 + wm * (BM / 2) + i * 16 + MF::row(lane, r);
-        const int64_t n = n0 + wn * (BN / 2) + j * 16 + (lane & 15);
-        if (m < M && n < N) {
-          S *c = C + (m + n * ldc) * NC;
-          const S xr = acc[0][i][j][r], xi = acc[NC - 1][i][j][r];
-          const S vr = NC == 1 ? alpha_r * xr : alpha_r * xr - alpha_i * xi;
-          c[0] = beta_one ? c[0] + vr : vr;
-          if (NC == 2) {
-            const S vi = alpha_r * xi + alpha_i * xr;
-            c[NC - 1] = beta_one ? c[NC - 1] + vi : vi;
-          }
-        }
-      }
 }
 
 // ---------------------------------------------------------------------------
@@ -748,28 +594,6 @@ struct TailSplit {
   int64_t rem = 0;
   int ksplit = 1;
 };
-template <typename S, int NC, int BM, int BN>
-int launch_wide(int opa, int opb, int cja, int cjb, int64_t M, int64_t N, int64_t K, const void *A, int64_t lda,
-                const void *B, int64_t ldb, void *C, int64_t ldc, double ar, double ai, int beta_one, int64_t batch,
-                int64_t sa, int64_t sb, int64_t sc, hipStream_t s) {
-  const int64_t gx = (M + BM - 1) / BM, gy = (N + BN - 1) / BN;
-  if (gx * gy > 0x7fffffffLL) return -4;
-  for (int64_t b0 = 0; b0 < batch; b0 += 65535) {  // batch entries go to grid.y, at most 65535 per launch
-    const dim3 grid((unsigned)(gx * gy), (unsigned)std::min<int64_t>(65535, batch - b0));
-    const S *a = (const S *)A + b0 * sa * NC, *b = (const S *)B + b0 * sb * NC;
-    S *c = (S *)C + b0 * sc * NC;
-#define TAL_WIDE(a_, b_)                                                                                          \
-  gemm_wide_kernel<S, NC, a_, b_, BM, BN><<<grid, dim3(256), 0, s>>>(                                             \
-      M, N, K, a, lda, b, ldb, c, ldc, (S)ar, (S)ai, (S)(cja ? -1 : 1), (S)(cjb ? -1 : 1), beta_one, gx, gy,      \
-      sa * NC, sb * NC, sc * NC)
-    if (opa == 0 && opb == 0) TAL_WIDE(0, 0);
-    else if (opa == 0) TAL_WIDE(0, 1);
-    else if (opb == 0) TAL_WIDE(1, 0);
-    else TAL_WIDE(1, 1);
-#undef TAL_WIDE
-  }
-  return hipGetLastError() == hipSuccess ? 0 : -2;
-}
 
 int op_code(char t) {
   switch (t) {
@@ -923,31 +747,6 @@ int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_
   return method == SPLIT_FP16X3
              ? launch_presplit<2>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, cmap, s)
              : launch_presplit<3>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, cmap, s);
-}
-
-int launch_gemm(int dk, char ta, char tb, int conja, int conjb, int64_t M, int64_t N, int64_t K, double ar, double ai,
-                const void *A, int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc,
-                hipStream_t s, int64_t batch, int64_t sa, int64_t sb, int64_t sc) {
-  const bool cplx = (dk == 14 || dk == 18);
-  const int opa = op_code(ta), opb = op_code(tb);
-  const int cja = (cplx && conja) ? 1 : 0, cjb = (cplx && conjb) ? 1 : 0;
-  if (opa < 0 || opb < 0 || M < 0 || N < 0 || K < 0 || !A || !B || !C || batch < 1) return -1;
-  if (M == 0 || N == 0) return 0;
-  if (ldc < std::max<int64_t>(1, M)) return -1;
-  if (lda < std::max<int64_t>(1, opa == 0 ? M : K)) return -1;
-  if (ldb < std::max<int64_t>(1, opb == 0 ? K : N)) return -1;
-  if (batch > 1 && (sa < 0 || sb < 0 || sc < ldc * N)) return -1;  // batch entries of C may not overlap
-#define TAL_GEMM_KIND(S, NC, BM, BN)                                                                              \
-  launch_wide<S, NC, BM, BN>(opa, opb, cja, cjb, M, N, K, A, lda, B, ldb, C, ldc, ar, ai, beta_one, batch, sa, sb, \
-                             sc, s)
-  switch (dk) {
-    case 8: return TAL_GEMM_KIND(double, 1, 128, 128);
-    case 4: return TAL_GEMM_KIND(float, 1, 128, 128);
-    case 18: return TAL_GEMM_KIND(double, 2, 64, 64);
-    case 14: return TAL_GEMM_KIND(float, 2, 64, 64);
-    default: return -1;
-  }
-#undef TAL_GEMM_KIND
 }
 
 }  // namespace tal

@@ -108,8 +108,11 @@ bool gemm_split_bf16_available();
 // operand and three products (fp16x3).
 enum SplitMethod { SPLIT_BF16X6 = 0, SPLIT_FP16X3 = 1 };
 
-// Split R4 GEMM with pre-split operands (same contract as launch_gemm for
-// dk = R4, batch 1); ws is device scratch of gemm_split_workspace(method, M,
+// Split R4 GEMM with pre-split operands:
+//   C(MxN, col-major, ldc) = ar * op(A) * op(B) + beta * C, beta in {0,1}.
+// ta: 'N' A is MxK (lda>=M); 'T' A is KxM (lda>=K).
+// tb: 'N' B is KxN (ldb>=K); 'T' B is NxK (ldb>=N).
+// ws is device scratch of gemm_split_workspace(method, M,
 // N, K) bytes, 16-byte aligned, that holds the planes of both operands.
 // cmap (device, M + N entries): element (m, n) of C is at C[cmap[m] +
 // cmap[M + n]] (elements), so the GEMM can read and write a tensor whose M and
@@ -118,17 +121,6 @@ size_t gemm_split_workspace(int method, int64_t M, int64_t N, int64_t K);
 int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_t K, double ar, const void *A,
                       int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc, void *ws,
                       hipStream_t s, const int64_t *cmap = nullptr);
-
-// C(MxN, col-major, ldc) = alpha * op(A) * op(B) + beta * C, beta in {0,1},
-// at any operand size (products the direct kernels cannot address).
-// ta: 'N' A is MxK (lda>=M); 'T' A is KxM (lda>=K).
-// tb: 'N' B is KxN (ldb>=K); 'T' B is NxK (ldb>=N).
-// conja/conjb conjugate complex operands.  Complex kinds use interleaved (re,im) storage.
-// batch > 1: that many independent products, entry q at A + q*sa, B + q*sb,
-// C + q*sc (strides in elements; C entries may not overlap).
-int launch_gemm(int dk, char ta, char tb, int conja, int conjb, int64_t M, int64_t N, int64_t K, double ar, double ai,
-                const void *A, int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc,
-                hipStream_t s, int64_t batch = 1, int64_t sa = 0, int64_t sb = 0, int64_t sc = 0);
 
 // Offsets of a C map: for the mixed-radix index m over extents ext[0..nm)
 // (first fastest), out[m] = sum of digit_t * str[t]; out[M + n] likewise

@@ -549,8 +549,6 @@ TtgtTemps ttgt_temp_bytes(const ContractPlan &plan, int dk, size_t lbytes, size_
   if (route == kRouteCopies) {
     if (plan.d_transpose && !plan.mat_d_in_place) t.d = dbytes;
     t.s = direct_choose(dk, plan.M, plan.N, plan.K, plan.batch).part_bytes;
-  } else if (route == kRouteWide) {
-    if (plan.d_transpose) t.d = dbytes;
   } else {
     int nm = 0, nn = 0;
     if (d_in_place(plan, &nm, &nn)) t.d = (size_t)(plan.M + plan.N) * sizeof(int64_t);  // the C map
@@ -635,12 +633,12 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
   if (gemm_start) (void)hipEventRecord(gemm_start, s);
   const bool d_back = plan.d_transpose && !in_place;
   if (!d_back) clock.done = done;
-  // hyper indices: plan.batch products of M x N x K, each operand strided by one matrix
-  const int64_t sa = plan.M * plan.K, sb = plan.K * plan.N, sc = plan.M * plan.N;
   if (route == kRouteCopies) {
     if (launch_direct(dk, plan.mat, A, B, C, ar, cplx ? ai : 0.0, aconj, bconj, acc, tmp.s, tmp.s_bytes, s))
       return TALSH_FAILURE;
-  } else if (route == kRouteSplit) {
+  } else {
+    // hyper indices: plan.batch products of M x N x K, each operand strided by one matrix
+    const int64_t sa = plan.M * plan.K, sb = plan.K * plan.N, sc = plan.M * plan.N;
     if (!tmp.w) return TALSH_FAILURE;
     for (int64_t q = 0; q < plan.batch; ++q)  // the planes workspace is reused in stream order
       if (launch_gemm_split(tmp.split, plan.a.op, plan.b.op, plan.M, plan.N, plan.K, ar,
@@ -648,10 +646,6 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
                             (const float *)B + q * sb, plan.b.ld, acc ? 1 : 0, (float *)C + q * sc,
                             std::max<int64_t>(1, plan.M), tmp.w, s, cmap))
         return TALSH_FAILURE;
-  } else if (launch_gemm(dk, plan.a.op, plan.b.op, aconj, bconj, plan.M, plan.N, plan.K, ar, cplx ? ai : 0.0, A,
-                         plan.a.ld, B, plan.b.ld, acc ? 1 : 0, C, std::max<int64_t>(1, plan.M), s, plan.batch, sa, sb,
-                         sc)) {
-    return TALSH_FAILURE;
   }
   if (gemm_end) (void)hipEventRecord(gemm_end, s);
   clock.done = done;

@@ -17,12 +17,11 @@ namespace tal {
 // A transpose moves 4.6 TB/s and takes about 4 us beside that.
 Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c) {
   DirectVariant v;
-  const bool mat_ok = direct_addressable(plan.mat, dk, &v);
   if (plan.direct_ok && direct_addressable(plan.direct, dk, &v) && v.mode < 3) {
     const DirectForm &f = plan.direct;
     const int esz = direct_elem(dk);
     const bool d_copy = plan.d_transpose && !plan.mat_d_in_place;
-    if (mat_ok && !plan.a.transpose && !plan.b.transpose && !d_copy) return kRouteCopies;  // nothing to copy
+    if (!plan.a.transpose && !plan.b.transpose && !d_copy) return kRouteCopies;  // nothing to copy
     const double avol = (double)f.avol * esz, bvol = (double)f.bvol * esz;
     const double dvol = (double)f.M * (double)f.N * (double)f.batch * esz;
     const bool ta = plan.swap ? plan.b.transpose : plan.a.transpose, tb = plan.swap ? plan.a.transpose : plan.b.transpose;
@@ -34,9 +33,9 @@ Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c) {
     if (plan.direct_run && plan.direct_run < 8) extra += 0.3 * gemm;
     if (plan.direct_conflict) extra += std::min(avol, bvol) > 4e6 ? 1e9 : 0.5 * gemm;
     if (plan.direct_scatter) extra += 4 * dvol / 4.6e6;
-    if (!mat_ok || copies > extra) return kRouteDirect;
+    if (copies > extra) return kRouteDirect;
   }
-  return mat_ok ? kRouteCopies : kRouteWide;
+  return kRouteCopies;
 }
 
 }  // namespace tal

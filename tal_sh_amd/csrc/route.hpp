@@ -8,8 +8,8 @@ namespace tal {
 
 // A plain product by the direct kernels straight from the tensors, or on copies
 // of the operands the planner transposes (with D written in place or through
-// D'); by the wide-address kernel on such copies; or by the fast-math GEMMs.
-enum Route { kRouteDirect, kRouteCopies, kRouteWide, kRouteSplit };
+// D'), or a product by the fast-math GEMMs on such copies.
+enum Route { kRouteDirect, kRouteCopies, kRouteSplit };
 
 // Of a plan without fast math; c: the direct kernels' choice for its product.
 Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c);

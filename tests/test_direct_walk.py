@@ -188,3 +188,13 @@ def test_launches_hold_fewer_threads_than_a_grid_can(walk, dk):
                         assert n > 0 and n * threads < 2 ** 32
                         at += n
                     assert at == units.value and walk.launch_units(units.value, at, threads) == 0
+
+
+def test_k_past_one_launch(walk):
+    for d, l, r, ext in (([], ["a", "b"], ["a", "b"], dict(a=65536, b=33000)),
+                         (["m", "n"], ["a", "m", "b"], ["b", "n", "a"], dict(a=65536, b=33000, m=2, n=3))):
+        pattern = "D(%s)+=L(%s)*R(%s)" % (",".join(d), ",".join(l), ",".join(r))
+        dims = [(ctypes.c_int * max(1, len(lab)))(*[ext[x] for x in lab]) for lab in (d, l, r)]
+        in_place = ctypes.c_int()
+        for dk in (4, 8, 14, 18):
+            assert walk.mat_addressable(pattern.encode(), *dims, dk, ctypes.byref(in_place)) == 1

@@ -115,3 +115,23 @@ def test_more_rows_than_one_grid_holds(talsh_gpu):
     for t in ten:
         t.destruct()
     torch.cuda.empty_cache()
+
+
+def test_more_contracted_indices_than_one_launch_takes(talsh_gpu):
+    """Longer than 2^31: ranges of 2^30 are summed one after the other. Sums of K products of -1, 0 and 1 stay far below
+    2^24 (standard deviation 2/3 sqrt(K) = 31,000), so the result is exact."""
+    ts = talsh_gpu
+    dims = [65536, 33000]
+    print("[case] contracted indices", dims, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    L, R = (torch.empty(dims[0] * dims[1], device="cuda").random_(-1, 2, generator=gen) for _ in range(2))
+    D = torch.full((1,), 5.0, device="cuda")
+    want = 5.0 - 2.0 * sum((L[at:at + (1 << 28)] * R[at:at + (1 << 28)]).sum(dtype=torch.float64).item()
+                           for at in range(0, L.numel(), 1 << 28))
+    torch.cuda.synchronize()
+    ten = [ts.Tensor(R4, d, ts.gpu_flat(0), ext=b.data_ptr()) for d, b in (([], D), (dims, L), (dims, R))]
+    ts.check(ts.contract("D()+=L(a,b)*R(a,b)", *ten, alpha=-2.0, accumulative=ts.YEP), "contract")
+    assert D.item() == want
+    for t in ten:
+        t.destruct()
+    torch.cuda.empty_cache()
