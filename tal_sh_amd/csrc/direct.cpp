@@ -37,7 +37,7 @@ DirectChoice direct_choose(int dk, int64_t M, int64_t N, int64_t K, int64_t batc
 }
 
 int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, void *D, double ar, double ai, bool conja,
-                  bool conjb, bool accumulate, void *ws, size_t ws_bytes, hipStream_t s) {
+                  bool conjb, bool accumulate, void *sums, hipStream_t s) {
   const int esz = direct_elem(dk);
   if (!esz || !A || !B || !D) return -1;
   if (f.K > kDirectMaxK) {
@@ -46,13 +46,13 @@ int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, voi
     for (int64_t k0 = 0; k0 < f.K; k0 += g.K) {
       g.K = g.k[0].ext = std::min(kDirectMaxK, f.K - k0);
       if (int e = launch_direct(dk, g, (const char *)A + k0 * f.k[0].s[0] * esz, (const char *)B + k0 * f.k[0].s[1] * esz,
-                                D, ar, ai, conja, conjb, accumulate || k0 > 0, ws, ws_bytes, s))
+                                D, ar, ai, conja, conjb, accumulate || k0 > 0, sums, s))
         return e;
     }
     return 0;
   }
   DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch);
-  if (c.part_bytes > ws_bytes || (c.part_bytes && !ws)) {  // no room for partial sums: whole tiles
+  if (c.part_bytes && !sums) {  // no room for partial sums: whole tiles
     c.whole = c.gx * c.gy;
     c.rem = 0;
     c.ksplit = 1;
@@ -78,7 +78,7 @@ int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, voi
   a.ksteps = c.ksteps;
   a.ar = ar;
   a.ai = ai;
-  a.part = ws;
+  a.part = sums;
   a.flags |= (accumulate ? kDirectBeta : 0) | (conja ? kDirectConjA : 0) | (conjb ? kDirectConjB : 0);
   const DirectLaunch launch =
       dk == 8 ? direct_launch_r8 : dk == 4 ? direct_launch_r4 : dk == 18 ? direct_launch_c8 : direct_launch_c4;

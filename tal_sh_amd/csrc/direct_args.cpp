@@ -178,9 +178,6 @@ const DirectTile *direct_tiles(int dk) {
   return dk == 8 ? r8 : dk == 4 ? r4 : dk == 18 ? c8 : c4;
 }
 
-// Most workspace a product's partial sums may take.
-constexpr size_t kMaxPart = (size_t)64 << 20;
-
 // Every tile shape is tried, both ways round.  A CU that gets u tiles (u may
 // be a fraction where tiles are split along K) takes max(unit, u * stream)
 // per 1024 of K.  The tiles that do not fill a last round over the CUs are cut
@@ -227,7 +224,7 @@ DirectChoice direct_choose(int dk, int64_t M, int64_t N, int64_t K, int64_t batc
         const double us = (double)(whole / cus) + (double)((rem * ks + cus - 1) / cus) * part;
         const double one = whole ? ti.unit : ti.unit * part;
         const size_t bytes = (size_t)rem * ks * ti.bm * ti.bn * esz;
-        if (bytes > kMaxPart) continue;
+        if (bytes > kSumsBytes) continue;
         consider(whole, rem, (int)ks, steps, std::max(one, us * ti.stream) * k + 5.0 + 2.0 * bytes / 3.5e6, bytes);
       }
     }

@@ -48,6 +48,9 @@ struct DirectTile {
 };
 const DirectTile *direct_tiles(int dk);
 
+// Most memory that the partial sums of a product's K ranges may take.
+constexpr size_t kSumsBytes = (size_t)64 << 20;
+
 // Tile shape and K split of a product on a GPU of `cus` compute units; depends on nothing else.
 struct DirectChoice {
   bool swap = false;  // A and B exchange roles

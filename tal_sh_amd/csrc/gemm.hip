@@ -628,20 +628,23 @@ static int64_t presplit_slots() {
 
 // K split of a partial last round of tiles: as many ranges as make it shortest,
 // counted in K steps.  A range costs about 4 steps beside its own (its first
-// loads, its partial sums written and read again): 5184^3 in fp16x3 has 861
+// loads) and the way of its partial sums through memory, 128 KB written and read
+// again (a step is 1.3 us of fp16x3, 2.3 of bf16x6): 5184^3 in fp16x3 has 861
 // tiles on 256 slots, and its 93 last ones run as 5 ranges each, 0.5 of a round
-// instead of a whole one (and 20 us of summing against 110 saved).
+// instead of a whole one (and 20 us of summing against 110 saved).  All ranges'
+// sums have to fit into kSumsBytes, two rounds of them.
 template <int NP>
-static TailSplit presplit_tail(int64_t M, int64_t N, int64_t K) {
+static TailSplit presplit_tail(int64_t M, int64_t N, int64_t K, bool room) {
   TailSplit t;
-  if (M <= 0 || N <= 0) return t;
+  if (M <= 0 || N <= 0 || !room) return t;
   const int64_t T = (round_up(M, PBM) / PBM) * (round_up(N, PBN) / PBN), slots = presplit_slots<NP>();
   if (slots <= 0) return t;
   const int64_t rem = T % slots, nks = round_up(std::max<int64_t>(K, 1), PBK) / PBK;
   if (rem == 0) return t;
-  int64_t best = nks;
-  for (int64_t ks = 2; ks <= 16 && ks * 8 <= nks; ++ks) {
-    const int64_t cost = (rem * ks + slots - 1) / slots * ((nks + ks - 1) / ks + 4);
+  double best = (double)nks;
+  for (int64_t ks = 2; ks <= 16 && ks * 8 <= nks && rem * ks * PBM * PBN * 4 <= (int64_t)kSumsBytes; ++ks) {
+    const double cost = (double)((rem * ks + slots - 1) / slots * ((nks + ks - 1) / ks + 4)) +
+                        (NP == 2 ? 0.033 : 0.019) * (double)(rem * ks);
     if (cost < best) {
       best = cost;
       t.rem = rem;
@@ -652,12 +655,11 @@ static TailSplit presplit_tail(int64_t M, int64_t N, int64_t K) {
 }
 
 // Workspace of the pre-split GEMM: the planes of op(A) and op(B) (NP planes
-// of 2-byte values each), for NP = 2 the row / column maxima, then the
-// partial sums of a K-split last round; each part starts on 256 bytes.
+// of 2-byte values each) and for NP = 2 the row / column maxima; each part
+// starts on 256 bytes.
 struct SplitLayout {
   int64_t Mp, Np, Kp;
-  size_t a, b, ua, ub, part, total;
-  TailSplit tail;
+  size_t a, b, ua, ub, total;
 };
 
 template <int NP>
@@ -666,21 +668,20 @@ static SplitLayout split_layout(int64_t M, int64_t N, int64_t K) {
   l.Mp = round_up(std::max<int64_t>(M, 1), PBM);
   l.Np = round_up(std::max<int64_t>(N, 1), PBN);
   l.Kp = round_up(std::max<int64_t>(K, 1), PBK);
-  l.tail = presplit_tail<NP>(M, N, K);
   l.a = 0;
   l.b = l.a + (size_t)round_up(2 * NP * l.Mp * l.Kp, 256);
   l.ua = l.b + (size_t)round_up(2 * NP * l.Np * l.Kp, 256);
   l.ub = l.ua + (NP == 2 ? (size_t)round_up(4 * l.Mp, 256) : 0);
-  l.part = l.ub + (NP == 2 ? (size_t)round_up(4 * l.Np, 256) : 0);
-  l.total = l.part + (l.tail.ksplit > 1 ? (size_t)l.tail.rem * l.tail.ksplit * PBM * PBN * sizeof(float) : 0);
+  l.total = l.ub + (NP == 2 ? (size_t)round_up(4 * l.Np, 256) : 0);
   return l;
 }
 
 template <int NP>
 static int launch_presplit(int opa, int opb, int64_t M, int64_t N, int64_t K, double ar, const void *A, int64_t lda,
                            const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc, void *ws,
-                           const int64_t *cmap, hipStream_t s) {
+                           void *sums, const int64_t *cmap, hipStream_t s) {
   const SplitLayout l = split_layout<NP>(M, N, K);
+  const TailSplit tail = presplit_tail<NP>(M, N, K, sums != nullptr);
   char *w = (char *)ws;
   uint4 *pa = (uint4 *)(w + l.a), *pb = (uint4 *)(w + l.b);
   uint32_t *ua = NP == 2 ? (uint32_t *)(w + l.ua) : nullptr, *ub = NP == 2 ? (uint32_t *)(w + l.ub) : nullptr;
@@ -695,7 +696,7 @@ static int launch_presplit(int opa, int opb, int64_t M, int64_t N, int64_t K, do
   p.nks = l.Kp / PBK;
   p.C = (float *)C;
   p.cmap = cmap;
-  p.part = (float *)(w + l.part);
+  p.part = (float *)sums;
   p.ua = ua;
   p.ub = ub;
   p.M = M;
@@ -703,9 +704,9 @@ static int launch_presplit(int opa, int opb, int64_t M, int64_t N, int64_t K, do
   p.ldc = ldc;
   p.gx = l.Mp / PBM;
   p.gy = l.Np / PBN;
-  p.rem = l.tail.rem;
+  p.rem = tail.rem;
   p.whole = p.gx * p.gy - p.rem;
-  p.ksplit = l.tail.ksplit;
+  p.ksplit = tail.ksplit;
   p.ksteps = (p.nks + p.ksplit - 1) / p.ksplit;
   p.beta_one = beta_one;
   p.alpha = (float)ar;
@@ -736,7 +737,7 @@ size_t gemm_split_workspace(int method, int64_t M, int64_t N, int64_t K) {
 
 int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_t K, double ar, const void *A,
                       int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc, void *ws,
-                      hipStream_t s, const int64_t *cmap) {
+                      void *sums, hipStream_t s, const int64_t *cmap) {
   const int opa = op_code(ta), opb = op_code(tb);
   if (opa < 0 || opb < 0 || M < 0 || N < 0 || K < 0 || !A || !B || !C || !ws || (uintptr_t)ws % 16) return -1;
   if (method != SPLIT_BF16X6 && method != SPLIT_FP16X3) return -1;
@@ -745,8 +746,8 @@ int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_
   if (lda < std::max<int64_t>(1, opa == 0 ? M : K)) return -1;
   if (ldb < std::max<int64_t>(1, opb == 0 ? K : N)) return -1;
   return method == SPLIT_FP16X3
-             ? launch_presplit<2>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, cmap, s)
-             : launch_presplit<3>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, cmap, s);
+             ? launch_presplit<2>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, sums, cmap, s)
+             : launch_presplit<3>(opa, opb, M, N, K, ar, A, lda, B, ldb, beta_one, C, ldc, ws, sums, cmap, s);
 }
 
 }  // namespace tal

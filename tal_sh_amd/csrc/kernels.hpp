@@ -9,6 +9,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "direct_args.hpp"
+
 namespace tal {
 
 // Events on the kernels of one operation (per host thread).
@@ -112,15 +114,16 @@ enum SplitMethod { SPLIT_BF16X6 = 0, SPLIT_FP16X3 = 1 };
 //   C(MxN, col-major, ldc) = ar * op(A) * op(B) + beta * C, beta in {0,1}.
 // ta: 'N' A is MxK (lda>=M); 'T' A is KxM (lda>=K).
 // tb: 'N' B is KxN (ldb>=K); 'T' B is NxK (ldb>=N).
-// ws is device scratch of gemm_split_workspace(method, M,
-// N, K) bytes, 16-byte aligned, that holds the planes of both operands.
+// ws is device scratch of gemm_split_workspace(method, M, N, K) bytes, 16-byte
+// aligned, that holds the planes of both operands; sums: kSumsBytes for the
+// partial sums of tiles cut along K, or null (none is cut).
 // cmap (device, M + N entries): element (m, n) of C is at C[cmap[m] +
 // cmap[M + n]] (elements), so the GEMM can read and write a tensor whose M and
 // N indices interleave in memory (ldc unused).
 size_t gemm_split_workspace(int method, int64_t M, int64_t N, int64_t K);
 int launch_gemm_split(int method, char ta, char tb, int64_t M, int64_t N, int64_t K, double ar, const void *A,
                       int64_t lda, const void *B, int64_t ldb, int beta_one, void *C, int64_t ldc, void *ws,
-                      hipStream_t s, const int64_t *cmap = nullptr);
+                      void *sums, hipStream_t s, const int64_t *cmap = nullptr);
 
 // Offsets of a C map: for the mixed-radix index m over extents ext[0..nm)
 // (first fastest), out[m] = sum of digit_t * str[t]; out[M + n] likewise

@@ -109,16 +109,6 @@ class Op {
     return TALSH_SUCCESS;
   }
   void *temp(int i) const { return temps_[i]; }
-  // One more temporary if the pool has room for it now: its index, else -1.
-  int acquire_optional(size_t bytes) {
-    void *p = nullptr;
-    int h = -1;
-    if (dev_alloc(g_, bytes, &p, &h)) return -1;
-    temps_.push_back(p);
-    temp_handles_.push_back(h);
-    temp_bytes_.push_back(bytes);
-    return (int)temps_.size() - 1;
-  }
 
   // Starts the task: stream, ordering against earlier work, input transfers.
   // clock: the kernels launched until end() carry dispatch timestamps, which
@@ -532,23 +522,17 @@ void ttgt_cache_clear() {
 // Depends on the plan, the kind, the fast-math mode and the device only.
 static Route plan_route(const ContractPlan &plan, int dk) {
   if (dk == R4 && rt().r4mode == R4_SPLIT_BF16) return kRouteSplit;
-  const DirectForm &f = plan.direct;
-  return contract_route(plan, dk, direct_choose(dk, f.M, f.N, f.K, f.batch));
+  return contract_route(plan, dk, direct_choose);
 }
 
 TtgtTemps ttgt_temp_bytes(const ContractPlan &plan, int dk, size_t lbytes, size_t rbytes, size_t dbytes) {
   TtgtTemps t;
   const Route route = plan_route(plan, dk);
-  if (route == kRouteDirect) {
-    const DirectForm &f = plan.direct;
-    t.s = direct_choose(dk, f.M, f.N, f.K, f.batch).part_bytes;
-    return t;
-  }
+  if (route == kRouteDirect) return t;
   if (plan.a.transpose) t.a = plan.swap ? rbytes : lbytes;
   if (plan.b.transpose) t.b = plan.swap ? lbytes : rbytes;
   if (route == kRouteCopies) {
     if (plan.d_transpose && !plan.mat_d_in_place) t.d = dbytes;
-    t.s = direct_choose(dk, plan.M, plan.N, plan.K, plan.batch).part_bytes;
   } else {
     int nm = 0, nn = 0;
     if (d_in_place(plan, &nm, &nn)) t.d = (size_t)(plan.M + plan.N) * sizeof(int64_t);  // the C map
@@ -569,7 +553,7 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
   const Route route = tmp.split >= 0 ? kRouteSplit : plan_route(plan, dk);
   if (route == kRouteDirect) {
     if (gemm_start) (void)hipEventRecord(gemm_start, s);
-    if (launch_direct(dk, plan.direct, L, R, D, ar, cplx ? ai : 0.0, lconj, rconj, acc, tmp.s, tmp.s_bytes, s))
+    if (launch_direct(dk, plan.direct, L, R, D, ar, cplx ? ai : 0.0, lconj, rconj, acc, tmp.sums, s))
       return TALSH_FAILURE;
     if (gemm_end) (void)hipEventRecord(gemm_end, s);
     return TALSH_SUCCESS;
@@ -634,7 +618,7 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
   const bool d_back = plan.d_transpose && !in_place;
   if (!d_back) clock.done = done;
   if (route == kRouteCopies) {
-    if (launch_direct(dk, plan.mat, A, B, C, ar, cplx ? ai : 0.0, aconj, bconj, acc, tmp.s, tmp.s_bytes, s))
+    if (launch_direct(dk, plan.mat, A, B, C, ar, cplx ? ai : 0.0, aconj, bconj, acc, tmp.sums, s))
       return TALSH_FAILURE;
   } else {
     // hyper indices: plan.batch products of M x N x K, each operand strided by one matrix
@@ -644,7 +628,7 @@ int enqueue_ttgt(const DigitalPattern &p, const ContractPlan &plan, int dk, bool
       if (launch_gemm_split(tmp.split, plan.a.op, plan.b.op, plan.M, plan.N, plan.K, ar,
                             (const float *)A + q * sa, plan.a.ld,
                             (const float *)B + q * sb, plan.b.ld, acc ? 1 : 0, (float *)C + q * sc,
-                            std::max<int64_t>(1, plan.M), tmp.w, s, cmap))
+                            std::max<int64_t>(1, plan.M), tmp.w, tmp.sums, s, cmap))
         return TALSH_FAILURE;
   }
   if (gemm_end) (void)hipEventRecord(gemm_end, s);
@@ -918,16 +902,13 @@ int talshTensorContract(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *lt
   if (tb.d) { id = (int)temps.size(); temps.push_back(tb.d); }
   if (tb.w) { iw = (int)temps.size(); temps.push_back(tb.w); }
   if (int e = op.acquire(temps)) return deferred(g, e);
-  // room for partial sums only helps: without it the product runs in whole tiles
-  const int is = tb.s ? op.acquire_optional(tb.s) : -1;
   if (int e = op.begin(dk, copy_ctrl)) return e;
   TtgtBuffers bufs;
   bufs.a = ia >= 0 ? op.temp(ia) : nullptr;
   bufs.b = ib >= 0 ? op.temp(ib) : nullptr;
   bufs.d = id >= 0 ? op.temp(id) : nullptr;
   bufs.w = iw >= 0 ? op.temp(iw) : nullptr;
-  bufs.s = is >= 0 ? op.temp(is) : nullptr;
-  bufs.s_bytes = is >= 0 ? tb.s : 0;
+  bufs.sums = stream_sums(g, op.stream());
   bufs.split = tb.split;
   op.gemm_events(tb.a || tb.b || tb.d, tb.d);
   if (int e = enqueue_ttgt(p, plan, dk, acc, scale_real, scale_imag, op.operand(0).dptr, op.operand(1).dptr,

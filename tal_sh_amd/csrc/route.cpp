@@ -15,7 +15,7 @@ namespace tal {
 // in 128 x 128 tiles short runs, and any runs by table, cost 40 %; D written 8
 // bytes apart, about four times its bytes.
 // A transpose moves 4.6 TB/s and takes about 4 us beside that.
-Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c) {
+Route contract_route(const ContractPlan &plan, int dk, DirectChooser choose) {
   DirectVariant v;
   if (plan.direct_ok && direct_addressable(plan.direct, dk, &v) && v.mode < 3) {
     const DirectForm &f = plan.direct;
@@ -27,6 +27,7 @@ Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c) {
     const bool ta = plan.swap ? plan.b.transpose : plan.a.transpose, tb = plan.swap ? plan.a.transpose : plan.b.transpose;
     const double copies =
         (2 * ((ta ? avol : 0) + (tb ? bvol : 0) + (d_copy ? dvol : 0))) / 4.6e6 + ((ta || tb) ? 4 : 0) + (d_copy ? 4 : 0);
+    const DirectChoice c = choose(dk, f.M, f.N, f.K, f.batch);
     const double gemm = c.us;
     double extra = 0;
     if (plan.direct_krun) extra += (c.tile ? 0.25 : plan.direct_krun < 32 || v.mode == 2 ? 0.4 : 0.05) * gemm;

@@ -11,7 +11,10 @@ namespace tal {
 // D'), or a product by the fast-math GEMMs on such copies.
 enum Route { kRouteDirect, kRouteCopies, kRouteSplit };
 
-// Of a plan without fast math; c: the direct kernels' choice for its product.
-Route contract_route(const ContractPlan &plan, int dk, const DirectChoice &c);
+// direct_choose on the GPU at hand.
+using DirectChooser = DirectChoice (*)(int dk, int64_t M, int64_t N, int64_t K, int64_t batch);
+
+// Of a plan without fast math.
+Route contract_route(const ContractPlan &plan, int dk, DirectChooser choose);
 
 }  // namespace tal

@@ -214,6 +214,13 @@ size_t image_bytes(const talsh_tens_t *t, int i) {
 }
 
 // ------------------------------------------------------------------ memory
+void *stream_sums(int g, hipStream_t s) {
+  const Device &d = rt().gpus[g];
+  for (size_t i = 0; d.sums && i < d.streams.size(); ++i)
+    if (d.streams[i] == s) return (char *)d.sums + i * kSumsBytes;
+  return nullptr;
+}
+
 int dev_alloc(int g, size_t bytes, void **p, int *handle) {
   const int e = rt().gpus[g].arena.alloc(bytes, p, handle);
   if (rt().log_mem)
@@ -484,6 +491,12 @@ int talshInit(size_t *host_buf_size, int *host_arg_max, int ngpus, int gpu_list[
     d.hip_id = id;
     d.mem_total = tot;
     size_t want = r.dev_buffer_request ? r.dev_buffer_request : (size_t)(0.80 * (double)fr);
+    // before the pool, which may be asked to take all the rest
+    if (hipMalloc(&d.sums, r.nstreams * kSumsBytes) != hipSuccess) {
+      d.sums = nullptr;
+      (void)hipGetLastError();
+    }
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess) return TALSH_FAILURE;
     want = std::min(want, fr);
     void *base = nullptr;
     while (want >= (64u << 20) && hipMalloc(&base, want) != hipSuccess) want = want / 10 * 9;
@@ -538,6 +551,8 @@ int talshShutdown(void) {
     d.free_events.clear();
     for (auto s : d.streams) (void)hipStreamDestroy(s);
     d.streams.clear();
+    if (d.sums) (void)hipFree(d.sums);
+    d.sums = nullptr;
     (void)hipFree(d.base);
     d.on = false;
   }

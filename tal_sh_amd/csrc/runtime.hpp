@@ -54,6 +54,7 @@ struct Device {
   size_t mem_total = 0;
   Arena arena;
   std::vector<hipStream_t> streams;
+  void *sums = nullptr;  // kSumsBytes per stream (stream_sums)
   // per stream: (completion event, weight) of tasks not yet seen complete, oldest first
   std::vector<std::deque<std::pair<EvRef, double>>> backlog;
   std::vector<hipEvent_t> free_events;
@@ -127,6 +128,13 @@ size_t image_bytes(const talsh_tens_t *t, int i);  // bytes of image i's body
 
 // Whether nothing that was submitted to GPU g is still running (completed tasks are dropped from the backlog).
 bool device_idle(int g);
+
+// Device memory for the partial sums of products that are cut along K, for
+// work on this stream of GPU g: its users follow one another there.  Apart from
+// the pool, so that neither a call's acceptance nor the order of its sums
+// depends on what else holds pool memory at the moment.  Null if talshInit found
+// no room for it (products then run uncut).
+void *stream_sums(int g, hipStream_t s);
 
 // Device memory (buffer pool) and host memory (pinned pool, malloc fallback).
 int dev_alloc(int g, size_t bytes, void **p, int *handle);

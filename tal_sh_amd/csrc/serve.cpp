@@ -83,7 +83,7 @@ int estimate(talshAmdServer *s, talshAmdServer::Req *q) {
   if (!resident(r.rtens, s->g)) need += br;
   // the TTGT temporaries talshTensorContract will take from the pool
   const tal::TtgtTemps t = tal::ttgt_temp_bytes(plan, dk, bl, br, bd);
-  need += t.a + t.b + t.d + t.w + t.s;
+  need += t.a + t.b + t.d + t.w;
   q->need = need;
   q->flops = ((dk == C4 || dk == C8) ? 8.0 : 2.0) * (double)plan.M * (double)plan.N * (double)plan.K *
              (double)plan.batch;

@@ -26,7 +26,6 @@
 #include <vector>
 
 #include "contract.hpp"
-#include "direct.hpp"
 #include "plan.hpp"
 #include "runtime.hpp"
 #include "talsh_amd.h"
@@ -244,7 +243,6 @@ int talshTensorContractXL(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *
     for (int j = 0; j < p.rrank; ++j)
       if (rid[j] < nd) N *= t[rid[j]];
     if (dk == R4 && r.r4mode == R4_SPLIT_BF16) b += gemm_split_workspace(r.split_method, M, N, K);
-    else b += direct_choose(dk, M, N, K, 1).part_bytes;
     return b;
   };
   size_t budget = dev.arena.largest_free() / 10 * 9;
@@ -424,8 +422,7 @@ int talshTensorContractXL(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *
       grow(want.b, have.b, tmp.b, fb);
       grow(want.d, have.d, tmp.d, want.d == pdv ? dv : 0);  // a D' temporary, or the GEMM's small offset table
       grow(want.w, have.w, tmp.w, 0);
-      grow(want.s, have.s, tmp.s, 0);
-      tmp.s_bytes = have.s;
+      tmp.sums = stream_sums(g, s);
       tmp.split = want.split;
       if (err) break;
       const void *lp = fetch(hl, l_in_place, p.lrank, ld, ol.data(), pl.data(), lbuf, s);

@@ -209,8 +209,11 @@ int route_of(const char *pattern, const int *ddims, const int *ldims, const int 
   DigitalPattern p;
   ContractPlan plan;
   if (parse_pattern(pattern, &p) || plan_contraction(p, ddims, ldims, rdims, 1, &plan)) return -1;
-  const DirectForm &d = plan.direct;
-  const Route r = contract_route(plan, dk, direct_choose(dk, d.M, d.N, d.K, d.batch, cus));
+  static int on;
+  on = cus;
+  const Route r = contract_route(plan, dk, [](int kind, int64_t M, int64_t N, int64_t K, int64_t batch) {
+    return direct_choose(kind, M, N, K, batch, on);
+  });
   const DirectForm &f = r == kRouteDirect ? plan.direct : plan.mat;
   const DirectChoice c = direct_choose(dk, f.M, f.N, f.K, f.batch, cus);
   DirectArgs a;
