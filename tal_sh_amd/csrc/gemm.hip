@@ -272,12 +272,13 @@ constexpr int kSplitRows = 8;
 template <int KC, int NP>
 __global__ __launch_bounds__(256) void split_planes_kernel(const float *__restrict__ X, int64_t ld, int64_t R,
                                                            int64_t K, int64_t nks, uint4 *__restrict__ P,
-                                                           int64_t plane, int vec, const uint32_t *__restrict__ U) {
+                                                           int64_t plane, int vec, const uint32_t *__restrict__ U,
+                                                           int64_t first) {
   const int tid = threadIdx.x;
   constexpr int ROWS = KC ? kSplitRows : 64, STEPS = 64 / ROWS;  // of a block
-  const int64_t nkb = (nks + STEPS - 1) / STEPS, rg = blockIdx.x / nkb;
+  const int64_t block = first + blockIdx.x, nkb = (nks + STEPS - 1) / STEPS, rg = block / nkb;
   const int64_t r = rg * ROWS + (KC ? (tid >> 2) % ROWS : tid & 63);
-  const int64_t ks = (blockIdx.x - rg * nkb) * STEPS + (KC ? tid / (4 * ROWS) : 0);
+  const int64_t ks = (block - rg * nkb) * STEPS + (KC ? tid / (4 * ROWS) : 0);
   const int c = KC ? tid & 3 : tid >> 6;
   if (ks >= nks) return;
   const int64_t k0 = ks * PBK + c * 8;
@@ -562,7 +563,6 @@ int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, 
                   uint32_t *U, hipStream_t s) {
   const int64_t nks = Kp / PBK, plane = Rp * Kp / 8;
   const int64_t steps = kcont ? 64 / kSplitRows : 1, nblk = Rp / (64 / steps) * ((nks + steps - 1) / steps);
-  if (nblk > 0x7fffffffLL) return -4;
   const int vec = ((uintptr_t)X % 16 == 0) && ld % 4 == 0;
   if (NP == 2 && kcont) {  // maxima and planes in one pass over HBM
     if (Rp / 2 > 0x7fffffffLL) return -4;
@@ -580,10 +580,13 @@ int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, 
       row_absmax_kernel<<<grid, dim3(256), 0, s>>>(X, ld, R, K, kseg, U);
     }
   }
-  if (kcont)
-    split_planes_kernel<1, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
-  else
-    split_planes_kernel<0, NP><<<dim3((unsigned)nblk), dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U);
+  // a grid holds fewer than 2^32 threads: short rows fill a block to an eighth, so 134 million of them take two
+  constexpr int64_t kMost = 0xffffffffu / 256;
+  for (int64_t first = 0; first < nblk; first += kMost) {
+    const dim3 grid((unsigned)std::min(kMost, nblk - first));
+    if (kcont) split_planes_kernel<1, NP><<<grid, dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U, first);
+    else split_planes_kernel<0, NP><<<grid, dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U, first);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

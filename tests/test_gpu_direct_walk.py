@@ -135,3 +135,27 @@ def test_more_contracted_indices_than_one_launch_takes(talsh_gpu):
     for t in ten:
         t.destruct()
     torch.cuda.empty_cache()
+
+
+def test_more_short_rows_than_one_grid_splits(talsh_gpu):
+    """Fast math (bf16x6, exact for small whole numbers): 140 million rows of 8 contracted indices."""
+    ts = talsh_gpu
+    M, K = 140000000, 8
+    print("[case] short rows", M, K, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    L = torch.empty(M * K, device="cuda").random_(-8, 9, generator=gen)
+    R = torch.empty(K, device="cuda").random_(-8, 9, generator=gen)
+    D = torch.full((M,), 5.0, device="cuda")
+    torch.cuda.synchronize()
+    ten = [ts.Tensor(R4, d, ts.gpu_flat(0), ext=b.data_ptr()) for d, b in (([M, 1], D), ([K, M], L), ([K, 1], R))]
+    ts.check(ts.fast_math(True, ts.SPLIT_BF16X6), "fast math")
+    try:
+        ts.check(ts.contract("D(a,b)+=L(k,a)*R(k,b)", *ten, alpha=1.0, accumulative=ts.YEP), "contract")
+    finally:
+        ts.fast_math(False)
+    for at in range(0, M, 1 << 24):
+        b = slice(at, min(M, at + (1 << 24)))
+        assert torch.equal(D[b], 5.0 + (L.view(M, K)[b] * R).sum(1)), at
+    for t in ten:
+        t.destruct()
+    torch.cuda.empty_cache()
