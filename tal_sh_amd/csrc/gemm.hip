@@ -219,11 +219,12 @@ int split_rows_log(int64_t nks, int64_t Rp) {
 __global__ __launch_bounds__(kSplitThreads) void split_rows_f16_kernel(const float *__restrict__ X, int64_t ld,
                                                                        int64_t R, int64_t K, int64_t nks,
                                                                        uint4 *__restrict__ P, int64_t plane, int vec,
-                                                                       uint32_t *__restrict__ U, int rows_log) {
+                                                                       uint32_t *__restrict__ U, int rows_log,
+                                                                       int64_t first) {
   __shared__ uint32_t red[kSplitThreads / 4];
   const int tid = threadIdx.x, c = tid & 3, row = tid >> 2 & ((1 << rows_log) - 1);
   const int ks0 = tid >> (2 + rows_log), round = kSplitThreads / 4 >> rows_log;  // K steps per round of the block
-  const int64_t r = ((int64_t)blockIdx.x << rows_log) + row, n = r < R ? K : 0;
+  const int64_t r = ((first + blockIdx.x) << rows_log) + row, n = r < R ? K : 0;
   const float *x = X + r * ld;
   if (tid < kSplitThreads / 4) red[tid] = 0;
   float v[kHeld][8];
@@ -565,28 +566,28 @@ int split_operand(bool kcont, const float *X, int64_t ld, int64_t R, int64_t K, 
   const int64_t steps = kcont ? 64 / kSplitRows : 1, nblk = Rp / (64 / steps) * ((nks + steps - 1) / steps);
   const int vec = ((uintptr_t)X % 16 == 0) && ld % 4 == 0;
   if (NP == 2 && kcont) {  // maxima and planes in one pass over HBM
-    if (Rp / 2 > 0x7fffffffLL) return -4;
+    if (Rp / 2 > 0x7fffffffLL) return -4;  // blocks are numbered in 31 bits
     const int rows_log = split_rows_log(nks, Rp);  // at most the 128 rows that Rp is a multiple of
-    split_rows_f16_kernel<<<dim3((unsigned)(Rp >> rows_log)), dim3(kSplitThreads), 0, s>>>(X, ld, R, K, nks, P, plane,
-                                                                                         vec, U, rows_log);
+    launch_grids(Rp >> rows_log, kSplitThreads, [&](int64_t first, dim3 grid, bool) {
+      split_rows_f16_kernel<<<grid, dim3(kSplitThreads), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U, rows_log, first);
+    });
     return hipGetLastError() == hipSuccess ? 0 : -2;
   }
   if constexpr (NP == 2) {
     fill_u32_kernel<<<dim3((unsigned)((Rp + 255) / 256)), dim3(256), 0, s>>>(U, Rp);
     if (R > 0 && K > 0) {
       const int64_t kseg = std::max<int64_t>(512, round_up((K + 65534) / 65535, 256));
-      if ((R + 63) / 64 > 0x7fffffffLL) return -4;
-      const dim3 grid((unsigned)((R + 63) / 64), (unsigned)((K + kseg - 1) / kseg));
-      row_absmax_kernel<<<grid, dim3(256), 0, s>>>(X, ld, R, K, kseg, U);
+      launch_grids((R + 63) / 64, 256, [&](int64_t first, dim3 grid, bool) {
+        grid.y = (unsigned)((K + kseg - 1) / kseg);
+        row_absmax_kernel<<<grid, dim3(256), 0, s>>>(X + first * 64, ld, R - first * 64, K, kseg, U + first * 64);
+      });
     }
   }
-  // a grid holds fewer than 2^32 threads: short rows fill a block to an eighth, so 134 million of them take two
-  constexpr int64_t kMost = 0xffffffffu / 256;
-  for (int64_t first = 0; first < nblk; first += kMost) {
-    const dim3 grid((unsigned)std::min(kMost, nblk - first));
+  // short rows fill a block to an eighth: 134 million of them take two grids
+  launch_grids(nblk, 256, [&](int64_t first, dim3 grid, bool) {
     if (kcont) split_planes_kernel<1, NP><<<grid, dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U, first);
     else split_planes_kernel<0, NP><<<grid, dim3(256), 0, s>>>(X, ld, R, K, nks, P, plane, vec, U, first);
-  }
+  });
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -44,6 +44,16 @@ inline void launch_last(F kernel, dim3 grid, dim3 block, hipStream_t s, A... arg
   }
 }
 
+// Blocks [0, nblk) of `threads` in grids of fewer than 2^32 threads: a larger one
+// is refused, or cut short without an error.  launch(first, grid, last): blocks
+// first, first + 1, ...; last: no other grid follows.
+template <typename F>
+inline void launch_grids(int64_t nblk, unsigned threads, F launch) {
+  const int64_t most = 0xffffffffu / threads;
+  for (int64_t at = 0; at < nblk; at += most)
+    launch(at, dim3((unsigned)(nblk - at < most ? nblk - at : most)), nblk - at <= most);
+}
+
 // A kernel of a timestamped operation; last: no other follows it.
 template <bool last = true, typename F, typename... A>
 inline void launch_clocked(F kernel, dim3 grid, dim3 block, hipStream_t s, A... args) {

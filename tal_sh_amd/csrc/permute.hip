@@ -129,6 +129,7 @@ struct PermArgsT {
   uint32_t nta, mga, sha;      // tiles along a, b and c, with dividers
   uint32_t ntb, mgb, shb;
   uint32_t ntc, mgc, shc;
+  uint32_t first;              // block of the grid's first workgroup
   int64_t ea, eb, ec;          // tile-dim extents
   int64_t isb, isc;            // input strides of b and c (a has stride 1)
   int64_t osa, osb, osc;       // output strides of a, b, c
@@ -255,7 +256,7 @@ template <typename T, int TA, int V, int OP>
 __global__ __launch_bounds__(kThreads) void perm_rows_kernel(const T *__restrict__ src, T *__restrict__ dst,
                                                              PermArgs p, typename Real<T>::type ar,
                                                              typename Real<T>::type ai, int conj) {
-  perm_rows_body<T, TA, V, OP>(src, dst, p, blockIdx.x, ar, ai, conj);
+  perm_rows_body<T, TA, V, OP>(src, dst, p, p.first + blockIdx.x, ar, ai, conj);
 }
 
 // Offset of line l0 + q * LINES of a tile's lines (i fast with extent E, k
@@ -338,7 +339,7 @@ template <typename T, int TA, int TB, int V, int OP>
 __global__ __launch_bounds__(tile_threads<TB>()) void perm_tile_kernel(const T *__restrict__ src, T *__restrict__ dst,
                                                              PermArgs p, typename Real<T>::type ar,
                                                              typename Real<T>::type ai, int conj) {
-  perm_tile_body<T, TA, TB, V, OP>(src, dst, p, blockIdx.x, ar, ai, conj);
+  perm_tile_body<T, TA, TB, V, OP>(src, dst, p, p.first + blockIdx.x, ar, ai, conj);
 }
 
 // Two permutation copies of one kind and tile shape in one launch (the A and
@@ -489,26 +490,33 @@ int grid_for(int64_t n) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(b, 1 << 22));
 }
 
+// The blocks of a permutation; its args' `first` is set for every grid.
+template <typename T, typename F>
+void launch_blocks(F kernel, unsigned threads, const T *src, T *dst, PermArgs p, typename Real<T>::type ar,
+                   typename Real<T>::type ai, int conj, int64_t nblk, hipStream_t s) {
+  launch_grids(nblk, threads, [&](int64_t first, dim3 grid, bool last) {
+    p.first = (uint32_t)first;
+    if (last) launch_clocked(kernel, grid, dim3(threads), s, src, dst, p, ar, ai, conj);
+    else launch_clocked<false>(kernel, grid, dim3(threads), s, src, dst, p, ar, ai, conj);
+  });
+}
+
 template <typename T, int TA, int V>
 void launch_rows(const T *src, T *dst, const PermArgs &p, int op, typename Real<T>::type ar,
                  typename Real<T>::type ai, int conj, int64_t nblk, hipStream_t s) {
   if (op == PERM_COPY)
-    launch_clocked(perm_rows_kernel<T, TA, V, PERM_COPY>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p, ar, ai,
-                                                                                          conj);
+    launch_blocks(perm_rows_kernel<T, TA, V, PERM_COPY>, kThreads, src, dst, p, ar, ai, conj, nblk, s);
   else
-    launch_clocked(perm_rows_kernel<T, TA, V, PERM_ADD>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p, ar, ai,
-                                                                                         conj);
+    launch_blocks(perm_rows_kernel<T, TA, V, PERM_ADD>, kThreads, src, dst, p, ar, ai, conj, nblk, s);
 }
 
 template <typename T, int TA, int TB, int V>
 void launch_tile(const T *src, T *dst, const PermArgs &p, int op, typename Real<T>::type ar,
                  typename Real<T>::type ai, int conj, int64_t nblk, hipStream_t s) {
   if (op == PERM_COPY)
-    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_COPY>, dim3((unsigned)nblk), dim3(tile_threads<TB>()), s, src, dst, p, ar, ai,
-                                                                                              conj);
+    launch_blocks(perm_tile_kernel<T, TA, TB, V, PERM_COPY>, tile_threads<TB>(), src, dst, p, ar, ai, conj, nblk, s);
   else
-    launch_clocked(perm_tile_kernel<T, TA, TB, V, PERM_ADD>, dim3((unsigned)nblk), dim3(tile_threads<TB>()), s, src, dst, p, ar, ai,
-                                                                                             conj);
+    launch_blocks(perm_tile_kernel<T, TA, TB, V, PERM_ADD>, tile_threads<TB>(), src, dst, p, ar, ai, conj, nblk, s);
 }
 
 // Widest access (elements) for type T: 16 bytes.
@@ -883,7 +891,7 @@ int launch_perm_pair_typed(const T *src0, T *dst0, int rank0, const int *dims0, 
   if (int e = plan_perm(src0, dst0, rank0, dims0, o2n0, &a)) return e;
   if (int e = plan_perm(src1, dst1, rank1, dims1, o2n1, &b)) return e;
   const bool pair = a.mode >= 2 && a.mode == b.mode && a.ta == b.ta && a.tb == b.tb && a.vec == b.vec &&
-                    a.p.nouter <= kPairOuter && b.p.nouter <= kPairOuter && a.nblk + b.nblk <= 0x7fffffffLL;
+                    a.p.nouter <= kPairOuter && b.p.nouter <= kPairOuter && a.nblk + b.nblk <= 0xffffffffLL / 512;  // one grid
   if (!pair) {
     if (int e = launch_plan(src0, dst0, a, PERM_COPY, 1.0, 0.0, 0, s)) return e;
     return launch_plan(src1, dst1, b, PERM_COPY, 1.0, 0.0, 0, s);
@@ -964,7 +972,7 @@ struct SliceArgs {
   int nrd;           // row dimensions
   int rx_log;        // log2 of threads along the run
   int64_t L;         // run length (elements)
-  int64_t nrows, nchunk;
+  int64_t nrows, nchunk, first;  // first: block of the grid's first workgroup
   int64_t src0, dst0;
   int64_t re[kMaxRank], rss[kMaxRank], rds[kMaxRank];  // row extents, source / destination strides
 };
@@ -988,7 +996,7 @@ template <typename T, int V, int OP, bool NARROW>
 __global__ __launch_bounds__(kThreads) void slice_kernel(const T *__restrict__ src, T *__restrict__ dst, SliceArgs p) {
   const int rx = 1 << p.rx_log, ry = kThreads >> p.rx_log;
   const int tx = threadIdx.x & (rx - 1), ty = threadIdx.x >> p.rx_log;
-  const int64_t chunk = (int64_t)blockIdx.x % p.nchunk, blk = (int64_t)blockIdx.x / p.nchunk;
+  const int64_t id = p.first + blockIdx.x, chunk = id % p.nchunk, blk = id / p.nchunk;
   const int64_t e = (chunk * rx + tx) * V;
   if (e >= p.L) return;
   int64_t so[kSliceRows], dof[kSliceRows];
@@ -1073,10 +1081,15 @@ int launch_slice_typed(int mode, const T *src, T *dst, int rank, const int *sdim
   const int64_t nblk = p.nchunk * ((p.nrows + ry * kSliceRows - 1) / (ry * kSliceRows));
   if (nblk > 0x7fffffffLL) return -4;
   const bool narrow = p.nrows <= 0xffffffffLL;  // row indices and extents fit 32 bits
-#define TAL_SLICE_LAUNCH(VV, NW)                                                                                   \
-  (accumulative                                                                                                  \
-       ? launch_clocked(slice_kernel<T, VV, PERM_ADD, NW>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p) \
-       : launch_clocked(slice_kernel<T, VV, PERM_COPY, NW>, dim3((unsigned)nblk), dim3(kThreads), s, src, dst, p))
+  auto run = [&](auto kernel) {
+    launch_grids(nblk, kThreads, [&](int64_t at, dim3 grid, bool last) {
+      p.first = at;
+      if (last) launch_clocked(kernel, grid, dim3(kThreads), s, src, dst, p);
+      else launch_clocked<false>(kernel, grid, dim3(kThreads), s, src, dst, p);
+    });
+  };
+#define TAL_SLICE_LAUNCH(VV, NW) \
+  (accumulative ? run(slice_kernel<T, VV, PERM_ADD, NW>) : run(slice_kernel<T, VV, PERM_COPY, NW>))
   if (V > 1) {
     if (narrow)
       TAL_SLICE_LAUNCH(VW, true);
