@@ -79,6 +79,7 @@ int launch_direct(int dk, const DirectForm &f, const void *A, const void *B, voi
   a.ar = ar;
   a.ai = ai;
   a.part = sums;
+  for (int cus = device_cus(); cus > 1; cus >>= 1) a.flags += 1 << kDirectCuShift;
   a.flags |= (accumulate ? kDirectBeta : 0) | (conja ? kDirectConjA : 0) | (conjb ? kDirectConjB : 0);
   const DirectLaunch launch =
       dk == 8 ? direct_launch_r8 : dk == 4 ? direct_launch_r4 : dk == 18 ? direct_launch_c8 : direct_launch_c4;

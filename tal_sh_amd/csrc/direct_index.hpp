@@ -138,7 +138,8 @@ enum DirectFlags {
   kDirectBeta = 1,    // D is accumulated
   kDirectConjA = 2, kDirectConjB = 4,
   kDirectAlongN = 8,  // D is stored along n (its contiguous index is an n index), else along m
-  kDirectGroupA = 16, kDirectGroupB = 32, kDirectGroupDm = 64, kDirectGroupDn = 128
+  kDirectGroupA = 16, kDirectGroupB = 32, kDirectGroupDm = 64, kDirectGroupDn = 128,
+  kDirectCuShift = 8  // from this bit on: log2 of the GPU's compute units (a power of two in every partition mode)
 };
 struct DirectArgs {
   const void *A, *B;

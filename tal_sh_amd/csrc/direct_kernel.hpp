@@ -265,11 +265,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
-  // The second workgroup of each CU gets the matrix cores first: equals, the two
-  // go through their K steps together and wait together (4096^3 R4 993 -> 985
-  // us, 4026 x 3990 by 3654 982 -> 968, R8 1913 -> 1903; no difference for the
-  // smaller tiles, and four levels of priority cost R4 23 %).
-  if (BM * BN == 128 * 128 && (blockIdx.x >> 8 & 1)) __builtin_amdgcn_s_setprio(1);
   // units: the whole tiles, then the K ranges of the others
   int u = p.first + (int)blockIdx.x, tile, kpart = 0;
   const bool part = u >= p.whole;
@@ -292,6 +287,13 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(OC
   const int m0 = bx * BM, n0 = by * BN;
   const int kbeg = kpart * p.ksteps * KB;
   const int kend = part ? min(p.K, kbeg + p.ksteps * KB) : p.K;
+  // The second workgroup of each CU gets the matrix cores first: equals, the two
+  // go through their K steps together and wait together (4096^3 R4 993 -> 985
+  // us, 4026 x 3990 by 3654 982 -> 968, R8 1913 -> 1903; no difference for the
+  // smaller tiles, and four levels of priority cost R4 23 %).  Every other round
+  // over the CUs is taken to be the second workgroups: so the first two rounds
+  // are dealt, later workgroups go where one ended and may meet an equal.
+  if (BM * BN == 128 * 128 && (blockIdx.x >> (p.flags >> kDirectCuShift) & 1)) __builtin_amdgcn_s_setprio(1);
   // A number with one dimension in an operand is linear there, and its offset
   // from the tile's origin fits 32 bits (the host checks): the origin goes
   // into the 64-bit base.
