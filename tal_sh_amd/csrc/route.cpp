@@ -6,14 +6,18 @@
 namespace tal {
 
 // Straight from the tensors where the transposes would cost more than the
-// reads in place do.  Measured (R8): a K step that walks runs of k costs 4 %
-// of a product in 128 x 128 tiles (9216^3: 21.99 -> 22.66 ms) and about a
-// quarter in smaller ones (1024^3: 41 -> 50 us), there with runs of any length,
-// as offsets then come from tables (runs of 20-24 by copies and in place: R8
-// 930 x 957 by 616 60 -> 56 us, 1480 x 1189 by 280 55 -> 51, C4 311 x 336 by
-// 600 40 -> 34, C8 550 x 552 by 420 64 -> 65; runs of 32, R8 1024^3, 72 -> 79);
-// in 128 x 128 tiles short runs, and any runs by table, cost 40 %; D written 8
-// bytes apart, about four times its bytes.
+// reads in place do.  Measured: a K step that walks runs of k costs up to 5 % of
+// a product in a kind's largest tiles, 128 x 128 real (R8 9216^3: 21.99 -> 22.66
+// ms) and 64 x 64 complex (1600^3 by copies of both operands and in place: C8
+// 552 -> 517 us, C4 291 -> 282; 4624 x 4624 by 4096 10,700 -> 10,460 and 5,160
+// -> 5,180), and about a quarter in smaller ones (R8 1024^3: 41 -> 50 us), there
+// with runs of any length, as offsets then come from tables (runs of 20-24 by
+// copies and in place: R8 930 x 957 by 616 60 -> 56 us, 1480 x 1189 by 280 55 ->
+// 51, C4 311 x 336 by 600 40 -> 34, C8 550 x 552 by 420 64 -> 65; runs of 32, R8
+// 1024^3, 72 -> 79); in 128 x 128 tiles short runs, and any runs by table, cost
+// 40 % (complex tiles are held to the same line, though runs of 16 cost them
+// little: C8 1600^3 549 by copies, 518 in place); D written 8 bytes apart, about
+// four times its bytes.
 // A transpose moves 4.6 TB/s and takes about 4 us beside that.
 Route contract_route(const ContractPlan &plan, int dk, DirectChooser choose) {
   DirectVariant v;
