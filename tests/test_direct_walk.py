@@ -198,3 +198,57 @@ def test_k_past_one_launch(walk):
         in_place = ctypes.c_int()
         for dk in (4, 8, 14, 18):
             assert walk.mat_addressable(pattern.encode(), *dims, dk, ctypes.byref(in_place)) == 1
+
+
+# Products by tile shape (its number in direct_tiles; complex kinds have one shape for 0 and 1): a, b and k with partial
+# tiles and partial K steps, 16-byte and element loads, and with k of two dimensions (a, b, i, j).
+LAYOUTS = ["D(a,b)+=L(a,k)*R(k,b)", "D(a,b)+=L(k,a)*R(k,b)", "D(b,a)+=L(a,k)*R(b,k)", "D(a,b)+=L(k,a)*R(b,k)"]
+RUN_LAYOUTS = ["D(a,b)+=L(i,a,j)*R(i,j,b)", "D(a,b)+=L(i,a,j)*R(b,i,j)", "D(b,a)+=L(a,i,j)*R(j,b,i)"]
+SMALL = [(129, 65, 259), (15, 1, 1), (33, 31, 7)]
+TILES = {
+    8: {0: [(16390, 2052, 70), (16389, 2051, 259)], 1: [(4100, 2052, 70), (4097, 2051, 133)],
+        2: [(8200, 66, 70), (8201, 65, 133)], 3: [(130, 66, 70)] + SMALL},
+    4: {0: [(4100, 8196, 260), (8197, 8199, 67)], 1: [(8200, 2052, 132), (8200, 2052, 130)],
+        2: [(2052, 2052, 68), (8200, 66, 70)], 3: [(132, 68, 68)] + SMALL},
+    18: {0: [(2500, 1598, 259)], 2: [(8200, 66, 70)], 3: SMALL},
+    14: {0: [(4100, 2052, 70), (4097, 2051, 133)], 2: [(8200, 66, 70), (8201, 65, 133)], 3: [(130, 66, 70)] + SMALL}}
+TILE_RUNS = {
+    8: {0: [(16390, 2052, 33, 4), (16390, 2052, 36, 6)], 1: [(4097, 2052, 17, 3), (8200, 1030, 16, 5), (4097, 2052, 3, 11)],
+        2: [(8200, 66, 17, 3), (8200, 66, 20, 7), (8200, 66, 5, 51)],
+        3: [(131, 31, 17, 3), (130, 34, 20, 7), (129, 33, 5, 51)]},
+    4: {0: [(16390, 1030, 33, 4)], 1: [(8200, 2052, 17, 3)], 2: [(8200, 66, 33, 4), (8200, 68, 36, 5), (8200, 66, 17, 5)],
+        3: [(131, 31, 33, 4), (132, 36, 36, 7), (129, 33, 5, 51)]},
+    18: {0: [(65537, 33, 5, 51)], 2: [(8200, 66, 17, 3), (8200, 66, 3, 51)], 3: [(131, 31, 17, 3), (129, 33, 3, 51)]},
+    14: {0: [(4097, 2052, 33, 4), (4097, 2052, 36, 7), (33000, 33, 5, 51)],
+         2: [(8200, 66, 17, 3), (8200, 66, 20, 7), (8200, 66, 5, 51)],
+         3: [(131, 31, 17, 3), (130, 34, 20, 7), (129, 33, 5, 51)]}}
+
+
+@pytest.mark.parametrize("dk", (4, 8, 14, 18))
+def test_tiles_are_chosen(walk, dk):
+    """The shapes above take the tiles they are listed under, with both load widths, and walk or look up their runs."""
+    wide = {4: 4, 8: 2, 14: 2, 18: 1}[dk]
+    out = (ctypes.c_int * 3)()
+
+    def route(pattern, ext):
+        dims = [(ctypes.c_int * len(lab))(*[ext[x] for x in lab]) for lab in labels_of(pattern)]
+        return walk.route_of(pattern.encode(), *dims, dk, 256, out)
+
+    assert set(TILES[dk]) == set(TILE_RUNS[dk]) == ({0, 1, 2, 3} if dk in (4, 8) else {0, 2, 3})
+    for tile, sizes in TILES[dk].items():
+        widths = set()
+        for size in sizes:
+            for pattern in LAYOUTS:
+                assert route(pattern, dict(zip("abk", size))) == ROUTE_COPIES, (pattern, size)
+                # as D(b,a), two shapes of equal cost may change places
+                assert out[0] == 0 and (out[2] == tile or pattern == LAYOUTS[2]), (pattern, size)
+                widths.add(out[1])
+        assert widths == {1, wide}, (tile, widths)
+    modes = set()
+    for tile, sizes in TILE_RUNS[dk].items():
+        for size in sizes:
+            for pattern in RUN_LAYOUTS[:2]:
+                assert route(pattern, dict(zip("abij", size))) == 0, (pattern, size)
+                assert out[2] == tile and out[0] in (1, 2), (pattern, size)
+                modes.add((tile, out[0]))
+    assert {m for _, m in modes} == {1, 2}

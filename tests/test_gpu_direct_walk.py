@@ -43,7 +43,9 @@ def check(ts, dk, pattern, ext, largest=8):
     m, n = [x for x in d if x in l], [x for x in d if x in r]
     total = math.prod(ext[x] for x in k) * largest ** 2 * (2 if dk in (C4, C8) else 1) + largest
     assert total < (2 ** 24 if dk in (R4, C4) else 2 ** 53)
-    want = matrix(body[0], d, ext, m, n) + matrix(body[1], l, ext, m, k) @ matrix(body[2], r, ext, k, n)
+    left = matrix(body[1], l, ext, m, k)
+    want = matrix(body[0], d, ext, m, n) + (left.conj().resolve_conj() if "L+(" in pattern else left) @ matrix(
+        body[2], r, ext, k, n)
     torch.cuda.synchronize()
     ten = [ts.Tensor(dk, [ext[x] for x in lab], ts.gpu_flat(0), ext=b.data_ptr()) for lab, b in zip(labels, body)]
     ts.check(ts.contract(pattern, ten[0], ten[1], ten[2], alpha=1.0, accumulative=ts.YEP), "contract")
