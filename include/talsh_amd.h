@@ -31,7 +31,8 @@ int talshAmdSetFastMathSplit(int method);
 int talshAmdGetFastMathSplit(void);
 
 /* Size in bytes of the per-GPU buffer pool taken at talshInit (default: 80 %
- * of the free device memory).  Must be called before talshInit. */
+ * of the free device memory).  Must be called before talshInit, which takes 64
+ * MiB per stream beside it, for the partial sums of products cut along K. */
 int talshAmdSetDeviceBufferSize(size_t bytes);
 
 /* Number of HIP streams per GPU used for tasks (default 4, at most 32).
