@@ -149,7 +149,8 @@ FAR = {8: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=8400000, p=37, q=24)),      # 16-byt
            ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=30, k=2200001)),     # both along k, element loads
            ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=140, k=2200002)),
            ("D(a,b)+=L(k,a)*R(b,k)", dict(a=129, b=31, k=2200000)),
-           ("D(b,a)+=L(a,k)*R(k,b)", dict(a=30, b=135, k=2150002))],
+           ("D(b,a)+=L(a,k)*R(k,b)", dict(a=30, b=135, k=2150002)),
+           ("D(a,b,h)+=L(a,k,h)*R(k,b,h)", dict(a=8400001, b=5, k=7, h=3))],  # batch entries
        4: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=16800000, p=35, q=24)),
            ("D(a,q)+=L(a,p)*R(q,p)", dict(a=16800001, p=64, q=33)),
            ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=33, k=4400001)),
@@ -158,6 +159,18 @@ FAR = {8: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=8400000, p=37, q=24)),      # 16-byt
             ("D(a,b)+=L(k,a)*R(k,b)", dict(a=130, b=33, k=1100001))],
        14: [("D(a,q)+=L(a,p)*R(p,q)", dict(a=8400001, p=35, q=24)),
             ("D(a,b)+=L(k,a)*R(b,k)", dict(a=130, b=33, k=2200001))]}
+
+
+# Operands of 2 GiB and more whose tiles are reached by 32-bit offsets from a 64-bit base.
+LARGE = [("D(a,b)+=L(a,k)*R(k,b)", dict(a=100003, b=37, k=2700)), ("D(a,b)+=L(a,k)*R(k,b)", dict(a=100002, b=38, k=2702)),
+         ("D(b,a)+=L(k,a)*R(b,k)", dict(a=2701, b=65, k=100003)), ("D(a,b)+=L(a,k)*R(k,b)", dict(a=4000, b=70, k=70001))]
+
+
+def test_large_operands_take_a_moving_base(walk):
+    for pattern, ext in LARGE:
+        dims = [(ctypes.c_int * len(lab))(*[ext[x] for x in lab]) for lab in labels_of(pattern)]
+        out = (ctypes.c_int * 3)()
+        assert walk.route_of(pattern.encode(), *dims, 8, 256, out) in (0, ROUTE_COPIES) and out[0] == 1, (pattern, ext)
 
 
 @pytest.mark.parametrize("dk", (4, 8, 14, 18))

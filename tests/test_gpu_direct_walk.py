@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from tal_common import C4, C8, R4, R8
-from test_direct_walk import BACKWARDS, FAR, SHORT_RUNS, high_rank, labels_of
+from test_direct_walk import BACKWARDS, FAR, LARGE, SHORT_RUNS, high_rank, labels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +22,24 @@ def matrix(body, labels, ext, rows, cols):
     order = [len(labels) - 1 - labels.index(x) for x in rows + cols]
     return body.view([ext[x] for x in labels][::-1]).permute(order).reshape(
         math.prod([ext[x] for x in rows]), -1).to(torch.complex128 if body.is_complex() else torch.float64).contiguous()
+
+
+def check_batch(ts, dk, pattern, ext, body, h):
+    """A hyper index that runs slowest in every tensor: one product per entry."""
+    labels = labels_of(pattern)
+    assert all(lab[-1] == h for lab in labels)
+    part = [[b.view(ext[h], -1)[q] for b in body] for q in range(ext[h])]
+    d, l, r = (lab[:-1] for lab in labels)
+    k = [x for x in l if x in r]
+    m, n = [x for x in d if x in l], [x for x in d if x in r]
+    want = [matrix(p[0], d, ext, m, n) + matrix(p[1], l, ext, m, k) @ matrix(p[2], r, ext, k, n) for p in part]
+    torch.cuda.synchronize()
+    ten = [ts.Tensor(dk, [ext[x] for x in lab], ts.gpu_flat(0), ext=b.data_ptr()) for lab, b in zip(labels, body)]
+    ts.check(ts.contract(pattern, *ten, alpha=1.0, accumulative=ts.YEP), "contract")
+    for p, w in zip(part, want):
+        assert torch.equal(matrix(p[0], d, ext, m, n), w)
+    for t in ten:
+        t.destruct()
 
 
 def check(ts, dk, pattern, ext, largest=8):
@@ -40,6 +58,10 @@ def check(ts, dk, pattern, ext, largest=8):
         body.append((torch.complex(draw(n), draw(n)) if dk in (C4, C8) else draw(n)).to(DTYPE[dk]))
     d, l, r = labels
     k = [x for x in l if x in r and x not in d]
+    h = [x for x in d if x in l and x in r]
+    if h:
+        check_batch(ts, dk, pattern, ext, body, h[0])
+        return
     m, n = [x for x in d if x in l], [x for x in d if x in r]
     total = math.prod(ext[x] for x in k) * largest ** 2 * (2 if dk in (C4, C8) else 1) + largest
     assert total < (2 ** 24 if dk in (R4, C4) else 2 ** 53)
@@ -90,6 +112,13 @@ def test_high_ranks(talsh_gpu, seed):
     assert np.array_equal(mat(0, d, m, n), want)
     for t in ten:
         t.destruct()
+
+
+@pytest.mark.parametrize("case", LARGE)
+def test_large_operands(talsh_gpu, case):
+    """2 GiB and more, within reach of a base that moves along k."""
+    check(talsh_gpu, R8, *case)
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("dk,case", [(dk, i) for dk in FAR for i in range(len(FAR[dk]))])
